@@ -17,6 +17,7 @@ Volumes are (N, C, H, W, D) fp16 channels_last_3d tensors.  Eight kinds of calls
 Sizes run from the deepest levels of such a network (a few hundred thousand elements, where launches and host time
 count) over ordinary training patches to the whole volume (1, 64, 350, 350, 128); extents need not be even.
 """
+import itertools
 import math
 
 import torch
@@ -295,3 +296,106 @@ _TOLERANCE = {
 
 def tolerance(case):
     return _TOLERANCE[case['kind']]
+
+
+def _conv64(x, taps):
+    """Depthwise 3x3x3 convolution with zero padding of an (N, H, W, D, C) tensor."""
+    _, h, w, d, _ = x.shape
+    padded = torch.nn.functional.pad(x, (0, 0, 1, 1, 1, 1, 1, 1))
+    y = torch.zeros_like(x)
+    for i, j, k in itertools.product(range(3), repeat=3):
+        y = y + padded[:, i:i + h, j:j + w, k:k + d] * taps[i, j, k]
+    return y
+
+
+def _taps_grad64(x, grad):
+    _, h, w, d, c = x.shape
+    padded = torch.nn.functional.pad(x, (0, 0, 1, 1, 1, 1, 1, 1))
+    out = torch.empty(3, 3, 3, c, device=x.device, dtype=x.dtype)
+    for i, j, k in itertools.product(range(3), repeat=3):
+        out[i, j, k] = (padded[:, i:i + h, j:j + w, k:k + d] * grad).sum((0, 1, 2, 3))
+    return out
+
+
+def _pool64(x):
+    """2x2x2 ceil-mode average over the voxels that exist, and the statistics of the result."""
+    def halved(t):
+        t = torch.nn.functional.pad(t, (0, 0, *(e for n in reversed(t.shape[1:4]) for e in (0, n % 2))))
+        n, h, w, d, c = t.shape
+        return t.view(n, h // 2, 2, w // 2, 2, d // 2, 2, c).sum((2, 4, 6))
+
+    pooled = halved(x) / halved(torch.ones_like(x[:1, ..., :1]))
+    return pooled, *_stats64(pooled)
+
+
+def _stats64(x):
+    return x.mean((0, 1, 2, 3)), (x * x).mean((0, 1, 2, 3))
+
+
+def exact(case, seed):
+    """The outputs of `run` in plain torch and 64 bits.  Bytes are no computed numbers: None stands in their place."""
+    kind = case['kind']
+    s = {}
+    for key, t in prepare(case, seed).items():
+        if torch.is_tensor(t):
+            t = t.detach().double()
+            s[key] = t.permute(0, 2, 3, 4, 1) if t.ndim == 5 else t
+
+    def volume(t):
+        return t.detach().permute(0, 4, 1, 2, 3)
+
+    def grads(outputs, upstream, names):
+        got = torch.autograd.grad(outputs, [s[k] for k in names], upstream)
+        return {k: volume(g) if g.ndim == 5 else g for k, g in zip(names, got)}
+
+    def differentiable(*names):
+        for k in names:
+            s[k] = s[k].requires_grad_(True)
+
+    if kind == 'conv':
+        return volume(_conv64(s['x'], s['taps']))
+    if kind == 'conv_grad':
+        dtaps = _taps_grad64(s['x'], s['grad'])
+        if case['want'] == 'w':
+            return dtaps
+        return volume(_conv64(s['grad'], s['taps'].flip(0, 1, 2))), dtaps
+    if kind == 'norm_pool':
+        mean, sqmean = _stats64(s['x'])
+        _, scale, shift = _fold(mean, sqmean, s['gamma'], s['beta'])
+        act = torch.relu(s['x'] * scale + shift)
+        pooled, pmean, psqmean = _pool64(act)
+        return {'mean': mean, 'sqmean': sqmean, 'act': volume(act), 'pooled': volume(pooled), 'pmean': pmean,
+                'psqmean': psqmean}
+    if kind == 'join':
+        s['z'] = s['x'] + s['y']
+        differentiable('z', 'gamma', 'beta')
+        mean, sqmean = _stats64(s['z'])
+        _, scale, shift = _fold(mean, sqmean, s['gamma'], s['beta'])
+        pooled, pmean, psqmean = _pool64(torch.relu(s['z'] * scale + shift))
+        g = grads((pooled, pmean, psqmean), (s['grad'], s['grad_mean'], s['grad_sqmean']), ('z', 'gamma', 'beta'))
+        return {'z': volume(s['z']), 'mean': mean.detach(), 'sqmean': sqmean.detach(), 'pooled': volume(pooled),
+                'pmean': pmean.detach(), 'psqmean': psqmean.detach(), 'dx': g['z'], 'dgamma': g['gamma'],
+                'dbeta': g['beta']}
+    if kind == 'block':
+        names = ('x', 'taps', 'gamma', 'beta', 'mix')
+        differentiable(*names)
+        y = _conv64(s['x'], s['taps'])
+        _, scale, shift = _fold(*_stats64(y), s['gamma'], s['beta'])
+        out = torch.relu(y * scale + shift) @ s['mix'] + s['x']
+        return {'out': volume(out), **{'d' + k: g for k, g in grads(out, s['grad'], names).items()}}
+    if kind == 'linear':
+        differentiable('x', 'mix')
+        out = torch.relu(s['x']) @ s['mix'] + s['skip']
+        return {'out': volume(out), **{'d' + k: g for k, g in grads(out, s['grad'], ('x', 'mix')).items()}}
+    if kind == 'bottleneck':
+        names = ('x', 'up', 'down', 'bias')
+        differentiable(*names)
+        out = torch.relu(s['x'] @ s['up'] + s['bias']) @ s['down'] + s['skip']
+        return {'out': volume(out), **{'d' + k: g for k, g in grads(out, s['grad'], names).items()}}
+    if kind == 'int8':
+        y = torch.relu(_conv64(s['x'], s['taps']) * s['scale'] + s['shift']) @ s['mix']
+        return {'q': None, 'qscale': y.abs().amax() / 127, 'y': volume(y)}
+    if kind == 'quant':
+        level = ((s['x'].clamp(-WINDOW, WINDOW) + WINDOW) / (2 * WINDOW) * 255).floor()
+        return {'q': None, 'back': volume(level * (2 * WINDOW / 255) - WINDOW)}
+    raise ValueError(kind)
