@@ -7,8 +7,8 @@
 // The op moves 2*V*(2*CIN + COUT) bytes: it is HBM-bound; both products run on v_mfma_f32_32x32x16_f16 so
 // that the arithmetic stays a fraction of the memory time.
 //
-// A workgroup of four wavefronts loops over tiles of 64 voxels.  The tile of x and of g is staged through LDS
-// (global -> registers one tile ahead -> LDS, rows of 16-byte chunks).
+// A workgroup of four wavefronts loops over tiles of 64 to 256 voxels (lb_tile).  The tile of x and of g is staged
+// through LDS (global -> registers one tile ahead -> LDS, rows of 16-byte chunks).
 //  * dx is computed transposed, dx^T[ci, v] = Wm[ci, :] . g^T[:, v]: the A operand is a 32-row block of Wm
 //    (16-byte fragments pre-arranged in LDS), the B operand is one 16-byte chunk of a voxel's g row.  One
 //    (32 voxels x 32 input channels) block per wavefront; the fp32 result is rounded to fp16, bounced through
@@ -28,28 +28,35 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kLbThreads = 256;
 constexpr int kLbWaves = kLbThreads / kWave;
-constexpr int kLbTile = 64;  // voxels per tile
+
+// Voxels per tile.  A tile's loads are all a workgroup has in flight, three workgroups run on a compute unit, and the
+// memory system needs about 40 KB in flight per compute unit: 64 voxels are enough from 96 channels (Cin + Cout) on,
+// fewer channels take tiles of the same bytes.
+constexpr int lb_tile(int cin, int cout) { return cin + cout >= 96 ? 64 : cin + cout >= 48 ? 128 : 256; }
 
 template <int CIN, int COUT>
 struct LbCfg {
+    static constexpr int TILE = lb_tile(CIN, COUT);
     static constexpr int MTI = (CIN + 31) / 32, MTO = (COUT + 31) / 32;  // 32-channel blocks
     static constexpr int KSO = COUT / 16;                                 // k steps of the dx product
-    static constexpr int KSV = kLbTile / 16;                              // k steps (voxels) of the dW product
+    static constexpr int KSV = TILE / 16;                                 // k steps (voxels) of the dW product
     static constexpr int XP = CIN, GP = COUT, DP = CIN;  // dense rows (halves); swizzled: SwizzledRows / BounceTile in common.hpp
-    static constexpr int NBD = 2 * MTI;                                   // dx blocks (32 voxels x 32 channels) per tile
+    static constexpr int NVT = TILE / 32;                                  // 32-voxel blocks
+    static constexpr int NBD = NVT * MTI;                                 // dx blocks (32 voxels x 32 channels) per tile
     static constexpr int NBW = MTI * MTO;                                 // dW blocks
     static constexpr int KSPL = NBW >= kLbWaves ? 1 : kLbWaves / NBW;     // voxel split when blocks are few
     static constexpr int BPW = NBW >= kLbWaves ? NBW / kLbWaves : 1;      // dW blocks per wavefront
-    static constexpr int NXC = kLbTile * CIN / 8, NGC = kLbTile * COUT / 8;  // 16-byte chunks per tile
+    static constexpr int NXC = TILE * CIN / 8, NGC = TILE * COUT / 8;  // 16-byte chunks per tile
     static constexpr int NLX = (NXC + kLbThreads - 1) / kLbThreads, NLG = (NGC + kLbThreads - 1) / kLbThreads;
     static constexpr int XS_OFF = 0;
-    static constexpr int GS_OFF = XS_OFF + kLbTile * XP * 2;
-    static constexpr int DS_OFF = GS_OFF + kLbTile * GP * 2;
-    static constexpr int WL_OFF = (DS_OFF + kLbTile * DP * 2 + 15) / 16 * 16;
+    static constexpr int GS_OFF = XS_OFF + TILE * XP * 2;
+    static constexpr int DS_OFF = GS_OFF + TILE * GP * 2;
+    static constexpr int WL_OFF = (DS_OFF + TILE * DP * 2 + 15) / 16 * 16;
     static constexpr int LDS_BYTES = WL_OFF + MTI * KSO * 64 * 16;
     static_assert(CIN % 16 == 0 && CIN <= 128 && COUT % 16 == 0 && COUT <= 128, "channels in {16,32,64,128}");
     static_assert(NBW % kLbWaves == 0 || kLbWaves % NBW == 0, "blocks divide over the wavefronts");
     static_assert(KSV % KSPL == 0, "voxel steps divide over the split");
+    static_assert(KSPL == 1 || LDS_BYTES >= KSPL * CIN * COUT * 4, "the sums of the split fit the tiles' LDS");
 };
 
 template <int CIN, int COUT>
@@ -90,10 +97,10 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
 #pragma unroll
         for (int i = 0; i < 16; ++i) wacc[bb][i] = 0.0f;
 
-    const int64_t ntiles = (V + kLbTile - 1) / kLbTile;
+    const int64_t ntiles = (V + Cfg::TILE - 1) / Cfg::TILE;
     half8_t xpre[NLX], gpre[NLG];
     auto prefetch = [&](int64_t tile) {
-        const int64_t v0 = tile * kLbTile;
+        const int64_t v0 = tile * Cfg::TILE;
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kLbThreads;
@@ -111,7 +118,7 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
     int64_t tile = blockIdx.x;
     if (tile < ntiles) prefetch(tile);
     for (; tile < ntiles; tile += gridDim.x) {
-        const int64_t v0 = tile * kLbTile;
+        const int64_t v0 = tile * Cfg::TILE;
         // ---- stage the tile (rows past V are zero: they add nothing to dW) ----
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
@@ -131,7 +138,7 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
         for (int bd = 0; bd < (Cfg::NBD + kLbWaves - 1) / kLbWaves; ++bd) {
             const int blk = wave + bd * kLbWaves;
             if (blk < Cfg::NBD) {  // wavefront-uniform
-                const int vt = blk % 2, mt = blk / 2;
+                const int vt = blk % Cfg::NVT, mt = blk / Cfg::NVT;
                 // chunk 2 s + hl of the lane's voxel row: the swizzle is an XOR, so step s is the offset of step 0 ^ 32 s
                 const int grow = GT::chunk16(32 * vt + il, hl);
                 float16_t acc;
@@ -190,8 +197,10 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
         __syncthreads();
     }
 
-    // ---- partial dW of this workgroup: row (blockIdx, kpart) of the workspace, [CIN][COUT] fp32 ----
-    float* out = ws + ((int64_t)blockIdx.x * KSPL + kpart) * (CIN * COUT);
+    // ---- partial dW of this workgroup: row blockIdx of the workspace, [CIN][COUT] fp32 ----
+    // Wavefronts that split the voxels add their sums in LDS first (the tiles are done: the loop ends in a barrier).
+    float* out = ws + (int64_t)blockIdx.x * (CIN * COUT);
+    float* part = KSPL > 1 ? reinterpret_cast<float*>(smem) + kpart * (CIN * COUT) : out;
 #pragma unroll
     for (int bb = 0; bb < BPW; ++bb) {
         const int blk = wb0 + bb * kLbWaves;
@@ -200,14 +209,24 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int ci = 32 * mi + 8 * (i / 4) + 4 * hl + i % 4;
-            if (ci < CIN && co < COUT) out[ci * COUT + co] = wacc[bb][i];
+            if (ci < CIN && co < COUT) part[ci * COUT + co] = wacc[bb][i];
+        }
+    }
+    if constexpr (KSPL > 1) {
+        __syncthreads();
+        const float* all = reinterpret_cast<const float*>(smem);
+        for (int j = t; j < CIN * COUT; j += kLbThreads) {
+            float sum = all[j];
+#pragma unroll
+            for (int k = 1; k < KSPL; ++k) sum += all[k * (CIN * COUT) + j];
+            out[j] = sum;
         }
     }
 }
 
-static int lb_blocks(int64_t V)
+static int lb_blocks(int64_t V, int cin, int cout)
 {
-    const int64_t ntiles = (V + kLbTile - 1) / kLbTile;
+    const int64_t ntiles = ceil_div64(V, lb_tile(cin, cout));
     return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, 768));  // three workgroups per CU
 }
 
@@ -216,21 +235,15 @@ static int launch_lb(const half_t* x, const half_t* g, const half_t* Wm, half_t*
                      int64_t V, hipStream_t s)
 {
     using Cfg = LbCfg<CIN, COUT>;
-    const int blocks = lb_blocks(V);
+    const int blocks = lb_blocks(V, CIN, COUT);
     hipLaunchKernelGGL((relu_linear_bwd_kernel<CIN, COUT>), dim3(blocks), dim3(kLbThreads), 0, s, x, g, Wm, dx, ws, V);
     int rc = check_launch("relu_linear_bwd");
     if (rc != KEROPS_OK) return rc;
     if (dw_dtype == KEROPS_DTYPE_F16)
-        launch_reduce_rows_f16(ws, blocks * Cfg::KSPL, CIN * COUT, (half_t*)dW, (half_t*)dW, CIN * COUT, 1.0, s);
+        launch_reduce_rows_f16(ws, blocks, CIN * COUT, (half_t*)dW, (half_t*)dW, CIN * COUT, 1.0, s);
     else
-        launch_reduce_rows(ws, blocks * Cfg::KSPL, CIN * COUT, (float*)dW, (float*)dW, CIN * COUT, 1.0, s);
+        launch_reduce_rows(ws, blocks, CIN * COUT, (float*)dW, (float*)dW, CIN * COUT, 1.0, s);
     return check_launch("relu_linear_bwd_reduce");
-}
-
-static int lb_kspl(int Cin, int Cout)
-{
-    const int nbw = ((Cin + 31) / 32) * ((Cout + 31) / 32);
-    return nbw >= kLbWaves ? 1 : kLbWaves / nbw;
 }
 
 }  // namespace kerops
@@ -249,7 +262,7 @@ extern "C" int64_t kerops_relu_linear_bwd_workspace_bytes(int64_t V, int32_t Cin
         set_error("relu_linear_bwd: built for Cin, Cout in {16,32,64,128} (got %d -> %d)", Cin, Cout);
         return KEROPS_E_UNSUPPORTED_C;
     }
-    return (int64_t)lb_blocks(V) * lb_kspl(Cin, Cout) * Cin * Cout * (int64_t)sizeof(float);
+    return (int64_t)lb_blocks(V, Cin, Cout) * Cin * Cout * (int64_t)sizeof(float);
 }
 
 extern "C" int kerops_relu_linear_bwd_f16(const void* x, const void* g, const void* Wm, void* dx, float* dW,
