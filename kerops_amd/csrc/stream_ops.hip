@@ -255,7 +255,7 @@ __device__ __forceinline__ uint32_t bytes_word(const u32x2_t& v, int k) { return
 __device__ __forceinline__ void set_bytes_word(uint32_t& v, int, uint32_t w) { v = w; }
 __device__ __forceinline__ void set_bytes_word(u32x2_t& v, int k, uint32_t w) { v[k] = w; }
 
-template <typename T, int U, bool FAST>
+template <typename T, int U, bool FAST, bool STREAM>
 __global__ __launch_bounds__(kStreamMaxThreads) void quant_u8_kernel(const T* __restrict__ x, uint8_t* __restrict__ q,
                                                                      int64_t numel, float window, float r_two_w,
                                                                      int segments)
@@ -285,17 +285,17 @@ __global__ __launch_bounds__(kStreamMaxThreads) void quant_u8_kernel(const T* __
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(xv + i + u * wk.su);
 #pragma unroll
-        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(one(v[u]), qv + i + u * wk.su);
+        for (int u = 0; u < U; ++u) store_result<STREAM>(qv + i + u * wk.su, one(v[u]));
     }
     for (int64_t i = wk.tail; i < nunits; i += wk.T)
-        __builtin_nontemporal_store(one(__builtin_nontemporal_load(xv + i)), qv + i);
+        store_result<STREAM>(qv + i, one(__builtin_nontemporal_load(xv + i)));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         for (int64_t k = nunits * E; k < numel; ++k)
             q[k] = (uint8_t)quant_u8_one<FAST>(to_f32(x[k]), window, two_w, r_two_w);
     }
 }
 
-template <typename T, int U>
+template <typename T, int U, bool STREAM>
 __global__ __launch_bounds__(kStreamMaxThreads) void dequant_u8_kernel(const uint8_t* __restrict__ q,
                                                                        T* __restrict__ out, int64_t numel,
                                                                        float window, int segments)
@@ -320,10 +320,10 @@ __global__ __launch_bounds__(kStreamMaxThreads) void dequant_u8_kernel(const uin
 #pragma unroll
         for (int u = 0; u < U; ++u) b[u] = __builtin_nontemporal_load(qv + i + u * wk.su);
 #pragma unroll
-        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(one(b[u]), ov + i + u * wk.su);
+        for (int u = 0; u < U; ++u) store_result<STREAM>(ov + i + u * wk.su, one(b[u]));
     }
     for (int64_t i = wk.tail; i < nunits; i += wk.T)
-        __builtin_nontemporal_store(one(__builtin_nontemporal_load(qv + i)), ov + i);
+        store_result<STREAM>(ov + i, one(__builtin_nontemporal_load(qv + i)));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         for (int64_t k = nunits * E; k < numel; ++k)
             out[k] = (T)__fsub_rn(__fmul_rn((float)q[k], scale), window);
@@ -735,16 +735,27 @@ extern "C" int kerops_quant_u8_window(const void* x, int32_t dtype, void* q, int
     const bool fast = window >= 0x1p-60f && window <= 0x1p60f;
     const float r_two_w = fast ? (float)(1.0 / (double)two_w) : 0.0f;
     const int seg = sh.segment != 1;
-#define KEROPS_QU8_GO(T, Uv, F)                                                                                  \
-    hipLaunchKernelGGL((quant_u8_kernel<T, Uv, F>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const T*)x, (uint8_t*)q, \
-                       numel, window, r_two_w, seg)
+    const bool cached = numel <= kCachedResultBytes;
+#define KEROPS_QU8_GO(T, Uv, F)                                                                                      \
+    if (cached)                                                                                                      \
+        hipLaunchKernelGGL((quant_u8_kernel<T, Uv, F, false>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const T*)x, \
+                           (uint8_t*)q, numel, window, r_two_w, seg);                                                \
+    else                                                                                                             \
+        hipLaunchKernelGGL((quant_u8_kernel<T, Uv, F, true>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const T*)x,  \
+                           (uint8_t*)q, numel, window, r_two_w, seg)
 #define KEROPS_QU8_T(T)                            \
     if (sh.unroll() == 8) {                        \
-        if (fast) KEROPS_QU8_GO(T, 8, true);       \
-        else KEROPS_QU8_GO(T, 8, false);           \
+        if (fast) {                                \
+            KEROPS_QU8_GO(T, 8, true);             \
+        } else {                                   \
+            KEROPS_QU8_GO(T, 8, false);            \
+        }                                          \
     } else {                                       \
-        if (fast) KEROPS_QU8_GO(T, 4, true);       \
-        else KEROPS_QU8_GO(T, 4, false);           \
+        if (fast) {                                \
+            KEROPS_QU8_GO(T, 4, true);             \
+        } else {                                   \
+            KEROPS_QU8_GO(T, 4, false);            \
+        }                                          \
     }
     if (dtype == KEROPS_DTYPE_F16) {
         KEROPS_QU8_T(half_t)
@@ -771,13 +782,19 @@ extern "C" int kerops_dequant_u8_window(const void* q, void* out, int32_t dtype,
     if (rc != KEROPS_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int seg = sh.segment != 1;
-#define KEROPS_DQ_T(T)                                                                                              \
-    if (sh.unroll() == 8) {                                                                                         \
-        hipLaunchKernelGGL((dequant_u8_kernel<T, 8>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const uint8_t*)q,   \
-                           (T*)out, numel, window, seg);                                                            \
-    } else {                                                                                                        \
-        hipLaunchKernelGGL((dequant_u8_kernel<T, 4>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const uint8_t*)q,   \
-                           (T*)out, numel, window, seg);                                                            \
+    const bool cached = numel * (dtype == KEROPS_DTYPE_F32 ? 4 : 2) <= kCachedResultBytes;
+#define KEROPS_DQ_GO(T, Uv)                                                                                         \
+    if (cached)                                                                                                     \
+        hipLaunchKernelGGL((dequant_u8_kernel<T, Uv, false>), dim3(sh.blocks), dim3(sh.threads), 0, s,              \
+                           (const uint8_t*)q, (T*)out, numel, window, seg);                                         \
+    else                                                                                                            \
+        hipLaunchKernelGGL((dequant_u8_kernel<T, Uv, true>), dim3(sh.blocks), dim3(sh.threads), 0, s,               \
+                           (const uint8_t*)q, (T*)out, numel, window, seg)
+#define KEROPS_DQ_T(T)         \
+    if (sh.unroll() == 8) {    \
+        KEROPS_DQ_GO(T, 8);    \
+    } else {                   \
+        KEROPS_DQ_GO(T, 4);    \
     }
     if (dtype == KEROPS_DTYPE_F16) {
         KEROPS_DQ_T(half_t)
@@ -787,6 +804,7 @@ extern "C" int kerops_dequant_u8_window(const void* q, void* out, int32_t dtype,
         KEROPS_DQ_T(float)
     }
 #undef KEROPS_DQ_T
+#undef KEROPS_DQ_GO
     return check_launch("dequant_u8_window");
 }
 
