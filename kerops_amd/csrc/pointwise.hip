@@ -31,7 +31,16 @@ struct PwCfg {
     static constexpr int TILE_HALVES = 32 * COUT;    // dense rows, swizzled: BounceTile in common.hpp
     static constexpr int OUT_CHUNKS = 32 * COUT / 8; // 16-byte chunks of one output tile
     static_assert(CIN % 16 == 0 && CIN <= 128, "CIN in {16,32,64,128}");
-    static_assert(COUT % 8 == 0 && COUT <= 128, "COUT in {16,32,64,128}");
+    static_assert(COUT % 16 == 0 && COUT <= 128, "COUT in {16,32,64,128}");
+    // Workgroups per compute unit of the persistent loop: as few as keep the memory pipe full.  Two have 32 KB and more
+    // of x and residual in flight from 64 channels (CIN + COUT) on; narrower tiles take three.  (us at 64 M elements of
+    // x and residual together with 2 / 3 / 4 / 8 workgroups: 16 -> 16 39.4 / 34.1 / 34.5 / 36.0, 32 -> 32 34.7 / 35.7 /
+    // 35.9 / 37.6, 64 -> 128 40.0 / 41.5 / 41.5 / 41.5.  More than fit the LDS, as four at 64 -> 128, also leave a
+    // second round that fills a part of the chip.)
+    static constexpr int PER_CU = CIN + COUT >= 64 ? 2 : 3;
+    // Without a residual a tile has half the bytes: four, where their LDS fits.
+    static constexpr int LDS_BYTES = kPwWaves * TILE_HALVES * 2 + MT * KS * 64 * 16 + 2 * CIN * 4 + 64;
+    static constexpr int PER_CU_NO_ADD = 160 * 1024 / LDS_BYTES < 4 ? 160 * 1024 / LDS_BYTES : 4;
 };
 
 // AFFINE: x is first mapped to fp16(max(fma(x, scale[c], shift[c]), 0)), the arithmetic of the batch-norm + ReLU
@@ -78,6 +87,7 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
 
     // B fragments of a tile: this lane's voxel, chunks 2q+hl.  A tile index past the end reads the last voxel (the
     // loads are unconditional, the tile is then never used).
+    half8_t xb[KS], xn[KS];
     auto load_x = [&](int64_t tidx, half8_t(&xb)[KS]) {
         int64_t v = tidx * 32 + vl;
         if (v >= V) v = V - 1;  // ragged last tile: clamp the read, the write is masked
@@ -89,29 +99,32 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
             else xb[q] = load_c8(x + v * CIN + 8 * (2 * q + hl));
         }
     };
-    // Without a residual the loads of the next tile are issued before this tile's arithmetic and stores: the wait
-    // for them at the top of the next round then leaves the stores in flight, and the memory pipe never drains
-    // between tiles (7 % faster at 32 -> 32 channels, 3 % at 64 -> 128).  With the residual as a third stream the
-    // same prefetch is 2-4 % slower than loading each tile where it is used, so those variants do that.
-    constexpr bool PIPE = !HAS_ADD;
-    half8_t xb[KS];
-    if constexpr (PIPE) load_x((int64_t)blockIdx.x * kPwWaves + wave, xb);
+    // residual chunks of a tile, in the order in which the results leave the LDS tile; the same clamp
+    constexpr int NC = Cfg::OUT_CHUNKS / kWave;
+    half8_t ab[HAS_ADD ? NC : 1];
+    auto load_add = [&](int64_t tidx, int k) {
+        const int c = k * kWave + lane;
+        int64_t v = tidx * 32 + c / (COUT / 8);
+        if (v >= V) v = V - 1;
+        ab[k] = load_c8_nt(add + v * COUT + (c % (COUT / 8)) * 8);
+    };
+    // Without a residual the loads of the next tile are issued before this tile's arithmetic and stores.  With one they
+    // are issued as soon as this tile has used its registers: the x fragments behind the matrix instructions, a residual
+    // chunk behind the store of its sum.  Both streams of a tile are then in flight while the previous one is stored.
+    // (Loading a residual chunk where it is added costs one memory latency per chunk: 64 -> 128 channels with residual
+    // at 0.88 M voxels 130 us, now 103, i.e. 4.4 and 5.5 TB/s; 128 -> 128 at 0.26 M 54 and 39 us.)
+    const int64_t first = (int64_t)blockIdx.x * kPwWaves + wave;
+    load_x(first, xb);
+    if constexpr (HAS_ADD) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) load_add(first, k);
+    }
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kPwWaves + wave;
         const bool live = tidx < ntiles;
         const int64_t v0 = tidx * 32;
-        half8_t xn[KS];
-        if constexpr (PIPE) load_x(tidx + tiles_per_round, xn);
+        if constexpr (!HAS_ADD) load_x(tidx + tiles_per_round, xn);
         if (live) {
-            if constexpr (!PIPE) {
-                int64_t v = v0 + vl;
-                if (v >= V) v = V - 1;
-#pragma unroll
-                for (int q = 0; q < KS; ++q) {
-                    if constexpr (CIN <= 32) xb[q] = load_c8_nt(x + v * CIN + 8 * (2 * q + hl));
-                    else xb[q] = load_c8(x + v * CIN + 8 * (2 * q + hl));
-                }
-            }
             if constexpr (AFFINE) {
 #pragma unroll
                 for (int q = 0; q < KS; ++q) {
@@ -157,6 +170,7 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
                     }
                 }
         }
+        if constexpr (HAS_ADD) load_x(tidx + tiles_per_round, xb);
         // the tile is private to the wavefront and its LDS operations complete in issue order: no workgroup
         // barrier, the wavefronts of a workgroup run independently
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -164,29 +178,28 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (live) {
 #pragma unroll
-            for (int c0 = 0; c0 < Cfg::OUT_CHUNKS; c0 += kWave) {
-                const int c = c0 + lane;
+            for (int k = 0; k < NC; ++k) {
+                const int c = k * kWave + lane;
                 const int row = c / (COUT / 8), cc = c % (COUT / 8);
-                if (c < Cfg::OUT_CHUNKS && v0 + row < V) {
-                    half8_t o = Tile::read(my, row, cc);
-                    const int64_t off = (v0 + row) * COUT + cc * 8;
-                    if (HAS_ADD) {
-                        const half8_t a8 = load_c8_nt(add + off);
+                half8_t o = Tile::read(my, row, cc);
+                if constexpr (HAS_ADD) {
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)o[j] + (float)a8[j]);  // fp16 add, RNE
-                    }
+                    for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)o[j] + (float)ab[k][j]);  // fp16 add, RNE
+                }
+                if (v0 + row < V) {
                     if (ABSMAX) {
 #pragma unroll
                         for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf((float)o[j]));
                     }
-                    store_c8_nt(out + off, o);
+                    store_c8_nt(out + (v0 + row) * COUT + cc * 8, o);
                 }
+                if constexpr (HAS_ADD) load_add(tidx + tiles_per_round, k);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if constexpr (PIPE) {
+        if constexpr (!HAS_ADD) {
 #pragma unroll
             for (int q = 0; q < KS; ++q) xb[q] = xn[q];
         }
@@ -233,6 +246,10 @@ static int launch_pw(const half_t* x, const half_t* Wm, const half_t* add, half_
         set_error("pointwise: the running max is built without residual add and without the affine map");
         return KEROPS_E_BADARG;
     }
+    using Cfg = PwCfg<CIN, COUT>;
+    if (!absmax)
+        blocks = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kPwWaves),
+                                                             (int64_t)(add ? Cfg::PER_CU : Cfg::PER_CU_NO_ADD) * device_geometry().cus));
     if (scale) {  // the affine map ends in a ReLU of its own
         if (add) {
             hipLaunchKernelGGL((pointwise_kernel<CIN, COUT, false, true, false, true>), dim3(blocks), dim3(kPwThreads), 0,
