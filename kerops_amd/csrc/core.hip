@@ -66,10 +66,8 @@ namespace kerops {
 // (columns below split) or out1.  A workgroup owns 16 columns; its 64 row slices take interleaved rows with four
 // loads in flight each (a single dependent chain over hundreds of rows took longer than the pass it finishes),
 // then the slices are combined by a fixed tree in LDS.
-// OutT: fp32, or fp16 = the fp32 result rounded once (what a cast of it gives, without the cast's launch).
-template <class OutT>
 __global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restrict__ ws, int nrows, int ncols,
-                                                           OutT* __restrict__ out0, OutT* __restrict__ out1,
+                                                           float* __restrict__ out0, float* __restrict__ out1,
                                                            int split, double scale)
 {
     __shared__ double part[64][17];
@@ -98,25 +96,75 @@ __global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restri
     if (sl == 0 && j < ncols) {
         const double v = part[0][lo] * scale;
         if (j < split) {
-            out0[j] = (OutT)(float)v;
+            out0[j] = (float)v;
         } else {
-            out1[j - split] = (OutT)(float)v;
+            out1[j - split] = (float)v;
         }
+    }
+}
+
+// The same sums where the columns come in whole groups of 32: a workgroup owns 32 of them (a 128-byte line of every
+// row), its 128 row slices take 16 bytes per lane and four rows at once.  The slices of a wavefront are combined in
+// registers, the wavefronts' sums in LDS, in a fixed order.  (768 rows of 8192 columns: 6.9 us, 9.5 with 64 bytes
+// of a row per workgroup and 4 bytes per lane.)
+// Out0, Out1: fp32, or fp16 = the fp32 result rounded once (what a cast of it gives, without the cast's launch).
+template <class Out0, class Out1>
+__global__ __launch_bounds__(1024) void reduce_lines_kernel(const float* __restrict__ ws, int nrows, int ncols,
+                                                            Out0* __restrict__ out0, Out1* __restrict__ out1,
+                                                            int split, double scale)
+{
+    __shared__ double part[16][33];
+    const int t = threadIdx.x, l = t % 8, sl = t / 8;
+    const float4_t* col = reinterpret_cast<const float4_t*>(ws + blockIdx.x * 32) + l;
+    const int64_t pitch = ncols / 4;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    int r = sl;
+    for (; r + 384 < nrows; r += 512) {
+        const float4_t a = col[r * pitch], b = col[(r + 128) * pitch], c = col[(r + 256) * pitch],
+                       d = col[(r + 384) * pitch];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[k] += ((double)a[k] + (double)b[k]) + ((double)c[k] + (double)d[k]);
+    }
+    for (; r < nrows; r += 128) {
+        const float4_t a = col[r * pitch];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[k] += (double)a[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int off = 32; off >= 8; off >>= 1) s[k] += __shfl_xor(s[k], off, 64);
+        if (t % kWave < 8) part[t / kWave][4 * l + k] = s[k];
+    }
+    __syncthreads();
+    if (t < 32) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) v += part[w][t];
+        v *= scale;
+        const int j = blockIdx.x * 32 + t;
+        if (j < split) out0[j] = (Out0)(float)v;
+        else out1[j - split] = (Out1)(float)v;
     }
 }
 
 void launch_reduce_rows(const float* ws, int nrows, int ncols, float* out0, float* out1, int split, double scale,
                         hipStream_t stream)
 {
-    hipLaunchKernelGGL(reduce_rows_kernel<float>, dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream, ws, nrows, ncols,
+    if (ncols % 32 == 0) {
+        hipLaunchKernelGGL((reduce_lines_kernel<float, float>), dim3(ncols / 32), dim3(1024), 0, stream, ws, nrows, ncols,
+                           out0, out1, split, scale);
+        return;
+    }
+    hipLaunchKernelGGL(reduce_rows_kernel, dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream, ws, nrows, ncols,
                        out0, out1, split, scale);
 }
 
-void launch_reduce_rows_f16(const float* ws, int nrows, int ncols, half_t* out0, half_t* out1, int split, double scale,
+void launch_reduce_rows_f16(const float* ws, int nrows, int ncols, half_t* out0, float* out1, int split,
                             hipStream_t stream)
 {
-    hipLaunchKernelGGL(reduce_rows_kernel<half_t>, dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream, ws, nrows, ncols,
-                       out0, out1, split, scale);
+    hipLaunchKernelGGL((reduce_lines_kernel<half_t, float>), dim3(ncols / 32), dim3(1024), 0, stream, ws, nrows, ncols,
+                       out0, out1, split, 1.0);
 }
 
 }  // namespace kerops

@@ -29,7 +29,7 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 constexpr int kLbThreads = 256;
 constexpr int kLbWaves = kLbThreads / kWave;
 
-// Voxels per tile.  A tile's loads are all a workgroup has in flight, three workgroups run on a compute unit, and the
+// Voxels per tile.  A tile's loads are all a workgroup has in flight, two workgroups run on a compute unit, and the
 // memory system needs about 40 KB in flight per compute unit: 64 voxels are enough from 96 channels (Cin + Cout) on,
 // fewer channels take tiles of the same bytes.
 constexpr int lb_tile(int cin, int cout) { return cin + cout >= 96 ? 64 : cin + cout >= 48 ? 128 : 256; }
@@ -224,10 +224,13 @@ __global__ __launch_bounds__(kLbThreads) void relu_linear_bwd_kernel(const half_
     }
 }
 
+// Two workgroups per compute unit: what the LDS holds at 128 -> 128 channels, and a third only adds a row to the
+// partial sums (64 -> 128 at 0.35 M voxels: 43.4 us with two, 47.7 with three; 128 -> 128 at 0.26 M: 54.8 and 67.7;
+// 16 -> 16 at 2.1 M: 39.2 and 39.5).
 static int lb_blocks(int64_t V, int cin, int cout)
 {
     const int64_t ntiles = ceil_div64(V, lb_tile(cin, cout));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, 768));  // three workgroups per CU
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, 2 * device_geometry().cus));
 }
 
 template <int CIN, int COUT>
@@ -240,7 +243,7 @@ static int launch_lb(const half_t* x, const half_t* g, const half_t* Wm, half_t*
     int rc = check_launch("relu_linear_bwd");
     if (rc != KEROPS_OK) return rc;
     if (dw_dtype == KEROPS_DTYPE_F16)
-        launch_reduce_rows_f16(ws, blocks, CIN * COUT, (half_t*)dW, (half_t*)dW, CIN * COUT, 1.0, s);
+        launch_reduce_rows_f16(ws, blocks, CIN * COUT, (half_t*)dW, nullptr, CIN * COUT, s);
     else
         launch_reduce_rows(ws, blocks, CIN * COUT, (float*)dW, (float*)dW, CIN * COUT, 1.0, s);
     return check_launch("relu_linear_bwd_reduce");
