@@ -64,8 +64,8 @@ extern "C" {
  * (kerops_hip_version() of the loaded library must equal the KEROPS_HIP_VERSION it was compiled
  * against).  100: first interface; 200: launch-shape knobs (waves, segment) on the stream entry points,
  * kerops_dwconv_wgrad_noalloc_f16, KEROPS_DTYPE_BF16; 210: the *_f16_out variants (weight gradients written as fp16 by the
- * reduction kernels), scale output of kerops_quant_i8_sym_f16. */
-#define KEROPS_HIP_VERSION 210
+ * reduction kernels), scale output of kerops_quant_i8_sym_f16; 211: kerops_bnrelu_linear_bwd_f16. */
+#define KEROPS_HIP_VERSION 211
 
 int kerops_hip_version(void);
 const char* kerops_last_error_string(void);
@@ -293,6 +293,18 @@ int kerops_relu_linear_bwd_f16(const void* x, const void* g, const void* Wm, voi
 int kerops_relu_linear_bwd_f16_out(const void* x, const void* g, const void* Wm, void* dx, void* dW, int32_t dw_dtype,
                                    void* workspace, int64_t workspace_bytes, int64_t V, int32_t Cin, int32_t Cout,
                                    void* stream);
+
+/* Backward of kerops_bnrelu_pointwise_f16 with respect to x, scale, shift and Wm, one pass over x and g:
+ *   z[v, ci]  = fp16(max(fma(x[v, ci], scale[ci], shift[ci]), 0))
+ *   gz[v, ci] = z[v, ci] > 0 ? fp16(sum_co g[v, co] * Wm[ci, co]) : 0
+ *   gm[v, ci] = x[v, ci] * scale[ci] > -shift[ci] ? gz[v, ci] : 0
+ *   dx = fp16(scale * gm);  daffine[0][ci] = sum_v x * gm;  daffine[1][ci] = sum_v gm;  dW[ci, co] = sum_v z * g
+ * i.e. kerops_bnrelu_fwd_f16, kerops_relu_linear_bwd_f16_out and kerops_bnrelu_bwd_f16, without z and gz in memory.
+ * scale, shift [Cin] fp32, daffine [2][Cin] fp32, dW as dw_dtype (F32 or F16).  Cin, Cout in {16,32,64,128}. */
+int64_t kerops_bnrelu_linear_bwd_workspace_bytes(int64_t V, int32_t Cin, int32_t Cout);
+int kerops_bnrelu_linear_bwd_f16(const void* x, const float* scale, const float* shift, const void* g, const void* Wm,
+                                 void* dx, void* dW, int32_t dw_dtype, float* daffine, void* workspace,
+                                 int64_t workspace_bytes, int64_t V, int32_t Cin, int32_t Cout, void* stream);
 
 /* Inverted-bottleneck pointwise block on MFMA, the hidden activation stays in registers:
  *   hid = relu(fp16(x @ Wup) + bias);  out = fp16(hid @ Wdown) + add       (fp16 adds)

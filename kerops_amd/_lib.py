@@ -18,7 +18,7 @@ KEROPS_E_WORKSPACE = -3
 KEROPS_E_LAUNCH = -4
 
 # KEROPS_HIP_VERSION of include/kerops_hip.h that SIGNATURES below mirrors
-HEADER_VERSION = 210
+HEADER_VERSION = 211
 
 DTYPE_TAGS = {torch.float16: 0, torch.float32: 1, torch.bfloat16: 2}
 # result types the gradient reduction kernels write themselves (the *_f16_out entry points)
@@ -76,6 +76,8 @@ SIGNATURES = {
     'kerops_relu_linear_bwd_workspace_bytes': (_i64, [_i64, _i32, _i32]),
     'kerops_relu_linear_bwd_f16': (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _p]),
     'kerops_relu_linear_bwd_f16_out': (ctypes.c_int, [_p, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i32, _i32, _p]),
+    'kerops_bnrelu_linear_bwd_workspace_bytes': (_i64, [_i64, _i32, _i32]),
+    'kerops_bnrelu_linear_bwd_f16': (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _p, _i32, _p, _p, _i64, _i64, _i32, _i32, _p]),
     'kerops_dwsep_block_workspace_bytes': (_i64, [_i32, _i32, _i32, _i32, _i32, _i32]),
     'kerops_dwsep_block_f16': (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _p,
                                               _i64, _p]),

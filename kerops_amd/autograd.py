@@ -15,8 +15,8 @@ from .ops.addition import AddStats, AddStatsBackward
 from .ops.avgpool import AvgPoolCeilStats, AvgPoolCeilStatsBackward
 from .ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
 from .ops.conv import DWConv, DWConvBackward, DWConvStats, DWConvWGRAD
-from .ops.linear import (ApplyBNReLULinearAdd, LinBReLULinAdd, LinBReLULinBackward, ReLULinearAdd,
-                         ReLULinearBackward)
+from .ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, LinBReLULinAdd, LinBReLULinBackward,
+                         ReLULinearAdd, ReLULinearBackward)
 from .ops.stats import Stats, StatsBackward
 
 
@@ -165,8 +165,8 @@ class DWConvStatsFn(torch.autograd.Function):
 class ApplyBNReLULinearAddFn(torch.autograd.Function):
     """out = ReLULinearAdd(ApplyBNReLU(x, bn_weight, bn_bias), weight, add_other) in one forward pass.
 
-    The normalised activation is not kept: backward recomputes it (one ApplyBNReLU pass, the time the forward
-    saved) and then runs the two backward ops of the composition."""
+    The normalised activation is not kept: backward recomputes it inside its one pass over x and the upstream
+    gradient."""
 
     @staticmethod
     def forward(ctx, x, bn_weight, bn_bias, weight, add_other):
@@ -177,8 +177,6 @@ class ApplyBNReLULinearAddFn(torch.autograd.Function):
     def backward(ctx, grad_out):
         x, bn_weight, bn_bias, weight = ctx.saved_tensors
         grad_out = _cl3d(grad_out)
-        z = ApplyBNReLU(x, bn_weight, bn_bias)
-        grad_z, grad_w = ReLULinearBackward(z, grad_out, weight, out_dtype=weight.dtype)
-        dx, dbw, dbb = ApplyBNReLUBackward(x, bn_weight.float(), bn_bias.float(), grad_z)
+        dx, dbw, dbb, grad_w = ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad_out, weight)
         return (dx, dbw.reshape(bn_weight.shape).to(bn_weight.dtype), dbb.reshape(bn_bias.shape).to(bn_bias.dtype),
                 grad_w, grad_out)

@@ -23,7 +23,7 @@ def warps(in_channels):
 
 @confexc(KeyError)
 def dblock(in_channels):
-    # voxels per tile of the gfx950 kernel
+    # accepted as in the reference; the gfx950 kernel chooses its tile from both channel counts
     return {16: 64, 32: 64, 64: 64, 128: 64}[in_channels]
 
 
@@ -60,7 +60,7 @@ def ReLULinearBackward(
     assert out_channels in _BUILT, 'the MFMA kernel is built for 16, 32, 64 or 128 output channels'
     # num_warps, D_block and ILP are accepted with any positive value, as in the reference
     # (kerops/ops/linear/relu_linear_backward.py:20-24), and not used: the gfx950 kernel always runs 4
-    # wavefronts on tiles of 64 voxels
+    # wavefronts on tiles of 64 to 256 voxels
     assert int(num_warps) > 0 and int(D_block) > 0 and int(ILP) > 0
     require_cuda(x, grad, weight)
 
@@ -77,3 +77,37 @@ def ReLULinearBackward(
               weight_grad.data_ptr(), _lib.GW_DTYPES[weight_grad.dtype], ws.data_ptr(), ws_bytes, V, in_channels,
               out_channels, _lib.stream_of(x))
     return x_grad, (weight_grad if direct else weight_grad.to(out_dtype))
+
+
+def ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad, weight):
+    """Gradients of ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other) in one pass over x and grad.
+    Returns (dx like x, bn_weight_grad fp32, bn_bias_grad fp32, weight_grad fp16): dx bit-identical to ApplyBNReLU,
+    ReLULinearBackward and ApplyBNReLUBackward in a row, the sums in another order.  The residual's gradient is grad
+    itself.  An addition to the reference's op set; host side of kerops_bnrelu_linear_bwd_f16."""
+    in_channels = x.shape[1]
+    out_channels = grad.shape[1]
+
+    assert x.ndim == grad.ndim == 5
+    assert list(x.shape[2:]) == list(grad.shape[2:])
+    assert x.shape[0] == grad.shape[0]
+    assert list(weight.shape) == [in_channels, out_channels]
+    assert x.dtype == weight.dtype == grad.dtype == torch.float16
+    assert bn_weight.numel() == bn_bias.numel() == in_channels
+    assert x.is_contiguous(memory_format=torch.channels_last_3d)
+    assert grad.is_contiguous(memory_format=torch.channels_last_3d)
+    assert in_channels in _BUILT and out_channels in _BUILT, 'built for 16, 32, 64 or 128 channels on either side'
+    require_cuda(x, bn_weight, bn_bias, grad, weight)
+
+    weight = weight.contiguous()
+    scale = bn_weight.to(torch.float32).contiguous()
+    shift = bn_bias.to(torch.float32).contiguous()
+    V = x.numel() // in_channels
+    ws_bytes = _lib.query('kerops_bnrelu_linear_bwd_workspace_bytes', V, in_channels, out_channels)
+    ws = _lib.workspace(ws_bytes, x.device)
+    x_grad = torch.empty_like(x)
+    weight_grad = torch.empty_like(weight)
+    affine_grad = torch.empty([2, in_channels], dtype=torch.float32, device=x.device)
+    _lib.call('kerops_bnrelu_linear_bwd_f16', x.data_ptr(), scale.data_ptr(), shift.data_ptr(), grad.data_ptr(),
+              weight.data_ptr(), x_grad.data_ptr(), weight_grad.data_ptr(), _lib.GW_DTYPES[torch.float16],
+              affine_grad.data_ptr(), ws.data_ptr(), ws_bytes, V, in_channels, out_channels, _lib.stream_of(x))
+    return x_grad, affine_grad[0], affine_grad[1], weight_grad

@@ -1,0 +1,103 @@
+"""Sizes at which the tile loops, the launch rules and the result-store rules of the GPU kernels change: one voxel less and
+more than a tile, one workgroup's tiles, the first second round of the persistent loops, and the size limit between
+cached and streaming stores.  Expected values come from the CPU oracle or from the unfused ops that it pins."""
+import pytest
+import torch
+
+import oracle
+from conftest import cpu_gen, rand_cl3d
+from kerops_amd.ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
+from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, ReLULinearAdd,
+                                   ReLULinearBackward)
+from kerops_amd.ops.quantization import DequantUint8Window, QuantUint8Window
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+CHANNELS = [(16, 16), (16, 32), (32, 16), (16, 128), (128, 16), (32, 64), (64, 64), (64, 128), (128, 128)]
+
+
+def bits(t):
+    return t.contiguous().view(torch.int16)
+
+
+def flat(g, v, c):
+    return rand_cl3d(g, 1, c, v, 1, 1)
+
+
+def matrix(g, cin, cout):
+    return (torch.randn(cin, cout, generator=g) / cin ** 0.5).half()
+
+
+@pytest.mark.parametrize('cin,cout', CHANNELS)
+@pytest.mark.parametrize('v', [1, 63, 65, 127, 129, 255, 257])
+def test_relu_linear_backward_tile_edges(cin, cout, v):
+    g = cpu_gen(v * 1000 + cin + cout)
+    x, grad, w = flat(g, v, cin), flat(g, v, cout), matrix(g, cin, cout)
+    dx, dw = ReLULinearBackward(x.to(DEV), grad.to(DEV), w.to(DEV), out_dtype=torch.float32)
+    ref_dx, ref_dw = oracle.relu_linear_bwd(x, grad, w)
+    # fp32 sums of at most 128 products against fp64, then one rounding to fp16
+    assert (dx.cpu().float() - ref_dx.float()).abs().max() <= 2.0 ** -9 * max(1.0, ref_dx.abs().max().item())
+    # fp32 sums of at most 257 products: 257 * 2^-24
+    assert ((dw.cpu().double() - ref_dw).norm() / ref_dw.norm()).item() < 257 * 2.0 ** -24
+
+
+# (131109 voxels: more than two tiles for some workgroups of every channel pair, a ragged last tile)
+@pytest.mark.parametrize('cin,cout', CHANNELS)
+@pytest.mark.parametrize('v', [1, 63, 65, 127, 129, 257, 131109])
+def test_bnrelu_linear_backward_equals_its_parts(cin, cout, v):
+    g = cpu_gen(v * 7 + cin + cout)
+    x, grad, w = flat(g, v, cin), flat(g, v, cout), matrix(g, cin, cout).to(DEV)
+    scale, shift = torch.randn(cin, generator=g), torch.randn(cin, generator=g) * 0.3
+    scale[0], shift[1] = 0.0, 0.0
+    xd, gd, sd, bd = x.to(DEV), grad.to(DEV), scale.to(DEV), shift.to(DEV)
+    z = ApplyBNReLU(xd, sd, bd)
+    gz, dw_ref = ReLULinearBackward(z, gd, w)
+    dx_ref, _, _ = ApplyBNReLUBackward(xd, sd, bd, gz)
+    dx, dscale, dshift, dw = ApplyBNReLULinearBackward(xd, sd, bd, gd, w)
+    assert torch.equal(bits(dx), bits(dx_ref))
+    # the same fp32 products in another order of rows, rounded once to fp16: neighbouring values at most
+    assert (dw.float() - dw_ref.float()).abs().max().item() <= 2.0 ** -10 * dw_ref.abs().max().item()
+    _, ref_scale, ref_shift = oracle.bnrelu_bwd(x, scale, shift, gz.cpu())
+    # each result goes through at most 2^9 dependent fp32 additions (a thread's rows, lanes, wavefronts; the rows of the
+    # workgroups are added in fp64): 2^9 * 2^-24 of the summed magnitudes
+    gzf = gz.float()
+    size = gzf.abs().sum((0, 2, 3, 4)).max().item() + (gzf * xd.float()).abs().sum((0, 2, 3, 4)).max().item()
+    for got, ref in ((dscale, ref_scale), (dshift, ref_shift)):
+        assert got.dtype == torch.float32 and got.shape == (cin,)
+        assert (got.cpu().double() - ref).abs().max().item() <= 2.0 ** -15 * size + 1e-30
+
+
+# 2 or 3 workgroups of 128 voxels per compute unit: 65536 or 98304 voxels a round
+@pytest.mark.parametrize('cin,cout', CHANNELS)
+@pytest.mark.parametrize('v', [1, 31, 33, 127, 129, 65569, 98400])
+def test_pointwise_residual_tiles_and_rounds(cin, cout, v):
+    g = cpu_gen(v + cin * cout)
+    x, add, w = flat(g, v, cin), flat(g, v, cout), matrix(g, cin, cout)
+    scale, shift = torch.rand(cin, generator=g) + 0.5, torch.randn(cin, generator=g) * 0.3
+    out = ReLULinearAdd(x.to(DEV), w.to(DEV), add.to(DEV)).cpu()
+    ref = oracle.pointwise(x, w, add=add, relu_in=True)
+    # fp16(product) may be a neighbour of the oracle's, then one more rounding of the sum
+    assert (out.float() - ref.float()).abs().max() <= 2.0 ** -9 * max(1.0, ref.abs().max().item())
+    fused = ApplyBNReLULinearAdd(x.to(DEV), scale.to(DEV), shift.to(DEV), w.to(DEV), add.to(DEV))
+    z = ApplyBNReLU(x.to(DEV), scale.to(DEV), shift.to(DEV))
+    assert torch.equal(bits(fused), bits(ReLULinearAdd(z, w.to(DEV), add.to(DEV))))
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
+def test_quantiser_store_rule(dtype):
+    # results up to 128 MB are stored plainly, larger ones with the streaming hint: the same values on both sides
+    limit = 128 << 20
+    back = limit // dtype.itemsize
+    gen = torch.Generator(DEV).manual_seed(5)
+    for n in (limit, limit + 8):
+        x = torch.randn(n, device=DEV, generator=gen).to(dtype)
+        q = QuantUint8Window(x, 2.5)
+        for lo, hi in ((0, 4099), (n - 4099, n)):
+            assert torch.equal(q[lo:hi].cpu(), oracle.quant_u8_window(x[lo:hi].cpu(), 2.5))
+        half = QuantUint8Window(x[:n // 2].clone(), 2.5)
+        assert torch.equal(q[:n // 2], half)
+    for n in (back, back + 8):
+        part = q[:n].clone()
+        out = DequantUint8Window(part, dtype, 2.5)
+        assert torch.equal(out[:n // 2], DequantUint8Window(part[:n // 2].clone(), dtype, 2.5))
+        assert torch.equal(out[n - 4099:].cpu(), oracle.dequant_u8_window(part[n - 4099:].cpu(), dtype, 2.5))
