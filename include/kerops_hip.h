@@ -34,10 +34,10 @@
  *    returns KEROPS_E_BADARG.
  *    For kerops_dwconv_fwd_f16 and kerops_dwconv_wgrad_f16 with the matrix-core
  *    kernels, h_chunk > 0 cuts H into uniform chunks of that many rows, one per
- *    workgroup; h_chunk = 0 is the balanced split: as many workgroups as the GPU
- *    holds at once, in groups that each own an equal, contiguous share of the
+ *    workgroup; h_chunk = -g is the balanced split: as many workgroups as the GPU
+ *    holds at once, in groups of g that each own an equal, contiguous share of the
  *    (bundle of neighbouring patches, row) sequence and march over it in step;
- *    h_chunk = -g selects that split with groups of g workgroups (for the weight
+ *    h_chunk = 0 takes the split that a cost model finds faster (for the weight
  *    gradient g must be a multiple of C / 64 when C > 64).
  */
 #ifndef KEROPS_HIP_H

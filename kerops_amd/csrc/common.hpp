@@ -227,7 +227,7 @@ static inline bool volume_exceeds_i64(int N, int H, int W, int D, int C)
 // H_chunk sweeps of the forward and weight-gradient kernels at 14 shapes from 96^3 x 16 to 350 x 350 x 128 x 128
 // channels: the choice is the sweep's optimum or within 2 % of it (a variant that charges half a round for a
 // partial last round instead of a whole one was up to 15 % off).
-static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup)
+static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup, double* best_cost = nullptr)
 {
     int best_h = H;
     double best = 1e300;
@@ -243,6 +243,7 @@ static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup)
             best_h = h;
         }
     }
+    if (best_cost) *best_cost = best;
     return best_h;
 }
 // Balanced split of the H-marching kernels.  The tiles of the tensor, in their linear order (slab fastest, then
@@ -280,8 +281,9 @@ static inline double balanced_cost(const BalancedSplit& b, int H, int row_len, i
     return (share + 2 + setup + crossings * 5.0) * (1.0 + 0.1 / rows) * (1.0 + 0.004 * H / share) * spread;
 }
 // slab_mult: the group size must be a multiple of it (kernels that keep per-slab state across bundles)
-static inline BalancedSplit pick_balanced(int H, int64_t tiles, int row_len, int slots, int setup, int slab_mult,
-                                          int xcds)
+template <typename Cost>
+static inline BalancedSplit best_balanced(int H, int64_t tiles, int row_len, int slots, int slab_mult, Cost cost,
+                                          double* cost_out)
 {
     BalancedSplit best = make_balanced(H, tiles, slots, slab_mult);
     double best_cost = 1e300;
@@ -289,7 +291,7 @@ static inline BalancedSplit pick_balanced(int H, int64_t tiles, int row_len, int
         if (g < 1 || g > slots || g % slab_mult != 0) return;
         if (g >= tiles + row_len && g > slab_mult) return;  // more than a row of idle members
         const BalancedSplit b = make_balanced(H, tiles, slots, (int)g);
-        const double c = balanced_cost(b, H, row_len, slots, setup, xcds);
+        const double c = cost(b);
         if (c < best_cost) {
             best_cost = c;
             best = b;
@@ -299,7 +301,43 @@ static inline BalancedSplit pick_balanced(int H, int64_t tiles, int row_len, int
     for (int f = 2; f <= 8; f *= 2)                                           // parts of a long row
         if (row_len % f == 0) consider(row_len / f);
     consider(slab_mult);
+    *cost_out = best_cost;
     return best;
+}
+// The split of a launch: the balanced one, or (h_chunk > 0) uniform chunks of h_chunk rows.
+// Where a group's share is a whole column of the volume or more, every group crosses into other bundles and the cost
+// above decides.  Where it is less, the launch lasts as long as the groups that do cross (two halo planes and a pipeline
+// refill, about eight plane steps), and chunks of equal length without any crossing are often faster although they
+// leave workgroup slots empty: the cheaper of the two, with the crossing counted in full, is taken.  Measured over 24
+// shapes of 4 to 400 M elements, C = 8..128, forward / fused backward / weight gradient each, against the balanced
+// split alone: 5.5 % faster on average, between 0.77 and 1.01 of its time ((2,32,96,96,96) forward 55.6 -> 52.7 us,
+// (2,128,45,51,37) backward 47.6 -> 43.4, (1,128,34,71,55) forward 24.2 -> 18.5), 1.3 % behind the best of all splits.
+struct MarchSplit {
+    BalancedSplit b;
+    int h_chunk;
+};
+static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int setup, int slab_mult, int xcds)
+{
+    double cost;
+    const BalancedSplit whole = best_balanced(
+        H, tiles, row_len, slots, slab_mult,
+        [&](const BalancedSplit& b) { return balanced_cost(b, H, row_len, slots, setup, xcds); }, &cost);
+    if ((whole.units + whole.ngroups - 1) / whole.ngroups >= H) return {whole, 0};
+    const BalancedSplit part = best_balanced(
+        H, tiles, row_len, slots, slab_mult,
+        [&](const BalancedSplit& b) {
+            const int64_t share = (b.units + b.ngroups - 1) / b.ngroups;
+            const bool aligned = b.units % b.ngroups == 0 && H % share == 0;  // no share crosses
+            const double crossing = share < H ? (aligned ? 0.0 : 8.0) : 8.0 * (double)share / H;
+            const double spread = (int)b.group > slots / xcds ? 1.04 : 1.0;
+            return ((double)share + 2 + setup + crossing) * (1.0 + 0.1 * row_len / (double)b.group) *
+                   (1.0 + 0.02 * (double)H / (double)share) * spread;
+        },
+        &cost);
+    double uniform_cost;
+    const int h = pick_h_chunk(H, tiles, slots, setup, &uniform_cost);
+    if (uniform_cost <= cost) return {part, h};
+    return {part, 0};
 }
 // offsets inside one (W, D, C) plane are 32-bit in the convolution kernels (W, D, C positive)
 static inline bool plane_exceeds_i32(int W, int D, int C)

@@ -931,19 +931,21 @@ static int plan_fwd_mfma(FwdArgs& a, int N, int h_chunk, bool balanced_ok = fals
     const DeviceGeometry geo = device_geometry();
     a.n_xcd = (uint32_t)geo.xcds;
     const int slots = geo.resident_workgroups(NT);  // 2 workgroups of 512 threads or 4 of 256 per compute unit
-    // h_chunk 0: balanced split with the group size of the cost model (-g: groups of g workgroups) for the kernels
-    // that support it; > 0: uniform chunks of that many rows
+    // h_chunk 0: the split of the cost model (pick_split; -g: balanced in groups of g workgroups) for the kernels that
+    // support the balanced one; > 0: uniform chunks of that many rows
     if (h_chunk < 0 || (h_chunk == 0 && balanced_ok)) {
         const int64_t tiles = (int64_t)N * a.n_wt * a.n_dt * a.n_slab;
-        const BalancedSplit b = h_chunk < 0 ? make_balanced(a.H, tiles, slots, -h_chunk)
-                                            : pick_balanced(a.H, tiles, a.n_dt * a.n_slab, slots, 6,
-                                                            per_slab_state ? a.n_slab : 1, geo.xcds);
+        const MarchSplit split =
+            h_chunk < 0 ? MarchSplit{make_balanced(a.H, tiles, slots, -h_chunk), 0}
+                        : pick_split(a.H, tiles, a.n_dt * a.n_slab, slots, 6, per_slab_state ? a.n_slab : 1, geo.xcds);
+        const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && tiles + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {
             set_error("dwconv_fwd: too many plane steps for the balanced split");
             return KEROPS_E_BADARG;
         }
-        if (fits) {
+        h_chunk = split.h_chunk;
+        if (fits && h_chunk == 0) {
             a.bal_group = b.group;
             a.bal_q = (uint32_t)(b.units / b.ngroups);
             a.bal_r = (uint32_t)(b.units % b.ngroups);

@@ -377,7 +377,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NT >= 512 ? 4 : 3) void dwconv_wgrad_
         for (int e = 0; e < 2; ++e) acc[kw][e] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     // Work of this workgroup: one (tile, row range) segment with uniform chunks, or, in the balanced split, its
-    // group's contiguous share [u, u_end) of the (bundle of bal_group tiles, row) sequence (see pick_balanced).
+    // group's contiguous share [u, u_end) of the (bundle of bal_group tiles, row) sequence (see pick_split).
     const bool balanced = a.bal_group > 0;
     uint32_t u = 0, u_end = 0, member = 0;  // wavefront-uniform, kept in scalar registers
     uint32_t ws_row = ws_slot;  // the workgroup's row of partial sums; row % slabs is its slab
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_bwd_split_kernel(const WgAr
     // size is a multiple of the slab count)
 
     // Work of this workgroup: one (tile, row range) segment with uniform chunks, or, in the balanced split, its
-    // group's contiguous share [u, u_end) of the (bundle of bal_group tiles, row) sequence (see pick_balanced).
+    // group's contiguous share [u, u_end) of the (bundle of bal_group tiles, row) sequence (see pick_split).
     // Both roles walk the same segments with the same sequence of workgroup barriers.
     const bool balanced = a.bal_group > 0;
     uint32_t u = 0, u_end = 0, member = 0;  // wavefront-uniform, kept in scalar registers
@@ -1069,7 +1069,7 @@ __global__ __launch_bounds__(1024) void wgrad_reduce_kernel(const float* __restr
 struct WgPlan {
     int cg, tile_w, tile_d, cl, h_chunk, n_wt, n_dt, n_hc, n_slab, n_xcd = 8;
     int64_t nblocks;
-    uint32_t bal_group = 0, bal_q = 0, bal_r = 0, n_tiles = 0;  // balanced split (bal_group > 0), see pick_balanced
+    uint32_t bal_group = 0, bal_q = 0, bal_r = 0, n_tiles = 0;  // balanced split (bal_group > 0), see pick_split
 };
 
 static int plan_wgrad(int N, int H, int W, int D, int C, int tile_w, int tile_d, int h_chunk, int lane_channels,
@@ -1121,23 +1121,25 @@ static int plan_wgrad(int N, int H, int W, int D, int C, int tile_w, int tile_d,
     p->n_xcd = geo.xcds;
     const int slots = geo.resident_workgroups(big_wg ? 512 : 256);
     p->bal_group = 0;
-    // h_chunk 0: balanced split with the group size of the cost model (-g: groups of g workgroups; matrix-core
-    // kernels only); > 0: uniform chunks of that many rows
+    // h_chunk 0: the split of the cost model (pick_split; -g: balanced in groups of g workgroups; matrix-core kernels
+    // only); > 0: uniform chunks of that many rows
     if (lane_channels >= 16 && h_chunk <= 0) {
         if (h_chunk < 0 && (-h_chunk) % p->n_slab != 0) {
             set_error("dwconv_wgrad: the group size of the balanced split must be a multiple of the slab count %d",
                       p->n_slab);
             return KEROPS_E_BADARG;
         }
-        const BalancedSplit b = h_chunk < 0 ? make_balanced(H, per_plane, slots, -h_chunk)
-                                            : pick_balanced(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab,
-                                                            geo.xcds);
+        const MarchSplit split =
+            h_chunk < 0 ? MarchSplit{make_balanced(H, per_plane, slots, -h_chunk), 0}
+                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab, geo.xcds);
+        const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && per_plane + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {
             set_error("dwconv_wgrad: too many plane steps for the balanced split");
             return KEROPS_E_BADARG;
         }
-        if (fits) {
+        h_chunk = split.h_chunk;
+        if (fits && h_chunk == 0) {
             p->bal_group = b.group;
             p->bal_q = (uint32_t)(b.units / b.ngroups);
             p->bal_r = (uint32_t)(b.units % b.ngroups);
@@ -1274,23 +1276,25 @@ static int plan_bwd(int N, int H, int W, int D, int C, int h_chunk, WgPlan* p)
     p->n_xcd = geo.xcds;
     const int slots = geo.resident_workgroups(512);  // two workgroups of 512 threads per compute unit
     p->bal_group = 0;
-    // h_chunk 0: balanced split with the group size of the cost model (-g: groups of g workgroups); > 0: uniform
-    // chunks of that many rows
+    // h_chunk 0: the split of the cost model (pick_split; -g: balanced in groups of g workgroups); > 0: uniform chunks
+    // of that many rows
     if (h_chunk <= 0) {
         if (h_chunk < 0 && (-h_chunk) % p->n_slab != 0) {
             set_error("dwconv_bwd: the group size of the balanced split must be a multiple of the slab count %d",
                       p->n_slab);
             return KEROPS_E_BADARG;
         }
-        const BalancedSplit b = h_chunk < 0 ? make_balanced(H, per_plane, slots, -h_chunk)
-                                            : pick_balanced(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab,
-                                                            geo.xcds);
+        const MarchSplit split =
+            h_chunk < 0 ? MarchSplit{make_balanced(H, per_plane, slots, -h_chunk), 0}
+                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab, geo.xcds);
+        const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && per_plane + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {
             set_error("dwconv_bwd: too many plane steps for the balanced split");
             return KEROPS_E_BADARG;
         }
-        if (fits) {
+        h_chunk = split.h_chunk;
+        if (fits && h_chunk == 0) {
             p->bal_group = b.group;
             p->bal_q = (uint32_t)(b.units / b.ngroups);
             p->bal_r = (uint32_t)(b.units % b.ngroups);
@@ -1300,7 +1304,7 @@ static int plan_bwd(int N, int H, int W, int D, int C, int h_chunk, WgPlan* p)
             p->nblocks = (int64_t)b.group * b.ngroups;
             return KEROPS_OK;
         }
-        h_chunk = pick_h_chunk(H, per_plane, slots, 8);
+        if (h_chunk == 0) h_chunk = pick_h_chunk(H, per_plane, slots, 8);
     }
     p->h_chunk = std::min(h_chunk, H);
     p->n_hc = ceil_div(H, p->h_chunk);

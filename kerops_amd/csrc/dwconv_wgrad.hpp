@@ -14,7 +14,7 @@ struct WgArgs {
     int H, W, D, C;
     int n_wt, n_dt, n_hc, n_slab, h_chunk;
     uint32_t nblocks;
-    // balanced split (matrix-core weight-gradient kernel): bal_group > 0 switches it on, see pick_balanced
+    // balanced split (matrix-core weight-gradient kernel): bal_group > 0 switches it on, see pick_split
     uint32_t bal_group, bal_q, bal_r;  // workgroups per group; bundles * H plane steps = groups * bal_q + bal_r
     uint32_t n_tiles;                  // tiles in the tensor
     uint32_t n_xcd;                    // accelerator dies of the device: the logical workgroup order follows them

@@ -79,8 +79,8 @@ def DWConvWGRAD(
     count) are accepted and not used (the library fixes the wavefronts per workgroup with the patch shape, and
     a workgroup marches over rows of H instead of 2*ILP of them); a (W_block, D_block) pair the library is not
     built with runs on the nearest built patch shape of the same kernel family.
-    H_chunk > 0: rows one workgroup marches over; 0: the balanced split (groups of workgroups share out the
-    rows of all patches evenly); -g: that split with groups of g workgroups.  The split fixes the order of the
+    H_chunk > 0: rows one workgroup marches over; 0: the faster, by a cost model, of such chunks and the balanced
+    split (groups of workgroups share out the rows of all patches evenly); -g: the balanced split with groups of g.  The split fixes the order of the
     fp32 additions: the same call always returns the same bits, different splits differ in the last bits.
     """
     channels = x.shape[1]

@@ -5,8 +5,9 @@ import pytest
 import torch
 
 import oracle
-from conftest import cpu_gen, rand_cl3d
+from conftest import cpu_gen, rand_cl3d, rand_dw_weight
 from kerops_amd.ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
+from kerops_amd.ops.conv import DWConv, DWConvBackward, DWConvStats, DWConvWGRAD
 from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, ReLULinearAdd,
                                    ReLULinearBackward)
 from kerops_amd.ops.quantization import DequantUint8Window, QuantUint8Window
@@ -101,3 +102,28 @@ def test_quantiser_store_rule(dtype):
         out = DequantUint8Window(part, dtype, 2.5)
         assert torch.equal(out[:n // 2], DequantUint8Window(part[:n // 2].clone(), dtype, 2.5))
         assert torch.equal(out[n - 4099:].cpu(), oracle.dequant_u8_window(part[n - 4099:].cpu(), dtype, 2.5))
+
+
+# few patches (chunks of H without crossing), shares that cross patches, odd extents, one plane, two channel slabs
+@pytest.mark.parametrize('shape', [(1, 8, 64, 64, 32), (2, 32, 13, 24, 40), (1, 128, 34, 21, 19), (1, 16, 1, 33, 37),
+                                   (3, 64, 47, 17, 9), (1, 64, 96, 9, 9)])
+def test_built_in_split_of_the_march(shape):
+    n, c, h, w, d = shape
+    g = cpu_gen(sum(shape))
+    x, grad = rand_cl3d(g, n, c, h, w, d).to(DEV), rand_cl3d(g, n, c, h, w, d).to(DEV)
+    _, wk = rand_dw_weight(g, c)
+    wd = wk.to(DEV)
+    # one workgroup per patch, no chunks: the same output and input gradient bit for bit
+    y = DWConv(x, wd)
+    assert torch.equal(bits(y), bits(DWConv(x, wd, H_chunk=h)))
+    ys, mean, sqmean = DWConvStats(x, wd)
+    assert torch.equal(bits(ys), bits(y))
+    rmean, rsq = oracle.stats(y.cpu())
+    assert torch.allclose(mean.cpu().double(), rmean, rtol=1e-5, atol=1e-6)
+    assert torch.allclose(sqmean.cpu().double(), rsq, rtol=1e-5, atol=1e-6)
+    dx, gw = DWConvBackward(x, grad, wd, out_dtype=torch.float32)
+    assert torch.equal(bits(dx), bits(DWConvBackward(x, grad, wd, H_chunk=h)[0]))
+    ref = oracle.dwconv_wgrad(x.cpu(), grad.cpu())
+    for got in (gw, DWConvWGRAD(x, grad, out_dtype=torch.float32)):
+        # fp32 sums of at most a few thousand products a workgroup, then fp64: the bound of the weight-gradient tests
+        assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < 1e-5
