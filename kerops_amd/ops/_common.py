@@ -36,8 +36,8 @@ def stream_waves(num_warps):
     with 4, 8 or 16 wavefronts of 64 lanes.  Every reference-valid value is mapped to the nearest built count
     (ties go to the smaller one); 0 leaves the choice to the library."""
     n = int(num_warps)
-    if n == 0:
-        return 0
+    if n == 0 or n in BUILT_WAVES:
+        return n
     assert n > 0, 'num_warps must be positive'
     return min(BUILT_WAVES, key=lambda w: (abs(w - n), w))
 

@@ -7,7 +7,7 @@ import torch
 
 from ... import _lib
 from ...settings import ConfigurableArg, confexc, configure
-from .._common import cl3d, nearest_conv_shape, next_power_of_2, require_cuda
+from .._common import nearest_conv_shape, next_power_of_2, require_cuda
 from .variants import FWD_VARIANTS
 
 # gfx950 launch table, keyed by channel count like the reference's `warps` / `dblock`
@@ -68,26 +68,23 @@ def DWConv(
     workgroup with the patch shape (4, or 8 for 512-thread patches); D_block (any power of two) is the tile
     extent along D, and a (W_block, D_block) pair the library is not built with runs on the nearest built patch
     shape of the same kernel family.  W_block (tile extent along W), H_chunk (> 0: rows one workgroup marches
-    over; 0: the balanced split, in which groups of workgroups share out the rows of all patches evenly; -g:
-    that split with groups of g workgroups) and lane_channels (16 = matrix-core kernels, the default; 2 or 4 =
+    over; 0: the faster, by a cost model, of such chunks and the balanced split, in which groups of workgroups
+    share out the rows of all patches evenly; -g: the balanced split with groups of g workgroups) and lane_channels (16 = matrix-core kernels, the default; 2 or 4 =
     vector kernels with that many channels per lane) are additional gfx950 knobs.
     """
-    channels = x.shape[1]
-
     assert x.ndim == 5
+    bsize, channels, H, W, D = x.shape
     assert x.is_contiguous(memory_format=torch.channels_last_3d)
     assert x.dtype == weight.dtype == torch.float16
     assert channels == next_power_of_2(channels)
-    assert list(weight.shape) == [3, 3, 3, channels]
+    assert weight.shape == (3, 3, 3, channels)
     assert D_block == next_power_of_2(D_block)
     {'float32': None, 'float16': None}[ACCTYPE]
     assert int(num_warps) > 0
     require_cuda(x, weight)
 
-    bsize, _, H, W, D = x.shape
     weight = weight.contiguous()
-    output = torch.empty_like(x)
-    assert cl3d(output)
+    output = torch.empty_like(x)  # channels_last_3d like x
 
     w_block, d_block, lane_c = nearest_conv_shape(FWD_VARIANTS, channels, W_block, D_block, lane_channels)
     _lib.call(

@@ -63,14 +63,26 @@ def table_key(channels=None, nbytes=None):
     return str(int(channels)) if channels else 'default'
 
 
-def stream_shape(op, channels=None, nbytes=None):
-    """The shape an op would use for a tensor with `channels` channels and `nbytes` bytes (zeros = built-in)."""
+_BUILT_IN = dict.fromkeys(KEYS, 0)
+
+
+def _find(op, channels, nbytes):
+    """The table's own entry (not a copy): the size class, else the channel count, else the op's default."""
     entry = _table.get(op)
     if entry:
-        for key in (table_key(channels, nbytes), str(int(channels)) if channels else 'default', 'default'):
-            if key in entry:
-                return dict(entry[key])
-    return dict.fromkeys(KEYS, 0)
+        if nbytes is not None and nbytes < SMALL_BYTES and 'small' in entry:
+            return entry['small']
+        if channels:
+            shape = entry.get(str(int(channels)))
+            if shape is not None:
+                return shape
+        return entry.get('default', _BUILT_IN)
+    return _BUILT_IN
+
+
+def stream_shape(op, channels=None, nbytes=None):
+    """The shape an op would use for a tensor with `channels` channels and `nbytes` bytes (zeros = built-in)."""
+    return dict(_find(op, channels, nbytes))
 
 
 def set_stream_shape(op, blocks=0, num_warps=0, segment=0, key='default'):
@@ -87,7 +99,7 @@ def stream_knob(op, key, arg='x'):
         if t is None or not hasattr(t, 'shape'):
             return stream_shape(op)[key]
         channels = t.shape[1] if t.ndim == 5 else None
-        return stream_shape(op, channels, t.numel() * t.element_size())[key]
+        return _find(op, channels, t.numel() * t.element_size())[key]
 
     knob.__name__ = f'{op}_{key}'
     # `configure` hands a configurator the positional arguments named by its own parameters

@@ -40,10 +40,20 @@ class ConfiguredFunction:
 
     def _refresh(self):
         self._conf_params = {k: _param_names(c) for k, c in self.configurators.items() if callable(c)}
-        # positions of those parameters among the wrapped function's positional arguments
-        self._conf_index = {k: [self.usual_args.index(p) for p in names if p in self.usual_args]
-                            for k, names in self._conf_params.items()}
+        # per configurable argument the positions of those parameters among the wrapped function's ordinary arguments
+        # (one position as a number); None: a parameter that is not among them, left to the general path of __call__
+        plan = []
+        for name in self.configurable_args:
+            index = [self.usual_args.index(p) if p in self.usual_args else None for p in self._conf_params.get(name, [])]
+            if None in index:
+                plan = None
+                break
+            plan.append((name, index[0] if len(index) == 1 else index))
+        self._plan = plan
         self._config_set = frozenset(self.configurable_args)
+        # defaults of the trailing ordinary arguments
+        self._defaults = tuple(p.default for p in (self.signature.parameters[a] for a in self.usual_args)
+                               if p.default is not inspect.Parameter.empty)
 
     def __repr__(self):
         lines = [f'{self.origin_function.__name__}{self.signature}']
@@ -66,23 +76,20 @@ class ConfiguredFunction:
         return conf(*[positional[self.usual_args.index(p)] for p in self._conf_params[name]])
 
     def __call__(self, *args, **kwargs):
-        # common case: every ordinary argument positional, keywords only for configurable ones; the general
-        # path below (Signature.bind) costs as much host time as a small kernel takes to run
-        if len(args) == len(self.usual_args) and self._config_set.issuperset(kwargs):
-            final = {}
-            for name in self.configurable_args:
-                if name in kwargs:
-                    final[name] = kwargs[name]
-                else:
-                    conf = self.configurators[name]
+        # common case: ordinary arguments positional or left at their defaults, keywords only for configurable ones;
+        # the general path below (Signature.bind) costs as much host time as a small kernel takes to run
+        missing = len(self.usual_args) - len(args)
+        if 0 <= missing <= len(self._defaults) and self._plan is not None and self._config_set.issuperset(kwargs):
+            if missing:
+                args += self._defaults[-missing:]
+            configurators = self.configurators
+            for name, index in self._plan:
+                if name not in kwargs:
+                    conf = configurators[name]
                     if callable(conf):
-                        index = self._conf_index[name]
-                        if len(index) != len(self._conf_params[name]):
-                            break  # a configurator parameter that is not a positional argument: general path
-                        conf = conf(*[args[i] for i in index])
-                    final[name] = conf
-            else:
-                return self.origin_function(*args, **final)
+                        conf = conf(args[index]) if type(index) is int else conf(*[args[i] for i in index])
+                    kwargs[name] = conf
+            return self.origin_function(*args, **kwargs)
         filled = dict.fromkeys(self.configurable_args, EmptyKwarg)
         filled.update(kwargs)
         bound = self.signature.bind(*args, **filled)

@@ -28,6 +28,19 @@ def test_configurators_fill_missing_kwargs():
     assert op.__name__ == 'op'
 
 
+def test_ordinary_arguments_by_position_keyword_or_default_agree():
+    x = FakeTensor(8)
+    assert op(x, 4) == op(x, y=4) == op(y=4, x=x) == (8, 4, 1, 7)
+    assert op(x, 4, b=9) == op(x, y=4, b=9) == (8, 4, 1, 9)
+    assert op(x, b=9) == op(x=x, b=9) == (8, 3, 1, 9)
+    with pytest.raises(TypeError):
+        op()
+    with pytest.raises(TypeError):
+        op(x, 4, 5)
+    with pytest.raises(TypeError):
+        op(x, 4, y=4)
+
+
 def test_explicit_kwargs_win():
     assert op(FakeTensor(8), a=99) == (8, 3, 99, 7)
     assert op(FakeTensor(8), b=0, a=None) == (8, 3, None, 0)
