@@ -80,20 +80,37 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     const int64_t ntiles = (V + 31) / 32;
     const int64_t tiles_per_round = (int64_t)gridDim.x * kMlpWaves;
     const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
+    // Loads of a tile (one past the end reads the last voxel and is never used): x fragments, and residual chunks in the
+    // order in which the results leave the LDS tile.  Those of the next tile are issued as soon as this tile has used
+    // the registers, so that both streams are in flight while the results are stored; loaded where they are used, a
+    // tile waits for memory twice (C = 64 at 1.96 M voxels 184 us, now 134; C = 32 at 0.4 M 18.9 and 17.5).
+    constexpr int NC = 32 * C / 8 / kWave;
+    half8_t xb[KS1], ab[NC];
+    auto load_x = [&](int64_t tidx) {
+        int64_t v = tidx * 32 + vl;
+        if (v >= V) v = V - 1;  // ragged last tile: clamp the read, the write is masked
+#pragma unroll
+        for (int s = 0; s < KS1; ++s) {
+            // rows of 128 bytes need the cache to hold the line until the row's other loads arrive
+            if constexpr (C <= 32) xb[s] = load_c8_nt(x + v * C + 16 * s + 8 * hl);
+            else xb[s] = load_c8(x + v * C + 16 * s + 8 * hl);
+        }
+    };
+    auto load_add = [&](int64_t tidx, int k) {
+        const int c = k * kWave + lane;
+        int64_t v = tidx * 32 + c / (C / 8);
+        if (v >= V) v = V - 1;
+        ab[k] = load_c8_nt(add + v * C + (c % (C / 8)) * 8);
+    };
+    const int64_t first = (int64_t)blockIdx.x * kMlpWaves + wave;
+    load_x(first);
+#pragma unroll
+    for (int k = 0; k < NC; ++k) load_add(first, k);
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kMlpWaves + wave;
         const bool live = tidx < ntiles;  // wavefront-uniform
         const int64_t v0 = tidx * 32;
         if (live) {
-            int64_t v = v0 + vl;
-            if (v >= V) v = V - 1;  // ragged last tile: clamp the read, the write is masked
-            half8_t xb[KS1];
-#pragma unroll
-            for (int s = 0; s < KS1; ++s) {
-                // rows of 128 bytes need the cache to hold the line until the row's other loads arrive
-                if constexpr (C <= 32) xb[s] = load_c8_nt(x + v * C + 16 * s + 8 * hl);
-                else xb[s] = load_c8(x + v * C + 16 * s + 8 * hl);
-            }
             // ---- first product, bias, ReLU: the B fragments of the second product ----
             half8_t hb[KS2];
 #pragma unroll
@@ -115,6 +132,7 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
                     }
                 }
             }
+            load_x(tidx + tiles_per_round);
             // ---- second product ----
 #pragma unroll
             for (int mo = 0; mo < MO; ++mo) {
@@ -139,29 +157,27 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
             // operations of one wavefront complete in issue order, so no workgroup barrier is needed ----
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int c0 = 0; c0 < 32 * C / 8; c0 += kWave) {
-                const int c = c0 + lane;
+            for (int k = 0; k < NC; ++k) {
+                const int c = k * kWave + lane;
                 const int row = c / (C / 8), cc = c % (C / 8);
-                if (c < 32 * C / 8 && v0 + row < V) {
-                    half8_t o = Tile::read(my, row, cc);
-                    const int64_t off = (v0 + row) * C + cc * 8;
-                    const half8_t a8 = load_c8_nt(add + off);
+                half8_t o = Tile::read(my, row, cc);
 #pragma unroll
-                    for (int jj = 0; jj < 8; ++jj) o[jj] = (half_t)((float)o[jj] + (float)a8[jj]);  // fp16 add, RNE
-                    store_c8_nt(out + off, o);
-                }
+                for (int jj = 0; jj < 8; ++jj) o[jj] = (half_t)((float)o[jj] + (float)ab[k][jj]);  // fp16 add, RNE
+                if (v0 + row < V) store_c8_nt(out + (v0 + row) * C + cc * 8, o);
+                load_add(tidx + tiles_per_round, k);
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
 }
 
-static int mlp_blocks(int64_t V)
+// Workgroups per compute unit: as few as keep 32 KB of x and residual in flight (us with 2 / 3 / 4 / 5 workgroups: C = 16
+// at 2.1 M voxels 41.3 / 35.7 / 35.4 / 35.4, C = 32 at 0.4 M 17.5 / 17.8 / 18.5 / 19.7, at 1.96 M 67.2 / 67.5 / 69.9 / 71.6,
+// C = 64 at 1.96 M 134 / 140 / 145 / 141).
+static int mlp_blocks(int64_t V, int C)
 {
-    const int64_t ntiles = (V + 31) / 32;
-    int64_t b = (ntiles + kMlpWaves - 1) / kMlpWaves;
-    if (b > 1024) b = 1024;
-    return (int)std::max<int64_t>(b, 1);
+    const int64_t per_cu = C >= 32 ? 2 : 4;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kMlpWaves), per_cu * device_geometry().cus));
 }
 
 }  // namespace kerops
@@ -179,7 +195,7 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
         set_error("lin_brelu_lin_add: non-positive size");
         return KEROPS_E_BADARG;
     }
-    const int blocks = mlp_blocks(V);
+    const int blocks = mlp_blocks(V, C);
     hipStream_t s = (hipStream_t)stream;
 #define KEROPS_MLP_CASE(CV)                                                                                      \
     if (C == CV) {                                                                                               \
