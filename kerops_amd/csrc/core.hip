@@ -103,10 +103,7 @@ __global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restri
     }
 }
 
-// The same sums where the columns come in whole groups of 32: a workgroup owns 32 of them (a 128-byte line of every
-// row), its 128 row slices take 16 bytes per lane and four rows at once.  The slices of a wavefront are combined in
-// registers, the wavefronts' sums in LDS, in a fixed order.  (768 rows of 8192 columns: 6.9 us, 9.5 with 64 bytes
-// of a row per workgroup and 4 bytes per lane.)
+// The same sums where the columns come in whole groups of 32.
 // Out0, Out1: fp32, or fp16 = the fp32 result rounded once (what a cast of it gives, without the cast's launch).
 template <class Out0, class Out1>
 __global__ __launch_bounds__(1024) void reduce_lines_kernel(const float* __restrict__ ws, int nrows, int ncols,
@@ -114,35 +111,9 @@ __global__ __launch_bounds__(1024) void reduce_lines_kernel(const float* __restr
                                                             int split, double scale)
 {
     __shared__ double part[16][33];
-    const int t = threadIdx.x, l = t % 8, sl = t / 8;
-    const float4_t* col = reinterpret_cast<const float4_t*>(ws + blockIdx.x * 32) + l;
-    const int64_t pitch = ncols / 4;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    int r = sl;
-    for (; r + 384 < nrows; r += 512) {
-        const float4_t a = col[r * pitch], b = col[(r + 128) * pitch], c = col[(r + 256) * pitch],
-                       d = col[(r + 384) * pitch];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[k] += ((double)a[k] + (double)b[k]) + ((double)c[k] + (double)d[k]);
-    }
-    for (; r < nrows; r += 128) {
-        const float4_t a = col[r * pitch];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[k] += (double)a[k];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-        for (int off = 32; off >= 8; off >>= 1) s[k] += __shfl_xor(s[k], off, 64);
-        if (t % kWave < 8) part[t / kWave][4 * l + k] = s[k];
-    }
-    __syncthreads();
-    if (t < 32) {
-        double v = 0.0;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) v += part[w][t];
-        v *= scale;
-        const int j = blockIdx.x * 32 + t;
+    const double v = sum_lines(ws, nrows, ncols, part) * scale;
+    const int j = blockIdx.x * 32 + threadIdx.x;
+    if (threadIdx.x < 32) {
         if (j < split) out0[j] = (Out0)(float)v;
         else out1[j - split] = (Out1)(float)v;
     }

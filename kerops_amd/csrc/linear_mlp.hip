@@ -83,7 +83,10 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     // Loads of a tile (one past the end reads the last voxel and is never used): x fragments, and residual chunks in the
     // order in which the results leave the LDS tile.  Those of the next tile are issued as soon as this tile has used
     // the registers, so that both streams are in flight while the results are stored; loaded where they are used, a
-    // tile waits for memory twice (C = 64 at 1.96 M voxels 184 us, now 134; C = 32 at 0.4 M 18.9 and 17.5).
+    // tile waits for memory twice (C = 64 at 1.96 M voxels 184 us, now 134; C = 16 at 2.1 M 37.1 and 35.4).
+    // At C = 32 four workgroups per compute unit hide the second wait as well, and there a block's forward and backward
+    // pass at 1.96 M voxels take 154 us against 156 with the early loads: each load stays where it is used.
+    constexpr bool EARLY = C != 32;
     constexpr int NC = 32 * C / 8 / kWave;
     half8_t xb[KS1], ab[NC];
     auto load_x = [&](int64_t tidx) {
@@ -103,14 +106,17 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
         ab[k] = load_c8_nt(add + v * C + (c % (C / 8)) * 8);
     };
     const int64_t first = (int64_t)blockIdx.x * kMlpWaves + wave;
-    load_x(first);
+    if constexpr (EARLY) {
+        load_x(first);
 #pragma unroll
-    for (int k = 0; k < NC; ++k) load_add(first, k);
+        for (int k = 0; k < NC; ++k) load_add(first, k);
+    }
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kMlpWaves + wave;
         const bool live = tidx < ntiles;  // wavefront-uniform
         const int64_t v0 = tidx * 32;
         if (live) {
+            if constexpr (!EARLY) load_x(tidx);
             // ---- first product, bias, ReLU: the B fragments of the second product ----
             half8_t hb[KS2];
 #pragma unroll
@@ -132,7 +138,7 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
                     }
                 }
             }
-            load_x(tidx + tiles_per_round);
+            if constexpr (EARLY) load_x(tidx + tiles_per_round);
             // ---- second product ----
 #pragma unroll
             for (int mo = 0; mo < MO; ++mo) {
@@ -161,22 +167,22 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
                 const int c = k * kWave + lane;
                 const int row = c / (C / 8), cc = c % (C / 8);
                 half8_t o = Tile::read(my, row, cc);
+                if constexpr (!EARLY) load_add(tidx, k);
 #pragma unroll
                 for (int jj = 0; jj < 8; ++jj) o[jj] = (half_t)((float)o[jj] + (float)ab[k][jj]);  // fp16 add, RNE
                 if (v0 + row < V) store_c8_nt(out + (v0 + row) * C + cc * 8, o);
-                load_add(tidx + tiles_per_round, k);
+                if constexpr (EARLY) load_add(tidx + tiles_per_round, k);
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
 }
 
-// Workgroups per compute unit: as few as keep 32 KB of x and residual in flight (us with 2 / 3 / 4 / 5 workgroups: C = 16
-// at 2.1 M voxels 41.3 / 35.7 / 35.4 / 35.4, C = 32 at 0.4 M 17.5 / 17.8 / 18.5 / 19.7, at 1.96 M 67.2 / 67.5 / 69.9 / 71.6,
-// C = 64 at 1.96 M 134 / 140 / 145 / 141).
+// Workgroups per compute unit (us with 2 / 3 / 4 / 5: C = 16 at 2.1 M voxels 41.3 / 35.7 / 35.4 / 35.4, C = 32 at 1.96 M
+// 89 / 71 / 67.3 / 67.2, C = 64 at 1.96 M 134 / 140 / 145 / 141)
 static int mlp_blocks(int64_t V, int C)
 {
-    const int64_t per_cu = C >= 32 ? 2 : 4;
+    const int64_t per_cu = C == 64 ? 2 : 4;
     return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kMlpWaves), per_cu * device_geometry().cus));
 }
 
@@ -225,270 +231,233 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
 // where a wavefront needs no LDS tiles and no workgroup barrier per tile; C = 64 runs the kernel below.
 //
 // A workgroup of four wavefronts loops over tiles of 64 voxels; x and g tiles are staged through LDS.
-// Phase A: per (32 voxels, 32 hidden channels) block a wavefront computes linup^T and (Wdown g^T) with the
-// same output layout, applies bias / ReLU / mask in registers and writes the hid and lg tiles to LDS.
-// Phase B: dx^T = Wup lg^T from the lg tile (bounced through LDS for 16-byte stores), and the three
-// reductions over voxels: the 32x32 blocks of dWdown = hid^T g and dWup = x^T lg take their fragments
-// (8 consecutive voxels of one channel) from the LDS tiles with 2-byte reads and stay in fp32 registers
-// for all tiles of the workgroup; dbias is a per-thread column sum of the lg tile.  Partials go to the
-// workspace, a second kernel adds them in a fixed order (fp64): deterministic, no atomics.
+// Phase A: wavefront w computes hidden block w (32 channels) of all 64 voxels, linup^T and (Wdown g^T) with the same
+// output layout, applies bias / ReLU / mask in registers and writes the hid and lg tiles to LDS.
+// Phase B: dx^T = Wup lg^T from the lg tile (one block of 32 voxels x 32 channels per wavefront, bounced through LDS for
+// 16-byte stores), and the reductions over voxels, four 32x32 blocks per wavefront: dWdown = hid^T g (even wavefronts)
+// and dWup = x^T lg (odd ones), which stay in fp32 registers for all tiles of the workgroup; their operands, 8 consecutive
+// voxels of one channel, are transposing LDS reads (SwizzledRows).  dbias adds up the lg operands that the odd wavefronts
+// read anyway.  The weight fragments of phase A are the same for every tile and stay in the wavefront's registers, so that
+// the LDS holds two workgroups per compute unit.  Partials go to the workspace, a second kernel adds them in a fixed order
+// (fp64): deterministic, no atomics.
+// Two workgroups of 256 registers per lane; with operands read from LDS in 2-byte pieces and the weights in LDS, one
+// workgroup per compute unit, the kernel took 705 us at 1.96 M voxels, now 247 (its HBM traffic at 6 TB/s: 125 us).
 namespace kerops {
 
-constexpr int kMbTile = 64;
-
-template <int C>
 struct MbCfg {
-    static constexpr int H = 2 * C;
-    static constexpr int MH = H / 32, MO = (C + 31) / 32;  // 32-channel blocks of hidden / in-out channels
+    static constexpr int C = 64, H = 128, TILE = 64;
+    static constexpr int MH = H / 32, MO = C / 32;         // 32-channel blocks of hidden / in-out channels
     static constexpr int KC = C / 16, KH = H / 16;         // k steps over C / over H
-    static constexpr int KV = kMbTile / 16;                // k steps over the voxels of a tile
-    static constexpr int XP = C + 8, HP = H + 8, DP = C;      // LDS row pitches in halves (the dx tile: dense rows, BounceTile)
-    static constexpr int NBA = 2 * MH;                     // phase A blocks (vt, mh)
-    static constexpr int NB6 = 2 * MO;                     // dx blocks (vt, mo)
-    static constexpr int NU = 2 * MH * MO;                 // reduction blocks: (type, mh, mc)
-    static constexpr int KSPL = NU >= kMlpWaves ? 1 : kMlpWaves / NU;
-    static constexpr int UPW = NU >= kMlpWaves ? NU / kMlpWaves : 1;
-    static constexpr int NXC = kMbTile * C / 8;            // 16-byte chunks of an x / g / dx tile
-    static constexpr int NLX = (NXC + kMlpThreads - 1) / kMlpThreads;
-    static constexpr int BPARTS = kMlpThreads / H;         // threads per hidden channel in the bias sum
+    static constexpr int KV = TILE / 16;                   // k steps over the voxels of a tile
+    static constexpr int NLX = TILE * C / 8 / kMlpThreads; // 16-byte chunks of an x / g / dx tile per thread
     static constexpr int RW = 2 * C * H + H;               // floats of one partial: dWup, dWdown, dbias
     static constexpr int XS_OFF = 0;
-    static constexpr int GS_OFF = XS_OFF + kMbTile * XP * 2;
-    static constexpr int HS_OFF = GS_OFF + kMbTile * XP * 2;
-    static constexpr int LS_OFF = HS_OFF + kMbTile * HP * 2;
-    static constexpr int DS_OFF = LS_OFF + kMbTile * HP * 2;
-    static constexpr int A1_OFF = (DS_OFF + kMbTile * DP * 2 + 15) / 16 * 16;
-    static constexpr int A3_OFF = A1_OFF + MH * KC * 64 * 16;
-    static constexpr int A6_OFF = A3_OFF + MH * KC * 64 * 16;
-    static constexpr int BS_OFF = A6_OFF + MO * KH * 64 * 16;
-    static constexpr int BH_OFF = BS_OFF + kMlpThreads * 4;  // fp16 copy of the bias
-    static constexpr int LDS_BYTES = BH_OFF + H * 2;
-    static_assert(C == 16 || C == 32 || C == 64, "C in {16,32,64}");
-    static_assert(KV % KSPL == 0 && kMbTile % BPARTS == 0, "even splits");
+    static constexpr int GS_OFF = XS_OFF + TILE * C * 2;
+    static constexpr int HS_OFF = GS_OFF + TILE * C * 2;
+    static constexpr int LS_OFF = HS_OFF + TILE * H * 2;
+    static constexpr int DS_OFF = LS_OFF + TILE * H * 2;
+    static constexpr int A6_OFF = DS_OFF + TILE * C * 2;   // fragments of the dx product [mo][s]
+    static constexpr int LDS_BYTES = A6_OFF + MO * KH * 64 * 16;
+    static_assert(RW % 32 == 0, "whole lines for the reduction");
+    static_assert(MH == kMlpWaves && 2 * MO == kMlpWaves, "one hidden block and one dx block per wavefront");
+    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per compute unit");
 };
 
-template <int C>
-__global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_bwd_kernel(const half_t* __restrict__ x,
-                                                                        const half_t* __restrict__ g,
-                                                                        const half_t* __restrict__ Wup,
-                                                                        const half_t* __restrict__ Wdown,
-                                                                        const half_t* __restrict__ bias,
-                                                                        half_t* __restrict__ dx, float* __restrict__ ws,
-                                                                        int64_t V)
+__global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_kernel(const half_t* __restrict__ x,
+                                                                           const half_t* __restrict__ g,
+                                                                           const half_t* __restrict__ Wup,
+                                                                           const half_t* __restrict__ Wdown,
+                                                                           const half_t* __restrict__ bias,
+                                                                           half_t* __restrict__ dx,
+                                                                           float* __restrict__ ws, int64_t V)
 {
-    using Cfg = MbCfg<C>;
-    constexpr int H = Cfg::H, MH = Cfg::MH, MO = Cfg::MO, KC = Cfg::KC, KH = Cfg::KH, KV = Cfg::KV;
-    constexpr int XP = Cfg::XP, HP = Cfg::HP, DP = Cfg::DP, NLX = Cfg::NLX, KSPL = Cfg::KSPL, UPW = Cfg::UPW;
+    using Cfg = MbCfg;
+    constexpr int C = Cfg::C, H = Cfg::H, KC = Cfg::KC, KH = Cfg::KH, KV = Cfg::KV, NLX = Cfg::NLX, TILE = Cfg::TILE;
+    using XT = SwizzledRows<C>;  // x and g tiles
+    using HT = SwizzledRows<H>;  // hid and lg tiles
     __shared__ __attribute__((aligned(16))) unsigned char smem[Cfg::LDS_BYTES];
-    half_t* xs = reinterpret_cast<half_t*>(smem + Cfg::XS_OFF);
-    half_t* gs = reinterpret_cast<half_t*>(smem + Cfg::GS_OFF);
-    half_t* hs = reinterpret_cast<half_t*>(smem + Cfg::HS_OFF);
-    half_t* ls = reinterpret_cast<half_t*>(smem + Cfg::LS_OFF);
-    half_t* ds = reinterpret_cast<half_t*>(smem + Cfg::DS_OFF);
-    half_t* a1 = reinterpret_cast<half_t*>(smem + Cfg::A1_OFF);
-    half8_t* a3 = reinterpret_cast<half8_t*>(smem + Cfg::A3_OFF);
-    half8_t* a6 = reinterpret_cast<half8_t*>(smem + Cfg::A6_OFF);
-    float* bred = reinterpret_cast<float*>(smem + Cfg::BS_OFF);
-    half_t* bsh = reinterpret_cast<half_t*>(smem + Cfg::BH_OFF);
+    unsigned char* xs = smem + Cfg::XS_OFF;
+    unsigned char* gs = smem + Cfg::GS_OFF;
+    unsigned char* hs = smem + Cfg::HS_OFF;
+    unsigned char* ls = smem + Cfg::LS_OFF;
+    unsigned char* ds = smem + Cfg::DS_OFF;
 
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    const int t = threadIdx.x, lane = t % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
     const int il = lane % 32, hl = lane / 32;
     const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
-    // fragments of the three per-voxel products (lane l: row l%32 of the block, k = 16 s + 8 (l/32) + 0..7)
-    // a1: linup^T = Wup^T x^T     -> Wup[k][32 mh + l%32]
-    for (int i = t; i < MH * KC * 64 * 8; i += kMlpThreads) {
-        const int j = i % 8, l = (i / 8) % 64, s = (i / 512) % KC, mh = i / (512 * KC);
-        a1[i] = Wup[(16 * s + 8 * (l / 32) + j) * H + 32 * mh + l % 32];
-    }
-    // a3: (Wdown g^T)             -> Wdown[32 mh + l%32][k .. k+7]
-    for (int i = t; i < MH * KC * 64; i += kMlpThreads) {
-        const int l = i % 64, s = (i / 64) % KC, mh = i / (64 * KC);
-        a3[i] = load_c8(Wdown + (32 * mh + l % 32) * C + 16 * s + 8 * (l / 32));
-    }
-    // a6: dx^T = Wup lg^T         -> Wup[32 mo + l%32][k .. k+7]
-    for (int i = t; i < MO * KH * 64; i += kMlpThreads) {
-        const int l = i % 64, s = (i / 64) % KH, mo = i / (64 * KH);
-        const int c = 32 * mo + l % 32;
-        a6[i] = c < C ? load_c8(Wup + c * H + 16 * s + 8 * (l / 32)) : z8;
-    }
-    for (int i = t; i < H; i += kMlpThreads) bsh[i] = bias[i];
-    const half8_t* a1f = reinterpret_cast<const half8_t*>(a1);
-
-    // reduction blocks of this wavefront: unit u = (type = u % 2, mh = (u / 2) % MH, mc = u / (2 MH));
-    // type 0: dWdown[h, c] = hid^T g, type 1: dWup[c, h] = x^T lg
-    const int u0 = Cfg::NU >= kMlpWaves ? wave : wave % Cfg::NU;
-    const int kpart = Cfg::NU >= kMlpWaves ? 0 : wave / Cfg::NU;
-    float16_t wacc[UPW];
+    // fragments of the three per-voxel products (lane: row il of the block, k = 16 s + 8 hl + 0..7)
+    half8_t a1[KC], a3[KC];
+    half4_t b4[4];
+    const int mo = wave / 2, vto = wave % 2;  // the wavefront's dx block
 #pragma unroll
-    for (int uu = 0; uu < UPW; ++uu)
+    for (int s = 0; s < KC; ++s) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) wacc[uu][i] = 0.0f;
-    float bacc = 0.0f;  // dbias: hidden channel t % H, voxels t / H + BPARTS * n
-    const int bh = t % H, bp = t / H;
+        for (int j = 0; j < 8; ++j) a1[s][j] = Wup[(16 * s + 8 * hl + j) * H + 32 * wave + il];  // linup^T = Wup^T x^T
+        a3[s] = load_c8(Wdown + (32 * wave + il) * C + 16 * s + 8 * hl);                        // Wdown g^T
+    }
+    half8_t* a6w = reinterpret_cast<half8_t*>(smem + Cfg::A6_OFF);  // dx^T = Wup lg^T
+    for (int i = t; i < Cfg::MO * KH * 64; i += kMlpThreads) {
+        const int l = i % 64, s = (i / 64) % KH, m = i / (64 * KH);
+        a6w[i] = load_c8(Wup + (32 * m + l % 32) * H + 16 * s + 8 * (l / 32));
+    }
+    const half8_t* a6 = a6w + mo * KH * 64 + lane;  // (the barrier behind the first staging covers it)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) b4[gq][jj] = bias[32 * wave + 8 * gq + 4 * hl + jj];
 
-    const int64_t ntiles = (V + kMbTile - 1) / kMbTile;
+    // reduction blocks of this wavefront, k = 0..3: hidden block mh = wave / 2 + 2 (k % 2), in-out block mc = k / 2;
+    // even wavefronts: dWdown[h, c] = hid^T g, odd ones: dWup[c, h] = x^T lg
+    float16_t wacc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) wacc[k][i] = 0.0f;
+    float bacc[2] = {0.0f, 0.0f};  // odd wavefronts: dbias of hidden block wave / 2 + 2 k, channel il
+    int hoff[2][2], xoff[2][2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        HT::tr_offsets(lane, wave / 2 + 2 * k, hoff[k]);
+        XT::tr_offsets(lane, k, xoff[k]);
+    }
+
+    const int64_t ntiles = (V + TILE - 1) / TILE;
     half8_t xpre[NLX], gpre[NLX];
     auto prefetch = [&](int64_t tile) {
-        const int64_t v0 = tile * kMbTile;
+        const int64_t v0 = tile * TILE;
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kMlpThreads;
             const int64_t v = v0 + c / (C / 8);
-            const bool ok = (c < Cfg::NXC) && (v < V);
-            xpre[j] = ok ? load_c8_nt(x + v * C + (c % (C / 8)) * 8) : z8;
-            gpre[j] = ok ? load_c8_nt(g + v * C + (c % (C / 8)) * 8) : z8;
+            xpre[j] = v < V ? load_c8_nt(x + v * C + (c % (C / 8)) * 8) : z8;
+            gpre[j] = v < V ? load_c8_nt(g + v * C + (c % (C / 8)) * 8) : z8;
         }
     };
 
     int64_t tile = blockIdx.x;
     if (tile < ntiles) prefetch(tile);
     for (; tile < ntiles; tile += gridDim.x) {
-        const int64_t v0 = tile * kMbTile;
+        const int64_t v0 = tile * TILE;
         // ---- stage the tile (rows past V are zero: they add nothing to the reductions) ----
+        // (the previous tile's x and g were last read before the barrier in front of its write-back)
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kMlpThreads;
-            if (c < Cfg::NXC) {
-                *reinterpret_cast<half8_t*>(xs + (c / (C / 8)) * XP + (c % (C / 8)) * 8) = xpre[j];
-                *reinterpret_cast<half8_t*>(gs + (c / (C / 8)) * XP + (c % (C / 8)) * 8) = gpre[j];
-            }
+            const int off = XT::chunk16(c / (C / 8), c % (C / 8));
+            *reinterpret_cast<half8_t*>(xs + off) = xpre[j];
+            *reinterpret_cast<half8_t*>(gs + off) = gpre[j];
         }
         __syncthreads();
         if (tile + gridDim.x < ntiles) prefetch(tile + gridDim.x);
 
-        // ---- phase A: hid and lg tiles, blocks (vt, mh) of 32 voxels x 32 hidden channels ----
+        // ---- phase A: hid and lg, 32 voxels x 32 hidden channels at a time ----
+#pragma unroll 1  // (unrolled, the offsets of both halves cost spilled registers)
+        for (int vt = 0; vt < 2; ++vt) {
+            const int row = 32 * vt + il;
+            // chunk 2 s + hl of the row: the swizzle is an XOR, so step s is the offset of step 0 ^ 32 s
+            const int xrow = XT::chunk16(row, hl);
+            float16_t up, dn;
 #pragma unroll
-        for (int ba = 0; ba < (Cfg::NBA + kMlpWaves - 1) / kMlpWaves; ++ba) {
-            const int blk = wave + ba * kMlpWaves;
-            if (blk < Cfg::NBA) {  // wavefront-uniform
-                const int vt = blk % 2, mh = blk / 2;
-                const int row = 32 * vt + il;
-                float16_t up, dn;
+            for (int i = 0; i < 16; ++i) up[i] = dn[i] = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) up[i] = dn[i] = 0.0f;
+            for (int s = 0; s < KC; ++s) {
+                const half8_t xb = *reinterpret_cast<const half8_t*>(xs + (xrow ^ (32 * s)));
+                const half8_t gb = *reinterpret_cast<const half8_t*>(gs + (xrow ^ (32 * s)));
+                up = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1[s], xb, up, 0, 0, 0);
+                dn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a3[s], gb, dn, 0, 0, 0);
+            }
+            // up[i], dn[i]: hidden channel 32 wave + 8 (i/4) + 4 hl + i%4 of voxel row
 #pragma unroll
-                for (int s = 0; s < KC; ++s) {
-                    const half8_t xb = *reinterpret_cast<const half8_t*>(xs + row * XP + 16 * s + 8 * hl);
-                    const half8_t gb = *reinterpret_cast<const half8_t*>(gs + row * XP + 16 * s + 8 * hl);
-                    up = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1f[(mh * KC + s) * 64 + lane], xb, up, 0, 0, 0);
-                    dn = __builtin_amdgcn_mfma_f32_32x32x16_f16(a3[(mh * KC + s) * 64 + lane], gb, dn, 0, 0, 0);
+            for (int gq = 0; gq < 4; ++gq) {
+                half4_t hv, lv;
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) {
+                    const half_t lin = (half_t)((float)(half_t)up[4 * gq + jj] + (float)b4[gq][jj]);  // fp16 add
+                    const bool pos = lin > (half_t)0;
+                    hv[jj] = pos ? lin : (half_t)0;
+                    lv[jj] = pos ? (half_t)dn[4 * gq + jj] : (half_t)0;
                 }
-                // up[i], dn[i]: hidden channel 32 mh + 8 (i/4) + 4 hl + i%4 of voxel row
-#pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    const int hc = 32 * mh + 8 * gq + 4 * hl;
-                    const half4_t b4 = *reinterpret_cast<const half4_t*>(bsh + hc);
-                    half4_t hv, lv;
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) {
-                        const half_t lin = (half_t)((float)(half_t)up[4 * gq + jj] + (float)b4[jj]);  // fp16 add
-                        const bool pos = lin > (half_t)0;
-                        hv[jj] = pos ? lin : (half_t)0;
-                        lv[jj] = pos ? (half_t)dn[4 * gq + jj] : (half_t)0;
-                    }
-                    // rows past V hold x = g = 0: hid = relu(bias) there, which must not reach dWdown ... but
-                    // it is multiplied by g = 0; lg = fp16(0) = 0, so dWup and dbias are unaffected as well
-                    *reinterpret_cast<half4_t*>(hs + row * HP + hc) = hv;
-                    *reinterpret_cast<half4_t*>(ls + row * HP + hc) = lv;
-                }
+                // rows past V hold x = g = 0: hid = relu(bias) there, which must not reach dWdown ... but
+                // it is multiplied by g = 0; lg = fp16(0) = 0, so dWup and dbias are unaffected as well
+                const int off = HT::chunk16(row, 4 * wave + gq) + 8 * hl;
+                *reinterpret_cast<half4_t*>(hs + off) = hv;
+                *reinterpret_cast<half4_t*>(ls + off) = lv;
             }
         }
         __syncthreads();
 
-        // ---- phase B1: dx^T blocks (vt, mo) from the lg tile ----
+        // ---- phase B1: the dx^T block (vto, mo) from the lg tile ----
+        {
+            const int row = 32 * vto + il;
+            const int lrow = HT::chunk16(row, hl);
+            float16_t acc;
 #pragma unroll
-        for (int b6 = 0; b6 < (Cfg::NB6 + kMlpWaves - 1) / kMlpWaves; ++b6) {
-            const int blk = wave + b6 * kMlpWaves;
-            if (blk < Cfg::NB6) {  // wavefront-uniform
-                const int vt = blk % 2, mo = blk / 2;
-                const int row = 32 * vt + il;
-                float16_t acc;
+            for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+            for (int s = 0; s < KH; ++s) {
+                const half8_t lb = *reinterpret_cast<const half8_t*>(ls + (lrow ^ (32 * s)));
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a6[64 * s], lb, acc, 0, 0, 0);
+            }
 #pragma unroll
-                for (int s = 0; s < KH; ++s) {
-                    const half8_t lb = *reinterpret_cast<const half8_t*>(ls + row * HP + 16 * s + 8 * hl);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a6[(mo * KH + s) * 64 + lane], lb, acc, 0, 0, 0);
-                }
+            for (int gq = 0; gq < 4; ++gq) {
+                half4_t o;
 #pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    const int c = 32 * mo + 8 * gq + 4 * hl;
-                    if (c < C) {
-                        half4_t o;
-#pragma unroll
-                        for (int jj = 0; jj < 4; ++jj) o[jj] = (half_t)acc[4 * gq + jj];
-                        *reinterpret_cast<half4_t*>(reinterpret_cast<unsigned char*>(ds) + BounceTile<C>::piece(row, 4 * mo + gq, hl)) = o;
-                    }
-                }
+                for (int jj = 0; jj < 4; ++jj) o[jj] = (half_t)acc[4 * gq + jj];
+                *reinterpret_cast<half4_t*>(ds + BounceTile<C>::piece(row, 4 * mo + gq, hl)) = o;
             }
         }
         // ---- phase B2: the reductions over the voxels of the tile ----
 #pragma unroll
-        for (int uu = 0; uu < UPW; ++uu) {
-            const int u = u0 + uu * kMlpWaves;
-            const int type = u % 2, mh = (u / 2) % MH, mc = u / (2 * MH);
-            const int cc = min(32 * mc + il, C - 1), hh = 32 * mh + il;
-            // A rows / B columns: type 0: (hid[:, hh], g[:, cc]); type 1: (x[:, cc], lg[:, hh])
-            const half_t* ap = type == 0 ? hs + hh : xs + cc;
-            const half_t* bp2 = type == 0 ? gs + cc : ls + hh;
-            const int apitch = type == 0 ? HP : XP, bpitch = type == 0 ? XP : HP;
+        for (int s = 0; s < KV; ++s) {
+            if (wave % 2 == 0) {
+                const half8_t hf[2] = {HT::read_tr(hs, hoff[0], s), HT::read_tr(hs, hoff[1], s)};
+                const half8_t gf[2] = {XT::read_tr(gs, xoff[0], s), XT::read_tr(gs, xoff[1], s)};
 #pragma unroll
-            for (int sp = 0; sp < KV / KSPL; ++sp) {
-                const int s = kpart + sp * KSPL;
-                half8_t af, bf;
+                for (int k = 0; k < 4; ++k)
+                    wacc[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hf[k % 2], gf[k / 2], wacc[k], 0, 0, 0);
+            } else {
+                const half8_t lf[2] = {HT::read_tr(ls, hoff[0], s), HT::read_tr(ls, hoff[1], s)};
+                const half8_t xf[2] = {XT::read_tr(xs, xoff[0], s), XT::read_tr(xs, xoff[1], s)};
 #pragma unroll
-                for (int jj = 0; jj < 8; ++jj) {
-                    af[jj] = ap[(16 * s + 8 * hl + jj) * apitch];
-                    bf[jj] = bp2[(16 * s + 8 * hl + jj) * bpitch];
-                }
-                wacc[uu] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, wacc[uu], 0, 0, 0);
+                for (int k = 0; k < 4; ++k)
+                    wacc[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[k / 2], lf[k % 2], wacc[k], 0, 0, 0);
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) bacc[k] += (float)lf[k][j];
             }
         }
-        // dbias: column sums of the lg tile
-#pragma unroll
-        for (int n = 0; n < kMbTile / Cfg::BPARTS; ++n) bacc += (float)ls[(bp + Cfg::BPARTS * n) * HP + bh];
         __syncthreads();
 
-        // ---- phase C: dx write-back, 16-byte chunks ----
+        // ---- phase C: dx write-back, 16-byte chunks (the dx tile is written next behind two barriers) ----
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kMlpThreads;
             const int row = c / (C / 8), cc = c % (C / 8);
-            if (c < Cfg::NXC && v0 + row < V) {
-                const half8_t o = BounceTile<C>::read(reinterpret_cast<const unsigned char*>(ds), row, cc);
-                store_c8_nt(dx + (v0 + row) * C + cc * 8, o);
-            }
+            if (v0 + row < V) store_c8_nt(dx + (v0 + row) * C + cc * 8, BounceTile<C>::read(ds, row, cc));
         }
-        __syncthreads();
     }
 
-    // ---- partials of this workgroup: row (blockIdx, kpart) = [dWup C*H][dWdown H*C][dbias H] ----
-    float* out = ws + ((int64_t)blockIdx.x * KSPL + kpart) * Cfg::RW;
+    // ---- partials of this workgroup: row blockIdx = [dWup C*H][dWdown H*C][dbias H] ----
+    float* out = ws + (int64_t)blockIdx.x * Cfg::RW;
 #pragma unroll
-    for (int uu = 0; uu < UPW; ++uu) {
-        const int u = u0 + uu * kMlpWaves;
-        const int type = u % 2, mh = (u / 2) % MH, mc = u / (2 * MH);
+    for (int k = 0; k < 4; ++k) {
+        const int mh = wave / 2 + 2 * (k % 2), mc = k / 2;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int ri = 8 * (i / 4) + 4 * hl + i % 4;  // row of the block held in register i
-            if (type == 0) {  // D[i = h][j = c]
-                const int h = 32 * mh + ri, c = 32 * mc + il;
-                if (c < C) out[C * H + h * C + c] = wacc[uu][i];
-            } else {  // D[i = c][j = h]
-                const int c = 32 * mc + ri, h = 32 * mh + il;
-                if (c < C) out[c * H + h] = wacc[uu][i];
-            }
+            if (wave % 2 == 0) out[C * H + (32 * mh + ri) * C + 32 * mc + il] = wacc[k][i];  // D[h][c]
+            else out[(32 * mc + ri) * H + 32 * mh + il] = wacc[k][i];                        // D[c][h]
         }
     }
-    bred[t] = bacc;
-    __syncthreads();
-    if (t < H) {
-        float s = 0.0f;
+    if (wave % 2 == 1) {
 #pragma unroll
-        for (int p = 0; p < Cfg::BPARTS; ++p) s += bred[p * H + t];
-        ws[((int64_t)blockIdx.x * KSPL) * Cfg::RW + 2 * C * H + t] = s;
-        for (int kp = 1; kp < KSPL; ++kp) ws[((int64_t)blockIdx.x * KSPL + kp) * Cfg::RW + 2 * C * H + t] = 0.0f;
+        for (int k = 0; k < 2; ++k) {
+            const float sum = bacc[k] + __shfl_xor(bacc[k], 32, 64);  // the two lane halves hold different voxels
+            if (hl == 0) out[2 * C * H + 32 * (wave / 2 + 2 * k) + il] = sum;
+        }
     }
 }
 
@@ -523,6 +492,7 @@ struct MtCfg {
     static constexpr int LOOP_BYTES = DS_OFF + kMlpWaves * 32 * DP * 2;
     static constexpr int LDS_BYTES = LOOP_BYTES > RW * 4 ? LOOP_BYTES : RW * 4;
     static_assert(C == 16 || C == 32, "one 32-channel block of in / out channels");
+    static_assert(RW % 32 == 0, "whole lines for the reduction");
 };
 
 // fp32 accumulator -> the two packed fp16 operands (registers 0..7 and 8..15)
@@ -1111,38 +1081,17 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_tr_kernel(
     for (int i = t; i < Cfg::RW; i += kMlpThreads) out[i] = red[i];
 }
 
-// sums the rows of the partial buffer in a fixed order (16 columns per workgroup, 64 interleaved row slices with four
-// loads in flight, fixed tree in LDS; fp64) and scatters the three results
+// sums the rows of the partial buffer in a fixed order (sum_lines in common.hpp) and scatters the three results
 // (OutT: fp32, or fp16 = the fp32 results rounded once)
 template <class OutT>
 __global__ __launch_bounds__(1024) void mlp_reduce_kernel(const float* __restrict__ ws, int nrows, int RW, int n_up,
                                                           int n_down, OutT* __restrict__ d_up,
                                                           OutT* __restrict__ d_down, OutT* __restrict__ d_bias)
 {
-    __shared__ double part[64][17];
-    const int lo = threadIdx.x % 16, sl = threadIdx.x / 16;
-    const int j = blockIdx.x * 16 + lo;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    if (j < RW) {
-        int r = sl;
-        for (; r + 192 < nrows; r += 256) {
-            const float a = ws[(int64_t)r * RW + j], b = ws[(int64_t)(r + 64) * RW + j];
-            const float c = ws[(int64_t)(r + 128) * RW + j], d = ws[(int64_t)(r + 192) * RW + j];
-            s0 += (double)a;
-            s1 += (double)b;
-            s2 += (double)c;
-            s3 += (double)d;
-        }
-        for (; r < nrows; r += 64) s0 += (double)ws[(int64_t)r * RW + j];
-    }
-    part[sl][lo] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    for (int w = 32; w > 0; w >>= 1) {
-        if (sl < w) part[sl][lo] += part[sl + w][lo];
-        __syncthreads();
-    }
-    if (sl == 0 && j < RW) {
-        const double v = part[0][lo];
+    __shared__ double part[16][33];
+    const double v = sum_lines(ws, nrows, RW, part);
+    const int j = blockIdx.x * 32 + threadIdx.x;
+    if (threadIdx.x < 32) {
         if (j < n_up) d_up[j] = (OutT)(float)v;
         else if (j < n_up + n_down) d_down[j - n_up] = (OutT)(float)v;
         else d_bias[j - n_up - n_down] = (OutT)(float)v;
@@ -1153,10 +1102,10 @@ static void launch_mlp_reduce(const float* ws, int nrows, int RW, int n_up, int 
                               void* d_bias, int dtype, hipStream_t s)
 {
     if (dtype == KEROPS_DTYPE_F16)
-        hipLaunchKernelGGL(mlp_reduce_kernel<half_t>, dim3(ceil_div(RW, 16)), dim3(1024), 0, s, ws, nrows, RW, n_up,
+        hipLaunchKernelGGL(mlp_reduce_kernel<half_t>, dim3(RW / 32), dim3(1024), 0, s, ws, nrows, RW, n_up,
                            n_down, (half_t*)d_up, (half_t*)d_down, (half_t*)d_bias);
     else
-        hipLaunchKernelGGL(mlp_reduce_kernel<float>, dim3(ceil_div(RW, 16)), dim3(1024), 0, s, ws, nrows, RW, n_up,
+        hipLaunchKernelGGL(mlp_reduce_kernel<float>, dim3(RW / 32), dim3(1024), 0, s, ws, nrows, RW, n_up,
                            n_down, (float*)d_up, (float*)d_down, (float*)d_bias);
 }
 
@@ -1167,15 +1116,7 @@ static int mb_blocks(int64_t V, int C)
         const int64_t ntiles = (V + 31) / 32;
         return (int)std::max<int64_t>(1, std::min<int64_t>((ntiles + kMlpWaves - 1) / kMlpWaves, C == 16 ? 768 : 512));
     }
-    const int64_t ntiles = (V + kMbTile - 1) / kMbTile;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, 512));
-}
-
-static int mb_kspl(int C)
-{
-    if (C <= 32) return 1;
-    const int nu = 2 * (2 * C / 32) * ((C + 31) / 32);
-    return nu >= kMlpWaves ? 1 : kMlpWaves / nu;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, MbCfg::TILE), 2 * device_geometry().cus));
 }
 
 }  // namespace kerops
@@ -1190,7 +1131,7 @@ extern "C" int64_t kerops_lin_brelu_lin_bwd_workspace_bytes(int64_t V, int32_t C
         set_error("lin_brelu_lin_bwd: built for C in {16,32,64} (got %d)", C);
         return KEROPS_E_UNSUPPORTED_C;
     }
-    return (int64_t)mb_blocks(V, C) * mb_kspl(C) * (4 * C * C + 2 * C) * (int64_t)sizeof(float);
+    return (int64_t)mb_blocks(V, C) * (4 * C * C + 2 * C) * (int64_t)sizeof(float);
 }
 
 extern "C" int kerops_lin_brelu_lin_bwd_f16(const void* x, const void* g, const void* Wup, const void* Wdown,
@@ -1252,20 +1193,16 @@ extern "C" int kerops_lin_brelu_lin_bwd_f16_out(const void* x, const void* g, co
         launch_mlp_reduce(ws, blocks, RW, 2 * 32 * 32, 2 * 32 * 32, dWup, dWdown, dbias, grad_dtype, s);
         return check_launch("lin_brelu_lin_bwd_reduce");
     }
-#define KEROPS_MB_CASE(CV)                                                                                        \
-    if (C == CV) {                                                                                                \
-        hipLaunchKernelGGL((lin_brelu_lin_bwd_kernel<CV>), dim3(blocks), dim3(kMlpThreads), 0, s,                \
-                           (const half_t*)x, (const half_t*)g, (const half_t*)Wup, (const half_t*)Wdown,         \
-                           (const half_t*)bias, (half_t*)dx, ws, V);                                             \
-        int rc = check_launch("lin_brelu_lin_bwd");                                                               \
-        if (rc != KEROPS_OK) return rc;                                                                           \
-        const int RW = MbCfg<CV>::RW;                                                                             \
-        launch_mlp_reduce(ws, blocks * MbCfg<CV>::KSPL, RW, 2 * CV * CV, 2 * CV * CV, dWup, dWdown, dbias,        \
-                          grad_dtype, s);                                                                         \
-        return check_launch("lin_brelu_lin_bwd_reduce");                                                          \
+    if (C == 64) {
+        hipLaunchKernelGGL(lin_brelu_lin_bwd_kernel, dim3(blocks), dim3(kMlpThreads), 0, s, (const half_t*)x,
+                           (const half_t*)g, (const half_t*)Wup, (const half_t*)Wdown, (const half_t*)bias, (half_t*)dx,
+                           ws, V);
+        int rc = check_launch("lin_brelu_lin_bwd");
+        if (rc != KEROPS_OK) return rc;
+        const int RW = MbCfg::RW;
+        launch_mlp_reduce(ws, blocks, RW, 2 * 64 * 64, 2 * 64 * 64, dWup, dWdown, dbias, grad_dtype, s);
+        return check_launch("lin_brelu_lin_bwd_reduce");
     }
-    KEROPS_MB_CASE(64)
-#undef KEROPS_MB_CASE
     set_error("lin_brelu_lin_bwd: built for C in {16,32,64} (got %d)", C);
     return KEROPS_E_UNSUPPORTED_C;
 }

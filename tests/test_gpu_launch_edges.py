@@ -8,8 +8,8 @@ import oracle
 from conftest import cpu_gen, rand_cl3d, rand_dw_weight
 from kerops_amd.ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
 from kerops_amd.ops.conv import DWConv, DWConvBackward, DWConvStats, DWConvWGRAD
-from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, ReLULinearAdd,
-                                   ReLULinearBackward)
+from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, LinBReLULinAdd,
+                                   LinBReLULinBackward, ReLULinearAdd, ReLULinearBackward)
 from kerops_amd.ops.quantization import DequantUint8Window, QuantUint8Window
 
 pytestmark = pytest.mark.gpu
@@ -127,3 +127,24 @@ def test_built_in_split_of_the_march(shape):
     for got in (gw, DWConvWGRAD(x, grad, out_dtype=torch.float32)):
         # fp32 sums of at most a few thousand products a workgroup, then fp64: the bound of the weight-gradient tests
         assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < 1e-5
+
+
+# 32769 voxels at 64 channels, 65553 at 16 and 32: a second tile for one workgroup of 512; 131109: ragged third tiles
+@pytest.mark.parametrize('c', [16, 32, 64])
+@pytest.mark.parametrize('v', [1, 31, 33, 63, 65, 32769, 65553, 131109])
+def test_inverted_bottleneck_tiles_and_rounds(c, v):
+    g = cpu_gen(c + v)
+    x, add, grad = flat(g, v, c), flat(g, v, c), flat(g, v, c)
+    up, down, bias = matrix(g, c, 2 * c), matrix(g, 2 * c, c), (torch.randn(2 * c, generator=g) * 0.3).half()
+    dev = [t.to(DEV) for t in (x, up, down, bias, add, grad)]
+    out = LinBReLULinAdd(*dev[:5]).cpu()
+    ref = oracle.lin_brelu_lin_add(x, up, down, bias, add)
+    # two products and two sums, each rounded to fp16: a hidden value may be a neighbour of the oracle's
+    assert (out.float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
+    got = LinBReLULinBackward(dev[0], dev[5], dev[1], dev[2], dev[3], out_dtype=torch.float32)
+    want = oracle.lin_brelu_lin_bwd(x, grad, up, down, bias)
+    for a, b in zip(got, want):
+        # the ReLU's mask can differ where a pre-activation rounds to the other side of zero (one in about 2^11 within
+        # a rounding of it), and a hidden value by one rounding
+        err = ((a.cpu().double() - b.double()).norm() / max(b.double().norm().item(), 1e-30)).item()
+        assert err < 2.0 ** -5 if v < 1000 else err < 2.0 ** -8, err
