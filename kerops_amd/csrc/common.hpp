@@ -227,7 +227,7 @@ static inline bool volume_exceeds_i64(int N, int H, int W, int D, int C)
 // H_chunk sweeps of the forward and weight-gradient kernels at 14 shapes from 96^3 x 16 to 350 x 350 x 128 x 128
 // channels: the choice is the sweep's optimum or within 2 % of it (a variant that charges half a round for a
 // partial last round instead of a whole one was up to 15 % off).
-static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup, double* best_cost = nullptr)
+static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup)
 {
     int best_h = H;
     double best = 1e300;
@@ -243,7 +243,6 @@ static inline int pick_h_chunk(int H, int64_t per_plane, int slots, int setup, d
             best_h = h;
         }
     }
-    if (best_cost) *best_cost = best;
     return best_h;
 }
 // Balanced split of the H-marching kernels.  The tiles of the tensor, in their linear order (slab fastest, then
@@ -331,13 +330,21 @@ static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots
             const double crossing = share < H ? (aligned ? 0.0 : 8.0) : 8.0 * (double)share / H;
             const double spread = (int)b.group > slots / xcds ? 1.04 : 1.0;
             return ((double)share + 2 + setup + crossing) * (1.0 + 0.1 * row_len / (double)b.group) *
-                   (1.0 + 0.02 * (double)H / (double)share) * spread;
+                   (1.0 + 0.004 * (double)H / (double)share) * spread;
         },
         &cost);
-    double uniform_cost;
-    const int h = pick_h_chunk(H, tiles, slots, setup, &uniform_cost);
-    if (uniform_cost <= cost) return {part, h};
-    return {part, 0};
+    // chunks that run in one round (never more workgroups, and partial sums, than the balanced split has)
+    int best_h = 0;
+    for (int c = 1; c <= 64 && c <= H && tiles * c <= slots; ++c) {
+        const int h = ceil_div(H, c);
+        if (ceil_div(H, h) != c) continue;  // the same split as a smaller c
+        const double uniform = ((double)h + 2 + setup) * (1.0 + 0.004 * c);
+        if (uniform <= cost) {
+            cost = uniform;
+            best_h = h;
+        }
+    }
+    return {part, best_h};
 }
 // offsets inside one (W, D, C) plane are 32-bit in the convolution kernels (W, D, C positive)
 static inline bool plane_exceeds_i32(int W, int D, int C)

@@ -227,3 +227,19 @@ def test_product_never_imports_the_oracle():
             if f.endswith(('.py', '.hip', '.hpp', '.h', '.cpp')):
                 text = open(os.path.join(dirpath, f)).read()
                 assert 'import oracle' not in text and 'from oracle' not in text and 'oracle/' not in text, f
+
+
+def test_built_in_split_never_exceeds_the_resident_workgroups():
+    # chunks of H are only taken where they run in one round: the partial sums of the built-in weight-gradient shapes
+    # fit the 4 MB that the entry point without a workspace owns, at any size
+    import random
+    lib = _lib.load()
+    rng = random.Random(3)
+    for _ in range(3000):
+        c = rng.choice((8, 16, 32, 64, 128))
+        n, h, w, d = rng.choice((1, 2, 4)), rng.randint(1, 400), rng.randint(1, 400), rng.randint(1, 256)
+        partial = 27 * min(c, 64) * 4
+        for need in (lib.kerops_dwconv_wgrad_workspace_bytes(n, h, w, d, c, 0, 0, 0, 0),
+                     lib.kerops_dwconv_bwd_workspace_bytes(n, h, w, d, c, 0)):
+            assert 0 < need <= 512 * partial < 4 << 20, (n, c, h, w, d, need // partial)
+        assert lib.kerops_dwconv_stats_workspace_bytes(n, h, w, d, c) <= 1024 * 2 * min(c, 64) * 4
