@@ -82,8 +82,9 @@ def ReLULinearBackward(
 def ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad, weight):
     """Gradients of ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other) in one pass over x and grad.
     Returns (dx like x, bn_weight_grad fp32, bn_bias_grad fp32, weight_grad fp16): dx bit-identical to ApplyBNReLU,
-    ReLULinearBackward and ApplyBNReLUBackward in a row, the sums in another order.  The residual's gradient is grad
-    itself.  An addition to the reference's op set; host side of kerops_bnrelu_linear_bwd_f16."""
+    ReLULinearBackward and ApplyBNReLUBackward in a row (kerops/ops/bnrelu.py:11-42,
+    kerops/ops/linear/relu_linear_backward.py:20-72, kerops/ops/bnrelu.py:45-82), the sums in another order.  The
+    residual's gradient is grad itself.  An addition to the reference's op set; host side of kerops_bnrelu_linear_bwd_f16."""
     in_channels = x.shape[1]
     out_channels = grad.shape[1]
 
