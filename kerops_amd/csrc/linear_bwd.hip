@@ -29,14 +29,21 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 constexpr int kLbThreads = 256;
 constexpr int kLbWaves = kLbThreads / kWave;
 
-// Voxels per tile.  A tile's loads are all a workgroup has in flight, two workgroups run on a compute unit, and the
-// memory system needs about 40 KB in flight per compute unit: 64 voxels are enough from 96 channels (Cin + Cout) on,
-// fewer channels take tiles of the same bytes.
-constexpr int lb_tile(int cin, int cout) { return cin + cout >= 96 ? 64 : cin + cout >= 48 ? 128 : 256; }
+// Voxels per tile.  A tile's loads are all a workgroup has in flight, two to four workgroups run on a compute unit, and
+// the memory system needs about 40 KB in flight per compute unit: 64 voxels, 128 where the rows are short.  us with 64 /
+// 128 voxels and the best workgroup count of each: 16 -> 64 at 0.9 M voxels 36.1 / 34.8, 16 -> 16 at 4 M 74.4 / 66.2
+// (256 voxels: 69.1), 32 -> 32 at 4 M 125.9 / 133.5, 64 -> 16 at 4096 6.1 / 6.7.
+// The AFFINE kernel has the registers of two workgroups on a compute unit and takes the tiles that fill them (16 -> 16 at
+// 4 M voxels 75.4 with 256, 83.1 with 128; 32 -> 32 140.4 with 128, 156.5 with 64 and three workgroups).
+constexpr int lb_tile(int cin, int cout, bool affine)
+{
+    if (affine) return cin + cout >= 96 ? 64 : cin + cout >= 48 ? 128 : 256;
+    return (cin == 16 && cout <= 64) || (cin == 32 && cout == 16) ? 128 : 64;
+}
 
-template <int CIN, int COUT>
+template <int CIN, int COUT, bool AFFINE>
 struct LbCfg {
-    static constexpr int TILE = lb_tile(CIN, COUT);
+    static constexpr int TILE = lb_tile(CIN, COUT, AFFINE);
     static constexpr int MTI = (CIN + 31) / 32, MTO = (COUT + 31) / 32;  // 32-channel blocks
     static constexpr int KSO = COUT / 16;                                 // k steps of the dx product
     static constexpr int KSV = TILE / 16;                                 // k steps (voxels) of the dW product
@@ -52,11 +59,12 @@ struct LbCfg {
     static constexpr int GS_OFF = XS_OFF + TILE * XP * 2;
     static constexpr int DS_OFF = GS_OFF + TILE * GP * 2;
     static constexpr int WL_OFF = (DS_OFF + TILE * DP * 2 + 15) / 16 * 16;
-    static constexpr int LDS_BYTES = WL_OFF + MTI * KSO * 64 * 16;
+    static constexpr int TILE_BYTES = WL_OFF + MTI * KSO * 64 * 16;
+    static constexpr int SPLIT_BYTES = KSPL > 1 ? KSPL * CIN * COUT * 4 : 0;  // the sums of the split, after the last tile
+    static constexpr int LDS_BYTES = TILE_BYTES > SPLIT_BYTES ? TILE_BYTES : SPLIT_BYTES;
     static_assert(CIN % 16 == 0 && CIN <= 128 && COUT % 16 == 0 && COUT <= 128, "channels in {16,32,64,128}");
     static_assert(NBW % kLbWaves == 0 || kLbWaves % NBW == 0, "blocks divide over the wavefronts");
     static_assert(KSV % KSPL == 0, "voxel steps divide over the split");
-    static_assert(KSPL == 1 || LDS_BYTES >= KSPL * CIN * COUT * 4, "the sums of the split fit the tiles' LDS");
 };
 
 // AFFINE: the op's input is z = fp16(max(fma(x, scale[c], shift[c]), 0)), formed from the loaded x on its way to LDS, and
@@ -75,7 +83,7 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
                                                                         const float* __restrict__ shift)
 {
     constexpr int CGI = CIN / 8, ROW = CIN * COUT + (AFFINE ? 2 * CIN : 0);  // ROW: floats of a row of the workspace
-    using Cfg = LbCfg<CIN, COUT>;
+    using Cfg = LbCfg<CIN, COUT, AFFINE>;
     constexpr int XP = Cfg::XP, GP = Cfg::GP, DP = Cfg::DP, KSO = Cfg::KSO, KSV = Cfg::KSV;
     constexpr int NLX = Cfg::NLX, NLG = Cfg::NLG, BPW = Cfg::BPW, KSPL = Cfg::KSPL;
     __shared__ __attribute__((aligned(16))) unsigned char smem[Cfg::LDS_BYTES];
@@ -266,13 +274,19 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
     }
 }
 
-// Two workgroups per compute unit: what the LDS holds at 128 -> 128 channels, and a third only adds a row to the
-// partial sums (64 -> 128 at 0.35 M voxels: 43.4 us with two, 47.7 with three; 128 -> 128 at 0.26 M: 54.8 and 67.7;
-// 16 -> 16 at 2.1 M: 39.2 and 39.5).
-static int lb_blocks(int64_t V, int cin, int cout)
+// Workgroups per compute unit (the AFFINE kernel: two).  Two: what the LDS holds at 128 -> 128 channels, and a third only adds a row to the
+// partial sums (64 -> 128 at 0.35 M voxels: 43.4 us with two, 47.7 with three; 128 -> 128 at 0.26 M: 54.8 and 67.7).
+// 16 -> 16 has the fewest bytes in flight and the shortest rows of sums and takes four.  In volumes of half a million
+// voxels and more, where the rows of sums are few against the tiles, three pay at 32 -> 32 (0.2 M voxels 13.7 us with
+// two, 14.5 with three; 0.9 M 36.9 and 34.8; 15.7 M 523 and 492) and 16 -> 128 (0.2 M 19.1 and 19.7; 0.9 M 57.6 and
+// 55.4; 4 M 231 and 219), and 16 -> 16 has one more than it needs (4 M: 68.9 with four, 66.2 with three).
+static int lb_blocks(int64_t V, int cin, int cout, bool affine)
 {
-    const int64_t ntiles = ceil_div64(V, lb_tile(cin, cout));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, 2 * device_geometry().cus));
+    const bool narrow = cin == 16 && cout == 16 && !affine;
+    int per_cu = narrow ? 4 : 2;
+    if (V >= (1 << 19) && !affine && (narrow || (cin == 32 && cout == 32) || (cin == 16 && cout == 128))) per_cu = 3;
+    const int64_t ntiles = ceil_div64(V, lb_tile(cin, cout, affine));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, per_cu * device_geometry().cus));
 }
 
 // daffine: the AFFINE kernel's [2][CIN] sums, null without scale and shift
@@ -280,7 +294,7 @@ template <int CIN, int COUT>
 static int launch_lb(const half_t* x, const float* scale, const float* shift, const half_t* g, const half_t* Wm,
                      half_t* dx, void* dW, int dw_dtype, float* daffine, float* ws, int64_t V, hipStream_t s)
 {
-    const int blocks = lb_blocks(V, CIN, COUT);
+    const int blocks = lb_blocks(V, CIN, COUT, scale != nullptr);
     if (scale)
         hipLaunchKernelGGL((relu_linear_bwd_kernel<CIN, COUT, true>), dim3(blocks), dim3(kLbThreads), 0, s, x, g, Wm, dx,
                            ws, V, scale, shift);
@@ -313,7 +327,7 @@ static int64_t lb_workspace(const char* op, int64_t V, int Cin, int Cout, bool a
         set_error("%s: built for Cin, Cout in {16,32,64,128} (got %d -> %d)", op, Cin, Cout);
         return KEROPS_E_UNSUPPORTED_C;
     }
-    return (int64_t)lb_blocks(V, Cin, Cout) * (Cin * Cout + (affine ? 2 * Cin : 0)) * (int64_t)sizeof(float);
+    return (int64_t)lb_blocks(V, Cin, Cout, affine) * (Cin * Cout + (affine ? 2 * Cin : 0)) * (int64_t)sizeof(float);
 }
 
 static int lb_run(const char* op, const void* x, const float* scale, const float* shift, const void* g, const void* Wm,

@@ -243,3 +243,15 @@ def test_built_in_split_never_exceeds_the_resident_workgroups():
                      lib.kerops_dwconv_bwd_workspace_bytes(n, h, w, d, c, 0)):
             assert 0 < need <= 512 * partial < 4 << 20, (n, c, h, w, d, need // partial)
         assert lib.kerops_dwconv_stats_workspace_bytes(n, h, w, d, c) <= 1024 * 2 * min(c, 64) * 4
+
+
+def test_linear_backward_takes_a_third_workgroup_in_large_volumes():
+    # rows of partial sums = workgroups: two per compute unit of 256, three where half a million voxels and more keep them
+    # busy (32 -> 32 lost 5 % at 15.7 M voxels with two, 16 -> 128 lost 6 % at 4 M)
+    lib = _lib.load()
+    for cin, cout in ((32, 32), (16, 128)):
+        small, large = (lib.kerops_relu_linear_bwd_workspace_bytes(v, cin, cout) for v in (200000, 4000000))
+        assert large * 2 == small * 3, (cin, cout, small, large)
+    # the widest pair holds two workgroups in LDS
+    assert (lib.kerops_relu_linear_bwd_workspace_bytes(4000000, 128, 128)
+            == lib.kerops_relu_linear_bwd_workspace_bytes(200000, 128, 128) == 512 * 128 * 128 * 4)
