@@ -19,7 +19,13 @@
 //    applied to the x fragment in registers).  The (32 x 32) output blocks are distributed over the
 //    wavefronts (with fewer than four blocks the wavefronts split the voxels instead) and accumulated in
 //    fp32 registers over all tiles of the workgroup; at the end every workgroup writes its partial
-//    [CIN][COUT] matrices to the workspace and a second kernel adds them in a fixed order (deterministic).
+//    [CIN][COUT] matrix to the workspace and a second kernel adds them in a fixed order (deterministic).
+//    A matrix instruction rounds its running sum twice, from a zero accumulator a little downwards (2e-9 on average, inputs
+//    ~ N(0, 1)).  Against the first, a block has two or more accumulators that take the voxel steps in turn; they and the
+//    sums of wavefronts that split the voxels are added in fp64 and rounded once for the row.  Against the second, odd
+//    workgroups work on -g and -Wm (the same bits of dx) and return minus their sum.  Relative error of dW against 64 bits,
+//    with one accumulator and fp32 sums of the split / now: 0.9 M voxels 16 -> 16 170e-9 / 94e-9, 64 -> 64 258e-9 /
+//    183e-9, 128 -> 128 268e-9 / 116e-9, at 1 % more time.
 #include "common.hpp"
 
 namespace kerops {
@@ -53,6 +59,10 @@ struct LbCfg {
     static constexpr int NBW = MTI * MTO;                                 // dW blocks
     static constexpr int KSPL = NBW >= kLbWaves ? 1 : kLbWaves / NBW;     // voxel split when blocks are few
     static constexpr int BPW = NBW >= kLbWaves ? NBW / kLbWaves : 1;      // dW blocks per wavefront
+    static constexpr int STEPS = KSV / KSPL;                               // voxel steps of a wavefront per tile and block
+    // Accumulators of a block.  128 -> 128 has registers for one: it starts a chain from zero in every tile.
+    static constexpr bool TILE_CHAIN = BPW == 4;
+    static constexpr int NSET = TILE_CHAIN ? 1 : KSPL == 4 && STEPS > 2 ? STEPS : 2;
     static constexpr int NXC = TILE * CIN / 8, NGC = TILE * COUT / 8;  // 16-byte chunks per tile
     static constexpr int NLX = (NXC + kLbThreads - 1) / kLbThreads, NLG = (NGC + kLbThreads - 1) / kLbThreads;
     static constexpr int XS_OFF = 0;
@@ -60,11 +70,62 @@ struct LbCfg {
     static constexpr int DS_OFF = GS_OFF + TILE * GP * 2;
     static constexpr int WL_OFF = (DS_OFF + TILE * DP * 2 + 15) / 16 * 16;
     static constexpr int TILE_BYTES = WL_OFF + MTI * KSO * 64 * 16;
-    static constexpr int SPLIT_BYTES = KSPL > 1 ? KSPL * CIN * COUT * 4 : 0;  // the sums of the split, after the last tile
+    static constexpr int SPLIT_BYTES = KSPL > 1 ? KSPL * CIN * COUT * 8 : 0;  // the sums of the split, after the last tile
     static constexpr int LDS_BYTES = TILE_BYTES > SPLIT_BYTES ? TILE_BYTES : SPLIT_BYTES;
     static_assert(CIN % 16 == 0 && CIN <= 128 && COUT % 16 == 0 && COUT <= 128, "channels in {16,32,64,128}");
     static_assert(NBW % kLbWaves == 0 || kLbWaves % NBW == 0, "blocks divide over the wavefronts");
     static_assert(KSV % KSPL == 0, "voxel steps divide over the split");
+    static_assert(LDS_BYTES >= kLbWaves * 2 * CIN * 8, "the sums of scale and shift fit the tiles' LDS");
+};
+
+// eight fp16 values (a float) with flipped signs where `signs` (0x80008000 or 0) says so
+__device__ __forceinline__ half8_t flip_signs(const half8_t& h, uint32_t signs)
+{
+    return __builtin_bit_cast(half8_t, __builtin_bit_cast(u32x4_t, h) ^ signs);
+}
+
+__device__ __forceinline__ float flip_sign(float f, uint32_t signs)
+{
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, f) ^ (signs & 0x80000000u));
+}
+
+// Sums over a wavefront's tiles of 2 x 8 values per lane, lane l holding the channels 8 (l % CGI) + 0..7.  A tile's values
+// of the four lanes l % 16 + {0, 16, 32, 48} are added in fp32 by two rounds of lane swaps that also deal the 16 sums out
+// to these lanes, four each; the tiles are added in fp64.  8 registers per lane where fp32 sums of all values take 16, and
+// no chain over the tiles (at 128 channels and 0.9 M voxels: relative error of dscale 140e-9 with the chain).
+template <int CGI>
+struct ChannelSums {
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    static __device__ __forceinline__ float swap32_add(float a, float b)  // lanes below 32: sum of a, the others: of b
+    {
+        const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                        false, false);
+        return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    }
+    static __device__ __forceinline__ float swap16_add(float a, float b)  // even rows of 16 lanes: sum of a, odd ones: of b
+    {
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                        false, false);
+        return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    }
+    __device__ __forceinline__ void add(const float (&v)[2][8])
+    {
+        float w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = swap32_add(v[0][k], v[1][k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum[k] += (double)swap16_add(w[k], w[k + 4]);
+    }
+    __device__ __forceinline__ void store(double* dst)  // dst[2][8 CGI]
+    {
+        const int lane = threadIdx.x % kWave, row = lane / 16;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+            for (int off = 8; off >= CGI; off >>= 1) sum[k] += __shfl_xor(sum[k], off, 64);
+            if (lane % 16 < CGI) dst[(row / 2) * 8 * CGI + (lane % CGI) * 8 + 4 * (row % 2) + k] = sum[k];
+        }
+    }
 };
 
 // AFFINE: the op's input is z = fp16(max(fma(x, scale[c], shift[c]), 0)), formed from the loaded x on its way to LDS, and
@@ -98,30 +159,42 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
     const int il = lane % 32, hl = lane / 32;
     const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
+    const uint32_t signs = blockIdx.x % 2 ? 0x80008000u : 0u;
+
     // A fragments of the dx product: wl[(mt*KSO + s)*64 + lane] = Wm[32 mt + il][16 s + 8 hl + 0..7]
     for (int i = t; i < Cfg::MTI * KSO * 64; i += kLbThreads) {
         const int l = i % 64, s = (i / 64) % KSO, mt = i / (64 * KSO);
         const int ci = 32 * mt + l % 32;
-        wl[i] = ci < CIN ? load_c8(Wm + ci * COUT + 16 * s + 8 * (l / 32)) : z8;
+        wl[i] = ci < CIN ? flip_signs(load_c8(Wm + ci * COUT + 16 * s + 8 * (l / 32)), signs) : z8;
     }
 
     // this wavefront's dW blocks (mi, ni) and its share of the voxel steps
     const int wb0 = Cfg::NBW >= kLbWaves ? wave : wave % Cfg::NBW;
     const int kpart = Cfg::NBW >= kLbWaves ? 0 : wave / Cfg::NBW;
-    float16_t wacc[BPW];
+    float16_t wacc[BPW][Cfg::NSET];
 #pragma unroll
     for (int bb = 0; bb < BPW; ++bb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) wacc[bb][i] = 0.0f;
+        for (int n = 0; n < Cfg::NSET; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) wacc[bb][n][i] = 0.0f;
+    int ndone = 0;  // tiles of this workgroup
 
-    float sc[AFFINE ? 8 : 1], sh[AFFINE ? 8 : 1], aacc[AFFINE ? 2 : 1][AFFINE ? 8 : 1];  // aacc: dscale, dshift
+    // dscale and dshift: this thread's values of FLUSH tiles (a chain of 8, 4 at 128 channels), and all of them
+    constexpr int FLUSH = (CIN == 128 ? 4 : 8) / NLX;
+    float sc[AFFINE ? 8 : 1], sh[AFFINE ? 8 : 1], aacc[2][8];
+    ChannelSums<CGI> asum;
+    auto clear_affine = [&]() {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) aacc[0][k] = aacc[1][k] = 0.0f;
+    };
     if constexpr (AFFINE) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             sc[j] = scale[(t % CGI) * 8 + j];
             sh[j] = shift[(t % CGI) * 8 + j];
-            aacc[0][j] = aacc[1][j] = 0.0f;
         }
+        clear_affine();
     }
 
     const int64_t ntiles = (V + Cfg::TILE - 1) / Cfg::TILE;
@@ -164,13 +237,14 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
 #pragma unroll
         for (int j = 0; j < NLG; ++j) {
             const int c = t + j * kLbThreads;
-            if (c < Cfg::NGC) *reinterpret_cast<half8_t*>(gs + GT::chunk16(c / (COUT / 8), c % (COUT / 8))) = gpre[j];
+            if (c < Cfg::NGC)
+                *reinterpret_cast<half8_t*>(gs + GT::chunk16(c / (COUT / 8), c % (COUT / 8))) = flip_signs(gpre[j], signs);
         }
         __syncthreads();
         if (tile + gridDim.x < ntiles) prefetch(tile + gridDim.x);
 
         // ---- dx^T blocks: (vt, mt) = 32 voxels x 32 input channels ----
-#pragma unroll
+#pragma unroll (Cfg::TILE_CHAIN && AFFINE ? 1 : 8)  // (128 -> 128: unrolled, it spills registers)
         for (int bd = 0; bd < (Cfg::NBD + kLbWaves - 1) / kLbWaves; ++bd) {
             const int blk = wave + bd * kLbWaves;
             if (blk < Cfg::NBD) {  // wavefront-uniform
@@ -200,6 +274,15 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
         }
 
         // ---- dW blocks: A = relu(x)^T (channel il of 8 consecutive voxels), B = g likewise ----
+        float16_t chain;  // TILE_CHAIN: the tile's sum of the block before, added behind the next block's instructions
+        auto add_chain = [&](int bb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                wacc[bb][0][i] += chain[i];
+                // (added here: left alone, the compiler keeps the chains of all blocks and adds them at the tile's end)
+                asm volatile("" : "+v"(wacc[bb][0][i]));
+            }
+        };
 #pragma unroll
         for (int bb = 0; bb < BPW; ++bb) {
             const int blk = wb0 + bb * kLbWaves;
@@ -207,17 +290,34 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
             int xoff[2], goff[2];  // transposing reads: lane = channel 32 mi + il / 32 ni + il, registers = 8 voxels
             XT::tr_offsets(lane, mi, xoff);
             GT::tr_offsets(lane, ni, goff);
-#pragma unroll
-            for (int sp = 0; sp < KSV / KSPL; ++sp) {
+            auto step = [&](int sp, float16_t c) {
                 const int s = kpart + sp * KSPL;
                 const half8_t af = __builtin_elementwise_max(XT::read_tr(xs, xoff, s), z8);  // relu(x), packed
-                const half8_t bf = GT::read_tr(gs, goff, s);
-                wacc[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf, wacc[bb], 0, 0, 0);
+                return __builtin_amdgcn_mfma_f32_32x32x16_f16(af, GT::read_tr(gs, goff, s), c, 0, 0, 0);
+            };
+            if constexpr (Cfg::TILE_CHAIN) {  // (AFFINE has no registers for a second chain)
+                float16_t next;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) next[i] = 0.0f;
+#pragma unroll
+                for (int sp = 0; sp < Cfg::STEPS; ++sp) next = step(sp, next);
+                if (!AFFINE && bb > 0) add_chain(bb - 1);
+                chain = next;
+                if constexpr (AFFINE) add_chain(bb);
+            } else if constexpr (Cfg::STEPS == 1) {
+                if (ndone % 2) wacc[bb][1] = step(0, wacc[bb][1]);
+                else wacc[bb][0] = step(0, wacc[bb][0]);
+            } else {
+#pragma unroll
+                for (int sp = 0; sp < Cfg::STEPS; ++sp) wacc[bb][sp % Cfg::NSET] = step(sp, wacc[bb][sp % Cfg::NSET]);
             }
         }
+        if constexpr (Cfg::TILE_CHAIN && !AFFINE) add_chain(BPW - 1);
+        ++ndone;
         __syncthreads();
 
         // ---- dx write-back: 16-byte chunks, masked by x > 0 ----
+        if constexpr (AFFINE && FLUSH == 1) clear_affine();
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kLbThreads;
@@ -240,13 +340,19 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
                 store_c8_nt(dx + (v0 + row) * CIN + cc * 8, o);
             }
         }
+        if constexpr (AFFINE) {
+            if (ndone % FLUSH == 0) {
+                asum.add(aacc);
+                if constexpr (FLUSH > 1) clear_affine();
+            }
+        }
         __syncthreads();
     }
 
     // ---- partial dW of this workgroup: row blockIdx of the workspace, [CIN][COUT] fp32 (AFFINE: and [2][CIN]) ----
     // Wavefronts that split the voxels add their sums in LDS first (the tiles are done: the loop ends in a barrier).
     float* out = ws + (int64_t)blockIdx.x * ROW;
-    float* part = KSPL > 1 ? reinterpret_cast<float*>(smem) + kpart * (CIN * COUT) : out;
+    double* part = reinterpret_cast<double*>(smem) + kpart * (CIN * COUT);
 #pragma unroll
     for (int bb = 0; bb < BPW; ++bb) {
         const int blk = wb0 + bb * kLbWaves;
@@ -255,22 +361,39 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int ci = 32 * mi + 8 * (i / 4) + 4 * hl + i % 4;
-            if (ci < CIN && co < COUT) part[ci * COUT + co] = wacc[bb][i];
+            if (ci >= CIN || co >= COUT) continue;
+            if constexpr (KSPL > 1) {
+                double sum = wacc[bb][0][i];
+#pragma unroll
+                for (int n = 1; n < Cfg::NSET; ++n) sum += (double)wacc[bb][n][i];
+                part[ci * COUT + co] = sum;
+            } else {
+                out[ci * COUT + co] = flip_sign(Cfg::NSET > 1 ? wacc[bb][0][i] + wacc[bb][Cfg::NSET - 1][i] : wacc[bb][0][i], signs);
+            }
         }
     }
     if constexpr (KSPL > 1) {
         __syncthreads();
-        const float* all = reinterpret_cast<const float*>(smem);
+        const double* all = reinterpret_cast<const double*>(smem);
         for (int j = t; j < CIN * COUT; j += kLbThreads) {
-            float sum = all[j];
+            double sum = all[j];
 #pragma unroll
             for (int k = 1; k < KSPL; ++k) sum += all[k * (CIN * COUT) + j];
-            out[j] = sum;
+            out[j] = flip_sign((float)sum, signs);
         }
     }
     if constexpr (AFFINE) {
         if constexpr (KSPL > 1) __syncthreads();  // the LDS sums have been read
-        block_channel_partials<2, 8>(aacc, CGI, reinterpret_cast<float*>(smem), out + CIN * COUT);
+        double* red = reinterpret_cast<double*>(smem);
+        if constexpr (FLUSH > 1) asum.add(aacc);
+        asum.store(red + wave * 2 * CIN);
+        __syncthreads();
+        if (t < 2 * CIN) {
+            double sum = 0.0;
+#pragma unroll
+            for (int wv = 0; wv < kLbWaves; ++wv) sum += red[wv * 2 * CIN + t];
+            out[CIN * COUT + t] = (float)sum;
+        }
     }
 }
 

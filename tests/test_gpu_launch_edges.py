@@ -42,7 +42,70 @@ def test_relu_linear_backward_tile_edges(cin, cout, v):
     assert ((dw.cpu().double() - ref_dw).norm() / ref_dw.norm()).item() < 257 * 2.0 ** -24
 
 
-# (131109 voxels: more than two tiles for some workgroups of every channel pair, a ragged last tile)
+# (input channels, output channels) -> voxels of a tile, workgroups from half a million voxels on, matrix instructions that
+# one accumulator of the weight gradient takes per tile
+LINEAR_TILES = {(16, 16): (128, 768, 1), (16, 32): (128, 512, 1), (32, 16): (128, 512, 1), (32, 32): (64, 768, 0.5),
+                (16, 64): (128, 512, 2), (64, 16): (64, 512, 1), (32, 64): (64, 512, 1), (64, 64): (64, 512, 2),
+                (16, 128): (64, 768, 2), (64, 128): (64, 512, 2), (128, 128): (64, 512, 4)}
+
+
+@pytest.mark.parametrize('cin,cout', LINEAR_TILES)
+def test_relu_linear_backward_many_tiles(cin, cout):
+    # every workgroup runs two tiles, some a third, ragged one
+    tile, workgroups, _ = LINEAR_TILES[cin, cout]
+    v = 2 * workgroups * tile + 3 * tile // 2 + 5
+    g = cpu_gen(cin + 3 * cout)
+    x, grad, w = flat(g, v, cin), flat(g, v, cout), matrix(g, cin, cout)
+    dx, dw = ReLULinearBackward(x.to(DEV), grad.to(DEV), w.to(DEV), out_dtype=torch.float32)
+    ref_dx, ref_dw = oracle.relu_linear_bwd(x, grad, w)
+    # fp32 sums of at most 128 products against fp64, then one rounding to fp16
+    assert (dx.cpu().float() - ref_dx.float()).abs().max() <= 2.0 ** -9 * max(1.0, ref_dx.abs().max().item())
+    # one voxel too many, missing or counted twice shifts dw by about 1 / sqrt(v), 4e-3 and more
+    assert ((dw.cpu().double() - ref_dw).norm() / ref_dw.norm()).item() < 2.0 ** -20
+
+
+# A rounding to fp32 leaves 0.42 * 2^-24 of its value (rms over the values of a binade).  Inputs ~ N(0, 1): a running sum of
+# n equal parts that is rounded r times a part ends with a relative error of 0.42 * 2^-24 * sqrt(r (n + 1) / 2).
+@pytest.mark.parametrize('cin,cout', LINEAR_TILES)
+def test_weight_gradient_error_of_large_volumes(cin, cout):
+    v = 900037
+    tile, workgroups, per_tile = LINEAR_TILES[cin, cout]
+    gen = torch.Generator(DEV).manual_seed(cin + cout)
+    x = torch.randn(v, cin, device=DEV, generator=gen).half()
+    grad = torch.randn(v, cout, device=DEV, generator=gen).half()
+    w = matrix(cpu_gen(), cin, cout).to(DEV)
+    _, dw = ReLULinearBackward(x.view(1, v, 1, 1, cin).permute(0, 4, 1, 2, 3), grad.view(1, v, 1, 1, cout).permute(0, 4, 1, 2, 3),
+                               w, out_dtype=torch.float32)
+    ref = torch.relu(x).double().t().contiguous() @ grad.double()
+    error = ((dw.double() - ref).norm() / ref.norm()).item()
+    tiles = v / tile / workgroups
+    if (cin, cout) == (128, 128):  # a chain of four instructions per tile, one addition per tile
+        parts = 2 * (4 + 1) / 2 + (tiles + 1) / 2
+    else:                          # chains over the tiles, each rounded twice per instruction
+        parts = 2 * (tiles * per_tile + 1) / 2
+    parts += 2                     # the row of the workgroup, the result
+    # a fifth above the expectation: the scatter over the results (256 of them at 16 -> 16), the downward part of the roundings
+    assert error < 1.2 * 0.42 * 2.0 ** -24 * parts ** 0.5, (error, parts)
+
+
+@pytest.mark.parametrize('cin,cout', [(16, 16), (64, 64), (128, 32), (128, 128)])
+def test_scale_and_shift_gradient_error_of_large_volumes(cin, cout):
+    v = 900037
+    gen = torch.Generator(DEV).manual_seed(cin - cout)
+    x = torch.randn(v, cin, device=DEV, generator=gen).half().view(1, v, 1, 1, cin).permute(0, 4, 1, 2, 3)
+    grad = torch.randn(v, cout, device=DEV, generator=gen).half().view(1, v, 1, 1, cout).permute(0, 4, 1, 2, 3)
+    w = matrix(cpu_gen(), cin, cout).to(DEV)
+    scale, shift = torch.rand(cin, device=DEV, generator=gen) + 0.5, torch.randn(cin, device=DEV, generator=gen) * 0.3
+    gz, _ = ReLULinearBackward(ApplyBNReLU(x, scale, shift), grad, w)
+    _, dscale, _, _ = ApplyBNReLULinearBackward(x, scale, shift, grad, w)
+    xl, gl = (t.permute(0, 2, 3, 4, 1).reshape(v, cin) for t in (x, gz))
+    ref = (xl.double() * gl.double() * (xl.float() * scale > -shift)).sum(0)
+    # chains of at most 8 values, two additions of lanes, the row, the result; 16 results: a factor of 1.5 for their scatter
+    parts = (8 + 1) / 2 + 2 + 2
+    assert ((dscale.double() - ref).norm() / ref.norm()).item() < 1.5 * 0.42 * 2.0 ** -24 * parts ** 0.5
+
+
+# (131109 voxels: a second tile for some workgroups of every channel pair, a ragged last tile)
 @pytest.mark.parametrize('cin,cout', CHANNELS)
 @pytest.mark.parametrize('v', [1, 63, 65, 127, 129, 257, 131109])
 def test_bnrelu_linear_backward_equals_its_parts(cin, cout, v):
