@@ -315,7 +315,12 @@ struct MarchSplit {
     BalancedSplit b;
     int h_chunk;
 };
-static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int setup, int slab_mult, int xcds)
+// one_row: most workgroups that may march over a single row, which reads three planes for one.  Alone on a compute unit
+// such a workgroup is still the faster one ((1,32,33,19,25), 198 of them: forward 6.26 us, 6.60 with two rows each); two
+// of them on a compute unit lose in the forward and weight-gradient kernels ((2,32,32,9,35), 384: forward 8.20 us, 6.81
+// with two rows each, weight gradient 12.2 and 10.9) and not in the fused backward (15.0 and 15.8).
+static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int setup, int slab_mult, int xcds,
+                                    int one_row)
 {
     double cost;
     const BalancedSplit whole = best_balanced(
@@ -333,11 +338,12 @@ static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots
                    (1.0 + 0.004 * (double)H / (double)share) * spread;
         },
         &cost);
-    // chunks that run in one round (never more workgroups, and partial sums, than the balanced split has)
+    // chunks that run in one round (never more workgroups, and partial sums, than fit the GPU at once)
     int best_h = 0;
     for (int c = 1; c <= 64 && c <= H && tiles * c <= slots; ++c) {
         const int h = ceil_div(H, c);
         if (ceil_div(H, h) != c) continue;  // the same split as a smaller c
+        if (h < 2 && c > 1 && tiles * c > one_row) break;
         const double uniform = ((double)h + 2 + setup) * (1.0 + 0.004 * c);
         if (uniform <= cost) {
             cost = uniform;

@@ -937,7 +937,8 @@ static int plan_fwd_mfma(FwdArgs& a, int N, int h_chunk, bool balanced_ok = fals
         const int64_t tiles = (int64_t)N * a.n_wt * a.n_dt * a.n_slab;
         const MarchSplit split =
             h_chunk < 0 ? MarchSplit{make_balanced(a.H, tiles, slots, -h_chunk), 0}
-                        : pick_split(a.H, tiles, a.n_dt * a.n_slab, slots, 6, per_slab_state ? a.n_slab : 1, geo.xcds);
+                        : pick_split(a.H, tiles, a.n_dt * a.n_slab, slots, 6, per_slab_state ? a.n_slab : 1, geo.xcds,
+                                     geo.cus);
         const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && tiles + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {

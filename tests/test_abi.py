@@ -255,3 +255,21 @@ def test_linear_backward_takes_a_third_workgroup_in_large_volumes():
     # the widest pair holds two workgroups in LDS
     assert (lib.kerops_relu_linear_bwd_workspace_bytes(4000000, 128, 128)
             == lib.kerops_relu_linear_bwd_workspace_bytes(200000, 128, 128) == 512 * 128 * 128 * 4)
+
+
+def test_built_in_split_gives_two_rows_where_workgroups_share_a_compute_unit():
+    # a workgroup that marches over one row of H reads three planes for it: only where each has a compute unit of its own
+    # (the fused backward, which keeps one row per workgroup up to all slots, is the faster for it)
+    lib = _lib.load()
+
+    def partials(name, n, c, h, w, d, rows):
+        wgrad = name == 'kerops_dwconv_wgrad_workspace_bytes'
+        return getattr(lib, name)(n, h, w, d, c, *((0, 0, rows, 0) if wgrad else (rows,))) // (27 * min(c, 64) * 4)
+
+    wgrad, fused = 'kerops_dwconv_wgrad_workspace_bytes', 'kerops_dwconv_bwd_workspace_bytes'
+    for shape in ((2, 32, 32, 9, 35), (2, 128, 10, 36, 11), (1, 16, 30, 57, 33), (1, 16, 26, 44, 43), (1, 32, 44, 32, 28)):
+        assert partials(wgrad, *shape, 1) > 256
+        assert 0 < partials(wgrad, *shape, 0) <= partials(wgrad, *shape, 2), shape
+        assert partials(fused, *shape, 0) == partials(fused, *shape, 1) <= 512, shape
+    for shape in ((1, 32, 33, 19, 25), (1, 64, 21, 11, 30), (4, 32, 12, 13, 15), (1, 32, 1, 64, 64)):
+        assert partials(wgrad, *shape, 0) == partials(wgrad, *shape, 1) <= 256, shape
