@@ -70,7 +70,7 @@ extern "C" int kerops_dwsep_block_f16(const void* x, const void* wt, const float
     int rc = dwconv_fwd_run(x, wt, t, scale, shift, N, H, W, D, Cin, 8, 8, 0, 16, stream);
     if (rc != KEROPS_OK) return rc;
     const int blocks = pointwise_blocks(V);
-    rc = pointwise_dispatch(t, (const half_t*)Wm, nullptr, (half_t*)y, amax_ws, V, Cin, Cout, false, true, blocks,
+    rc = pointwise_dispatch(t, (const half_t*)Wm, nullptr, (half_t*)y, amax_ws, V, Cin, Cout, false, true,
                             (hipStream_t)stream);
     if (rc != KEROPS_OK) return rc;
     launch_pw_absmax_final(amax_ws, blocks, absmax, (hipStream_t)stream);

@@ -32,15 +32,22 @@ struct PwCfg {
     static constexpr int OUT_CHUNKS = 32 * COUT / 8; // 16-byte chunks of one output tile
     static_assert(CIN % 16 == 0 && CIN <= 128, "CIN in {16,32,64,128}");
     static_assert(COUT % 16 == 0 && COUT <= 128, "COUT in {16,32,64,128}");
-    // Workgroups per compute unit of the persistent loop: as few as keep the memory pipe full.  Two have 32 KB and more
-    // of x and residual in flight from 64 channels (CIN + COUT) on; narrower tiles take three.  (us at 64 M elements of
-    // x and residual together with 2 / 3 / 4 / 8 workgroups: 16 -> 16 39.4 / 34.1 / 34.5 / 36.0, 32 -> 32 34.7 / 35.7 /
-    // 35.9 / 37.6, 64 -> 128 40.0 / 41.5 / 41.5 / 41.5.  More than fit the LDS, as four at 64 -> 128, also leave a
-    // second round that fills a part of the chip.)
-    static constexpr int PER_CU = CIN + COUT >= 64 ? 2 : 3;
-    // Without a residual a tile has half the bytes: four, where their LDS fits.
+    // Workgroups per compute unit of the persistent loop: as few as keep the memory pipe full, which also have the fewest
+    // prologues.  With a residual three up to 64 channels (CIN + COUT), whose tiles have the fewest bytes in flight, two
+    // above (us with 2 / 3 / 4 / 8: 16 -> 16 at 2.1 M voxels 39.4 / 34.1 / 34.5 / 36.0, 32 -> 32 at 0.9 M 31.1 / 30.4 /
+    // 31.1, 16 -> 64 at 0.9 M 43.6 / 44.7 / 44.8, 64 -> 128 at 0.35 M 40.0 / 41.5 / 41.5 / 41.5; more than fit the LDS,
+    // as four at 64 -> 128, also leave a second round that fills a part of the chip).  Widening from few channels three
+    // again in volumes above 3 M voxels (16 -> 64 at 15.7 M 814 / 763 / 767, 32 -> 64 888 / 858 / 843).
+    // Without a residual a tile has half the bytes: four, where their LDS fits (64 -> 128, 0.1 M voxels 16.1 with four,
+    // 13.2 with the three that fit, 4 M 284 and 285; 128 -> 128 24.3 with four, 18.6 with the two that fit, 4 M 387 and 391).
     static constexpr int LDS_BYTES = kPwWaves * TILE_HALVES * 2 + MT * KS * 64 * 16 + 2 * CIN * 4 + 64;
-    static constexpr int PER_CU_NO_ADD = 160 * 1024 / LDS_BYTES < 4 ? 160 * 1024 / LDS_BYTES : 4;
+    static constexpr int FITS = 160 * 1024 / LDS_BYTES;
+    static int64_t workgroups(int64_t V, bool add)
+    {
+        const bool three = CIN + COUT <= 64 || (CIN < COUT && CIN + COUT < 128 && V > 3 << 20);
+        const int per_cu = add ? (three ? 3 : 2) : (FITS < 4 ? FITS : 4);
+        return std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kPwWaves), (int64_t)per_cu * device_geometry().cus));
+    }
 };
 
 // AFFINE: x is first mapped to fp16(max(fma(x, scale[c], shift[c]), 0)), the arithmetic of the batch-norm + ReLU
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(256) void pw_absmax_final_kernel(const float* __res
     if (threadIdx.x == 0) out[0] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-static int pw_blocks(int64_t V)
+int pointwise_blocks(int64_t V)
 {
     const int64_t ntiles = (V + 31) / 32;
     int64_t b = (ntiles + kPwWaves - 1) / kPwWaves;
@@ -239,17 +246,13 @@ static int pw_blocks(int64_t V)
 
 template <int CIN, int COUT>
 static int launch_pw(const half_t* x, const half_t* Wm, const half_t* add, half_t* out, float* amax_ws, int64_t V,
-                     bool relu_in, bool absmax, int blocks, hipStream_t s, const float* scale = nullptr,
-                     const float* shift = nullptr)
+                     bool relu_in, bool absmax, hipStream_t s, const float* scale, const float* shift)
 {
     if (absmax && (add || scale)) {  // no instantiation keeps the running max next to a residual or the affine map
         set_error("pointwise: the running max is built without residual add and without the affine map");
         return KEROPS_E_BADARG;
     }
-    using Cfg = PwCfg<CIN, COUT>;
-    if (!absmax)
-        blocks = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kPwWaves),
-                                                             (int64_t)(add ? Cfg::PER_CU : Cfg::PER_CU_NO_ADD) * device_geometry().cus));
+    const int blocks = absmax ? pointwise_blocks(V) : (int)PwCfg<CIN, COUT>::workgroups(V, add != nullptr);
     if (scale) {  // the affine map ends in a ReLU of its own
         if (add) {
             hipLaunchKernelGGL((pointwise_kernel<CIN, COUT, false, true, false, true>), dim3(blocks), dim3(kPwThreads), 0,
@@ -278,12 +281,11 @@ static int launch_pw(const half_t* x, const half_t* Wm, const half_t* add, half_
 }
 
 int pointwise_dispatch(const half_t* x, const half_t* Wm, const half_t* add, half_t* out, float* amax_ws, int64_t V,
-                       int Cin, int Cout, bool relu_in, bool absmax, int blocks, hipStream_t s, const float* scale,
-                       const float* shift)
+                       int Cin, int Cout, bool relu_in, bool absmax, hipStream_t s, const float* scale, const float* shift)
 {
 #define KEROPS_PW_CASE(CI, CO)      \
     if (Cin == CI && Cout == CO)    \
-        return launch_pw<CI, CO>(x, Wm, add, out, amax_ws, V, relu_in, absmax, blocks, s, scale, shift);
+        return launch_pw<CI, CO>(x, Wm, add, out, amax_ws, V, relu_in, absmax, s, scale, shift);
     KEROPS_PW_CASE(16, 16)
     KEROPS_PW_CASE(16, 32)
     KEROPS_PW_CASE(32, 16)
@@ -304,8 +306,6 @@ int pointwise_dispatch(const half_t* x, const half_t* Wm, const half_t* add, hal
     set_error("pointwise: no kernel built for Cin=%d Cout=%d (both in {16,32,64,128})", Cin, Cout);
     return KEROPS_E_UNSUPPORTED_C;
 }
-
-int pointwise_blocks(int64_t V) { return pw_blocks(V); }
 
 void launch_pw_absmax_final(const float* ws, int n, float* out, hipStream_t s)
 {
@@ -328,7 +328,7 @@ extern "C" int kerops_pointwise_f16(const void* x, const void* Wm, const void* a
         return KEROPS_E_BADARG;
     }
     return pointwise_dispatch((const half_t*)x, (const half_t*)Wm, (const half_t*)add, (half_t*)out, nullptr, V, Cin,
-                              Cout, relu_in != 0, false, pw_blocks(V), (hipStream_t)stream);
+                              Cout, relu_in != 0, false, (hipStream_t)stream);
 }
 
 extern "C" int kerops_bnrelu_pointwise_f16(const void* x, const float* scale, const float* shift, const void* Wm,
@@ -345,5 +345,5 @@ extern "C" int kerops_bnrelu_pointwise_f16(const void* x, const float* scale, co
         return KEROPS_E_BADARG;
     }
     return pointwise_dispatch((const half_t*)x, (const half_t*)Wm, (const half_t*)add, (half_t*)out, nullptr, V, Cin,
-                              Cout, false, false, pw_blocks(V), (hipStream_t)stream, scale, shift);
+                              Cout, false, false, (hipStream_t)stream, scale, shift);
 }
