@@ -38,7 +38,7 @@ struct MlpCfg {
     static_assert(C == 16 || C == 32 || C == 64, "C in {16,32,64}");
 };
 
-template <int C>
+template <int C, bool EARLY>
 __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const half_t* __restrict__ x,
                                                                         const half_t* __restrict__ Wup,
                                                                         const half_t* __restrict__ Wdown,
@@ -81,12 +81,9 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     const int64_t tiles_per_round = (int64_t)gridDim.x * kMlpWaves;
     const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
     // Loads of a tile (one past the end reads the last voxel and is never used): x fragments, and residual chunks in the
-    // order in which the results leave the LDS tile.  Those of the next tile are issued as soon as this tile has used
+    // order in which the results leave the LDS tile.  EARLY: those of the next tile are issued as soon as this tile has used
     // the registers, so that both streams are in flight while the results are stored; loaded where they are used, a
-    // tile waits for memory twice (C = 64 at 1.96 M voxels 184 us, now 134; C = 16 at 2.1 M 37.1 and 35.4).
-    // At C = 32 four workgroups per compute unit hide the second wait as well, and there a block's forward and backward
-    // pass at 1.96 M voxels take 154 us against 156 with the early loads: each load stays where it is used.
-    constexpr bool EARLY = C != 32;
+    // tile waits for memory twice (mlp_early has the figures).
     constexpr int NC = 32 * C / 8 / kWave;
     half8_t xb[KS1], ab[NC];
     auto load_x = [&](int64_t tidx) {
@@ -178,11 +175,17 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     }
 }
 
-// Workgroups per compute unit (us with 2 / 3 / 4 / 5: C = 16 at 2.1 M voxels 41.3 / 35.7 / 35.4 / 35.4, C = 32 at 1.96 M
-// 89 / 71 / 67.3 / 67.2, C = 64 at 1.96 M 134 / 140 / 145 / 141)
+// Early loads (us with them and the best workgroup count / with late loads and four workgroups per compute unit): C = 16 at
+// 4096 voxels 3.1 / 3.2, 1 M 18.8 / 20.0, 15.7 M 252 / 265; C = 64 at 0.1 M 18.0 / 28.2, 15.7 M 1079 / 1381; C = 32 at
+// 4096 4.6 / 4.8, 0.1 M 7.9 / 9.0, 0.4 M 18.2 / 19.3, 1 M 37.4 / 38.2, 2 M 69.1 / 69.3, 2.5 M 86.8 / 87.0, 3 M 103.1 /
+// 101.9, 4 M 137.3 / 135.2, 15.7 M 534 to 552 / 528 to 533: there four workgroups hide the second wait as well, and volumes
+// above 2.6 M voxels load late.
+static bool mlp_early(int64_t V, int C) { return C != 32 || V <= 5 << 19; }
+// Workgroups per compute unit with early loads (us with 2 / 3 / 4: C = 16 at 2.0 M voxels 39.6 / 34.2 / 33.5, C = 32 at
+// 0.1 M 8.2 / 8.3 / 9.2 and at 2.0 M 71.3 / 68.5 / 70.2, C = 64 at 2.0 M 142 / 148 / 156)
 static int mlp_blocks(int64_t V, int C)
 {
-    const int64_t per_cu = C == 64 ? 2 : 4;
+    const int64_t per_cu = C == 64 ? 2 : C == 32 && mlp_early(V, C) ? 3 : 4;
     return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kMlpWaves), per_cu * device_geometry().cus));
 }
 
@@ -203,16 +206,17 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
     }
     const int blocks = mlp_blocks(V, C);
     hipStream_t s = (hipStream_t)stream;
-#define KEROPS_MLP_CASE(CV)                                                                                      \
-    if (C == CV) {                                                                                               \
-        hipLaunchKernelGGL((lin_brelu_lin_add_kernel<CV>), dim3(blocks), dim3(kMlpThreads), 0, s,               \
-                           (const half_t*)x, (const half_t*)Wup, (const half_t*)Wdown, (const half_t*)bias,     \
-                           (const half_t*)add, (half_t*)out, V);                                                \
-        return check_launch("lin_brelu_lin_add");                                                                \
+#define KEROPS_MLP_CASE(CV, EARLY)                                                                                      \
+    if (C == CV && mlp_early(V, C) == EARLY) {                                                                          \
+        hipLaunchKernelGGL((lin_brelu_lin_add_kernel<CV, EARLY>), dim3(blocks), dim3(kMlpThreads), 0, s, (const half_t*)x, \
+                           (const half_t*)Wup, (const half_t*)Wdown, (const half_t*)bias, (const half_t*)add,            \
+                           (half_t*)out, V);                                                                             \
+        return check_launch("lin_brelu_lin_add");                                                                       \
     }
-    KEROPS_MLP_CASE(16)
-    KEROPS_MLP_CASE(32)
-    KEROPS_MLP_CASE(64)
+    KEROPS_MLP_CASE(16, true)
+    KEROPS_MLP_CASE(32, true)
+    KEROPS_MLP_CASE(32, false)
+    KEROPS_MLP_CASE(64, true)
 #undef KEROPS_MLP_CASE
     set_error("lin_brelu_lin_add: built for C in {16,32,64} (got %d)", C);
     return KEROPS_E_UNSUPPORTED_C;

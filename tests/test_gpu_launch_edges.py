@@ -211,3 +211,19 @@ def test_inverted_bottleneck_tiles_and_rounds(c, v):
         # a rounding of it), and a hidden value by one rounding
         err = ((a.cpu().double() - b.double()).norm() / max(b.double().norm().item(), 1e-30)).item()
         assert err < 2.0 ** -5 if v < 1000 else err < 2.0 ** -8, err
+
+
+def test_inverted_bottleneck_is_the_same_with_early_and_late_loads():
+    # 32 channels load late above 2.6 M voxels: every voxel's result is its own, so the parts give the same bits
+    c, v = 32, (5 << 19) + 33
+    gen = torch.Generator(DEV).manual_seed(9)
+    x, add = (torch.randn(1, v, 1, 1, c, device=DEV, generator=gen).half().permute(0, 4, 1, 2, 3) for _ in range(2))
+    g = cpu_gen(9)
+    up, down, bias = (t.to(DEV) for t in (matrix(g, c, 2 * c), matrix(g, 2 * c, c), (torch.randn(2 * c, generator=g) * 0.3).half()))
+    out = LinBReLULinAdd(x, up, down, bias, add)
+    cut = 1 << 20
+    for part in (slice(0, cut), slice(cut, v)):
+        assert torch.equal(bits(out[:, :, part]), bits(LinBReLULinAdd(x[:, :, part], up, down, bias, add[:, :, part])))
+    tail = slice(v - 5000, v)
+    ref = oracle.lin_brelu_lin_add(*(t.cpu() for t in (x[:, :, tail], up, down, bias, add[:, :, tail])))
+    assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
