@@ -612,9 +612,13 @@ __device__ __forceinline__ void st_stream(_Float16* p, int64_t chunk, const type
 // Result stores with or without the hint.  Stores without it stay in the 256 MB memory-side cache: the pass that reads
 // the result next finds it there, and a result that is overwritten soon (a pool of buffers, one call after another) may
 // never reach memory.  That holds while result and reader fit the cache together, so results up to kCachedResultBytes
-// are stored plainly.  A window quantiser and its inverse on 33 M bf16 values (33 MB of bytes, 66 MB back): 37.0 us
-// with the hint, 33.9 without; a 268 MB int8 result: 142 us with, 151 without.
-constexpr int64_t kCachedResultBytes = 128ll << 20;
+// are stored plainly.  us with the hint / plainly, a window quantiser and its inverse: 33 M 16-bit values (31 MiB of bytes,
+// 63 MiB back) 38.5 / 36.0, 48 M 57.7 / 54.0, 64 M (bytes plain; values of 122 MiB hinted / plain) 66.0 / 69.8, 96 M (92 MiB
+// of bytes, values hinted) 103.8 / 96.0, 128 M (122 MiB) 133 / 123; 16 M fp32 values 33.8 / 30.5, 64 M (61 MiB of bytes)
+// 112.5 / 108.8, 96 M (92 MiB) 165 / 162.  A result that nothing reads: 16-bit bytes of 64 / 96 / 128 / 160 MiB 36.3 / 36.3,
+// 51.9 / 53.9, 68.2 / 71.3, 84.5 / 87.8; values of 64 / 96 / 128 / 160 MiB 20.6 / 19.8, 29.2 / 29.9, 35.8 / 39.6, 44.0 / 48.3; a
+// 268 MB int8 result 142 / 151.  Above 96 MiB what is gained with a reader is lost without one.
+constexpr int64_t kCachedResultBytes = 96ll << 20;
 // (The value is passed as a value: through a reference the compiler moves a load of quant_u8_kernel<16-bit type, 8> behind
 // the store of the previous value, one load in flight per wavefront instead of eight, 1.24 ms for 0.48 at 1.0 G values.)
 template <bool STREAM, typename T>

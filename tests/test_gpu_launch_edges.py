@@ -149,8 +149,8 @@ def test_pointwise_residual_tiles_and_rounds(cin, cout, v):
 
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
 def test_quantiser_store_rule(dtype):
-    # results up to 128 MB are stored plainly, larger ones with the streaming hint: the same values on both sides
-    limit = 128 << 20
+    # results up to 96 MiB are stored plainly, larger ones with the streaming hint: the same values on both sides
+    limit = 96 << 20
     back = limit // dtype.itemsize
     gen = torch.Generator(DEV).manual_seed(5)
     for n in (limit, limit + 8):
