@@ -273,3 +273,46 @@ def test_built_in_split_gives_two_rows_where_workgroups_share_a_compute_unit():
         assert partials(fused, *shape, 0) == partials(fused, *shape, 1) <= 512, shape
     for shape in ((1, 32, 33, 19, 25), (1, 64, 21, 11, 30), (4, 32, 12, 13, 15), (1, 32, 1, 64, 64)):
         assert partials(wgrad, *shape, 0) == partials(wgrad, *shape, 1) <= 256, shape
+
+
+def test_bnrelu_linear_backward_entry_point_refuses():
+    lib = _lib.load()
+    buf = (ctypes.c_char * 4096)()
+    at = (ctypes.addressof(buf) + 15) & ~15
+    need = lib.kerops_bnrelu_linear_bwd_workspace_bytes(100, 16, 32)
+    assert need == 1 * (16 * 32 + 2 * 16) * 4  # one workgroup: its weight gradient, its scale and shift sums
+
+    def call(x=at, scale=at, shift=at, g=at, wm=at, dx=at, dw=at, dtype=0, daffine=at, ws=at, nbytes=need, v=100, cin=16,
+             cout=32):
+        return lib.kerops_bnrelu_linear_bwd_f16(x, scale, shift, g, wm, dx, dw, dtype, daffine, ws, nbytes, v, cin, cout, None)
+
+    for bad in (dict(x=None), dict(scale=None), dict(shift=None), dict(g=None), dict(wm=None), dict(dx=None), dict(dw=None),
+                dict(daffine=None), dict(x=at + 8), dict(g=at + 2), dict(wm=at + 8), dict(dx=at + 8), dict(dtype=2),
+                dict(dtype=7), dict(v=0), dict(v=-5)):
+        assert call(**bad) == _lib.KEROPS_E_BADARG, bad
+        assert 'bnrelu_linear_bwd' in _lib.last_error()
+    for bad in (dict(ws=None), dict(ws=at + 4), dict(nbytes=need - 1), dict(nbytes=0), dict(nbytes=-1)):
+        assert call(**bad) == _lib.KEROPS_E_WORKSPACE, bad
+    for cin, cout in ((8, 16), (16, 8), (24, 16), (256, 16), (16, 0), (-16, 16)):
+        assert call(cin=cin, cout=cout) == _lib.KEROPS_E_UNSUPPORTED_C
+        assert lib.kerops_bnrelu_linear_bwd_workspace_bytes(100, cin, cout) == _lib.KEROPS_E_UNSUPPORTED_C
+    assert lib.kerops_bnrelu_linear_bwd_workspace_bytes(0, 16, 16) == _lib.KEROPS_E_BADARG
+
+
+def test_bnrelu_linear_backward_checks_its_tensors():
+    from kerops_amd.ops.linear import ApplyBNReLULinearBackward
+
+    def call(x=cl3d(1, 16, 4, 4, 4), scale=torch.zeros(16), shift=torch.zeros(16), grad=cl3d(1, 32, 4, 4, 4),
+             weight=torch.zeros(16, 32, dtype=torch.float16)):
+        return ApplyBNReLULinearBackward(x, scale, shift, grad, weight)
+
+    for bad in (dict(x=cl3d(1, 16, 4, 4, 4).float()), dict(x=torch.zeros(1, 16, 4, 4, 4, dtype=torch.float16)),
+                dict(grad=cl3d(1, 32, 4, 4, 5)), dict(grad=cl3d(2, 32, 4, 4, 4)), dict(scale=torch.zeros(8)),
+                dict(shift=torch.zeros(32)), dict(weight=torch.zeros(32, 16, dtype=torch.float16)),
+                dict(weight=torch.zeros(16, 32)), dict(grad=torch.zeros(1, 32, 4, 4, 4, dtype=torch.float16)),
+                dict(x=cl3d(1, 8, 4, 4, 4), scale=torch.zeros(8), shift=torch.zeros(8),
+                     weight=torch.zeros(8, 32, dtype=torch.float16))):
+        with pytest.raises(AssertionError):
+            call(**bad)
+    with pytest.raises(RuntimeError, match='no CPU path'):
+        call()

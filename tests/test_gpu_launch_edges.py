@@ -131,6 +131,51 @@ def test_bnrelu_linear_backward_equals_its_parts(cin, cout, v):
         assert (got.cpu().double() - ref).abs().max().item() <= 2.0 ** -15 * size + 1e-30
 
 
+def same_special(a, b):
+    """The same NaNs, infinities of the same sign, and the same values elsewhere (a NaN's own bits are not specified)."""
+    nan = torch.isnan(a)
+    return torch.equal(nan, torch.isnan(b)) and torch.equal(torch.where(nan, 0, a), torch.where(nan, 0, b))
+
+
+# channel pairs of every split of the weight gradient, two workgroups at least
+@pytest.mark.parametrize('cin,cout', [(16, 16), (32, 32), (16, 64), (64, 64), (128, 32), (128, 128)])
+@pytest.mark.parametrize('where', ['x', 'scale', 'shift', 'grad'])
+def test_bnrelu_linear_backward_of_special_values_equals_its_parts(cin, cout, where):
+    v = 700
+    g = cpu_gen(cin + cout)
+    x, grad, w = flat(g, v, cin), flat(g, v, cout), matrix(g, cin, cout).to(DEV)
+    scale, shift = torch.rand(cin, generator=g) + 0.5, torch.randn(cin, generator=g) * 0.3
+    scale[5], shift[6] = -0.75, 0.0
+    inf, nan = float('inf'), float('nan')
+    if where == 'x':  # one per channel, in different workgroups
+        for ch, (row, value) in enumerate([(3, inf), (300, -inf), (690, nan), (4, 65504.0), (301, -65504.0), (5, 6e-8), (6, -0.0)]):
+            x[0, ch, row] = value
+    elif where == 'scale':
+        scale[:5] = torch.tensor([inf, -inf, nan, 3e38, 1e-45])
+    elif where == 'shift':
+        shift[:5] = torch.tensor([inf, -inf, nan, 3e38, -0.0])
+    else:
+        for ch, (row, value) in enumerate([(3, inf), (300, -inf), (690, nan), (4, 65504.0), (301, 6e-8)]):
+            grad[0, ch, row] = value
+    xd, gd, sd, bd = x.to(DEV), grad.to(DEV), scale.to(DEV), shift.to(DEV)
+    z = ApplyBNReLU(xd, sd, bd)
+    gz, dw_ref = ReLULinearBackward(z, gd, w)
+    dx_ref, dscale_ref, dshift_ref = ApplyBNReLUBackward(xd, sd, bd, gz)
+    dx, dscale, dshift, dw = ApplyBNReLULinearBackward(xd, sd, bd, gd, w)
+    assert same_special(dx, dx_ref)
+    for got, ref, size in ((dw, dw_ref, None), (dscale, dscale_ref, xd.float() * gz.float()), (dshift, dshift_ref, gz.float())):
+        got, ref = got.double(), ref.double()
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        usual = torch.isfinite(ref)
+        assert torch.equal(torch.isinf(got), torch.isinf(ref)) and torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
+        # dw: neighbouring fp16 values; the sums: fp32 additions of the summed magnitudes, 2^9 in a row at most
+        if size is None:
+            bound = 2.0 ** -10 * ref.abs() + 2.0 ** -14
+        else:
+            bound = 2.0 ** -15 * size.double().abs().nan_to_num(0.0, 0.0, 0.0).sum((0, 2, 3, 4)) + 1e-30
+        assert ((got - ref).abs() <= bound)[usual].all()
+
+
 # 2 or 3 workgroups of 128 voxels per compute unit: 65536 or 98304 voxels a round
 @pytest.mark.parametrize('cin,cout', CHANNELS)
 @pytest.mark.parametrize('v', [1, 31, 33, 127, 129, 65569, 98400])
