@@ -307,10 +307,10 @@ static inline BalancedSplit best_balanced(int H, int64_t tiles, int row_len, int
 // Where a group's share is a whole column of the volume or more, every group crosses into other bundles and the cost
 // above decides.  Where it is less, the launch lasts as long as the groups that do cross (two halo planes and a pipeline
 // refill, about eight plane steps), and chunks of equal length without any crossing are often faster although they
-// leave workgroup slots empty: the cheaper of the two, with the crossing counted in full, is taken.  Measured over 24
-// shapes of 4 to 400 M elements, C = 8..128, forward / fused backward / weight gradient each, against the balanced
-// split alone: 5.5 % faster on average, between 0.77 and 1.01 of its time ((2,32,96,96,96) forward 55.6 -> 52.7 us,
-// (2,128,45,51,37) backward 47.6 -> 43.4, (1,128,34,71,55) forward 24.2 -> 18.5), 1.3 % behind the best of all splits.
+// leave workgroup slots empty: the cheaper of the two, with the crossing counted in full, is taken.  Measured over 180
+// volumes of 0.26 to 400 M elements, C = 8..128, against the balanced split alone: forward 8.8 % faster on average,
+// weight gradient 4.9, fused backward 6.8, between 0.54 and 1.04 of its time ((2,32,96,96,96) forward 55.6 -> 52.7 us,
+// (2,128,45,51,37) backward 47.6 -> 43.4, (1,128,34,71,55) forward 24.2 -> 18.5).
 struct MarchSplit {
     BalancedSplit b;
     int h_chunk;

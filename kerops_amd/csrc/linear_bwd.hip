@@ -40,7 +40,8 @@ constexpr int kLbWaves = kLbThreads / kWave;
 // 128 voxels and the best workgroup count of each: 16 -> 64 at 0.9 M voxels 36.1 / 34.8, 16 -> 16 at 4 M 74.4 / 66.2
 // (256 voxels: 69.1), 32 -> 32 at 4 M 125.9 / 133.5, 64 -> 16 at 4096 6.1 / 6.7.
 // The AFFINE kernel has the registers of two workgroups on a compute unit and takes the tiles that fill them (16 -> 16 at
-// 4 M voxels 75.4 with 256, 83.1 with 128; 32 -> 32 140.4 with 128, 156.5 with 64 and three workgroups).
+// 4 M voxels 75.4 with 256, 83.1 with 128; 32 -> 32 140.4 with 128, 156.5 with 64 and three workgroups; 77.0 and 140.8 with
+// the sums as they are now).
 constexpr int lb_tile(int cin, int cout, bool affine)
 {
     if (affine) return cin + cout >= 96 ? 64 : cin + cout >= 48 ? 128 : 256;

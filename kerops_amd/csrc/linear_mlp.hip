@@ -245,7 +245,8 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
 // the LDS holds two workgroups per compute unit.  Partials go to the workspace, a second kernel adds them in a fixed order
 // (fp64): deterministic, no atomics.
 // Two workgroups of 256 registers per lane; with operands read from LDS in 2-byte pieces and the weights in LDS, one
-// workgroup per compute unit, the kernel took 705 us at 1.96 M voxels, now 247 (its HBM traffic at 6 TB/s: 125 us).
+// workgroup per compute unit, the op with its reduction took 721 us at 1.96 M voxels, now 267 (its HBM traffic at 6 TB/s:
+// 125 us).
 namespace kerops {
 
 struct MbCfg {

@@ -99,7 +99,7 @@ def test_relu_linear_backward_matches_oracle(cin, cout, spatial):
 
 def test_relu_linear_backward_default_dtype_determinism_and_large():
     g = cpu_gen(77)
-    x = rand_cl3d(g, 2, 32, 37, 53, 16)   # V = 62 752: many tiles per workgroup, ragged last tile
+    x = rand_cl3d(g, 2, 32, 37, 53, 16)   # V = 62 752: 491 tiles, the last ragged, one per workgroup
     grad = rand_cl3d(g, 2, 16, 37, 53, 16)
     Wm = rand_pw(g, 32, 16)
     xd, gd, wd = x.to(DEV), grad.to(DEV), Wm.to(DEV)

@@ -105,7 +105,7 @@ def test_scale_and_shift_gradient_error_of_large_volumes(cin, cout):
     assert ((dscale.double() - ref).norm() / ref.norm()).item() < 1.5 * 0.42 * 2.0 ** -24 * parts ** 0.5
 
 
-# (131109 voxels: a second tile for some workgroups of every channel pair, a ragged last tile)
+# (131109 voxels: a second tile for one workgroup at least of every channel pair, a ragged last tile)
 @pytest.mark.parametrize('cin,cout', CHANNELS)
 @pytest.mark.parametrize('v', [1, 63, 65, 127, 129, 257, 131109])
 def test_bnrelu_linear_backward_equals_its_parts(cin, cout, v):
@@ -237,7 +237,8 @@ def test_built_in_split_of_the_march(shape):
         assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < 1e-5
 
 
-# 32769 voxels at 64 channels, 65553 at 16 and 32: a second tile for one workgroup of 512; 131109: ragged third tiles
+# backward: 32769 voxels at 64 channels, 65553 at 32: a second tile for one workgroup of 512; 131109: a second or ragged third
+# tile at every channel count, forward and backward
 @pytest.mark.parametrize('c', [16, 32, 64])
 @pytest.mark.parametrize('v', [1, 31, 33, 63, 65, 32769, 65553, 131109])
 def test_inverted_bottleneck_tiles_and_rounds(c, v):
