@@ -284,16 +284,23 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_bwd_kernel(const ha
 
 // Launch shape (blocks, waves, segment) as for the flat stream kernels; segment counts output chunks per thread and
 // step: 1 = interleaved (one window per thread in flight), 2 = contiguous runs of two chunks per thread (two
-// windows, 16 loads, in flight).  Built-in choices measured at (1,64,350,350,128).
+// windows, 16 loads, in flight).  Built-in choices by the size of the volume that is pooled; the largest measured at
+// (1,64,350,350,128).  GPU time per launch in a row of launches at 64 channels, inputs from memory:
+//   forward   24 / 48 / 96 / 192 MiB: (1280,4,1) or (256,4,1) 13.8 / 19.5 / 30.3 / 49.1 us, here 13.4 / 18.2 / 27.7 / 46.2
+//   backward  24 / 48 / 96 / 192 MiB: (768,4,1) or (256,4,1) 8.4 / 14.8 / 27.5 / 49.2, here 7.2 / 13.1 / 26.1 / 45.9
 struct PoolDefault {
+    int64_t below;  // bytes
     int blocks, waves, segment;
 };
-constexpr PoolDefault kDefPoolFwd{256, 4, 1};
-constexpr PoolDefault kDefPoolFwdBnRelu{256, 4, 2};
-constexpr PoolDefault kDefPoolBwd{256, 4, 1};
+constexpr int64_t kMiB = 1ll << 20, kAnySize = INT64_MAX;
+constexpr PoolDefault kDefPoolFwd[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 1}};
+constexpr PoolDefault kDefPoolFwdBnRelu[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 2}};
+constexpr PoolDefault kDefPoolBwd[] = {{20 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
+                                       {512 * kMiB, 256, 4, 2}, {kAnySize, 256, 4, 1}};
 constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
 
-static int pool_plan(const char* op, const PoolDefault& def, int N, int H, int W, int D, int C, int blocks, int waves,
+// `table`: the lines of one of the tables above, the last without a limit
+static int pool_plan(const char* op, const PoolDefault* table, int N, int H, int W, int D, int C, int blocks, int waves,
                      int segment, PoolDims* p, int64_t* nchunks, StreamShape* sh)
 {
     if (N <= 0 || H <= 0 || W <= 0 || D <= 0 || C <= 0 || !is_pow2(C)) {
@@ -308,6 +315,9 @@ static int pool_plan(const char* op, const PoolDefault& def, int N, int H, int W
         set_error("%s: tensor too large", op);
         return KEROPS_E_BADARG;
     }
+    const int64_t bytes = (int64_t)N * H * W * D * C * 2;
+    while (bytes >= table->below) ++table;
+    const PoolDefault& def = *table;
     if (waves == 0) waves = def.waves;
     if (segment == 0) segment = def.segment;
     if (!(waves == 4 || waves == 8 || waves == 16)) {

@@ -445,21 +445,50 @@ using namespace kerops;
 //   waves    wavefronts per workgroup: 4, 8 or 16
 //   segment  1 = interleaved walk, 4 or 8 = each workgroup step covers one contiguous run of that many
 //            chunks per thread (with C < 8 a request for 8 runs as 4)
-// Built-in choices: measured on MI355X at (1,64,350,350,128) with `python -m kerops_amd.tune --streams`.
+// Built-in choices by the size of the tensor (the fp16 volume; the wide side of a quantiser).  Workgroups of four
+// wavefronts win while a tensor is small: a workgroup of sixteen is placed on a compute unit only as a whole and pays
+// its slowest wavefront at either end.  GPU time per launch in a row of launches, inputs from memory, C = 16 and 64 alike:
+//   BN-ReLU            0.5 / 8 / 48 / 192 MiB: (256,16,8) or (1280,16,4) 6.1 / 7.9 / 20.4 / 67.0 us, here 2.8 / 4.9 / 18.7 / 65.3
+//   its backward       8 / 48 / 96 / 384 MiB: (768,4,1) or (1536,16,4) 13.0 / 34.2 / 78.8 / 215, here 12.6 / 31.9 / 55.1 / 196;
+//                      1.9 GiB 1002, 1011 with 256 workgroups
+//   add + statistics   8 / 48 / 96 / 1914 MiB: (1280,4,8) or (1280,16,8) 12.2 / 34.2 / 67.0 / 1048, here 12.1 / 31.4 / 54.3 / 1019
+//   its backward       2 / 24 / 64 MiB: (1536,16,1) or (512,4,4) 8.1 / 17.9 / 37.4, here 5.2 / 15.3 / 36.3
+//   statistics         0.5 / 48 / 96 MiB: (1536,16,8) or (256,4,8) 11.0 / 19.9 / 24.6, here 8.0 / 16.4 / 23.8
+//   window quantiser   2 / 24 / 64 / 128 MiB in: (512,16,8) or (256,4,8) 6.6 / 9.3 / 21.2 / 36.7, here 3.4 / 8.8 / 19.1 / 36.7
+//   its inverse        2 / 24 / 48 MiB out: (1536,16,8) 5.1 / 10.1 / 18.1, here 3.1 / 8.7 / 15.9
+//   int8 quantiser     16 / 48 / 96 MiB in: (256,4,4) or (4096,16,4) 10.2 / 26.8 / 29.0, here 7.2 / 15.6 / 27.9
+// Up to 4 % of a launch separates neighbouring lines of a table.  The shapes of the largest tensors were measured at
+// (1,64,350,350,128).
 namespace {
 
 struct StreamDefault {
     int blocks, waves, segment;
 };
-constexpr StreamDefault kDefStats{256, 4, 8};
-constexpr StreamDefault kDefAddStats{1280, 16, 8};
-constexpr StreamDefault kDefStatsBwd{4096, 16, 4};
-constexpr StreamDefault kDefAddStatsBwd{512, 4, 4};
-constexpr StreamDefault kDefBnReluFwd{1280, 16, 4};
-constexpr StreamDefault kDefBnReluBwd{1536, 16, 4};
-constexpr StreamDefault kDefQuantU8{256, 4, 8};
-constexpr StreamDefault kDefDequantU8{512, 4, 4};
-constexpr StreamDefault kDefQuantI8{4096, 16, 4};
+// the shape of the first line whose limit is above the tensor's size
+struct SizedDefault {
+    int64_t below;  // bytes
+    StreamDefault shape;
+};
+constexpr int64_t kMiB = 1ll << 20, kAnySize = INT64_MAX;
+constexpr SizedDefault kDefStats[] = {{384 * kMiB, {512, 4, 4}}, {kAnySize, {256, 4, 8}}};
+constexpr SizedDefault kDefAddStats[] = {{kAnySize, {256, 4, 1}}};
+constexpr SizedDefault kDefStatsBwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {4096, 16, 4}}};
+constexpr SizedDefault kDefAddStatsBwd[] = {{112 * kMiB, {1024, 4, 4}}, {kAnySize, {512, 4, 4}}};
+constexpr SizedDefault kDefBnReluFwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {1280, 16, 4}}};
+constexpr SizedDefault kDefBnReluBwd[] = {{1536 * kMiB, {256, 4, 1}}, {kAnySize, {1536, 16, 4}}};
+constexpr SizedDefault kDefQuantU8[] = {{56 * kMiB, {1536, 4, 4}}, {112 * kMiB, {1536, 4, 8}}, {kAnySize, {256, 4, 8}}};
+constexpr SizedDefault kDefDequantU8[] = {{3 * kMiB, {1024, 4, 1}}, {56 * kMiB, {2048, 4, 8}}, {kAnySize, {512, 4, 4}}};
+constexpr SizedDefault kDefQuantI8[] = {{160 * kMiB, {2048, 4, 4}}, {256 * kMiB, {1536, 16, 4}}, {kAnySize, {4096, 16, 4}}};
+// (called ahead of the argument checks)
+int64_t tensor_bytes(int64_t count, int size) { return count <= 0 ? 0 : count > kAnySize / size ? kAnySize : count * size; }
+int64_t channel_bytes(int64_t M, int C) { return M <= 0 || C <= 0 ? 0 : tensor_bytes(tensor_bytes(M, C), 2); }
+template <int N>
+const StreamDefault& default_shape(const SizedDefault (&table)[N], int64_t bytes)
+{
+    int i = 0;
+    while (i < N - 1 && bytes >= table[i].below) ++i;
+    return table[i].shape;
+}
 constexpr int kMaxStreamBlocks = 65536;
 constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
 
@@ -585,8 +614,8 @@ static int stats_common(const char* op, const StreamDefault& def, const void* x,
 extern "C" int kerops_stats_f16(const void* x, float* mean, float* sqmean, int64_t M, int32_t C, void* workspace,
                                 int64_t workspace_bytes, int32_t blocks, int32_t waves, int32_t segment, void* stream)
 {
-    return stats_common("stats", kDefStats, x, nullptr, nullptr, mean, sqmean, M, C, workspace, workspace_bytes, blocks,
-                        waves, segment, stream);
+    return stats_common("stats", default_shape(kDefStats, channel_bytes(M, C)), x, nullptr, nullptr, mean, sqmean, M, C,
+                        workspace, workspace_bytes, blocks, waves, segment, stream);
 }
 
 extern "C" int kerops_add_stats_f16(const void* x, const void* y, void* z, float* mean, float* sqmean, int64_t M,
@@ -597,8 +626,8 @@ extern "C" int kerops_add_stats_f16(const void* x, const void* y, void* z, float
         set_error("add_stats: null pointer");
         return KEROPS_E_BADARG;
     }
-    return stats_common("add_stats", kDefAddStats, x, y, z, mean, sqmean, M, C, workspace, workspace_bytes, blocks,
-                        waves, segment, stream);
+    return stats_common("add_stats", default_shape(kDefAddStats, channel_bytes(M, C)), x, y, z, mean, sqmean, M, C,
+                        workspace, workspace_bytes, blocks, waves, segment, stream);
 }
 
 static int stats_bwd_common(const char* op, const StreamDefault& def, const void* x, const void* add_grad,
@@ -637,8 +666,8 @@ static int stats_bwd_common(const char* op, const StreamDefault& def, const void
 extern "C" int kerops_stats_bwd_f16(const void* x, const float* mean_grad, const float* sqmean_grad, void* dx,
                                     int64_t M, int32_t C, int32_t blocks, int32_t waves, int32_t segment, void* stream)
 {
-    return stats_bwd_common("stats_bwd", kDefStatsBwd, x, nullptr, mean_grad, sqmean_grad, dx, M, C, blocks, waves,
-                            segment, stream);
+    return stats_bwd_common("stats_bwd", default_shape(kDefStatsBwd, channel_bytes(M, C)), x, nullptr, mean_grad,
+                            sqmean_grad, dx, M, C, blocks, waves, segment, stream);
 }
 
 extern "C" int kerops_add_stats_bwd_f16(const void* add_grad, const float* mean_grad, const float* sqmean_grad,
@@ -649,8 +678,8 @@ extern "C" int kerops_add_stats_bwd_f16(const void* add_grad, const float* mean_
         set_error("add_stats_bwd: null pointer");
         return KEROPS_E_BADARG;
     }
-    return stats_bwd_common("add_stats_bwd", kDefAddStatsBwd, add_result, add_grad, mean_grad, sqmean_grad, out, M, C,
-                            blocks, waves, segment, stream);
+    return stats_bwd_common("add_stats_bwd", default_shape(kDefAddStatsBwd, channel_bytes(M, C)), add_result, add_grad,
+                            mean_grad, sqmean_grad, out, M, C, blocks, waves, segment, stream);
 }
 
 extern "C" int kerops_bnrelu_fwd_f16(const void* x, const float* wv, const float* bv, void* y, int64_t M, int32_t C,
@@ -661,7 +690,8 @@ extern "C" int kerops_bnrelu_fwd_f16(const void* x, const float* wv, const float
     const int Vr = C >= 8 ? 8 : C;
     const int CG = C / Vr;
     StreamShape sh;
-    rc = resolve_shape("bnrelu_fwd", kDefBnReluFwd, M * CG, Vr == 8, blocks, waves, segment, &sh);
+    rc = resolve_shape("bnrelu_fwd", default_shape(kDefBnReluFwd, channel_bytes(M, C)), M * CG, Vr == 8, blocks, waves,
+                       segment, &sh);
     if (rc != KEROPS_OK) return rc;
     if (!x || !wv || !bv || !y || !aligned16(x) || !aligned16(y)) {
         set_error("bnrelu_fwd: null or misaligned pointer");
@@ -686,7 +716,8 @@ extern "C" int kerops_bnrelu_bwd_f16(const void* x, const float* wv, const float
     const int Vr = C >= 8 ? 8 : C;
     const int CG = C / Vr;
     StreamShape sh;
-    rc = resolve_shape("bnrelu_bwd", kDefBnReluBwd, M * CG, Vr == 8, blocks, waves, segment, &sh);
+    rc = resolve_shape("bnrelu_bwd", default_shape(kDefBnReluBwd, channel_bytes(M, C)), M * CG, Vr == 8, blocks, waves,
+                       segment, &sh);
     if (rc != KEROPS_OK) return rc;
     if (!x || !wv || !bv || !g || !dx || !dW || !dB || !aligned16(x) || !aligned16(g) || !aligned16(dx)) {
         set_error("bnrelu_bwd: null or misaligned pointer");
@@ -725,8 +756,8 @@ extern "C" int kerops_quant_u8_window(const void* x, int32_t dtype, void* q, int
         return KEROPS_E_BADARG;
     }
     StreamShape sh;
-    int rc = check_flat("quant_u8_window", kDefQuantU8, x, q, numel, numel / (dtype == KEROPS_DTYPE_F32 ? 4 : 8), blocks,
-                        waves, segment, &sh);
+    int rc = check_flat("quant_u8_window", default_shape(kDefQuantU8, tensor_bytes(numel, dtype == KEROPS_DTYPE_F32 ? 4 : 2)), x, q,
+                        numel, numel / (dtype == KEROPS_DTYPE_F32 ? 4 : 8), blocks, waves, segment, &sh);
     if (rc != KEROPS_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     // 1/(2w) correctly rounded to fp32: the double quotient rounded once more is exact for division
@@ -777,8 +808,8 @@ extern "C" int kerops_dequant_u8_window(const void* q, void* out, int32_t dtype,
         return KEROPS_E_BADARG;
     }
     StreamShape sh;
-    int rc = check_flat("dequant_u8_window", kDefDequantU8, q, out, numel, numel / (dtype == KEROPS_DTYPE_F32 ? 4 : 8),
-                        blocks, waves, segment, &sh);
+    int rc = check_flat("dequant_u8_window", default_shape(kDefDequantU8, tensor_bytes(numel, dtype == KEROPS_DTYPE_F32 ? 4 : 2)), q,
+                        out, numel, numel / (dtype == KEROPS_DTYPE_F32 ? 4 : 8), blocks, waves, segment, &sh);
     if (rc != KEROPS_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int seg = sh.segment != 1;
@@ -842,7 +873,8 @@ extern "C" int kerops_quant_i8_sym_f16(const void* y, const float* absmax, void*
                                        int32_t blocks, int32_t waves, int32_t segment, void* stream)
 {
     StreamShape sh;
-    int rc = check_flat("quant_i8_sym", kDefQuantI8, y, q, numel, numel / 8, blocks, waves, segment, &sh);
+    int rc = check_flat("quant_i8_sym", default_shape(kDefQuantI8, tensor_bytes(numel, 2)), y, q, numel, numel / 8, blocks,
+                        waves, segment, &sh);
     if (rc != KEROPS_OK) return rc;
     if (!absmax) {
         set_error("quant_i8_sym: null absmax");

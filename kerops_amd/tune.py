@@ -8,8 +8,8 @@ kerops/ops/conv/dwconv_wgrad.py:10-22); the tables in kerops_amd/ops/conv were m
     python -m kerops_amd.tune --channels 32 64 --apply          # and reconfigure the ops of this process
 
     python -m kerops_amd.tune --streams                         # the flat stream ops: (blocks, num_warps, segment)
-    python -m kerops_amd.tune --streams --all --write           # every channel count of the README table and the
-                                                                # small-tensor class; rewrites settings/stream_shapes.json
+    python -m kerops_amd.tune --streams --all --write           # every channel count of the README table; rewrites
+                                                                # settings/stream_shapes.json
 
 `tune(...)` returns {op: {C: (W_block, D_block, lane_channels, H_chunk, ms)}}; `apply(result)` installs the
 choices through the ops' `reconfigure`, the same mechanism a user of the reference has for overriding its tables.
@@ -181,9 +181,9 @@ def apply_streams(result, write=False, note='', key='default'):
 
 
 # `--streams --all`: the tensors behind each key of the stream table.  "default" (channel counts without an entry)
-# repeats the 64-channel measurement.
+# repeats the 64-channel measurement; "small" stays with the library's rule by size.
 STREAM_CLASSES = (('8', (1, 8, 350, 350, 128)), ('16', (1, 16, 350, 350, 128)), ('32', (1, 32, 350, 350, 128)),
-                  ('64', (1, 64, 350, 350, 128)), ('128', (1, 128, 350, 350, 128)), ('small', (2, 16, 64, 64, 64)))
+                  ('64', (1, 64, 350, 350, 128)), ('128', (1, 128, 350, 350, 128)))
 
 
 def main():

@@ -6,11 +6,14 @@ import torch
 
 import oracle
 from conftest import cpu_gen, rand_cl3d, rand_dw_weight
+from kerops_amd.ops.addition import AddStats, AddStatsBackward
+from kerops_amd.ops.avgpool import AvgPoolCeilStats, AvgPoolCeilStatsBackward
 from kerops_amd.ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
 from kerops_amd.ops.conv import DWConv, DWConvBackward, DWConvStats, DWConvWGRAD
 from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, LinBReLULinAdd,
                                    LinBReLULinBackward, ReLULinearAdd, ReLULinearBackward)
-from kerops_amd.ops.quantization import DequantUint8Window, QuantUint8Window
+from kerops_amd.ops.quantization import DequantUint8Window, QuantInt8Sym, QuantUint8Window
+from kerops_amd.ops.stats import Stats, StatsBackward
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
@@ -273,3 +276,49 @@ def test_inverted_bottleneck_is_the_same_with_early_and_late_loads():
     tail = slice(v - 5000, v)
     ref = oracle.lin_brelu_lin_add(*(t.cpu() for t in (x[:, :, tail], up, down, bias, add[:, :, tail])))
     assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
+
+
+# one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
+@pytest.mark.parametrize('mib', [3, 14, 20, 56, 112, 160])
+@pytest.mark.parametrize('off', [-1, 1])
+def test_stream_ops_either_side_of_a_size_line(mib, off):
+    c = 64
+    v = (mib << 20) // (2 * c) + off
+    gen = torch.Generator(DEV).manual_seed(mib)
+    x, y = (torch.randn(1, v, 1, 1, c, device=DEV, generator=gen).half().permute(0, 4, 1, 2, 3) for _ in range(2))
+    scale, shift = torch.rand(c, device=DEV, generator=gen) + 0.5, torch.randn(c, device=DEV, generator=gen)
+    one = dict(blocks=64, num_warps=4, segment=1)  # a shape of its own: every element is the same whatever the shape
+    peak = torch.full((1,), 5.0, device=DEV)
+    q = QuantUint8Window(x, 3.0)
+    pooled, pmean, psq = AvgPoolCeilStats(x)
+    z, zmean, zsq = AddStats(x, y)
+    dx, dscale, dshift = ApplyBNReLUBackward(x, scale, shift, y)
+    for got, ref in ((q, QuantUint8Window(x, 3.0, **one)),
+                     (DequantUint8Window(q, torch.float16, 3.0), DequantUint8Window(q, torch.float16, 3.0, **one)),
+                     (QuantInt8Sym(x, peak)[0], QuantInt8Sym(x, peak, **one)[0]),
+                     (ApplyBNReLU(x, scale, shift), ApplyBNReLU(x, scale, shift, **one)),
+                     (dx, ApplyBNReLUBackward(x, scale, shift, y, **one)[0]),
+                     (z, AddStats(x, y, **one)[0]),
+                     (StatsBackward(x, scale, shift), StatsBackward(x, scale, shift, **one)),
+                     (AddStatsBackward(x, scale, shift, y), AddStatsBackward(x, scale, shift, y, **one)),
+                     (pooled, AvgPoolCeilStats(x, **one)[0]),
+                     (AvgPoolCeilStatsBackward(pooled, scale, shift, pooled, tuple(x.shape)),
+                      AvgPoolCeilStatsBackward(pooled, scale, shift, pooled, tuple(x.shape), **one))):
+        assert torch.equal(got, ref)
+
+    def rows(t):
+        return t.permute(0, 2, 3, 4, 1).double().view(-1, c)
+
+    def sums(t):
+        return t.mean(0), (t * t).mean(0)
+
+    # the statistics are those of the averages ahead of their rounding to fp16
+    averages = torch.cat([rows(x)[:v // 2 * 2].view(-1, 2, c).mean(1), rows(x)[v // 2 * 2:]])
+    active = torch.where(dx == 0, 0.0, y.double())  # (scale > 0: the gradient is zero where the ReLU is, or y itself)
+    dscale_ref, dshift_ref = ((active * t).sum((0, 2, 3, 4)) for t in (x.double(), 1.0))
+    for got, ref in ((Stats(x), sums(rows(x))), ((zmean, zsq), sums(rows(z))), ((pmean, psq), sums(averages)),
+                     ((dscale, dshift), (dscale_ref, dshift_ref))):
+        # fp32 sums of a workgroup's values (chains of at most a few hundred, error below 2^-24 times their root), fp64
+        # from there; means of N(0, 1) values over v voxels are 1 / sqrt(v) in size
+        for a, b in zip(got, ref):
+            assert ((a.double() - b).norm() / b.norm()).item() < 1e-5
