@@ -304,10 +304,10 @@ static inline BalancedSplit best_balanced(int H, int64_t tiles, int row_len, int
     return best;
 }
 // The split of a launch: the balanced one, or (h_chunk > 0) uniform chunks of h_chunk rows.
-// Where a group's share is a whole column of the volume or more, every group crosses into other bundles and the cost
-// above decides.  Where it is less, the launch lasts as long as the groups that do cross (two halo planes and a pipeline
-// refill, about eight plane steps), and chunks of equal length without any crossing are often faster although they
-// leave workgroup slots empty: the cheaper of the two, with the crossing counted in full, is taken.  Measured over 180
+// Where a group's share of the balanced split is a whole column of the volume or more, every group crosses into other
+// bundles and the cost above decides.  Where it is less, the launch lasts as long as the groups that do cross (two halo
+// planes and a pipeline refill), and chunks of equal length without any crossing are often faster although they leave
+// workgroup slots empty: the cheaper of the two, with the crossing counted in full, is taken.  Measured over 180
 // volumes of 0.26 to 400 M elements, C = 8..128, against the balanced split alone: forward 8.8 % faster on average,
 // weight gradient 4.9, fused backward 6.8, between 0.54 and 1.04 of its time ((2,32,96,96,96) forward 55.6 -> 52.7 us,
 // (2,128,45,51,37) backward 47.6 -> 43.4, (1,128,34,71,55) forward 24.2 -> 18.5).
@@ -315,36 +315,54 @@ struct MarchSplit {
     BalancedSplit b;
     int h_chunk;
 };
-// one_row: most workgroups that may march over a single row, which reads three planes for one.  Alone on a compute unit
-// such a workgroup is still the faster one ((1,32,33,19,25), 198 of them: forward 6.26 us, 6.60 with two rows each); two
-// of them on a compute unit lose in the forward and weight-gradient kernels ((2,32,32,9,35), 384: forward 8.20 us, 6.81
-// with two rows each, weight gradient 12.2 and 10.9) and not in the fused backward (15.0 and 15.8).
-static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int setup, int slab_mult, int xcds,
-                                    int one_row)
+// What a launch costs beyond its plane steps, per kernel: fitted to every chunk length and a dozen group sizes at 150
+// volumes of 0.26 to 240 M elements each.
+struct MarchCost {
+    int setup;        // plane steps that a workgroup's prologue, pipeline fill and epilogue take
+    double crossing;  // plane steps that crossing into another bundle takes
+    // A workgroup that has a compute unit of its own steps faster than one of two, so half a round of longer chunks can
+    // beat a full round of short ones ((1,64,34,44,29) forward: 408 workgroups of two rows 9.8 us, 216 of four 8.9;
+    // fused backward 18.5 and 17.3): the ratio of the two, 1 where it does not pay.
+    double alone;
+    // Most workgroups that may march over a single row, which reads three planes for one.  Alone on a compute unit such a
+    // workgroup is still the faster one ((1,32,33,19,25), 198 of them: forward 6.26 us, 6.60 with two rows each); two of
+    // them on a compute unit lose in the forward and weight-gradient kernels ((2,32,32,9,35), 384: forward 8.20 us, 6.81
+    // with two rows each, weight gradient 12.2 and 10.9).
+    int one_row;
+};
+static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int slab_mult, const DeviceGeometry& geo,
+                                    const MarchCost& m)
 {
     double cost;
     const BalancedSplit whole = best_balanced(
         H, tiles, row_len, slots, slab_mult,
-        [&](const BalancedSplit& b) { return balanced_cost(b, H, row_len, slots, setup, xcds); }, &cost);
+        [&](const BalancedSplit& b) { return balanced_cost(b, H, row_len, slots, m.setup, geo.xcds); }, &cost);
     if ((whole.units + whole.ngroups - 1) / whole.ngroups >= H) return {whole, 0};
-    const BalancedSplit part = best_balanced(
-        H, tiles, row_len, slots, slab_mult,
-        [&](const BalancedSplit& b) {
-            const int64_t share = (b.units + b.ngroups - 1) / b.ngroups;
-            const bool aligned = b.units % b.ngroups == 0 && H % share == 0;  // no share crosses
-            const double crossing = share < H ? (aligned ? 0.0 : 8.0) : 8.0 * (double)share / H;
-            const double spread = (int)b.group > slots / xcds ? 1.04 : 1.0;
-            return ((double)share + 2 + setup + crossing) * (1.0 + 0.1 * row_len / (double)b.group) *
-                   (1.0 + 0.004 * (double)H / (double)share) * spread;
-        },
-        &cost);
+    auto occupancy = [&](int64_t workgroups) { return workgroups <= geo.cus ? m.alone : 1.0; };
+    auto part_cost = [&](const BalancedSplit& b) {
+        const int64_t share = (b.units + b.ngroups - 1) / b.ngroups;
+        const bool aligned = b.units % b.ngroups == 0 && H % share == 0;  // no share crosses
+        const double crossing = share < H ? (aligned ? 0.0 : m.crossing) : m.crossing * (double)share / H;
+        const double spread = (int)b.group > slots / geo.xcds ? 1.04 : 1.0;
+        return ((double)share + 2 + m.setup + crossing) * (1.0 + 0.1 * row_len / (double)b.group) *
+               (1.0 + 0.004 * (double)H / (double)share) * spread * occupancy((int64_t)b.group * b.ngroups);
+    };
+    BalancedSplit part = best_balanced(H, tiles, row_len, slots, slab_mult, part_cost, &cost);
+    if (m.alone < 1.0 && geo.cus < slots) {
+        double half;
+        const BalancedSplit b = best_balanced(H, tiles, row_len, geo.cus, slab_mult, part_cost, &half);
+        if (half < cost) {
+            cost = half;
+            part = b;
+        }
+    }
     // chunks that run in one round (never more workgroups, and partial sums, than fit the GPU at once)
     int best_h = 0;
     for (int c = 1; c <= 64 && c <= H && tiles * c <= slots; ++c) {
         const int h = ceil_div(H, c);
         if (ceil_div(H, h) != c) continue;  // the same split as a smaller c
-        if (h < 2 && c > 1 && tiles * c > one_row) break;
-        const double uniform = ((double)h + 2 + setup) * (1.0 + 0.004 * c);
+        if (h < 2 && c > 1 && tiles * c > m.one_row) break;
+        const double uniform = ((double)h + 2 + m.setup) * (1.0 + 0.004 * c) * occupancy(tiles * c);
         if (uniform <= cost) {
             cost = uniform;
             best_h = h;

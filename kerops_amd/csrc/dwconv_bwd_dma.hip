@@ -73,9 +73,6 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
     constexpr int CG = Cfg::CG, TD = Cfg::TD, TW = Cfg::TW, NT = Cfg::NT, SC = Cfg::SC, PB = Cfg::PB, PDP = Cfg::PDP;
     constexpr int NQ = Cfg::NQ, NSUB = Cfg::NSUB, RO = Cfg::RO, GSLOT = Cfg::GSLOT, XSLOT = Cfg::XSLOT, CPL = Cfg::CPL;
     constexpr int NGI = Cfg::NGI, NXI = Cfg::NXI, NGS = Cfg::NGS, NXS = Cfg::NXS, NWAVE = Cfg::NWAVE, PPB = Cfg::PPB;
-    // vector memory instructions a wavefront issues per step: the plane loads (g blocks twice when their interior
-    // chunks take the streaming hint), then, in the input-gradient role, one store per output row
-    constexpr int LOADS = (NTI ? 2 : 1) * NGI + NXI;
     __shared__ __attribute__((aligned(16))) unsigned char smem[Cfg::LDS_BYTES];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(void __attribute__((address_space(3)))*)smem;
 
@@ -194,9 +191,12 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
         __syncthreads();  // the zero fill is complete before any load writes LDS
         return true;
     };
-    // planes p of x and g (clamped into the volume; copies of a clamped plane are never used) into their ring slots
+    // planes p of x and g into their ring slots; planes outside the volume or past the segment's last one (he) are never
+    // used and not loaded (the steps' waits leave at most the stores behind the newest loads in flight, so they hold with
+    // or without loads)
     auto load_planes = [&](int p, int gs, int xs) {
-        const int64_t off = (int64_t)min(max(p, 0), H - 1) * plane_bytes;
+        if (p < 0 || p >= H || p > he) return;
+        const int64_t off = (int64_t)p * plane_bytes;
         const char* gplane = uniform_ptr(gn + off);
         const char* xplane = uniform_ptr(xn + off);
 #pragma unroll
@@ -224,21 +224,27 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
         // ---- input gradient: flipped weight operands, (kd' = 0, 1, 2, -) of one kh' per lane; the four registers of
         // an accumulator tile form a ring (see dwconv_fwd_mfma_segment): every step each lane hands its weights to the
         // next lane of its quad ----
+        // (unconditional 8-byte loads, the resting lane's zeroed afterwards: with a condition around them the compiler
+        // waited for each before the next, twelve trips to memory in a row)
         half4_t wA[3][CPL];
         {
             const int r0 = (1 - rr) & 3, c0 = cslab + q * CPL;
+            const half_t* wrow = a.wt + (2 - min(r0, 2)) * 9 * C + c0;
+            u32x2_t w9[9];
 #pragma unroll
-            for (int kw = 0; kw < 3; ++kw)
+            for (int k = 0; k < 9; ++k) w9[k] = *reinterpret_cast<const u32x2_t*>(wrow + k * C);
 #pragma unroll
-                for (int e = 0; e < CPL; ++e) {
-                    half4_t v = {(half_t)0, (half_t)0, (half_t)0, (half_t)0};
-                    if (r0 < 3) {
+            for (int kw = 0; kw < 3; ++kw) {
+                uint32_t lo[3], hi[3];
 #pragma unroll
-                        for (int kd = 0; kd < 3; ++kd)
-                            v[kd] = a.wt[(((2 - r0) * 3 + (2 - kw)) * 3 + (2 - kd)) * C + c0 + e];
-                    }
-                    wA[kw][e] = v;
+                for (int kd = 0; kd < 3; ++kd) {
+                    const u32x2_t v = w9[(2 - kw) * 3 + (2 - kd)];
+                    lo[kd] = r0 < 3 ? v[0] : 0u;
+                    hi[kd] = r0 < 3 ? v[1] : 0u;
                 }
+                split_operands3(lo, wA[kw][0], wA[kw][1]);
+                split_operands3(hi, wA[kw][2], wA[kw][3]);
+            }
         }
         // g operand: lane rr = j reads the staged positions pgrp + j + k, k = 0..2
         int boff[3];
@@ -271,9 +277,9 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
 #pragma unroll
             for (int o = 0; o < RO; ++o) masked_store8_stream(dxn, 0u, u32x2_t{0u, 0u}, 0);
 
-            auto step = [&](auto ring, int p, bool live) {
+            auto step = [&](auto ring, int p) {
                 constexpr int DONE = (decltype(ring)::value + 3) & 3;  // register of dx plane p-1, complete after this step
-                const bool gin = live && (p >= 0) && (p < H) && (p <= he);
+                const bool gin = (p >= 0) && (p < H);
                 wait_loads_in_flight<RO>();  // this step's planes have landed; the stores behind them may be in flight
                 __syncthreads();
                 load_planes_first(p + 1, gs_load, xs_load);
@@ -304,7 +310,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
                     }
                 }
                 const int ho = p - 1;
-                const bool store = live && (ho >= hs) && (ho < he);
+                const bool store = ho >= hs;
                 char* dplane = const_cast<char*>(uniform_ptr(dxn + (int64_t)max(ho, 0) * plane_bytes));
 #pragma unroll
                 for (int o = 0; o < RO; ++o) {
@@ -325,12 +331,25 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
                     for (int e = 0; e < CPL; ++e) wA[kw][e] = quad_rotate_up(wA[kw][e]);
                 gs = gs + 1 == NGS ? 0 : gs + 1;
             };
-            // groups of four steps (the ring's period); both roles run the same number of steps, so their barriers match
-            for (int p = hs - 1; p <= he + 1; p += 4) {
-                step(std::integral_constant<int, 0>{}, p, true);
-                step(std::integral_constant<int, 1>{}, p + 1, p + 1 <= he + 1);
-                step(std::integral_constant<int, 2>{}, p + 2, p + 2 <= he + 1);
-                step(std::integral_constant<int, 3>{}, p + 3, p + 3 <= he + 1);
+            // The steps p = hs - 1 .. he, no more (rounding a segment up to whole groups of four and loading past its
+            // end cost a short march up to 4.7 us: (1,64,28,128,128) in chunks of 14 rows MARCH_BWD_START -> MARCH_BWD_NOW
+            // us); both roles run the same number, so their barriers match.  A group of four is the ring's period.
+            for (int p = hs - 1;; p += 4) {
+                step(std::integral_constant<int, 0>{}, p);
+                if (p + 1 > he) break;
+                step(std::integral_constant<int, 1>{}, p + 1);
+                if (p + 2 > he) break;
+                step(std::integral_constant<int, 2>{}, p + 2);
+                if (p + 3 > he) break;
+                step(std::integral_constant<int, 3>{}, p + 3);
+                if (p + 4 > he) break;
+            }
+            // the weights go on to where the next segment starts
+            for (int i = (he - hs + 2) & 3; i != 0; i = (i + 1) & 3) {
+#pragma unroll
+                for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+                    for (int e = 0; e < CPL; ++e) wA[kw][e] = quad_rotate_up(wA[kw][e]);
             }
         }  // segments
         wait_loads_in_flight<0>();
@@ -370,12 +389,10 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
             // lane j reads the x slot of plane P + j - 1 = p - 2 + j: its slot index runs behind the newest plane's
             int xslot_lane = (NXS + r2 - 2) % NXS;
             load_planes(hs - 1, 0, 0);
-            // as many steps as the other role runs (groups of four), so that the barriers match
-            const int nsteps = (he - hs + 3 + 3) / 4 * 4;
-            for (int i = 0; i < nsteps; ++i) {
-                const int p = hs - 1 + i;
+            // as many steps as the other role runs, so that the barriers match
+            for (int p = hs - 1; p <= he; ++p) {
                 const int P = p - 1;  // g plane P meets the x planes P-1, P, P+1 = p, the newest one staged
-                const bool on = (p <= he + 1) && (P >= hs) && (P < he);
+                const bool on = P >= hs;
                 wait_loads_in_flight<0>();
                 __syncthreads();
                 load_planes_first(p + 1, gs_load, xs_load);

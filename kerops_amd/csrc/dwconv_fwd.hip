@@ -543,20 +543,22 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     // the three steps that add to it, so no register is moved between steps.  At step s (x plane hp = hs - 1 + s)
     // register i takes kh = (s + 1 - i) % 4 (3 = none: zero weights), i.e. every step each lane hands its weights
     // to the next lane of its quad (one DPP move per dword); a march of 4n steps leaves them where they started.
+    // (Nine unconditional loads of channel pairs, the resting lane's zeroed afterwards: a condition around the loads makes
+    // the compiler wait for each before the next, six trips to memory in a row before the first plane.)
     half4_t wA[3][2];
     {
         const int r0 = (1 - rr) & 3;
+        const half_t* wrow = a.wt + (min(r0, 2) * 9) * C + c0;
+        uint32_t w9[9];
 #pragma unroll
-        for (int kw = 0; kw < 3; ++kw)
+        for (int k = 0; k < 9; ++k) w9[k] = *reinterpret_cast<const uint32_t*>(wrow + k * C);
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                half4_t v = {(half_t)0, (half_t)0, (half_t)0, (half_t)0};
-                if (r0 < 3) {
+        for (int kw = 0; kw < 3; ++kw) {
+            uint32_t r[3];
 #pragma unroll
-                    for (int kd = 0; kd < 3; ++kd) v[kd] = a.wt[((r0 * 3 + kw) * 3 + kd) * C + c0 + e];
-                }
-                wA[kw][e] = v;
-            }
+            for (int kd = 0; kd < 3; ++kd) r[kd] = r0 < 3 ? w9[kw * 3 + kd] : 0u;
+            split_operands3(r, wA[kw][0], wA[kw][1]);
+        }
     }
     float esc[2] = {1.0f, 1.0f}, esh[2] = {0.0f, 0.0f};
     if (EPI) {
@@ -628,8 +630,9 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         for (int e = 0; e < 2; ++e) T[o][e] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     // Global loads run two planes ahead of the arithmetic, into two register sets used alternately.
-    // They are unconditional (plane indices are clamped; planes that do not exist are never used):
-    // the compiler's wait-count bookkeeping is exact only on branch-free paths.
+    // In the loop they are unconditional (plane indices are clamped to what the march uses, so at its ends they find
+    // the plane in the L2; the copies are never used): the compiler's wait-count bookkeeping is exact only on
+    // branch-free paths.
     // (the fused pointwise mode has no registers to spare for the second set and runs one plane ahead)
     // Planes in flight per workgroup: measured at (1,C,350,350,128), one plane ahead is faster with 8 and with 64
     // channels per slab (C = 8: 4 % for the plain kernel, 10 % with the statistics; C = 64, 128: 1 %), two planes
@@ -637,8 +640,9 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     // of a group further apart, and the halo lines they share leave the L2 before the neighbour asks for them.
     constexpr int AHEAD = MODE == 2 ? 1 : (SC == 8 || (SC == 64 && MODE != 3)) ? 1 : 2;
     half8_t xpre0[NLDX], xpre1[NLDX];
+    const int hp_last = min(he, H - 1);
     auto prefetch = [&](int hp, half8_t(&xpre)[NLDX]) {
-        const char* xplane = reinterpret_cast<const char*>(xn + min(max(hp, 0), H - 1) * plane_stride);
+        const char* xplane = reinterpret_cast<const char*>(xn + min(max(hp, 0), hp_last) * plane_stride);
 #pragma unroll
         for (int j = 0; j < NLDX; ++j) {
             // nobody else reads the interior chunks: with the hint they do not push shared lines out of the L2
@@ -650,9 +654,9 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     };
 
     int parity = 0;
-    auto step = [&](auto ring, int hp, half8_t(&xpre)[NLDX], bool live) {
+    auto step = [&](auto ring, int hp, half8_t(&xpre)[NLDX], auto tail) {
         constexpr int DONE = (decltype(ring)::value + 3) & 3;  // register of output plane hp-1, complete after this step
-        const bool xin = live && (hp >= 0) && (hp < H);  // wavefront-uniform
+        const bool xin = (hp >= 0) && (hp < H);  // wavefront-uniform
         unsigned char* xbuf = smem + parity * XSLOT;
 #pragma unroll
         for (int j = 0; j < NLDX; ++j) {
@@ -665,7 +669,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         // path, and loads queued behind other wavefronts' stores reach memory late (measured at C = 64: 0.703 ->
         // 0.694 ms; the same order without the priority, or the priority without the order, changes nothing).
         __builtin_amdgcn_s_setprio(3);
-        prefetch(hp + AHEAD, xpre);
+        if (!decltype(tail)::value || hp + AHEAD <= hp_last) prefetch(hp + AHEAD, xpre);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(0);
         flush_row(parity ^ 1);
@@ -692,7 +696,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         }
         // register DONE of every tile is the finished output plane hp-1
         const int ho = hp - 1;
-        const bool finished = live && (ho >= hs);
+        const bool finished = ho >= hs;
         pending_row = finished ? ho : -1;
         if (finished) {  // workgroup-uniform
             unsigned char* otile = smem + OT_OFF + parity * OT_BYTES;
@@ -794,24 +798,23 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     // The steps hp = hs-1 .. he run in groups of four (the period of the accumulator ring; the register sets
     // alternate inside a group), in a loop whose only exit is at its end: an exit between two steps would give the
     // loop a second way into its first step, on which the newest set is the oldest, and the compiler's wait before
-    // that step's staging writes would cover every load in flight.  A count that does not divide ends with steps
-    // that stage planes nobody reads, compute and store nothing.
+    // that step's staging writes would cover every load in flight.  The one to three steps that are left follow the
+    // loop in code of their own and load what they need (running a fourth of a group on empty cost a short march up to
+    // 3 us: (1,64,30,128,128) in chunks of 15 rows MARCH_FWD_START -> MARCH_FWD_NOW us).
     using std::integral_constant;
-    if constexpr (AHEAD == 1) {
-        for (int hp = hs - 1; hp <= he; hp += 4) {
-            step(integral_constant<int, 0>{}, hp, xpre0, true);
-            step(integral_constant<int, 1>{}, hp + 1, xpre0, hp + 1 <= he);
-            step(integral_constant<int, 2>{}, hp + 2, xpre0, hp + 2 <= he);
-            step(integral_constant<int, 3>{}, hp + 3, xpre0, hp + 3 <= he);
-        }
-    } else {
-        for (int hp = hs - 1; hp <= he; hp += 4) {
-            step(integral_constant<int, 0>{}, hp, xpre0, true);
-            step(integral_constant<int, 1>{}, hp + 1, xpre1, hp + 1 <= he);
-            step(integral_constant<int, 2>{}, hp + 2, xpre0, hp + 2 <= he);
-            step(integral_constant<int, 3>{}, hp + 3, xpre1, hp + 3 <= he);
-        }
+    constexpr std::false_type loop{};
+    constexpr std::true_type tail{};
+    half8_t(&xodd)[NLDX] = AHEAD == 1 ? xpre0 : xpre1;
+    int hp = hs - 1;
+    for (; hp + 3 <= he; hp += 4) {
+        step(integral_constant<int, 0>{}, hp, xpre0, loop);
+        step(integral_constant<int, 1>{}, hp + 1, xodd, loop);
+        step(integral_constant<int, 2>{}, hp + 2, xpre0, loop);
+        step(integral_constant<int, 3>{}, hp + 3, xodd, loop);
     }
+    if (hp <= he) step(integral_constant<int, 0>{}, hp, xpre0, tail);
+    if (hp + 1 <= he) step(integral_constant<int, 1>{}, hp + 1, xodd, tail);
+    if (hp + 2 <= he) step(integral_constant<int, 2>{}, hp + 2, xpre0, tail);
     if constexpr (BOUNCE) {
         __syncthreads();
         flush_row(parity ^ 1);
@@ -937,8 +940,8 @@ static int plan_fwd_mfma(FwdArgs& a, int N, int h_chunk, bool balanced_ok = fals
         const int64_t tiles = (int64_t)N * a.n_wt * a.n_dt * a.n_slab;
         const MarchSplit split =
             h_chunk < 0 ? MarchSplit{make_balanced(a.H, tiles, slots, -h_chunk), 0}
-                        : pick_split(a.H, tiles, a.n_dt * a.n_slab, slots, 6, per_slab_state ? a.n_slab : 1, geo.xcds,
-                                     geo.cus);
+                        : pick_split(a.H, tiles, a.n_dt * a.n_slab, slots, per_slab_state ? a.n_slab : 1, geo,
+                                     MarchCost{6, 8.0, 0.75, geo.cus});
         const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && tiles + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {

@@ -1131,7 +1131,7 @@ static int plan_wgrad(int N, int H, int W, int D, int C, int tile_w, int tile_d,
         }
         const MarchSplit split =
             h_chunk < 0 ? MarchSplit{make_balanced(H, per_plane, slots, -h_chunk), 0}
-                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab, geo.xcds, geo.cus);
+                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, p->n_slab, geo, MarchCost{8, 8.0, 1.0, geo.cus});
         const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && per_plane + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {
@@ -1286,7 +1286,7 @@ static int plan_bwd(int N, int H, int W, int D, int C, int h_chunk, WgPlan* p)
         }
         const MarchSplit split =
             h_chunk < 0 ? MarchSplit{make_balanced(H, per_plane, slots, -h_chunk), 0}
-                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, 8, p->n_slab, geo.xcds, slots);
+                        : pick_split(H, per_plane, p->n_dt * p->n_slab, slots, p->n_slab, geo, MarchCost{5, 3.0, 0.8, slots});
         const BalancedSplit& b = split.b;
         const bool fits = b.units < (1LL << 31) && per_plane + b.group < (1LL << 31);  // 32-bit counters in the kernel
         if (!fits && h_chunk < 0) {
