@@ -225,7 +225,8 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
         // an accumulator tile form a ring (see dwconv_fwd_mfma_segment): every step each lane hands its weights to the
         // next lane of its quad ----
         // (unconditional 8-byte loads, the resting lane's zeroed afterwards: with a condition around them the compiler
-        // waited for each before the next, twelve trips to memory in a row)
+        // waited for each before the next, twelve trips to memory in a row; (1,64,28,128,128) in chunks of 14 rows
+        // 42.2 -> 41.5 us)
         half4_t wA[3][CPL];
         {
             const int r0 = (1 - rr) & 3, c0 = cslab + q * CPL;
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
                 gs = gs + 1 == NGS ? 0 : gs + 1;
             };
             // The steps p = hs - 1 .. he, no more (rounding a segment up to whole groups of four and loading past its
-            // end cost a short march up to 4.7 us: (1,64,28,128,128) in chunks of 14 rows MARCH_BWD_START -> MARCH_BWD_NOW
+            // end cost a short march up to 4.7 us: (1,64,28,128,128) in chunks of 14 rows 46.9 -> 42.2
             // us); both roles run the same number, so their barriers match.  A group of four is the ring's period.
             for (int p = hs - 1;; p += 4) {
                 step(std::integral_constant<int, 0>{}, p);

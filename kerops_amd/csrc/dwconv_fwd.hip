@@ -544,7 +544,8 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     // register i takes kh = (s + 1 - i) % 4 (3 = none: zero weights), i.e. every step each lane hands its weights
     // to the next lane of its quad (one DPP move per dword); a march of 4n steps leaves them where they started.
     // (Nine unconditional loads of channel pairs, the resting lane's zeroed afterwards: a condition around the loads makes
-    // the compiler wait for each before the next, six trips to memory in a row before the first plane.)
+    // the compiler wait for each before the next, six trips to memory in a row before the first plane; (1,64,30,128,128)
+    // in chunks of 15 rows 29.2 -> 27.4 us.)
     half4_t wA[3][2];
     {
         const int r0 = (1 - rr) & 3;
@@ -800,7 +801,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     // loop a second way into its first step, on which the newest set is the oldest, and the compiler's wait before
     // that step's staging writes would cover every load in flight.  The one to three steps that are left follow the
     // loop in code of their own and load what they need (running a fourth of a group on empty cost a short march up to
-    // 3 us: (1,64,30,128,128) in chunks of 15 rows MARCH_FWD_START -> MARCH_FWD_NOW us).
+    // 3 us: (1,64,30,128,128) in chunks of 15 rows 30.6 -> 29.2 us).
     using std::integral_constant;
     constexpr std::false_type loop{};
     constexpr std::true_type tail{};

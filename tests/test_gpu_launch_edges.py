@@ -322,3 +322,21 @@ def test_stream_ops_either_side_of_a_size_line(mib, off):
         # from there; means of N(0, 1) values over v voxels are 1 / sqrt(v) in size
         for a, b in zip(got, ref):
             assert ((a.double() - b).norm() / b.norm()).item() < 1e-5
+
+
+# marches of 3 to 8 plane steps and more: every remainder of the groups of four, one and several segments of a workgroup, at
+# both ends of the volume and inside it
+@pytest.mark.parametrize('c,w,d', [(8, 9, 67), (16, 9, 33), (32, 17, 17), (64, 9, 9), (128, 9, 9)])
+@pytest.mark.parametrize('h_chunk', [1, 2, 3, 4, 5, 6, 7, -2, -6])
+def test_depthwise_marches_of_any_length(c, w, d, h_chunk):
+    g = cpu_gen(c + h_chunk)
+    n, h = 2, 13
+    x, grad = rand_cl3d(g, n, c, h, w, d).to(DEV), rand_cl3d(g, n, c, h, w, d).to(DEV)
+    wt = rand_dw_weight(g, c)[1].to(DEV)
+    # a chunk of the whole height, which the oracle tests pin: an output does not depend on the march that computes it
+    assert torch.equal(bits(DWConv(x, wt, H_chunk=h_chunk)), bits(DWConv(x, wt, H_chunk=h)))
+    dx, gw = DWConvBackward(x, grad, wt, H_chunk=h_chunk, out_dtype=torch.float32)
+    dx_ref, gw_ref = DWConvBackward(x, grad, wt, H_chunk=h, out_dtype=torch.float32)
+    assert torch.equal(bits(dx), bits(dx_ref))
+    # fp32 sums of a few thousand products in another order
+    assert ((gw - gw_ref).norm() / gw_ref.norm()).item() < 1e-5
