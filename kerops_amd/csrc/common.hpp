@@ -130,6 +130,29 @@ __device__ __forceinline__ void masked_store16_stream(void* sbase, uint32_t voff
                  : "s"(sbase), "v"(voff), "v"(data), "s"(mask)
                  : "memory");
 }
+
+// ---- plane access with the hardware's bounds check ---------------------------------------------------------
+// A buffer access whose byte offset is not below the resource's size does nothing: a load returns zeros, a store is
+// dropped, no memory is touched.  So a plane that does not exist has size 0 and a lane without a voxel an offset past
+// every plane, and no condition stands around the instruction: the compiler's wait-count bookkeeping is exact only on
+// branch-free paths (behind a conditional store it waits for every access in flight).
+typedef __amdgpu_buffer_rsrc_t plane_rsrc_t;
+constexpr uint32_t kNoVoxel = 0xfffffff0u;  // no offset below the bytes of a plane of at most 2^31 - 8 fp16 elements
+__device__ __forceinline__ plane_rsrc_t plane_rsrc(const void* plane, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(plane), 0, (int)bytes, 0x27000);
+}
+template <bool STREAM>
+__device__ __forceinline__ half8_t plane_load16(plane_rsrc_t r, uint32_t voff)
+{
+    return __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, 0, STREAM ? 2 : 0));
+}
+template <bool STREAM>
+__device__ __forceinline__ void plane_store16(plane_rsrc_t r, uint32_t voff, half8_t v)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, (int)voff, 0, STREAM ? 2 : 0);
+}
+
 constexpr int64_t kStreamInteriorMinBytes = 384ll << 20;
 
 // Order in which the 16-byte chunks of a staged plane (a TW x TD patch with its one-voxel halo, CG chunks per

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::WPE) void dwconv_fwd_kernel(const Fwd
 // 576 of the 1024 multiply-adds of an instruction are useful; per x row, four positions and 16
 // channels the cost is 3 matrix instructions, the operand comes from LDS as three dwords (two
 // channels per lane and position) split into the even and the odd channel by byte permutes.
-// The arithmetic is a fraction of the memory time; global loads run two planes ahead.
+// The arithmetic is a fraction of the memory time; global loads run one plane ahead.
 template <int CG_, int TW_, int TD_, int NT_>
 struct FmCfg {
     static constexpr int CG = CG_, TW = TW_, TD = TD_, NT = NT_, NWAVE = NT_ / 64;
@@ -448,9 +448,9 @@ struct FmCfg {
     static constexpr int RO = TW / RSPLIT;                 // output rows per wavefront (it reads RO + 2 x rows)
     static constexpr int R = TW + 2;                       // x rows incl. halo
     static constexpr int PDP = (TD + 3 + 3) / 4 * 4;       // x positions per row: halo + one over-read, padded to 4
-    static constexpr int XSLOT = R * PDP * PB;
-    static constexpr int DUMP = 2 * XSLOT;
-    static constexpr int LDS_BYTES = DUMP + 16;
+    static constexpr int DUMP = R * PDP * PB;              // behind a staged plane: 16 bytes that nobody reads
+    static constexpr int XSLOT = DUMP + 16;
+    static constexpr int LDS_BYTES = 2 * XSLOT;
     static constexpr int NXCH = R * (TD + 2) * CG;
     static constexpr int NLDX = (NXCH + NT - 1) / NT;
     static_assert(TD % (4 * NSUB) == 0, "a row splits into whole position groups");
@@ -505,15 +505,12 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     const int w0 = wt_i * Cfg::TW, d0 = dt * TD;
     const int cslab = slab * SC;
     const int64_t plane_stride = (int64_t)W * D * C;
+    const uint32_t plane_bytes = (uint32_t)(plane_stride * 2);
     const half_t* xn = a.x + (int64_t)n * H * plane_stride;
     half_t* yn = a.y + (int64_t)n * H * plane_stride;
 
-    // positions that staging never writes (outside the volume, row padding) must read as zero
-    const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int o = t * 16; o < Cfg::LDS_BYTES; o += NT * 16) *reinterpret_cast<half8_t*>(smem + o) = z8;
-
-    // staging assignment, 16-byte chunks (8 channels of one position); lanes without a chunk inside the
-    // volume load the plane's first chunk and write it to the dump slot
+    // staging assignment, 16-byte chunks (8 channels of one position): a chunk outside the volume loads as zeros (see
+    // plane_rsrc), a lane without a chunk writes to the dump slot
     uint32_t xgo[NLDX];
     int xls[NLDX];
     typedef HaloOrder<Cfg::TW, TD, CG> Order;  // shared chunks first, interior chunks last
@@ -524,8 +521,8 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         Order::decode(ch, wq, dq, cq);
         const int w = w0 - 1 + wq, d = d0 - 1 + dq;
         const bool ok = (ch < Cfg::NXCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-        xgo[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
-        xls[j] = ok ? lds_swizzle<PB>(wq * PDP + dq, cq * 16) : -1;
+        xgo[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : kNoVoxel;
+        xls[j] = ch < Cfg::NXCH ? lds_swizzle<PB>(wq * PDP + dq, cq * 16) : Cfg::DUMP;
     }
 
     // lane = (block b, index rr); block = (channel pair q, position group sub)
@@ -578,12 +575,31 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     if constexpr (MODE == 2) {
         // pw^T fragments, pre-arranged so that lane l of block mt reads 16 contiguous bytes per k step:
         // [mt][s][l][8] = pw[16 s + 8 (l / 32) + 0..7][32 mt + l % 32]
+        // (16-byte loads of its rows, all in flight at once)
         half_t* pa = reinterpret_cast<half_t*>(smem + A_OFF);
-        for (int i = t; i < MT * KS * 64 * 8; i += NT) {
-            const int jj = i % 8, l = (i / 8) % 64, s2 = (i / 512) % KS, m2 = i / (512 * KS);
-            pa[i] = a.pw[(16 * s2 + 8 * (l / 32) + jj) * COUT + 32 * m2 + l % 32];
+        constexpr int NPW = SC * COUT / 8 / NT;
+        static_assert(NPW * 8 * NT == SC * COUT, "every thread loads the same number of chunks");
+        half8_t row8[NPW];
+#pragma unroll
+        for (int i = 0; i < NPW; ++i) row8[i] = *reinterpret_cast<const half8_t*>(a.pw + (t + i * NT) * 8);
+#pragma unroll
+        for (int i = 0; i < NPW; ++i) {
+            const int e = (t + i * NT) * 8, k = e / COUT, o = e % COUT;
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj)
+                pa[(((o / 32) * KS + k / 16) * 64 + ((k % 16) / 8) * 32 + o % 32 + jj) * 8 + k % 8] = row8[i][jj];
         }
     }
+    // its result leaves as NY2 chunks of 16 bytes per thread and plane
+    constexpr int NY2 = MODE == 2 ? NPOS * (COUT / 8) / NT : 0;
+    uint32_t y2go[NY2 > 0 ? NY2 : 1];
+#pragma unroll
+    for (int i = 0; i < NY2; ++i) {
+        const int c = t + i * NT, row = c / (COUT / 8), cc = c - row * (COUT / 8);
+        const int w = w0 + row / TD, d = d0 + row % TD;
+        y2go[i] = (w < W && d < D) ? (uint32_t)(((w * D + d) * COUT + cc * 8) * 2) : kNoVoxel;
+    }
+    const uint32_t y2_bytes = (uint32_t)((int64_t)W * D * COUT * 2);
     half_t* yn2 = MODE == 2 ? a.y2 + (int64_t)n * H * W * D * COUT : nullptr;
 
     // x operand: lane rr = j reads the positions pgrp + j + k (patch column = position + 1 - 1), k = 0..2
@@ -607,15 +623,14 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     const int ord = ot_swz(opos, ocq * 16);
     const int ow = w0 + opos / TD, odd = d0 + opos % TD;
     const bool ovalid = (ow < W) && (odd < D);
-    const uint32_t ogo = ovalid ? (uint32_t)(((ow * D + odd) * C + cslab + ocq * 8) * 2) : 0u;
+    const uint32_t ogo = ovalid ? (uint32_t)(((ow * D + odd) * C + cslab + ocq * 8) * 2) : kNoVoxel;
     int pending_row = -1;
-    auto flush_row = [&](int par) {  // stores the plane that the previous step left in output tile par
-        if (BOUNCE && pending_row >= 0) {  // workgroup-uniform
+    auto flush_row = [&](int par) {  // stores the plane that the previous step left in output tile par, if it did
+        if constexpr (BOUNCE) {
             const half8_t o8 = *reinterpret_cast<const half8_t*>(smem + OT_OFF + par * OT_BYTES + ord);
+            const char* yplane = uniform_ptr(reinterpret_cast<char*>(yn + max(pending_row, 0) * plane_stride));
             // written once, never re-read: streaming hint keeps L2 for the halo rows
-            if (ovalid)
-                __builtin_nontemporal_store(
-                    o8, reinterpret_cast<half8_t*>(reinterpret_cast<char*>(yn + pending_row * plane_stride) + ogo));
+            plane_store16<true>(plane_rsrc(yplane, pending_row >= 0 ? plane_bytes : 0u), ogo, o8);
         }
     };
     // mode 3: whether the lane's position pgrp + rr of the output rows ra .. ra+RO-1 lies inside the volume
@@ -630,39 +645,38 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
 #pragma unroll
         for (int e = 0; e < 2; ++e) T[o][e] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // Global loads run two planes ahead of the arithmetic, into two register sets used alternately.
-    // In the loop they are unconditional (plane indices are clamped to what the march uses, so at its ends they find
-    // the plane in the L2; the copies are never used): the compiler's wait-count bookkeeping is exact only on
-    // branch-free paths.
-    // (the fused pointwise mode has no registers to spare for the second set and runs one plane ahead)
-    // Planes in flight per workgroup: measured at (1,C,350,350,128), one plane ahead is faster with 8 and with 64
-    // channels per slab (C = 8: 4 % for the plain kernel, 10 % with the statistics; C = 64, 128: 1 %), two planes
-    // ahead with 16 and 32 (1-2 %), and three are slower everywhere: more planes in flight spread the workgroups
-    // of a group further apart, and the halo lines they share leave the L2 before the neighbour asks for them.
-    constexpr int AHEAD = MODE == 2 ? 1 : (SC == 8 || (SC == 64 && MODE != 3)) ? 1 : 2;
-    half8_t xpre0[NLDX], xpre1[NLDX];
+    // Global loads run one plane ahead of the arithmetic.  They are unconditional; planes outside the volume or past the
+    // march's last one have no bytes (see plane_rsrc).  So is the store behind them: a step waits for the loads of its
+    // plane and leaves the store of the step before in flight.  (With a condition around the store the compiler waited
+    // for it too: us before -> now, C = 16 / 64 at (2,C,45,51,37) 9.8 -> 9.0 / 15.9 -> 14.5, at (1,C,350,350,128)
+    // 203 -> 200 / 696 -> 688.)  Two planes ahead, in two register sets, are slower: (1,C,350,350,128) C = 8 / 32 / 64
+    // 102 / 375 / 733 us, 100 / 360 / 689 with one: the workgroups of a group spread further apart, and the halo lines
+    // they share leave the L2 before the neighbour asks for them.
+    half8_t xpre[NLDX];
     const int hp_last = min(he, H - 1);
-    auto prefetch = [&](int hp, half8_t(&xpre)[NLDX]) {
-        const char* xplane = reinterpret_cast<const char*>(xn + min(max(hp, 0), hp_last) * plane_stride);
+    auto prefetch = [&](int hp) {
+        const bool used = (hp >= 0) && (hp <= hp_last);
+        const plane_rsrc_t r = plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(xn + (used ? hp : 0) * plane_stride)),
+                                          used ? plane_bytes : 0u);
 #pragma unroll
         for (int j = 0; j < NLDX; ++j) {
             // nobody else reads the interior chunks: with the hint they do not push shared lines out of the L2
             if (NTI && Order::interior_only(j * NT))
-                xpre[j] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(xplane + xgo[j]));
+                xpre[j] = plane_load16<true>(r, xgo[j]);
             else
-                xpre[j] = *reinterpret_cast<const half8_t*>(xplane + xgo[j]);
+                xpre[j] = plane_load16<false>(r, xgo[j]);
         }
     };
 
     int parity = 0;
-    auto step = [&](auto ring, int hp, half8_t(&xpre)[NLDX], auto tail) {
+    // `out` (fused pointwise mode): whether the step has an output plane, all but the first two do
+    auto step = [&](auto ring, int hp, auto out) {
         constexpr int DONE = (decltype(ring)::value + 3) & 3;  // register of output plane hp-1, complete after this step
         const bool xin = (hp >= 0) && (hp < H);  // wavefront-uniform
         unsigned char* xbuf = smem + parity * XSLOT;
 #pragma unroll
         for (int j = 0; j < NLDX; ++j) {
-            unsigned char* dst = xls[j] >= 0 ? xbuf + xls[j] : smem + Cfg::DUMP;
-            *reinterpret_cast<half8_t*>(dst) = xpre[j];
+            *reinterpret_cast<half8_t*>(xbuf + xls[j]) = xpre[j];
         }
         __syncthreads();
         // The loads of the next plane go out first and at raised wave priority, the stores of the finished plane
@@ -670,7 +684,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         // path, and loads queued behind other wavefronts' stores reach memory late (measured at C = 64: 0.703 ->
         // 0.694 ms; the same order without the priority, or the priority without the order, changes nothing).
         __builtin_amdgcn_s_setprio(3);
-        if (!decltype(tail)::value || hp + AHEAD <= hp_last) prefetch(hp + AHEAD, xpre);
+        prefetch(hp + 1);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(0);
         flush_row(parity ^ 1);
@@ -697,7 +711,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         }
         // register DONE of every tile is the finished output plane hp-1
         const int ho = hp - 1;
-        const bool finished = ho >= hs;
+        const bool finished = MODE == 2 ? decltype(out)::value : ho >= hs;
         pending_row = finished ? ho : -1;
         if (finished) {  // workgroup-uniform
             unsigned char* otile = smem + OT_OFF + parity * OT_BYTES;
@@ -764,21 +778,24 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
                     }
                 }
                 __syncthreads();
-                half_t* y2plane = yn2 + (int64_t)ho * W * D * COUT;
+                const plane_rsrc_t r2 =
+                    plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(yn2 + (int64_t)ho * W * D * COUT)), y2_bytes);
 #pragma unroll
-                for (int c = t; c < NPOS * (COUT / 8); c += NT) {
-                    const int row = c / (COUT / 8), cc = c - row * (COUT / 8);
-                    const int w = w0 + row / TD, d = d0 + row % TD;
-                    if (w < W && d < D) {
-                        const half4_t lo = *reinterpret_cast<const half4_t*>(yt + row * RY + cc * 8);
-                        const half4_t hi = *reinterpret_cast<const half4_t*>(yt + row * RY + cc * 8 + 4);
-                        const half8_t o8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                for (int i = 0; i < NY2; ++i) {
+                    const int c = t + i * NT, row = c / (COUT / 8), cc = c - row * (COUT / 8);
+                    const half4_t lo = *reinterpret_cast<const half4_t*>(yt + row * RY + cc * 8);
+                    const half4_t hi = *reinterpret_cast<const half4_t*>(yt + row * RY + cc * 8 + 4);
+                    const half8_t o8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
-                        for (int jj = 0; jj < 8; ++jj) amax = fmaxf(amax, fabsf((float)o8[jj]));
-                        store_c8_nt(y2plane + ((int64_t)w * D + d) * COUT + cc * 8, o8);
-                    }
+                    for (int jj = 0; jj < 8; ++jj)
+                        amax = fmaxf(amax, y2go[i] != kNoVoxel ? fabsf((float)o8[jj]) : 0.0f);
+                    plane_store16<true>(r2, y2go[i], o8);
                 }
             }
+        } else if constexpr (MODE == 2) {
+            // as many stores, here of nothing, as a step with an output has
+#pragma unroll
+            for (int i = 0; i < NY2; ++i) plane_store16<true>(plane_rsrc(a.y2, 0u), kNoVoxel, half8_t{});
         }
         // the finished register rests for one step (its lane has zero weights then) and starts its next plane
         // from zero; the weights move on by one lane
@@ -793,29 +810,32 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         parity ^= 1;
     };
 
-    prefetch(hs - 1, xpre0);
-    if (AHEAD >= 2) prefetch(hs, xpre1);
-    __syncthreads();  // the one-off zero fill is complete before staging writes anything
-    // The steps hp = hs-1 .. he run in groups of four (the period of the accumulator ring; the register sets
-    // alternate inside a group), in a loop whose only exit is at its end: an exit between two steps would give the
-    // loop a second way into its first step, on which the newest set is the oldest, and the compiler's wait before
-    // that step's staging writes would cover every load in flight.  The one to three steps that are left follow the
-    // loop in code of their own and load what they need (running a fourth of a group on empty cost a short march up to
-    // 3 us: (1,64,30,128,128) in chunks of 15 rows 30.6 -> 29.2 us).
+    // (with a store behind it, here of nothing, as in the loop: the waits are then the same on both ways into it)
+    prefetch(hs - 1);
+    flush_row(1);
+    // The steps hp = hs-1 .. he; a group of four is the period of the accumulator ring.  Whatever step a march ends with,
+    // the accesses in flight are the same, so the waits stay exact.  (Rounding a march up to whole groups cost a short one
+    // up to 3 us: (1,64,30,128,128) in chunks of 15 rows 30.6 -> 29.2 us.)
     using std::integral_constant;
-    constexpr std::false_type loop{};
-    constexpr std::true_type tail{};
-    half8_t(&xodd)[NLDX] = AHEAD == 1 ? xpre0 : xpre1;
+    constexpr std::true_type yes{};
     int hp = hs - 1;
-    for (; hp + 3 <= he; hp += 4) {
-        step(integral_constant<int, 0>{}, hp, xpre0, loop);
-        step(integral_constant<int, 1>{}, hp + 1, xodd, loop);
-        step(integral_constant<int, 2>{}, hp + 2, xpre0, loop);
-        step(integral_constant<int, 3>{}, hp + 3, xodd, loop);
+    constexpr int R0 = MODE == 2 ? 2 : 0;  // ring position of the loop's first step
+    if constexpr (MODE == 2) {
+        // (steps without an output in code of their own: in the loop the stores stand behind no condition)
+        step(integral_constant<int, 0>{}, hp, std::false_type{});
+        step(integral_constant<int, 1>{}, hp + 1, std::false_type{});
+        hp += 2;
     }
-    if (hp <= he) step(integral_constant<int, 0>{}, hp, xpre0, tail);
-    if (hp + 1 <= he) step(integral_constant<int, 1>{}, hp + 1, xodd, tail);
-    if (hp + 2 <= he) step(integral_constant<int, 2>{}, hp + 2, xpre0, tail);
+    for (;; hp += 4) {
+        step(integral_constant<int, R0>{}, hp, yes);
+        if (hp + 1 > he) break;
+        step(integral_constant<int, R0 + 1>{}, hp + 1, yes);
+        if (hp + 2 > he) break;
+        step(integral_constant<int, (R0 + 2) % 4>{}, hp + 2, yes);
+        if (hp + 3 > he) break;
+        step(integral_constant<int, (R0 + 3) % 4>{}, hp + 3, yes);
+        if (hp + 4 > he) break;
+    }
     if constexpr (BOUNCE) {
         __syncthreads();
         flush_row(parity ^ 1);
