@@ -33,19 +33,16 @@ struct PwCfg {
     static_assert(CIN % 16 == 0 && CIN <= 128, "CIN in {16,32,64,128}");
     static_assert(COUT % 16 == 0 && COUT <= 128, "COUT in {16,32,64,128}");
     // Workgroups per compute unit of the persistent loop: as few as keep the memory pipe full, which also have the fewest
-    // prologues.  With a residual three up to 64 channels (CIN + COUT), whose tiles have the fewest bytes in flight, two
-    // above (us with 2 / 3 / 4 / 8: 16 -> 16 at 2.1 M voxels 39.4 / 34.1 / 34.5 / 36.0, 32 -> 32 at 0.9 M 31.1 / 30.4 /
-    // 31.1, 16 -> 64 at 0.9 M 43.6 / 44.7 / 44.8, 64 -> 128 at 0.35 M 40.0 / 41.5 / 41.5 / 41.5; more than fit the LDS,
-    // as four at 64 -> 128, also leave a second round that fills a part of the chip).  Widening from few channels three
-    // again in volumes above 3 M voxels (16 -> 64 at 15.7 M 814 / 763 / 767, 32 -> 64 888 / 858 / 843).
+    // prologues.  With a residual two, at 16 -> 16, whose tiles have the fewest bytes, three (us with 2 / 3 / 4: 16 -> 16 at
+    // 0.9 M voxels 16.3 / 15.7 / 15.8, 32 -> 32 at 0.9 M 29.7 / 31.4 / 31.4 and at 4 M 126 / 136 / 139, 64 -> 32 at 2 M
+    // 84.8 / 91.3 / 89.9, 64 -> 128 at 0.9 M 99.0 / 100.2 / 99.3, 16 -> 64 at 4 M 197 / 198 / 200).
     // Without a residual a tile has half the bytes: four, where their LDS fits (64 -> 128, 0.1 M voxels 16.1 with four,
     // 13.2 with the three that fit, 4 M 284 and 285; 128 -> 128 24.3 with four, 18.6 with the two that fit, 4 M 387 and 391).
     static constexpr int LDS_BYTES = kPwWaves * TILE_HALVES * 2 + MT * KS * 64 * 16 + 2 * CIN * 4 + 64;
     static constexpr int FITS = 160 * 1024 / LDS_BYTES;
     static int64_t workgroups(int64_t V, bool add)
     {
-        const bool three = CIN + COUT <= 64 || (CIN < COUT && CIN + COUT < 128 && V > 3 << 20);
-        const int per_cu = add ? (three ? 3 : 2) : (FITS < 4 ? FITS : 4);
+        const int per_cu = add ? (CIN + COUT == 32 ? 3 : 2) : (FITS < 4 ? FITS : 4);
         return std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kPwWaves), (int64_t)per_cu * device_geometry().cus));
     }
 };
@@ -68,14 +65,76 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
     __shared__ float red[kPwWaves];
     __shared__ __attribute__((aligned(16))) float aff[AFFINE ? 2 * CIN : 4];  // [scale | shift]
 
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    const int t = threadIdx.x, lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
     const int vl = lane % 32, hl = lane / 32;
+    const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
-    // A fragments: wfrag[((mt*KS + s)*64 + l)*8 + j] = Wm[16 s + 8 (l/32) + j][32 mt + l%32]
-    for (int i = t; i < MT * KS * 64 * 8; i += kPwThreads) {
-        const int j = i % 8, l = (i / 8) % 64, s = (i / 512) % KS, mt = i / (512 * KS);
-        const int co = 32 * mt + l % 32;
-        wfrag[i] = (co < COUT) ? Wm[(16 * s + 8 * (l / 32) + j) * COUT + co] : (half_t)0;
+    // The rows of Wm, 16 bytes at a time and all at once; they go to LDS behind the first tile's loads: one trip to memory
+    // for both (two-byte loads ahead of everything else: 32 -> 32 at 50000 voxels with residual 5.1 us, now 4.0; 64 -> 128
+    // 11.5, 8.2; 128 -> 128 15.8, 12.4).
+    constexpr int NWC = CIN * COUT / 8, NLW = (NWC + kPwThreads - 1) / kPwThreads;
+    const plane_rsrc_t wr = plane_rsrc(Wm, CIN * COUT * 2);
+    half8_t wpre[NLW];
+#pragma unroll
+    for (int i = 0; i < NLW; ++i) wpre[i] = plane_load16<false>(wr, (uint32_t)(t + i * kPwThreads) * 16);
+
+    float amax = 0.0f;
+    const int64_t ntiles = (V + 31) / 32;
+    const int64_t tiles_per_round = (int64_t)gridDim.x * kPwWaves;
+    const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
+    unsigned char* my = reinterpret_cast<unsigned char*>(tile[wave]);
+
+    // The tile's part of a tensor with `row` bytes per voxel; voxels past V and tiles past the last have no bytes (loads give
+    // zeros, stores are dropped), so nothing stands behind a condition and the compiler's waits are exact: a tile's x
+    // fragments are waited for with the stores of the one before in flight.
+    auto tile_rsrc = [&](const half_t* p, int64_t tidx, int row) {
+        const int64_t v0 = tidx < ntiles ? tidx * 32 : 0;
+        const int rows = tidx < ntiles ? (int)std::min<int64_t>(V - v0, 32) : 0;
+        return plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(p) + v0 * row), (uint32_t)(rows * row));
+    };
+    // B fragments of a tile: this lane's voxel, chunks 2q+hl
+    half8_t xb[KS], xn[KS];
+    auto load_x = [&](int64_t tidx, half8_t(&xb)[KS]) {
+        const plane_rsrc_t r = tile_rsrc(x, tidx, 2 * CIN);
+        // a load instruction touches 32 bytes of every voxel row: rows of 128 bytes and more need the cache to hold the
+        // line until the row's other loads arrive, so only narrow rows stream
+#pragma unroll
+        for (int q = 0; q < KS; ++q) xb[q] = plane_load16<(CIN <= 32)>(r, (uint32_t)(vl * 2 * CIN + 16 * (2 * q + hl)));
+    };
+    // residual chunks of a tile, in the order in which the results leave the LDS tile
+    constexpr int NC = Cfg::OUT_CHUNKS / kWave;
+    half8_t ab[HAS_ADD ? NC : 1];
+    // Without a residual the loads of the next tile are issued before this tile's arithmetic and stores.  With one they
+    // are issued as soon as this tile has used its registers: the x fragments behind the matrix instructions, a residual
+    // chunk behind the store of its sum.  Both streams of a tile are then in flight while the previous one is stored.
+    // (Loading a residual chunk where it is added costs one memory latency per chunk: 64 -> 128 channels with residual
+    // at 0.88 M voxels 130 us, now 103, i.e. 4.4 and 5.5 TB/s; 128 -> 128 at 0.26 M 54 and 39 us.)
+    const int64_t first = (int64_t)blockIdx.x * kPwWaves + wave;
+    load_x(first, xb);
+    // (with the loads and stores in the order of the loop, stores of nothing, so that the waits are the same on both ways
+    // into it)
+    {
+        const plane_rsrc_t ar = tile_rsrc(add, first, 2 * COUT);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            plane_store16<true>(plane_rsrc(out, 0u), 0u, z8);
+            if constexpr (HAS_ADD) ab[k] = plane_load16<true>(ar, (uint32_t)(k * kWave + lane) * 16);
+        }
+    }
+    // A fragments: wfrag[((mt*KS + s)*64 + l)*8 + j] = Wm[16 s + 8 (l/32) + j][32 mt + l%32]; 16 output channels fill half
+    // a block, the other half is zero
+#pragma unroll
+    for (int i = 0; i < NLW; ++i) {
+        const int c = t + i * kPwThreads, ci = c * 8 / COUT, co = c * 8 % COUT;
+        if (c < NWC) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                wfrag[((co / 32 * KS + ci / 16) * 64 + ci % 16 / 8 * 32 + co % 32 + j) * 8 + ci % 8] = wpre[i][j];
+        }
+    }
+    if constexpr (COUT == 16) {
+        for (int i = t; i < KS * 32; i += kPwThreads)
+            *reinterpret_cast<half8_t*>(wfrag + ((i / 32 * 64 + i % 32 / 16 * 32 + 16 + i % 16) * 8)) = z8;
     }
     if constexpr (AFFINE) {
         for (int i = t; i < CIN; i += kPwThreads) {
@@ -85,53 +144,11 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
     }
     __syncthreads();
     const half8_t* wa = reinterpret_cast<const half8_t*>(wfrag) + lane;
-
-    float amax = 0.0f;
-    const int64_t ntiles = (V + 31) / 32;
-    const int64_t tiles_per_round = (int64_t)gridDim.x * kPwWaves;
-    const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
-    unsigned char* my = reinterpret_cast<unsigned char*>(tile[wave]);
-
-    // B fragments of a tile: this lane's voxel, chunks 2q+hl.  A tile index past the end reads the last voxel (the
-    // loads are unconditional, the tile is then never used).
-    half8_t xb[KS], xn[KS];
-    auto load_x = [&](int64_t tidx, half8_t(&xb)[KS]) {
-        int64_t v = tidx * 32 + vl;
-        if (v >= V) v = V - 1;  // ragged last tile: clamp the read, the write is masked
-#pragma unroll
-        for (int q = 0; q < KS; ++q) {
-            // a load instruction touches 32 bytes of every voxel row: rows of 128 bytes and more need the
-            // cache to hold the line until the row's other loads arrive, so only narrow rows stream
-            if constexpr (CIN <= 32) xb[q] = load_c8_nt(x + v * CIN + 8 * (2 * q + hl));
-            else xb[q] = load_c8(x + v * CIN + 8 * (2 * q + hl));
-        }
-    };
-    // residual chunks of a tile, in the order in which the results leave the LDS tile; the same clamp
-    constexpr int NC = Cfg::OUT_CHUNKS / kWave;
-    half8_t ab[HAS_ADD ? NC : 1];
-    auto load_add = [&](int64_t tidx, int k) {
-        const int c = k * kWave + lane;
-        int64_t v = tidx * 32 + c / (COUT / 8);
-        if (v >= V) v = V - 1;
-        ab[k] = load_c8_nt(add + v * COUT + (c % (COUT / 8)) * 8);
-    };
-    // Without a residual the loads of the next tile are issued before this tile's arithmetic and stores.  With one they
-    // are issued as soon as this tile has used its registers: the x fragments behind the matrix instructions, a residual
-    // chunk behind the store of its sum.  Both streams of a tile are then in flight while the previous one is stored.
-    // (Loading a residual chunk where it is added costs one memory latency per chunk: 64 -> 128 channels with residual
-    // at 0.88 M voxels 130 us, now 103, i.e. 4.4 and 5.5 TB/s; 128 -> 128 at 0.26 M 54 and 39 us.)
-    const int64_t first = (int64_t)blockIdx.x * kPwWaves + wave;
-    load_x(first, xb);
-    if constexpr (HAS_ADD) {
-#pragma unroll
-        for (int k = 0; k < NC; ++k) load_add(first, k);
-    }
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kPwWaves + wave;
-        const bool live = tidx < ntiles;
         const int64_t v0 = tidx * 32;
         if constexpr (!HAS_ADD) load_x(tidx + tiles_per_round, xn);
-        if (live) {
+        {
             if constexpr (AFFINE) {
 #pragma unroll
                 for (int q = 0; q < KS; ++q) {
@@ -148,7 +165,6 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
                 }
             }
             if (RELU_IN) {
-                const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
                 for (int q = 0; q < KS; ++q) xb[q] = __builtin_elementwise_max(xb[q], z8);  // packed maximum
             }
@@ -183,25 +199,23 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (live) {
+        const plane_rsrc_t outr = tile_rsrc(out, tidx, 2 * COUT), addr = tile_rsrc(add, tidx + tiles_per_round, 2 * COUT);
 #pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                const int c = k * kWave + lane;
-                const int row = c / (COUT / 8), cc = c % (COUT / 8);
-                half8_t o = Tile::read(my, row, cc);
-                if constexpr (HAS_ADD) {
+        for (int k = 0; k < NC; ++k) {
+            const int c = k * kWave + lane;
+            const int row = c / (COUT / 8), cc = c % (COUT / 8);
+            half8_t o = Tile::read(my, row, cc);
+            if constexpr (HAS_ADD) {
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)o[j] + (float)ab[k][j]);  // fp16 add, RNE
-                }
-                if (v0 + row < V) {
-                    if (ABSMAX) {
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf((float)o[j]));
-                    }
-                    store_c8_nt(out + (v0 + row) * COUT + cc * 8, o);
-                }
-                if constexpr (HAS_ADD) load_add(tidx + tiles_per_round, k);
+                for (int j = 0; j < 8; ++j) o[j] = (half_t)((float)o[j] + (float)ab[k][j]);  // fp16 add, RNE
             }
+            if (ABSMAX) {
+                const bool inside = v0 + row < V;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) amax = fmaxf(amax, inside ? fabsf((float)o[j]) : 0.0f);
+            }
+            plane_store16<true>(outr, (uint32_t)c * 16, o);
+            if constexpr (HAS_ADD) ab[k] = plane_load16<true>(addr, (uint32_t)c * 16);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
