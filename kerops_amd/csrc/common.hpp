@@ -153,6 +153,15 @@ __device__ __forceinline__ void plane_store16(plane_rsrc_t r, uint32_t voff, hal
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, (int)voff, 0, STREAM ? 2 : 0);
 }
 
+// The rows [v0, v0 + rows) of a [V][row_bytes / 2] tensor; rows that do not exist (past V, or v0 < 0) have no bytes, so a
+// tile's accesses stand behind no condition.  (v0 wavefront-uniform, rows * row_bytes < 2^31)
+__device__ __forceinline__ plane_rsrc_t rows_rsrc(const half_t* p, int64_t v0, int rows, int64_t V, int row_bytes)
+{
+    const bool some = v0 >= 0 && v0 < V;
+    const int n = some ? (int)std::min<int64_t>(V - v0, rows) : 0;
+    return plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(p) + (some ? v0 : 0) * row_bytes), (uint32_t)(n * row_bytes));
+}
+
 constexpr int64_t kStreamInteriorMinBytes = 384ll << 20;
 
 // Order in which the 16-byte chunks of a staged plane (a TW x TD patch with its one-voxel halo, CG chunks per

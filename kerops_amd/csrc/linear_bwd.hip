@@ -204,14 +204,11 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
     }
 
     const int64_t ntiles = (V + Cfg::TILE - 1) / Cfg::TILE;
-    // The tile's part of a tensor with `row` bytes per voxel; rows past V and tiles past the last have no bytes, so nothing
-    // stands behind a condition and the wait for a tile's loads leaves the stores of the one before in flight (us with the
-    // conditions / now: 64 -> 64 at 0.05 / 0.9 M voxels 14.2 / 13.2, 66.5 / 64.3, with the batch-norm map at 0.9 M 77.8 / 73.0;
+    // The tile's part of a tensor with `row` bytes per voxel: nothing stands behind a condition and the wait for a tile's
+    // loads leaves the stores of the one before in flight (us with the conditions / now: 64 -> 64 at 0.05 / 0.9 M voxels 14.2 / 13.2, 66.5 / 64.3, with the batch-norm map at 0.9 M 77.8 / 73.0;
     // 128 -> 128 at 0.05 / 0.3 M 29.6 / 27.4, 60.9 / 56.5).
     auto tile_rsrc = [&](const half_t* p, int64_t tile, int row) {
-        const int64_t v0 = tile < ntiles ? tile * Cfg::TILE : 0;
-        const int rows = tile < ntiles ? (int)std::min<int64_t>(V - v0, Cfg::TILE) : 0;
-        return plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(p) + v0 * row), (uint32_t)(rows * row));
+        return rows_rsrc(p, tile * Cfg::TILE, Cfg::TILE, V, row);
     };
     half8_t xpre[NLX], gpre[NLG];
     auto prefetch = [&](int64_t tile) {  // (chunks past the tile: zeros)

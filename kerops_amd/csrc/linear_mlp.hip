@@ -38,7 +38,7 @@ struct MlpCfg {
     static_assert(C == 16 || C == 32 || C == 64, "C in {16,32,64}");
 };
 
-template <int C, bool EARLY>
+template <int C>
 __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const half_t* __restrict__ x,
                                                                         const half_t* __restrict__ Wup,
                                                                         const half_t* __restrict__ Wdown,
@@ -53,24 +53,32 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     half_t* a2 = reinterpret_cast<half_t*>(smem + Cfg::A2_OFF);
     half_t* bs = reinterpret_cast<half_t*>(smem + Cfg::B_OFF);
 
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    const int t = threadIdx.x, lane = t % kWave, wave = __builtin_amdgcn_readfirstlane(t / kWave);
     const int vl = lane % 32, hl = lane / 32;
 
     // a1[((mt*KS1 + s)*64 + l)*8 + j] = Wup[16 s + 8 (l/32) + j][32 mt + l%32]
-    for (int i = t; i < MT1 * KS1 * 64 * 8; i += kMlpThreads) {
-        const int j = i % 8, l = (i / 8) % 64, s = (i / 512) % KS1, mt = i / (512 * KS1);
-        a1[i] = Wup[(16 * s + 8 * (l / 32) + j) * HID + 32 * mt + l % 32];
-    }
     // a2[((mo*KS2 + s)*64 + l)*8 + j] = Wdown[hidden channel of (s = 2 mt + gp, l/32, j)][32 mo + l%32]
-    for (int i = t; i < MO * KS2 * 64 * 8; i += kMlpThreads) {
-        const int j = i % 8, l = (i / 8) % 64, s = (i / 512) % KS2, mo = i / (512 * KS2);
+    // All their loads are in flight at once and go to LDS behind the first tile's (the weights need not be aligned: two bytes
+    // each).  One after the other, ahead of the tile, they cost C = 32 at 20000
+    // voxels 1.9 us of 5.9, C = 64 at 5000 0.8 of 8.6.
+    constexpr int N1 = MT1 * KS1 * 512 / kMlpThreads, N2 = MO * KS2 * 512 / kMlpThreads;
+    static_assert(HID <= kMlpThreads, "a bias value per thread");
+    half_t w1[N1], w2[N2];
+#pragma unroll
+    for (int k = 0; k < N1; ++k) {
+        const int i = t + k * kMlpThreads, j = i % 8, l = (i / 8) % 64, s = (i / 512) % KS1, mt = i / (512 * KS1);
+        w1[k] = Wup[(16 * s + 8 * (l / 32) + j) * HID + 32 * mt + l % 32];
+    }
+#pragma unroll
+    for (int k = 0; k < N2; ++k) {
+        const int i = t + k * kMlpThreads, j = i % 8, l = (i / 8) % 64, s = (i / 512) % KS2, mo = i / (512 * KS2);
         const int mt = s / 2, gp = s % 2;
         const int ch = 32 * mt + 8 * (2 * gp + j / 4) + 4 * (l / 32) + j % 4;
         const int co = 32 * mo + l % 32;
-        a2[i] = co < C ? Wdown[ch * C + co] : (half_t)0;
+        const half_t w = Wdown[ch * C + co % C];
+        w2[k] = co < C ? w : (half_t)0;
     }
-    for (int i = t; i < HID; i += kMlpThreads) bs[i] = bias[i];
-    __syncthreads();
+    const half_t bias_t = bias[t % HID];
 
     const half8_t* a1f = reinterpret_cast<const half8_t*>(a1) + lane;
     const half8_t* a2f = reinterpret_cast<const half8_t*>(a2) + lane;
@@ -80,40 +88,39 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
     const int64_t ntiles = (V + 31) / 32;
     const int64_t tiles_per_round = (int64_t)gridDim.x * kMlpWaves;
     const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
-    // Loads of a tile (one past the end reads the last voxel and is never used): x fragments, and residual chunks in the
-    // order in which the results leave the LDS tile.  EARLY: those of the next tile are issued as soon as this tile has used
-    // the registers, so that both streams are in flight while the results are stored; loaded where they are used, a
-    // tile waits for memory twice (mlp_early has the figures).
+    // Loads of a tile: x fragments, and residual chunks in the order in which the results leave the LDS tile.  Those of the
+    // next tile are issued as soon as this tile has used the registers, so that both streams are in flight while the
+    // results are stored; loaded where they are used, a tile waits for memory twice (C = 64 at 0.1 M voxels 28.2 us, 18.0
+    // early, C = 32 9.0 and 7.8).  Nothing stands behind a condition (rows_rsrc), so a tile waits for its own loads and
+    // leaves the stores of the one before in flight (C = 16 at 0.9 M voxels 17.4 -> 16.2 us).
     constexpr int NC = 32 * C / 8 / kWave;
     half8_t xb[KS1], ab[NC];
     auto load_x = [&](int64_t tidx) {
-        int64_t v = tidx * 32 + vl;
-        if (v >= V) v = V - 1;  // ragged last tile: clamp the read, the write is masked
+        const plane_rsrc_t r = rows_rsrc(x, tidx * 32, 32, V, 2 * C);
+        // rows of 128 bytes need the cache to hold the line until the row's other loads arrive
 #pragma unroll
-        for (int s = 0; s < KS1; ++s) {
-            // rows of 128 bytes need the cache to hold the line until the row's other loads arrive
-            if constexpr (C <= 32) xb[s] = load_c8_nt(x + v * C + 16 * s + 8 * hl);
-            else xb[s] = load_c8(x + v * C + 16 * s + 8 * hl);
-        }
-    };
-    auto load_add = [&](int64_t tidx, int k) {
-        const int c = k * kWave + lane;
-        int64_t v = tidx * 32 + c / (C / 8);
-        if (v >= V) v = V - 1;
-        ab[k] = load_c8_nt(add + v * C + (c % (C / 8)) * 8);
+        for (int s = 0; s < KS1; ++s) xb[s] = plane_load16<(C <= 32)>(r, (uint32_t)(vl * 2 * C + 32 * s + 16 * hl));
     };
     const int64_t first = (int64_t)blockIdx.x * kMlpWaves + wave;
-    if constexpr (EARLY) {
-        load_x(first);
+    load_x(first);
+    {
+        // (with the loads and stores in the order of the loop, stores of nothing: the waits are the same on both ways in)
+        const plane_rsrc_t ar = rows_rsrc(add, first * 32, 32, V, 2 * C);
 #pragma unroll
-        for (int k = 0; k < NC; ++k) load_add(first, k);
+        for (int k = 0; k < NC; ++k) {
+            plane_store16<true>(plane_rsrc(out, 0u), 0u, half8_t{});
+            ab[k] = plane_load16<true>(ar, (uint32_t)(k * kWave + lane) * 16);
+        }
     }
+#pragma unroll
+    for (int k = 0; k < N1; ++k) a1[t + k * kMlpThreads] = w1[k];
+#pragma unroll
+    for (int k = 0; k < N2; ++k) a2[t + k * kMlpThreads] = w2[k];
+    if (t < HID) bs[t] = bias_t;
+    __syncthreads();
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kMlpWaves + wave;
-        const bool live = tidx < ntiles;  // wavefront-uniform
-        const int64_t v0 = tidx * 32;
-        if (live) {
-            if constexpr (!EARLY) load_x(tidx);
+        {
             // ---- first product, bias, ReLU: the B fragments of the second product ----
             half8_t hb[KS2];
 #pragma unroll
@@ -135,7 +142,7 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
                     }
                 }
             }
-            if constexpr (EARLY) load_x(tidx + tiles_per_round);
+            load_x(tidx + tiles_per_round);
             // ---- second product ----
 #pragma unroll
             for (int mo = 0; mo < MO; ++mo) {
@@ -159,33 +166,30 @@ __global__ __launch_bounds__(kMlpThreads) void lin_brelu_lin_add_kernel(const ha
             // ---- write-back of the wavefront's own tile: no other wavefront touches it, and the LDS
             // operations of one wavefront complete in issue order, so no workgroup barrier is needed ----
             __builtin_amdgcn_wave_barrier();
+            const plane_rsrc_t outr = rows_rsrc(out, tidx * 32, 32, V, 2 * C),
+                               addr = rows_rsrc(add, (tidx + tiles_per_round) * 32, 32, V, 2 * C);
 #pragma unroll
             for (int k = 0; k < NC; ++k) {
                 const int c = k * kWave + lane;
                 const int row = c / (C / 8), cc = c % (C / 8);
                 half8_t o = Tile::read(my, row, cc);
-                if constexpr (!EARLY) load_add(tidx, k);
 #pragma unroll
                 for (int jj = 0; jj < 8; ++jj) o[jj] = (half_t)((float)o[jj] + (float)ab[k][jj]);  // fp16 add, RNE
-                if (v0 + row < V) store_c8_nt(out + (v0 + row) * C + cc * 8, o);
-                if constexpr (EARLY) load_add(tidx + tiles_per_round, k);
+                plane_store16<true>(outr, (uint32_t)c * 16, o);
+                ab[k] = plane_load16<true>(addr, (uint32_t)c * 16);
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
 }
 
-// Early loads (us with them and the best workgroup count / with late loads and four workgroups per compute unit): C = 16 at
-// 4096 voxels 3.1 / 3.2, 1 M 18.8 / 20.0, 15.7 M 252 / 265; C = 64 at 0.1 M 18.0 / 28.2, 15.7 M 1079 / 1381; C = 32 at
-// 4096 4.6 / 4.8, 0.1 M 7.9 / 9.0, 0.4 M 18.2 / 19.3, 1 M 37.4 / 38.2, 2 M 69.1 / 69.3, 2.5 M 86.8 / 87.0, 3 M 103.1 /
-// 101.9, 4 M 137.3 / 135.2, 15.7 M 534 to 552 / 528 to 533: there four workgroups hide the second wait as well, and volumes
-// above 2.6 M voxels load late.
-static bool mlp_early(int64_t V, int C) { return C != 32 || V <= 5 << 19; }
-// Workgroups per compute unit with early loads (us with 2 / 3 / 4: C = 16 at 2.0 M voxels 39.6 / 34.2 / 33.5, C = 32 at
-// 0.1 M 8.2 / 8.3 / 9.2 and at 2.0 M 71.3 / 68.5 / 70.2, C = 64 at 2.0 M 142 / 148 / 156)
+// Workgroups per compute unit.  A workgroup begins with its weights, which small volumes notice most (us with 1 / 2 / 3):
+// C = 64 at 45000 voxels 10.9 / 12.8 / 13.0, 0.16 M 19.0 / 20.5 / 22.8, 0.2 M 24.1 / 23.5 / 27.1, 2.0 M 161 / 139 / 145;
+// C = 32 at 0.1 M 7.9 / 7.4 / 8.6, 0.9 M 39.4 / 31.9 / 33.9, 4.0 M 164 / 133 / 139; C = 16 (2 / 3 / 4) at 0.1 M 4.6 / 5.1
+// / 5.1, 0.25 M 7.2 / 6.8 / 7.6, 0.9 M 17.5 / 16.7 / 16.3, 2.0 M 34.7 / 33.6 / 33.5
 static int mlp_blocks(int64_t V, int C)
 {
-    const int64_t per_cu = C == 64 ? 2 : C == 32 && mlp_early(V, C) ? 3 : 4;
+    const int64_t per_cu = C == 64 ? (V < 180000 ? 1 : 2) : C == 32 || V < 140000 ? 2 : V < 500000 ? 3 : 4;
     return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kMlpWaves), per_cu * device_geometry().cus));
 }
 
@@ -206,17 +210,16 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
     }
     const int blocks = mlp_blocks(V, C);
     hipStream_t s = (hipStream_t)stream;
-#define KEROPS_MLP_CASE(CV, EARLY)                                                                                      \
-    if (C == CV && mlp_early(V, C) == EARLY) {                                                                          \
-        hipLaunchKernelGGL((lin_brelu_lin_add_kernel<CV, EARLY>), dim3(blocks), dim3(kMlpThreads), 0, s, (const half_t*)x, \
-                           (const half_t*)Wup, (const half_t*)Wdown, (const half_t*)bias, (const half_t*)add,            \
-                           (half_t*)out, V);                                                                             \
-        return check_launch("lin_brelu_lin_add");                                                                       \
+#define KEROPS_MLP_CASE(CV)                                                                                        \
+    if (C == CV) {                                                                                                 \
+        hipLaunchKernelGGL((lin_brelu_lin_add_kernel<CV>), dim3(blocks), dim3(kMlpThreads), 0, s, (const half_t*)x, \
+                           (const half_t*)Wup, (const half_t*)Wdown, (const half_t*)bias, (const half_t*)add,       \
+                           (half_t*)out, V);                                                                        \
+        return check_launch("lin_brelu_lin_add");                                                                  \
     }
-    KEROPS_MLP_CASE(16, true)
-    KEROPS_MLP_CASE(32, true)
-    KEROPS_MLP_CASE(32, false)
-    KEROPS_MLP_CASE(64, true)
+    KEROPS_MLP_CASE(16)
+    KEROPS_MLP_CASE(32)
+    KEROPS_MLP_CASE(64)
 #undef KEROPS_MLP_CASE
     set_error("lin_brelu_lin_add: built for C in {16,32,64} (got %d)", C);
     return KEROPS_E_UNSUPPORTED_C;
@@ -245,7 +248,7 @@ extern "C" int kerops_lin_brelu_lin_add_f16(const void* x, const void* Wup, cons
 // the LDS holds two workgroups per compute unit.  Partials go to the workspace, a second kernel adds them in a fixed order
 // (fp64): deterministic, no atomics.
 // Two workgroups of 256 registers per lane; with operands read from LDS in 2-byte pieces and the weights in LDS, one
-// workgroup per compute unit, the op with its reduction took 721 us at 1.96 M voxels, now 267 (its HBM traffic at 6 TB/s:
+// workgroup per compute unit, the op with its reduction took 721 us at 1.96 M voxels, now 247 (its HBM traffic at 6 TB/s:
 // 125 us).
 namespace kerops {
 
@@ -303,10 +306,15 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_kernel(const
         a3[s] = load_c8(Wdown + (32 * wave + il) * C + 16 * s + 8 * hl);                        // Wdown g^T
     }
     half8_t* a6w = reinterpret_cast<half8_t*>(smem + Cfg::A6_OFF);  // dx^T = Wup lg^T
-    for (int i = t; i < Cfg::MO * KH * 64; i += kMlpThreads) {
-        const int l = i % 64, s = (i / 64) % KH, m = i / (64 * KH);
-        a6w[i] = load_c8(Wup + (32 * m + l % 32) * H + 16 * s + 8 * (l / 32));
+    constexpr int N6 = Cfg::MO * KH * 64 / kMlpThreads;
+    half8_t w6[N6];
+#pragma unroll
+    for (int k = 0; k < N6; ++k) {
+        const int i = t + k * kMlpThreads, l = i % 64, s = (i / 64) % KH, m = i / (64 * KH);
+        w6[k] = load_c8(Wup + (32 * m + l % 32) * H + 16 * s + 8 * (l / 32));
     }
+#pragma unroll
+    for (int k = 0; k < N6; ++k) a6w[t + k * kMlpThreads] = w6[k];
     const half8_t* a6 = a6w + mo * KH * 64 + lane;  // (the barrier behind the first staging covers it)
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq)
@@ -329,22 +337,23 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_kernel(const
     }
 
     const int64_t ntiles = (V + TILE - 1) / TILE;
+    // (nothing behind a condition, see rows_rsrc: a tile waits for its loads and leaves the stores of the one before in
+    // flight: 273 -> 247 us at 2.0 M voxels)
     half8_t xpre[NLX], gpre[NLX];
     auto prefetch = [&](int64_t tile) {
-        const int64_t v0 = tile * TILE;
+        const plane_rsrc_t xr = rows_rsrc(x, tile * TILE, TILE, V, 2 * C), gr = rows_rsrc(g, tile * TILE, TILE, V, 2 * C);
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
-            const int c = t + j * kMlpThreads;
-            const int64_t v = v0 + c / (C / 8);
-            xpre[j] = v < V ? load_c8_nt(x + v * C + (c % (C / 8)) * 8) : z8;
-            gpre[j] = v < V ? load_c8_nt(g + v * C + (c % (C / 8)) * 8) : z8;
+            xpre[j] = plane_load16<true>(xr, (uint32_t)(t + j * kMlpThreads) * 16);
+            gpre[j] = plane_load16<true>(gr, (uint32_t)(t + j * kMlpThreads) * 16);
         }
     };
 
     int64_t tile = blockIdx.x;
-    if (tile < ntiles) prefetch(tile);
+    prefetch(tile);
+#pragma unroll
+    for (int j = 0; j < NLX; ++j) plane_store16<true>(plane_rsrc(dx, 0u), 0u, z8);  // (of nothing: as many as a tile's)
     for (; tile < ntiles; tile += gridDim.x) {
-        const int64_t v0 = tile * TILE;
         // ---- stage the tile (rows past V are zero: they add nothing to the reductions) ----
         // (the previous tile's x and g were last read before the barrier in front of its write-back)
 #pragma unroll
@@ -355,7 +364,7 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_kernel(const
             *reinterpret_cast<half8_t*>(gs + off) = gpre[j];
         }
         __syncthreads();
-        if (tile + gridDim.x < ntiles) prefetch(tile + gridDim.x);
+        prefetch(tile + gridDim.x);
 
         // ---- phase A: hid and lg, 32 voxels x 32 hidden channels at a time ----
 #pragma unroll 1  // (unrolled, the offsets of both halves cost spilled registers)
@@ -437,11 +446,12 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_kernel(const
         __syncthreads();
 
         // ---- phase C: dx write-back, 16-byte chunks (the dx tile is written next behind two barriers) ----
+        const plane_rsrc_t dr = rows_rsrc(dx, tile * TILE, TILE, V, 2 * C);
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
             const int c = t + j * kMlpThreads;
             const int row = c / (C / 8), cc = c % (C / 8);
-            if (v0 + row < V) store_c8_nt(dx + (v0 + row) * C + cc * 8, BounceTile<C>::read(ds, row, cc));
+            plane_store16<true>(dr, (uint32_t)c * 16, BounceTile<C>::read(ds, row, cc));
         }
     }
 
@@ -832,24 +842,35 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_tr_kernel(
     const int t = threadIdx.x, lane = t % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(t / kWave);  // scalar: tile indices stay wavefront-uniform
     const int il = lane % 32, hl = lane / 32;
-    const half8_t z8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
     // hidden channel (within a block of 32) that element j of reduction group `half` of lane half hl holds
     auto hperm = [](int half, int hl_, int j) { return 16 * half + 8 * (j / 4) + 4 * hl_ + j % 4; };
 
-    for (int i = t; i < MH * KC * 512; i += kMlpThreads) {
-        const int j = i % 8, l = (i / 8) % 64, s = (i / 512) % KC, mh = i / (512 * KC);
-        f1w[i] = Wup[(16 * s + 8 * (l / 32) + j) * H + 32 * mh + l % 32];
+    // (all loads in flight at once)
+    {
+        constexpr int N1 = MH * KC * 512 / kMlpThreads, N3 = 2 * MH * 512 / kMlpThreads;
+        static_assert(MH * KC * 64 == kMlpThreads && H <= kMlpThreads, "one chunk of Wdown, at most one bias value per thread");
+        half_t w1[N1], w3[N3];
+#pragma unroll
+        for (int k = 0; k < N1; ++k) {
+            const int i = t + k * kMlpThreads, j = i % 8, l = (i / 8) % 64, s = (i / 512) % KC, mh = i / (512 * KC);
+            w1[k] = Wup[(16 * s + 8 * (l / 32) + j) * H + 32 * mh + l % 32];
+        }
+#pragma unroll
+        for (int k = 0; k < N3; ++k) {
+            const int i = t + k * kMlpThreads, j = i % 8, l = (i / 8) % 64, f = i / 512;
+            w3[k] = Wup[(l % 32) * H + 32 * (f / 2) + hperm(f % 2, l / 32, j)];
+        }
+        const int l2 = t % 64, s2 = (t / 64) % KC, mh2 = t / (64 * KC);
+        const half8_t w2 = load_c8(Wdown + (32 * mh2 + l2 % 32) * C + 16 * s2 + 8 * (l2 / 32));
+        const half_t bias_t = bias[t % H];
+#pragma unroll
+        for (int k = 0; k < N1; ++k) f1w[t + k * kMlpThreads] = w1[k];
+#pragma unroll
+        for (int k = 0; k < N3; ++k) f3w[t + k * kMlpThreads] = w3[k];
+        reinterpret_cast<half8_t*>(smem + Cfg::F2_OFF)[t] = w2;
+        if (t < H) bsh[t] = bias_t;
     }
-    for (int i = t; i < MH * KC * 64; i += kMlpThreads) {
-        const int l = i % 64, s = (i / 64) % KC, mh = i / (64 * KC);
-        reinterpret_cast<half8_t*>(smem + Cfg::F2_OFF)[i] = load_c8(Wdown + (32 * mh + l % 32) * C + 16 * s + 8 * (l / 32));
-    }
-    for (int i = t; i < 2 * MH * 512; i += kMlpThreads) {
-        const int j = i % 8, l = (i / 8) % 64, f = i / 512;
-        f3w[i] = Wup[(l % 32) * H + 32 * (f / 2) + hperm(f % 2, l / 32, j)];
-    }
-    for (int i = t; i < H; i += kMlpThreads) bsh[i] = bias[i];
     __syncthreads();
 
     const half8_t* f1 = reinterpret_cast<const half8_t*>(smem + Cfg::F1_OFF) + lane;
@@ -907,59 +928,46 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_tr_kernel(
     const int64_t stride = (int64_t)gridDim.x * kMlpWaves;
     half8_t xn[KC], gn[KC];
     // one instruction fetches 16 whole rows (1 KB): lane -> 16-byte chunk lane % 4 of voxel 16 s + lane / 4
-    // (rows past V read the last voxel and are zeroed before use)
+    // (rows that do not exist: zeros)
     auto fetch = [&](int64_t tile) {
+        const plane_rsrc_t xr = rows_rsrc(x, tile * 32, 32, V, 2 * C), gr = rows_rsrc(g, tile * 32, 32, V, 2 * C);
 #pragma unroll
         for (int s = 0; s < KC; ++s) {
-            int64_t v = tile * 32 + 16 * s + lane / 4;
-            v = v < V ? v : V - 1;
-            xn[s] = load_c8_nt(x + v * C + (lane % 4) * 8);
-            gn[s] = load_c8_nt(g + v * C + (lane % 4) * 8);
+            xn[s] = plane_load16<true>(xr, (uint32_t)(s * kWave + lane) * 16);
+            gn[s] = plane_load16<true>(gr, (uint32_t)(s * kWave + lane) * 16);
         }
     };
 
-    // dx leaves one tile late: the wait for the operands of a tile then only covers stores issued a whole
-    // tile earlier (the memory counter retires loads and stores in issue order)
-    auto flush = [&](int64_t pv0, bool ragged) {
+    // dx leaves one tile late, behind the loads of the tile after it: the wait for the operands of a tile leaves the
+    // stores in flight (nothing stands behind a condition, see rows_rsrc)
+    auto flush = [&](int64_t pv0) {
+        const plane_rsrc_t dr = rows_rsrc(dx, pv0, 32, V, 2 * C);
 #pragma unroll
         for (int pass = 0; pass < 2; ++pass) {  // lane -> 16-byte chunk lane % 4 of row 16 pass + lane / 4
             const int row = 16 * pass + lane / 4, cc = lane % 4;
-            if (!ragged || pv0 + row < V) {
-                const half8_t o = *reinterpret_cast<const half8_t*>(dt + row * 64 + ((cc ^ tr_slot(row)) * 16));
-                // rows 8..15 and 24..31 hold the two 8-byte halves of a chunk swapped
-                const bool sw = (row >> 3) & 1;
-                const half8_t w = {sw ? o[4] : o[0], sw ? o[5] : o[1], sw ? o[6] : o[2], sw ? o[7] : o[3],
-                                   sw ? o[0] : o[4], sw ? o[1] : o[5], sw ? o[2] : o[6], sw ? o[3] : o[7]};
-                store_c8_nt(dx + (pv0 + row) * C + cc * 8, w);
-            }
+            const half8_t o = *reinterpret_cast<const half8_t*>(dt + row * 64 + ((cc ^ tr_slot(row)) * 16));
+            // rows 8..15 and 24..31 hold the two 8-byte halves of a chunk swapped
+            const bool sw = (row >> 3) & 1;
+            const half8_t w = {sw ? o[4] : o[0], sw ? o[5] : o[1], sw ? o[6] : o[2], sw ? o[7] : o[3],
+                               sw ? o[0] : o[4], sw ? o[1] : o[5], sw ? o[2] : o[6], sw ? o[3] : o[7]};
+            plane_store16<true>(dr, (uint32_t)(pass * kWave + lane) * 16, w);
         }
         wave_sync();
     };
 
     const int64_t first = (int64_t)blockIdx.x * kMlpWaves + wave;
     int64_t tile = first;
-    if (tile < ntiles) fetch(tile);
+    fetch(tile);
+    flush(-1);
     for (; tile < ntiles; tile += stride) {
-        const int64_t v0 = tile * 32;
         half8_t xc[KC], gc[KC];
 #pragma unroll
         for (int s = 0; s < KC; ++s) {
             xc[s] = xn[s];
             gc[s] = gn[s];
         }
-        if (v0 + 32 > V) {  // ragged last tile (wavefront-uniform)
-#pragma unroll
-            for (int s = 0; s < KC; ++s) {
-                const bool ok = v0 + 16 * s + lane / 4 < V;
-                xc[s] = ok ? xc[s] : z8;
-                gc[s] = ok ? gc[s] : z8;
-            }
-        }
-        if (tile != first) flush(v0 - stride * 32, false);  // an earlier tile of this wavefront is never ragged
-        {
-            const int64_t nt = tile + stride;
-            fetch(nt < ntiles ? nt : tile);
-        }
+        fetch(tile + stride);
+        flush(tile != first ? (tile - stride) * 32 : -1);
         __builtin_amdgcn_sched_barrier(0);
 
         // x and g into the tiles as fetched; back as the lane's own row (chunks hl and 2 + hl: the operands of the
@@ -1049,7 +1057,7 @@ __global__ __launch_bounds__(kMlpThreads, 2) void lin_brelu_lin_bwd_tr_kernel(
         }
         wave_sync();
     }
-    if (first < ntiles) flush((tile - stride) * 32, true);
+    if (first < ntiles) flush((tile - stride) * 32);
 
     // ---- the four wavefronts add their partials in LDS, wavefront 0 first: [dWup C*H][dWdown H*C][dbias H] ----
     float* red = reinterpret_cast<float*>(smem);

@@ -84,14 +84,9 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
     const int64_t nrounds = (ntiles + tiles_per_round - 1) / tiles_per_round;
     unsigned char* my = reinterpret_cast<unsigned char*>(tile[wave]);
 
-    // The tile's part of a tensor with `row` bytes per voxel; voxels past V and tiles past the last have no bytes (loads give
-    // zeros, stores are dropped), so nothing stands behind a condition and the compiler's waits are exact: a tile's x
-    // fragments are waited for with the stores of the one before in flight.
-    auto tile_rsrc = [&](const half_t* p, int64_t tidx, int row) {
-        const int64_t v0 = tidx < ntiles ? tidx * 32 : 0;
-        const int rows = tidx < ntiles ? (int)std::min<int64_t>(V - v0, 32) : 0;
-        return plane_rsrc(uniform_ptr(reinterpret_cast<const char*>(p) + v0 * row), (uint32_t)(rows * row));
-    };
+    // The tile's part of a tensor with `row` bytes per voxel: nothing stands behind a condition and the compiler's waits are
+    // exact, a tile's x fragments are waited for with the stores of the one before in flight.
+    auto tile_rsrc = [&](const half_t* p, int64_t tidx, int row) { return rows_rsrc(p, tidx * 32, 32, V, row); };
     // B fragments of a tile: this lane's voxel, chunks 2q+hl
     half8_t xb[KS], xn[KS];
     auto load_x = [&](int64_t tidx, half8_t(&xb)[KS]) {

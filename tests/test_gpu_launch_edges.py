@@ -278,6 +278,22 @@ def test_inverted_bottleneck_is_the_same_with_early_and_late_loads():
     assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
 
 
+# either side of the volumes at which the workgroups per compute unit change: every voxel's result is its own, so one part
+# of the volume gives the same bits as the whole
+@pytest.mark.parametrize('c, line', [(16, 140000), (16, 500000), (64, 180000)])
+def test_inverted_bottleneck_either_side_of_a_volume_line(c, line):
+    g = cpu_gen(c)
+    x, add = flat(g, line + 1, c), flat(g, line + 1, c)
+    up, down, bias = matrix(g, c, 2 * c), matrix(g, 2 * c, c), (torch.randn(2 * c, generator=g) * 0.3).half()
+    dev = [t.to(DEV) for t in (x, up, down, bias, add)]
+    out = LinBReLULinAdd(*dev)
+    below = LinBReLULinAdd(dev[0][:, :, :line - 1], *dev[1:4], dev[4][:, :, :line - 1])
+    assert torch.equal(bits(out[:, :, :line - 1]), bits(below))
+    tail = slice(line - 2000, line + 1)
+    ref = oracle.lin_brelu_lin_add(x[:, :, tail], up, down, bias, add[:, :, tail])
+    assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
+
+
 # one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
 @pytest.mark.parametrize('mib', [3, 14, 20, 56, 112, 160])
 @pytest.mark.parametrize('off', [-1, 1])
