@@ -359,7 +359,8 @@ struct MarchCost {
     // Most workgroups that may march over a single row, which reads three planes for one.  Alone on a compute unit such a
     // workgroup is still the faster one ((1,32,33,19,25), 198 of them: forward 6.26 us, 6.60 with two rows each); two of
     // them on a compute unit lose in the forward and weight-gradient kernels ((2,32,32,9,35), 384: forward 8.20 us, 6.81
-    // with two rows each, weight gradient 12.2 and 10.9).
+    // with two rows each, weight gradient 12.2 and 10.9) and not in the fused backward (15.0 and 15.8), which keeps to
+    // single rows wherever they fit.
     int one_row;
 };
 static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int slab_mult, const DeviceGeometry& geo,
@@ -395,7 +396,7 @@ static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots
         if (ceil_div(H, h) != c) continue;  // the same split as a smaller c
         if (h < 2 && c > 1 && tiles * c > m.one_row) break;
         const double uniform = ((double)h + 2 + m.setup) * (1.0 + 0.004 * c) * occupancy(tiles * c);
-        if (uniform <= cost) {
+        if (uniform <= cost || (h == 1 && m.one_row >= slots)) {
             cost = uniform;
             best_h = h;
         }
