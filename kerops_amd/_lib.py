@@ -4,12 +4,18 @@ There is no fallback: if the library has not been built, or a call returns an
 error code, a RuntimeError is raised.  `python -m kerops_amd.build` builds it.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
+import sys
 
 import torch
 
+from .settings import hardware_conf, stream_table
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, '_C', 'libkerops_hip.so')
+HOST_PATH = os.path.join(_HERE, '_C', 'kerops_host.so')
 
 KEROPS_OK = 0
 KEROPS_E_BADARG = -1
@@ -84,6 +90,11 @@ SIGNATURES = {
 }
 
 _lib = None
+# The native call path of the ops (csrc/host.cpp), there once the library is loaded
+host = None
+# op name -> (ConfiguredFunction, or None for a plain function; [(dictionary, or None for its configurators, key, value),
+# ...]: what has to be as it was at import for the native path to take a call)
+native_ops = {}
 
 
 class KeropsHipError(RuntimeError):
@@ -112,19 +123,61 @@ def load():
                 f'{LIB_PATH} reports interface version {built}, this binding was written for {HEADER_VERSION}: '
                 'rebuild the library (python -m kerops_amd.build)'
             )
+        _load_host(lib)
         _lib = lib
     return _lib
+
+
+def _load_host(lib):
+    global host
+    from .ops import addition, avgpool, bnrelu, conv, fused, linear, quantization, stats  # noqa: F401 (fill native_ops)
+    from .ops.conv import dwconv, dwconv_wgrad
+
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f'{HOST_PATH} is missing: build the HIP extension first (python -m kerops_amd.build)')
+    loader = importlib.machinery.ExtensionFileLoader('kerops_host', HOST_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('kerops_host', HOST_PATH, loader=loader))
+    loader.exec_module(module)
+    if module.HEADER_VERSION != HEADER_VERSION:
+        raise RuntimeError(f'{HOST_PATH} was built for interface version {module.HEADER_VERSION}, this binding for '
+                           f'{HEADER_VERSION}: rebuild the library (python -m kerops_amd.build)')
+    module.setup(
+        {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
+        {name: (None if op is None else op.__dict__, _helpers + entries) for name, (op, entries) in native_ops.items()},
+        sys.modules[__name__], stream_table.__dict__, hardware_conf.__dict__, dwconv.__dict__,
+        dwconv_wgrad.__dict__)
+    for name, (op, _) in native_ops.items():
+        if op is not None:
+            op.native = getattr(module, name)
+    host = module
+
+
+def native(*helpers):
+    """Decorator of an op that csrc/host.cpp can take.  `helpers`: names in the op's module that its configurators go by."""
+    def register(op):
+        origin = getattr(op, 'origin_function', op)
+        entries = [(origin.__globals__, name, origin.__globals__[name]) for name in helpers]
+        if origin is not op:
+            entries += [(None, name, conf) for name, conf in op.configurators.items()]
+        native_ops[origin.__name__] = (None if origin is op else op, entries)
+        return op
+
+    return register
 
 
 def last_error():
     return load().kerops_last_error_string().decode('utf-8', 'replace')
 
 
+def fail(name, code):
+    raise KeropsHipError(name, code, last_error())
+
+
 def call(name, *args):
     """Call an int-returning entry point and turn error codes into exceptions."""
     rc = getattr(load(), name)(*args)
     if rc != KEROPS_OK:
-        raise KeropsHipError(name, rc, last_error())
+        fail(name, rc)
     return rc
 
 
@@ -132,7 +185,7 @@ def query(name, *args):
     """Call a *_workspace_bytes function (negative result = error)."""
     n = getattr(load(), name)(*args)
     if n < 0:
-        raise KeropsHipError(name, int(n), last_error())
+        fail(name, int(n))
     return int(n)
 
 
@@ -154,3 +207,7 @@ def stream_of(t):
 def workspace(nbytes, device):
     """Scratch buffer owned by the caller side of the ABI (torch's caching allocator)."""
     return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
+
+
+_helpers = [(globals(), name, globals()[name]) for name in ('load', 'call', 'query', 'stream_of', 'workspace')]
+_helpers += [(vars(stream_table), name, getattr(stream_table, name)) for name in ('_find', 'stream_shape')]

@@ -1,4 +1,5 @@
-"""Build step: compile kerops_amd/csrc/*.hip for gfx950 into kerops_amd/_C/libkerops_hip.so.
+"""Build step: compile kerops_amd/csrc/*.hip for gfx950 into kerops_amd/_C/libkerops_hip.so, and csrc/host.cpp (the ops'
+native call path, host code against the installed torch) into kerops_amd/_C/kerops_host.so.
 
     python -m kerops_amd.build            # compile every source, link
     python -m kerops_amd.build --verbose
@@ -12,6 +13,7 @@ import argparse
 import glob
 import os
 import subprocess
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -19,6 +21,9 @@ CSRC = os.path.join(HERE, 'csrc')
 OUT_DIR = os.path.join(HERE, '_C')
 OBJ_DIR = os.path.join(OUT_DIR, 'obj')
 LIB_PATH = os.path.join(OUT_DIR, 'libkerops_hip.so')
+HOST_PATH = os.path.join(OUT_DIR, 'kerops_host.so')
+
+HOST_SOURCE = os.path.join(CSRC, 'host.cpp')
 
 ARCH = 'gfx950'
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
@@ -57,6 +62,26 @@ def _compile(src, verbose):
     return obj
 
 
+def _compile_host(verbose):
+    """The Python extension of the ops' native call path: host code only, against the installed torch."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1',
+           '-DUSE_ROCM=1', f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}']
+    cmd += ['-isystem', os.path.join(root, 'include'), '-isystem', os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
+            '-isystem', os.path.join(os.path.dirname(os.path.dirname(HIPCC)), 'include'),
+            '-isystem', sysconfig.get_paths()['include']]
+    cmd += ['-Wall', HOST_SOURCE, '-o', HOST_PATH, '-L' + os.path.join(root, 'lib')]
+    cmd += ['-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_hip', '-ltorch', '-ltorch_python']
+    if verbose:
+        print(' '.join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f'{cmd[0]} failed for {HOST_SOURCE}:\n{res.stderr}')
+    if res.stderr.strip():
+        print(res.stderr)
+
+
 def build(verbose=False, jobs=None):
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
@@ -64,7 +89,9 @@ def build(verbose=False, jobs=None):
         raise RuntimeError(f'no .hip sources under {CSRC}')
     jobs = jobs or min(len(srcs), os.cpu_count() or 1, 8)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host, verbose)
         objs = list(pool.map(lambda s: _compile(s, verbose), srcs))
+        host.result()
     cmd = [HIPCC, '-shared', '-fPIC', f'--offload-arch={ARCH}', '-o', LIB_PATH] + objs
     if verbose:
         print(' '.join(cmd), flush=True)

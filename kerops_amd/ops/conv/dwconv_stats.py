@@ -10,9 +10,14 @@ from ... import _lib
 from .._common import cl3d, next_power_of_2, require_cuda
 
 
+@_lib.native()
 def DWConvStats(x, weight):
     """Returns (y, mean, sqmean): y = DWConv(x, weight) (bit-identical), mean / sqmean = Stats(y)
     (fp32, per channel; fp32 partial sums per workgroup, added in fp64 in a fixed order)."""
+    if _lib.host is not None:
+        out = _lib.host.DWConvStats(x, weight)
+        if out is not None:
+            return out
     channels = x.shape[1]
 
     assert x.ndim == 5

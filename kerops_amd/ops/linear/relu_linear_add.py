@@ -19,6 +19,7 @@ def ilp(in_channels):
     return {16: 1, 32: 1, 64: 1, 128: 1}[in_channels]
 
 
+@_lib.native('ilp')
 @configure(num_warps=4, D_block=32, ILP=lambda x: ilp(x.shape[1]))
 def ReLULinearAdd(x, weight, add_other, *, num_warps: ConfigurableArg, D_block: ConfigurableArg,
                   ILP: ConfigurableArg):
@@ -45,11 +46,16 @@ def ReLULinearAdd(x, weight, add_other, *, num_warps: ConfigurableArg, D_block: 
     return output
 
 
+@_lib.native()
 def ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other):
     """ReLULinearAdd(ApplyBNReLU(x, bn_weight, bn_bias), weight, add_other) in one pass, bit-identical to that
     composition (kerops/ops/bnrelu.py:11-42 then kerops/ops/linear/relu_linear_add.py:20-52): the normalised
     activation is formed in registers from the loaded x fragments and never written.  An addition to the
     reference's op set; host side of kerops_bnrelu_pointwise_f16."""
+    if _lib.host is not None:
+        out = _lib.host.ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other)
+        if out is not None:
+            return out
     in_channels = x.shape[1]
     out_channels = add_other.shape[1]
 

@@ -27,6 +27,7 @@ def dblock(in_channels):
     return {16: 64, 32: 64, 64: 64, 128: 64}[in_channels]
 
 
+@_lib.native('warps', 'dblock')
 @configure(
     num_warps=lambda x: warps(x.shape[1]),
     D_block=lambda x: dblock(x.shape[1]),
@@ -79,12 +80,17 @@ def ReLULinearBackward(
     return x_grad, (weight_grad if direct else weight_grad.to(out_dtype))
 
 
+@_lib.native()
 def ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad, weight):
     """Gradients of ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other) in one pass over x and grad.
     Returns (dx like x, bn_weight_grad fp32, bn_bias_grad fp32, weight_grad fp16): dx bit-identical to ApplyBNReLU,
     ReLULinearBackward and ApplyBNReLUBackward in a row (kerops/ops/bnrelu.py:11-42,
     kerops/ops/linear/relu_linear_backward.py:20-72, kerops/ops/bnrelu.py:45-82), the sums in another order.  The
     residual's gradient is grad itself.  An addition to the reference's op set; host side of kerops_bnrelu_linear_bwd_f16."""
+    if _lib.host is not None:
+        out = _lib.host.ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad, weight)
+        if out is not None:
+            return out
     in_channels = x.shape[1]
     out_channels = grad.shape[1]
 

@@ -28,6 +28,9 @@ def _param_names(fn):
 
 
 class ConfiguredFunction:
+    # the op's native call path, if it has one and the library is loaded: returns None for a call that it does not take
+    native = None
+
     def __init__(self, origin_function, signature, configurable_args, usual_args, **configurators):
         self.origin_function = origin_function
         self.signature = signature
@@ -76,6 +79,10 @@ class ConfiguredFunction:
         return conf(*[positional[self.usual_args.index(p)] for p in self._conf_params[name]])
 
     def __call__(self, *args, **kwargs):
+        if self.native is not None:
+            out = self.native(*args, **kwargs)
+            if out is not None:
+                return out
         # common case: ordinary arguments positional or left at their defaults, keywords only for configurable ones;
         # the general path below (Signature.bind) costs as much host time as a small kernel takes to run
         missing = len(self.usual_args) - len(args)
