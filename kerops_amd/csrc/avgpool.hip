@@ -282,6 +282,96 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_bwd_kernel(const ha
         one(i, ld_stream<V>(inpgrad, i), ld_stream<V>(output, i), std::false_type{});
 }
 
+// Backward in the order of the gradient it writes, for voxel rows narrower than a 128-byte line (16-byte chunks): a thread
+// takes one output chunk of a pair of (h, w) rows, i.e. one pooled chunk seen from one of its D taps, and stores it to the
+// (up to) four rows, so every store of a wavefront is one run of 1 KB wherever the rows end.  The kernel above stores each
+// result to both taps: every second voxel row of an instruction, parts of lines ((2,8,121,156,118) 25.2 us, here 20.0:
+// pool_bwd_by_rows has more).
+// The price is each pooled chunk read (from the cache) and computed twice.
+// Everything goes through buffer descriptors that drop what does not exist: no load or store stands behind a condition,
+// and a step waits for its own loads and leaves the stores of the one before in flight.
+// Quotients by extents are products with their reciprocals (fast_divisor).
+struct FastDivisor {
+    uint32_t mul, shift;
+};
+// n / d for n < 2^31: (mulhi(n, mul) + n) >> shift with shift = ceil(log2 d), mul = floor(2^32 (2^shift - d) / d) + 1
+static FastDivisor fast_divisor(uint32_t d)
+{
+    uint32_t s = 0;
+    while ((1ull << s) < d) ++s;
+    return {(uint32_t)((((1ull << s) - d) << 32) / d + 1), s};
+}
+__device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDivisor d) { return (__umulhi(n, d.mul) + n) >> d.shift; }
+
+struct PoolRows {  // (output bytes below 2^32, so chunks and items are below 2^28)
+    uint32_t items, row, pooled_row;  // output chunks of all row pairs, of one, pooled chunks of a pooled row
+    uint32_t cg_shift;
+    FastDivisor by_row, by_wo, by_ho;
+    uint32_t bytes, pooled_bytes;  // of dx, and of the pooled tensors
+};
+
+template <int U>
+__global__ __launch_bounds__(kStreamMaxThreads) void avgpool_bwd_rows_kernel(
+    const half_t* __restrict__ inpgrad, const float* __restrict__ meangrad, const float* __restrict__ sqmeangrad,
+    const half_t* __restrict__ output, half_t* __restrict__ dx, const PoolDims p, const PoolRows q, float fMo)
+{
+    const uint32_t step = gridDim.x * blockDim.x, first = blockIdx.x * blockDim.x + threadIdx.x;
+    const plane_rsrc_t gr = plane_rsrc(inpgrad, q.pooled_bytes), orr = plane_rsrc(output, q.pooled_bytes), dr = plane_rsrc(dx, q.bytes);
+    // (every stride of the walk is a multiple of the channel groups: a thread keeps its own)
+    const uint32_t cg = first & (p.CG - 1);
+    float mg[8], sg[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        mg[j] = __fdiv_rn(meangrad[cg * 8 + j], fMo);
+        sg[j] = sqmeangrad[cg * 8 + j];
+    }
+    struct Item {
+        half8_t g, o;
+    };
+    auto load = [&](uint32_t i) {
+        const uint32_t prow = fast_div(i, q.by_row), j = i - prow * q.row;
+        const uint32_t chunk = prow * q.pooled_row + ((j >> (q.cg_shift + 1)) << q.cg_shift) + cg;
+        const uint32_t off = i < q.items ? chunk * 16 : kNoVoxel;
+        return Item{plane_load16<true>(gr, off), plane_load16<true>(orr, off)};
+    };
+    Item next[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) next[u] = load(first + u * step);
+    // (stores of nothing: the waits of the loop are the same on both ways in)
+#pragma unroll
+    for (int k = 0; k < 4 * U; ++k) plane_store16<true>(dr, kNoVoxel, half8_t{});
+    for (uint32_t i0 = first; i0 - threadIdx.x < q.items; i0 += U * step) {
+        Item cur[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) cur[u] = next[u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) next[u] = load(i0 + (U + u) * step);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t i = i0 + u * step;
+            const uint32_t prow = fast_div(i, q.by_row), j = i - prow * q.row;
+            const uint32_t t = fast_div(prow, q.by_wo), wO = prow - t * p.Wo;
+            const uint32_t n = fast_div(t, q.by_ho), hO = t - n * p.Ho;
+            const bool h1 = 2 * hO + 1 < (uint32_t)p.H, w1 = 2 * wO + 1 < (uint32_t)p.W, d1 = ((j >> q.cg_shift) | 1) < (uint32_t)p.D;
+            // the window holds 2^k voxels: the product with 2^-k is the correctly rounded quotient
+            const float inv = __builtin_bit_cast(float, (127u - (uint32_t)h1 - (uint32_t)w1 - (uint32_t)d1) << 23);
+            half8_t res;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float s = __fdiv_rn(__fmul_rn(__fmul_rn(2.0f, (float)cur[u].o[c]), sg[c]), fMo);
+                res[c] = (half_t)__fmul_rn(__fadd_rn(__fadd_rn((float)cur[u].g[c], mg[c]), s), inv);
+            }
+            const uint32_t off = (((n * p.H + 2 * hO) * p.W + 2 * wO) * q.row + j) * 16;
+            const bool live = i < q.items;
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    plane_store16<true>(dr, live && (a == 0 || h1) && (b == 0 || w1) ? off + (a * p.W + b) * q.row * 16 : kNoVoxel, res);
+        }
+    }
+}
+
 // Launch shape (blocks, waves, segment) as for the flat stream kernels; segment counts output chunks per thread and
 // step: 1 = interleaved (one window per thread in flight), 2 = contiguous runs of two chunks per thread (two
 // windows, 16 loads, in flight).  Built-in choices by the size of the volume that is pooled; the largest measured at
@@ -297,11 +387,35 @@ constexpr PoolDefault kDefPoolFwd[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 
 constexpr PoolDefault kDefPoolFwdBnRelu[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 2}};
 constexpr PoolDefault kDefPoolBwd[] = {{20 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
                                        {512 * kMiB, 256, 4, 2}, {kAnySize, 256, 4, 1}};
+// in output order (segment: output chunks per thread and step); us with (512,4,1) / (512,4,2): C = 8, 4 MiB 3.9 / 4.2, 11 6.4 /
+// 5.7, 49 15.9 / 16.1, 67 20.1 / 20.8, 184 48.3 / 50.2; C = 16, 9 MiB 6.1 / 5.5, 17 8.0 / 6.6, 100 27.0 / 25.5, 368 91.4 / 91.2; C = 32,
+// 95 MiB 26.3 / 24.6; 256 workgroups are too few (67 MiB 27.5, 368 137), 1024 to 4096 no better
+constexpr PoolDefault kDefPoolBwdRows[] = {{6 * kMiB, 512, 4, 1}, {kAnySize, 512, 4, 2}};
+constexpr PoolDefault kDefPoolBwdRows8[] = {{6 * kMiB, 512, 4, 1}, {64 * kMiB, 512, 4, 2}, {kAnySize, 512, 4, 1}};
 constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
+
+// Backward: the condition of the redistributing stores (PERM), and where the kernel in output order is the faster one.
+// us with results stored from where they are computed or redistributed, each with its best shape / in output order:
+//   8 channels   (1,8,90,91,93) 7.9 / 5.7, (2,8,121,156,118) 25.2 / 20.0, (2,8,200,201,150) 59.2 / 48.1
+//   16 channels  (1,16,80,85,83) 10.4 / 6.6, (2,16,90,101,121) 24.8 / 19.7, (2,16,200,201,150) 109 / 91
+//   32 channels  (1,32,60,61,59) 5.7 / 6.1, (1,32,81,87,85) 13.9 / 12.7, (1,32,150,150,150) 54.4 / 50.0, (1,32,200,201,150) 95 / 88
+//   redistributed (1,8,128,128,128) 9.4 / 9.1, (1,16,128,128,128) 17.2 / 16.5, (1,16,160,160,128) 26.1 / 25.3,
+//                 (1,8,350,350,128) 54.8 / 57.1, (1,16,350,350,128) 109 / 114, (1,32,350,350,128) 226 / 236
+static bool pool_bwd_permutes(int D, int C)
+{
+    return C >= 8 && C < 64 && D % 2 == 0 && ((int64_t)ceil_div(D, 2) * (C / 8)) % kWave == 0;
+}
+static bool pool_bwd_by_rows(int N, int H, int W, int D, int C)
+{
+    if (N <= 0 || H <= 0 || W <= 0 || D <= 0 || volume_exceeds_i64(N, H, W, D, C)) return false;
+    const int64_t bytes = (int64_t)N * H * W * D * C * 2;
+    return (C == 8 || C == 16 || (C == 32 && bytes >= 24 * kMiB)) && bytes <= (int64_t)kNoVoxel &&  // (32-bit offsets)
+           !(bytes >= 192 * kMiB && pool_bwd_permutes(D, C));
+}
 
 // `table`: the lines of one of the tables above, the last without a limit
 static int pool_plan(const char* op, const PoolDefault* table, int N, int H, int W, int D, int C, int blocks, int waves,
-                     int segment, PoolDims* p, int64_t* nchunks, StreamShape* sh)
+                     int segment, PoolDims* p, int64_t* nchunks, StreamShape* sh, int items_per_chunk = 1)
 {
     if (N <= 0 || H <= 0 || W <= 0 || D <= 0 || C <= 0 || !is_pow2(C)) {
         set_error("%s: extents must be positive and C a power of two", op);
@@ -349,7 +463,7 @@ static int pool_plan(const char* op, const PoolDefault* table, int N, int H, int
     // (never beyond what a workspace query with blocks = 0 sizes for)
     if (blocks <= 0)
         blocks = std::min(kMaxDefaultBlocks, std::max(1, (int)((int64_t)def.blocks * device_geometry().cus / 256)));
-    sh->blocks = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(*nchunks, (int64_t)sh->threads * segment), blocks));
+    sh->blocks = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div64(*nchunks * items_per_chunk, (int64_t)sh->threads * segment), blocks));
     return KEROPS_OK;
 }
 
@@ -446,7 +560,9 @@ extern "C" int kerops_avgpool_ceil_stats_bwd_f16(const void* inpgrad, const floa
     PoolDims p;
     int64_t nchunks = 0;
     StreamShape sh;
-    int rc = pool_plan("avgpool_ceil_stats_bwd", kDefPoolBwd, N, H, W, D, C, blocks, waves, segment, &p, &nchunks, &sh);
+    const bool rows = pool_bwd_by_rows(N, H, W, D, C);
+    int rc = pool_plan("avgpool_ceil_stats_bwd", !rows ? kDefPoolBwd : C == 8 ? kDefPoolBwdRows8 : kDefPoolBwdRows, N, H, W, D, C,
+                       blocks, waves, segment, &p, &nchunks, &sh, rows ? 2 : 1);
     if (rc != KEROPS_OK) return rc;
     if (!inpgrad || !meangrad || !sqmeangrad || !output || !dx || !aligned16(inpgrad) || !aligned16(output) ||
         !aligned16(dx)) {
@@ -456,7 +572,26 @@ extern "C" int kerops_avgpool_ceil_stats_bwd_f16(const void* inpgrad, const floa
     const float fMo = (float)((int64_t)N * p.Ho * p.Wo * p.Do);
     const int seg = sh.segment != 1;
     // redistribute the results for whole-line stores where a voxel row is narrower than a 128-byte line
-    const bool perm = C >= 8 && C < 64 && D % 2 == 0 && ((int64_t)p.Do * p.CG) % kWave == 0;
+    const bool perm = pool_bwd_permutes(D, C);
+    if (rows) {
+        PoolRows q;
+        q.row = (uint32_t)D * p.CG;
+        q.pooled_row = (uint32_t)p.Do * p.CG;
+        q.items = (uint32_t)((int64_t)N * p.Ho * p.Wo) * q.row;
+        q.cg_shift = (uint32_t)__builtin_ctz(p.CG);
+        q.by_row = fast_divisor(q.row);
+        q.by_wo = fast_divisor((uint32_t)p.Wo);
+        q.by_ho = fast_divisor((uint32_t)p.Ho);
+        q.bytes = (uint32_t)((int64_t)N * H * W * D * C * 2);
+        q.pooled_bytes = (uint32_t)(nchunks * 16);
+#define KEROPS_POOLB_ROWS(Uv)                                                                                        \
+    hipLaunchKernelGGL((avgpool_bwd_rows_kernel<Uv>), dim3(sh.blocks), dim3(sh.threads), 0, (hipStream_t)stream,        \
+                       (const half_t*)inpgrad, meangrad, sqmeangrad, (const half_t*)output, (half_t*)dx, p, q, fMo)
+        if (sh.segment == 2) KEROPS_POOLB_ROWS(2);
+        else KEROPS_POOLB_ROWS(1);
+#undef KEROPS_POOLB_ROWS
+        return check_launch("avgpool_ceil_stats_bwd");
+    }
 #define KEROPS_POOLB_GO(Uv)                                                                                          \
     KEROPS_DISPATCH_V(C, {                                                                                           \
         if (perm && V == 8)                                                                                          \

@@ -294,6 +294,25 @@ def test_inverted_bottleneck_either_side_of_a_volume_line(c, line):
     assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
 
 
+# the pooling backward in output order (8, 16 and, from 24 MiB on, 32 channels): single rows and voxels, runs of a wavefront
+# that end inside a row, many rounds of one workgroup, both sides of the 32-channel line
+@pytest.mark.parametrize('c,shape', [(8, (1, 1, 1, 1)), (8, (2, 3, 5, 7)), (8, (1, 2, 1, 65)), (8, (1, 9, 8, 64)), (16, (1, 1, 6, 31)),
+                                     (16, (3, 4, 5, 33)), (16, (1, 6, 7, 128)), (32, (1, 71, 73, 75)), (32, (1, 71, 73, 76)),
+                                     (32, (1, 64, 64, 96)), (32, (1, 64, 64, 95))])
+@pytest.mark.parametrize('knobs', [{}, dict(blocks=1, segment=1), dict(blocks=3, segment=2, num_warps=8)])
+def test_pool_backward_rows(c, shape, knobs):
+    n, h, w, d = shape
+    if knobs and n * h * w * d > 100000:
+        knobs = dict(knobs, blocks=knobs['blocks'] * 40)
+    g = cpu_gen(h * w + d)
+    small = (n, c, (h + 1) // 2, (w + 1) // 2, (d + 1) // 2)
+    grad, pooled = rand_cl3d(g, *small), rand_cl3d(g, *small)
+    mg, sg = torch.randn(c, generator=g), torch.randn(c, generator=g)
+    dx = AvgPoolCeilStatsBackward(*(t.to(DEV) for t in (grad, mg, sg, pooled)), (n, c, h, w, d), **knobs)
+    # the same operations in the same order
+    assert torch.equal(bits(dx.cpu()), bits(oracle.avgpool_ceil_stats_bwd(grad, mg, sg, pooled, (n, c, h, w, d))))
+
+
 # one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
 @pytest.mark.parametrize('mib', [3, 14, 20, 56, 112, 160])
 @pytest.mark.parametrize('off', [-1, 1])
