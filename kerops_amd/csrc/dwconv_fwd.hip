@@ -1017,26 +1017,17 @@ static int launch_fwd_mfma(const FwdArgs& base, int N, int h_chunk, hipStream_t 
     return check_launch("dwconv_fwd");
 }
 
-// Adds the per-workgroup sums of one channel in a fixed order (fp64) and divides by the number of voxels:
-// one workgroup per (statistic, channel); row r of the workspace belongs to slab r % n_slab.
-__global__ __launch_bounds__(256) void dwconv_stats_reduce_kernel(const float* __restrict__ ws, uint32_t nblocks,
-                                                                  int n_slab, int SC, double inv_count,
-                                                                  float* __restrict__ mean, float* __restrict__ sqmean)
+// Adds the per-workgroup sums in a fixed order (fp64, sum_columns) and divides by the number of voxels: one workgroup per
+// slab and 16 of its 2 SC columns (SC sums, SC sums of squares); row r of the workspace belongs to slab r % n_slab.
+__global__ __launch_bounds__(1024) void dwconv_stats_reduce_kernel(const float* __restrict__ ws, uint32_t nblocks,
+                                                                   int n_slab, int SC, double inv_count,
+                                                                   float* __restrict__ mean, float* __restrict__ sqmean)
 {
-    __shared__ double part[256];
-    const int C = n_slab * SC;
-    const int st = blockIdx.x / C, c = blockIdx.x % C;
-    const int slab = c / SC, ch = c % SC;
-    double s = 0.0;
-    for (uint32_t r = slab + (uint32_t)n_slab * threadIdx.x; r < nblocks; r += (uint32_t)n_slab * 256)
-        s += (double)ws[(int64_t)r * 2 * SC + st * SC + ch];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) (st == 0 ? mean : sqmean)[c] = (float)(part[0] * inv_count);
+    __shared__ double part[16][17];
+    const int slab = blockIdx.x % n_slab, j = (int)(blockIdx.x / n_slab) * 16 + threadIdx.x % 16;
+    const int nrows = ((int)nblocks - slab + n_slab - 1) / n_slab;
+    const double v = sum_columns(ws + (int64_t)slab * 2 * SC, nrows, (int64_t)n_slab * 2 * SC, j, 2 * SC, part) * inv_count;
+    if (threadIdx.x < 16 && j < 2 * SC) (j < SC ? mean : sqmean)[slab * SC + j % SC] = (float)v;
 }
 
 // launch shape of the convolution + statistics kernel for a channel count (the default shapes of dwconv_fwd_run)
@@ -1297,7 +1288,7 @@ extern "C" int kerops_dwconv_stats_f16(const void* x, const void* wt, void* y, f
     });
     if (rc != KEROPS_OK) return rc;
     const double inv_count = 1.0 / ((double)N * H * W * D);
-    hipLaunchKernelGGL(dwconv_stats_reduce_kernel, dim3(2 * C), dim3(256), 0, s, (const float*)workspace, a.nblocks,
+    hipLaunchKernelGGL(dwconv_stats_reduce_kernel, dim3(a.n_slab * ceil_div(2 * std::min(C, 64), 16)), dim3(1024), 0, s, (const float*)workspace, a.nblocks,
                        a.n_slab, std::min(C, 64), inv_count, mean, sqmean);
     return check_launch("dwconv_stats_reduce");
 }

@@ -1031,38 +1031,20 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_bwd_split_kernel(const WgAr
 }
 
 // Second pass, fixed summation order (deterministic).  The workspace holds one row per (n, h-chunk, w-patch,
-// d-patch) of width RW = slabs*27*SC floats.  A workgroup owns 16 columns, its 64 row slices sum interleaved rows
-// (four loads in flight), the slices are combined in LDS in a fixed order and the result is scattered to the
-// [27][C] layout.  One launch: at 128^3-class shapes a second small launch was 5 % of the whole op.
+// d-patch) of width RW = slabs*27*SC floats.  A workgroup owns 16 columns (sum_columns, in fp64), the result is scattered to
+// the [27][C] layout.  One launch: at 128^3-class shapes a second small launch was 5 % of the whole op.
 // OutT: fp32, or fp16 = the sum rounded once (what a cast of the fp32 result gives, without its launch).
 template <class OutT>
 __global__ __launch_bounds__(1024) void wgrad_reduce_kernel(const float* __restrict__ ws, OutT* __restrict__ gw,
                                                             int n_rows, int RW, int SC, int C)
 {
-    __shared__ float part[64][17];
-    const int cl = threadIdx.x % 16, slice = threadIdx.x / 16;
-    const int col = blockIdx.x * 16 + cl;
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-    if (col < RW) {
-        int r = slice;
-        for (; r + 192 < n_rows; r += 256) {
-            s0 += ws[(int64_t)r * RW + col];
-            s1 += ws[(int64_t)(r + 64) * RW + col];
-            s2 += ws[(int64_t)(r + 128) * RW + col];
-            s3 += ws[(int64_t)(r + 192) * RW + col];
-        }
-        for (; r < n_rows; r += 64) s0 += ws[(int64_t)r * RW + col];
-    }
-    part[slice][cl] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    for (int w = 32; w > 0; w >>= 1) {
-        if (slice < w) part[slice][cl] += part[slice + w][cl];
-        __syncthreads();
-    }
-    if (slice == 0 && col < RW) {
+    __shared__ double part[16][17];
+    const int col = blockIdx.x * 16 + threadIdx.x % 16;
+    const double v = sum_columns(ws, n_rows, RW, col, RW, part);
+    if (threadIdx.x < 16 && col < RW) {
         const int slab = col / (27 * SC), rem = col % (27 * SC);
         const int tap = rem / SC, cs = rem % SC;
-        gw[tap * C + slab * SC + cs] = (OutT)part[0][cl];
+        gw[tap * C + slab * SC + cs] = (OutT)(float)v;
     }
 }
 
