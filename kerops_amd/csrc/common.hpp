@@ -694,36 +694,6 @@ static inline int stream_blocks_default(int64_t work_items, int preferred = 768)
     return (int)b;
 }
 
-// Sum NACC*V per-thread accumulators over the threads of a workgroup that own the same
-// channel group (thread t owns group t % CG, CG <= 64 a power of two) and write the
-// workgroup's partial [NACC][CG*V] to `dst`.  `red` is LDS of kStreamWaves*NACC*CG*V floats.
-template <int NACC, int V>
-__device__ __forceinline__ void block_channel_partials(float (&acc)[NACC][V], int CG, float* red, float* dst)
-{
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
-    const int cols = CG * V;
-#pragma unroll
-    for (int a = 0; a < NACC; ++a)
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            float v = acc[a][j];
-            for (int off = 32; off >= CG; off >>= 1) v += __shfl_xor(v, off, 64);
-            acc[a][j] = v;
-        }
-    if (lane < CG) {
-#pragma unroll
-        for (int a = 0; a < NACC; ++a)
-#pragma unroll
-            for (int j = 0; j < V; ++j) red[(wave * NACC + a) * cols + lane * V + j] = acc[a][j];
-    }
-    __syncthreads();
-    for (int o = t; o < NACC * cols; o += kStreamThreads) {
-        float s = 0.0f;
-#pragma unroll
-        for (int wv = 0; wv < kStreamWaves; ++wv) s += red[wv * NACC * cols + o];
-        dst[o] = s;
-    }
-}
 
 // ---- launch shape of the flat stream kernels ------------------------------------------------------------
 // A stream kernel walks its 16-byte chunks in steps of U chunks per thread (all U loads of a stream are issued
@@ -756,33 +726,62 @@ struct ChunkWalk {
 };
 constexpr int kStreamMaxThreads = 1024;
 
-// block_channel_partials for any workgroup size up to 1024 threads: the wavefronts hand their sums over in
-// rounds of four through the same 4-slot LDS buffer; thread o keeps the running sums of the outputs
-// o, o + threads, ... (at most NACC*512 / 256 = 2*NACC of them) and adds the rounds in a fixed order.
+// Sums of N values per lane over the lanes of a wavefront with the same lane % CG (CG <= 64 a power of two), pairs first at a
+// distance of 32 lanes, then 16, ...  A step halves the values that a lane goes on with: it hands the other half of them to
+// its partner, so N = 16 takes 8 + 4 + 2 + 1 exchanges, each step's in flight together, and one for every step after that.
+// (A butterfly per value is N log2(64 / CG) exchanges one after the other, 96 at CG = 1: Stats of (1,8,64,64,32) 10.7 us, here 5.4,
+// AddStats of (1,16,128,128,128) 40.4 and 36.1.)
+// `store(base, v)`: called with the N >> steps values that the lane has, the first of them number `base`, by one lane each.
+template <int N, int OFF = 32, class Store>
+__device__ __forceinline__ void wave_sums(float (&v)[N], int CG, int lane, int base, int spare, Store store)
+{
+    if constexpr (OFF > 0) {
+        if (OFF >= CG) {  // (uniform)
+            if constexpr (N > 1) {
+                const bool up = (lane & OFF) != 0;
+                float w[N / 2];
+#pragma unroll
+                for (int k = 0; k < N / 2; ++k) {
+                    const float keep = up ? v[N / 2 + k] : v[k], give = up ? v[k] : v[N / 2 + k];
+                    w[k] = keep + __shfl_xor(give, OFF, 64);
+                }
+                wave_sums<N / 2, OFF / 2>(w, CG, lane, base + (up ? N / 2 : 0), spare, store);
+            } else {
+                float w[1] = {v[0] + __shfl_xor(v[0], OFF, 64)};
+                wave_sums<1, OFF / 2>(w, CG, lane, base, spare | OFF, store);  // both partners hold the sum
+            }
+            return;
+        }
+    }
+    if ((lane & spare) == 0) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) store(base + k, v[k]);
+    }
+}
+
+// Sum NACC*V per-thread accumulators over the threads of a workgroup (up to 1024) that own the same channel group
+// (thread t owns group t % CG, CG <= 64 a power of two) and write the workgroup's partial [NACC][CG*V] to `dst`.  The
+// wavefronts hand their sums over in rounds of four through LDS (`red`: 4*NACC*CG*V floats); thread o keeps the running
+// sums of the outputs o, o + threads, ... (at most NACC*512 / 256 = 2*NACC of them) and adds the rounds in a fixed order.
 template <int NACC, int V>
 __device__ __forceinline__ void block_channel_partials_any(float (&acc)[NACC][V], int CG, float* red, float* dst)
 {
     const int t = threadIdx.x, lane = t % kWave, wave = t / kWave, nthr = blockDim.x, nwaves = nthr / kWave;
     const int cols = CG * V, nout = NACC * cols;
+    float flat[NACC * V];
 #pragma unroll
     for (int a = 0; a < NACC; ++a)
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-            float v = acc[a][j];
-            for (int off = 32; off >= CG; off >>= 1) v += __shfl_xor(v, off, 64);
-            acc[a][j] = v;
-        }
+        for (int j = 0; j < V; ++j) flat[a * V + j] = acc[a][j];
     constexpr int kMine = 2 * NACC;
     float run[kMine];
 #pragma unroll
     for (int m = 0; m < kMine; ++m) run[m] = 0.0f;
     for (int r = 0; r < nwaves; r += 4) {
-        if (wave >= r && wave < r + 4 && lane < CG) {
-#pragma unroll
-            for (int a = 0; a < NACC; ++a)
-#pragma unroll
-                for (int j = 0; j < V; ++j) red[((wave - r) * NACC + a) * cols + lane * V + j] = acc[a][j];
-        }
+        if (wave >= r && wave < r + 4)
+            wave_sums<NACC * V>(flat, CG, lane, 0, 0, [&](int k, float v) {
+                red[((wave - r) * NACC + k / V) * cols + (lane & (CG - 1)) * V + k % V] = v;
+            });
         __syncthreads();
 #pragma unroll
         for (int m = 0; m < kMine; ++m) {
