@@ -385,7 +385,7 @@ struct PoolDefault {
 constexpr int64_t kMiB = 1ll << 20, kAnySize = INT64_MAX;
 constexpr PoolDefault kDefPoolFwd[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 1}};
 constexpr PoolDefault kDefPoolFwdBnRelu[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 2}};
-constexpr PoolDefault kDefPoolBwd[] = {{20 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
+constexpr PoolDefault kDefPoolBwd[] = {{32 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
                                        {512 * kMiB, 256, 4, 2}, {kAnySize, 256, 4, 1}};
 // in output order (segment: output chunks per thread and step); us with (512,4,1) / (512,4,2): C = 8, 4 MiB 3.9 / 4.2, 11 6.4 /
 // 5.7, 49 15.9 / 16.1, 67 20.1 / 20.8, 184 48.3 / 50.2; C = 16, 9 MiB 6.1 / 5.5, 17 8.0 / 6.6, 100 27.0 / 25.5, 368 91.4 / 91.2; C = 32,

@@ -314,7 +314,7 @@ def test_pool_backward_rows(c, shape, knobs):
 
 
 # one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
-@pytest.mark.parametrize('mib', [3, 14, 20, 56, 112, 160])
+@pytest.mark.parametrize('mib', [3, 14, 20, 40, 56, 112, 160])
 @pytest.mark.parametrize('off', [-1, 1])
 def test_stream_ops_either_side_of_a_size_line(mib, off):
     c = 64
