@@ -8,6 +8,7 @@ import importlib.machinery
 import importlib.util
 import os
 import sys
+import weakref
 
 import torch
 
@@ -148,7 +149,7 @@ def _load_host(lib):
         dwconv_wgrad.__dict__)
     for name, (op, _) in native_ops.items():
         if op is not None:
-            op.native = getattr(module, name)
+            op.native, op.native_for = getattr(module, name), weakref.ref(op)
     host = module
 
 

@@ -28,8 +28,11 @@ def _param_names(fn):
 
 
 class ConfiguredFunction:
-    # the op's native call path, if it has one and the library is loaded: returns None for a call that it does not take
+    # The op's native call path, if it has one and the library is loaded: returns None for a call that it does not take.
+    # It goes by the configurators of the object it was made for (`native_for`, a weak reference), so a copy of an op, or
+    # another object that `functools.wraps` has given this one's attributes, calls its Python function.
     native = None
+    native_for = None
 
     def __init__(self, origin_function, signature, configurable_args, usual_args, **configurators):
         self.origin_function = origin_function
@@ -58,6 +61,9 @@ class ConfiguredFunction:
         self._defaults = tuple(p.default for p in (self.signature.parameters[a] for a in self.usual_args)
                                if p.default is not inspect.Parameter.empty)
 
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in ('native', 'native_for')}
+
     def __repr__(self):
         lines = [f'{self.origin_function.__name__}{self.signature}']
         for name, conf in self.configurators.items():
@@ -79,7 +85,7 @@ class ConfiguredFunction:
         return conf(*[positional[self.usual_args.index(p)] for p in self._conf_params[name]])
 
     def __call__(self, *args, **kwargs):
-        if self.native is not None:
+        if self.native is not None and self.native_for() is self:
             out = self.native(*args, **kwargs)
             if out is not None:
                 return out

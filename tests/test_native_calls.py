@@ -1,5 +1,8 @@
 """The native call path of the ops against their Python functions: the same results, shapes, strides and types wherever it
 takes a call, and None for every call that it leaves to them."""
+import copy
+import functools
+
 import pytest
 import torch
 from torch.overrides import TorchFunctionMode
@@ -112,6 +115,35 @@ def test_missing_native_calls_fail_loudly(monkeypatch):
     monkeypatch.setattr(_lib, 'HOST_PATH', _lib.HOST_PATH + '.none')
     with pytest.raises(RuntimeError, match='build the HIP extension'):
         _lib.load()
+
+
+def _clone(op):
+    return functools.wraps(op)(type(op)(op.origin_function, op.signature, op.configurable_args, op.usual_args, **op.configurators))
+
+
+COPIES = {'copy': copy.copy, 'deepcopy': copy.deepcopy, 'wraps': _clone}
+
+
+@pytest.mark.parametrize('how', COPIES)
+def test_a_copy_goes_by_its_own_configurators(host, monkeypatch, how):
+    taken = []
+    monkeypatch.setattr(DWConvBackward, 'native', lambda *args, **kwargs: taken.append(args))
+    other = COPIES[how](DWConvBackward)
+    for op, native in ((DWConvBackward, True), (other, False)):
+        with pytest.raises(RuntimeError, match='no CPU path'):
+            op(*arguments('DWConvBackward', 'plain', 'cpu'))
+        assert bool(taken) == native
+        taken.clear()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('how', COPIES)
+def test_a_reconfigured_copy_and_its_original(host, how):
+    args = arguments('DWConvBackward', 'plain', DEV)
+    other = COPIES[how](DWConvBackward)
+    other.reconfigure(**{**DWConvBackward.configurators, 'out_dtype': torch.float32})
+    assert other(*args)[1].dtype == torch.float32 and DWConvBackward(*args)[1].dtype == torch.float16
+    assert host.DWConvBackward(*args) is not None
 
 
 # (16-channel forms only where the fused block, built for 64 input channels, is not the op)
