@@ -138,10 +138,16 @@ def _load_host(lib):
         raise RuntimeError(f'{HOST_PATH} is missing: build the HIP extension first (python -m kerops_amd.build)')
     loader = importlib.machinery.ExtensionFileLoader('kerops_host', HOST_PATH)
     module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('kerops_host', HOST_PATH, loader=loader))
-    loader.exec_module(module)
-    if module.HEADER_VERSION != HEADER_VERSION:
-        raise RuntimeError(f'{HOST_PATH} was built for interface version {module.HEADER_VERSION}, this binding for '
-                           f'{HEADER_VERSION}: rebuild the library (python -m kerops_amd.build)')
+    try:
+        loader.exec_module(module)
+    except ImportError as e:
+        raise RuntimeError(f'{HOST_PATH} does not load ({e}): rebuild the library (python -m kerops_amd.build)') from e
+    # the extension reads objects of torch and of the interpreter by the layouts of the headers it was compiled with
+    built = (module.HEADER_VERSION, module.TORCH_VERSION, module.PYTHON_VERSION)
+    here = (HEADER_VERSION, str(torch.__version__), sys.hexversion >> 16)
+    if built != here:
+        raise RuntimeError(f'{HOST_PATH} was built for (interface, torch, Python) {built}, this is {here}: '
+                           'rebuild the library (python -m kerops_amd.build)')
     module.setup(
         {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
         {name: (None if op is None else op.__dict__, _helpers + entries) for name, (op, entries) in native_ops.items()},

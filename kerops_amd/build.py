@@ -67,7 +67,8 @@ def _compile_host(verbose):
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1',
-           '-DUSE_ROCM=1', f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}']
+           '-DUSE_ROCM=1', f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+           f'-DKEROPS_TORCH_VERSION="{torch.__version__}"']
     cmd += ['-isystem', os.path.join(root, 'include'), '-isystem', os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
             '-isystem', os.path.join(os.path.dirname(os.path.dirname(HIPCC)), 'include'),
             '-isystem', sysconfig.get_paths()['include']]

@@ -906,6 +906,11 @@ PyMODINIT_FUNC PyInit_kerops_host()
     k_fwd_variants = name("FWD_VARIANTS"), k_wgrad_variants = name("WGRAD_VARIANTS"), k_out_dtype = name("out_dtype");
     k_configurators = name("configurators");
     PyObject* m = PyModule_Create(&definition);
-    if (m && PyModule_AddIntConstant(m, "HEADER_VERSION", KEROPS_HIP_VERSION) != 0) Py_CLEAR(m);
+    // what the binding compares before it calls anything else: the layouts of torch's and the interpreter's objects that
+    // this file was compiled with are those of these versions only
+    if (m && (PyModule_AddIntConstant(m, "HEADER_VERSION", KEROPS_HIP_VERSION) != 0 ||
+              PyModule_AddStringConstant(m, "TORCH_VERSION", KEROPS_TORCH_VERSION) != 0 ||
+              PyModule_AddIntConstant(m, "PYTHON_VERSION", PY_VERSION_HEX >> 16) != 0))
+        Py_CLEAR(m);
     return m;
 }

@@ -2,6 +2,7 @@
 takes a call, and None for every call that it leaves to them."""
 import copy
 import functools
+import sys
 
 import pytest
 import torch
@@ -115,6 +116,16 @@ def test_missing_native_calls_fail_loudly(monkeypatch):
     monkeypatch.setattr(_lib, 'HOST_PATH', _lib.HOST_PATH + '.none')
     with pytest.raises(RuntimeError, match='build the HIP extension'):
         _lib.load()
+
+
+@pytest.mark.parametrize('owner,name,value', [(torch, '__version__', '2.9.1+rocm6.4'), (sys, 'hexversion', sys.hexversion + (1 << 16)),
+                                              (_lib, 'HEADER_VERSION', _lib.HEADER_VERSION + 1)])
+def test_native_calls_built_for_another_version_are_refused(host, monkeypatch, owner, name, value):
+    lib = _lib.load()
+    monkeypatch.setattr(owner, name, value)
+    with pytest.raises(RuntimeError, match='rebuild the library'):
+        _lib._load_host(lib)
+    assert _lib.host is host
 
 
 def _clone(op):
