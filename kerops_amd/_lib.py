@@ -8,6 +8,7 @@ import importlib.machinery
 import importlib.util
 import os
 import sys
+import types
 import weakref
 
 import torch
@@ -150,7 +151,8 @@ def _load_host(lib):
                            'rebuild the library (python -m kerops_amd.build)')
     module.setup(
         {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES},
-        {name: (None if op is None else op.__dict__, _helpers + entries) for name, (op, entries) in native_ops.items()},
+        {name: (None if op is None else op.__dict__, [(globals(), '_lib', lib)] + entries)
+         for name, (op, entries) in native_ops.items()},
         sys.modules[__name__], stream_table.__dict__, hardware_conf.__dict__, dwconv.__dict__,
         dwconv_wgrad.__dict__)
     for name, (op, _) in native_ops.items():
@@ -159,17 +161,59 @@ def _load_host(lib):
     host = module
 
 
-def native(*helpers):
-    """Decorator of an op that csrc/host.cpp can take.  `helpers`: names in the op's module that its configurators go by."""
-    def register(op):
-        origin = getattr(op, 'origin_function', op)
-        entries = [(origin.__globals__, name, origin.__globals__[name]) for name in helpers]
-        if origin is not op:
-            entries += [(None, name, conf) for name, conf in op.configurators.items()]
-        native_ops[origin.__name__] = (None if origin is op else op, entries)
-        return op
+# names that csrc/host.cpp reads on every call instead of relying on what they were at import
+_LIVE = frozenset(('_lib', 'host', '_table', 'SMALL_BYTES', 'L1_CACHE_BYTES', '_WAVES', '_TILE_D', '_TILE_W', '_LANE_C', 'FWD_VARIANTS',
+                   'WGRAD_VARIANTS'))
 
-    return register
+
+def _codes(code):
+    yield code
+    for const in code.co_consts:
+        if isinstance(const, types.CodeType):
+            yield from _codes(const)
+
+
+def _relied(function, found):
+    """Adds to `found` ({(id of a dictionary, key): (dictionary, key, value)}) every module-level name that `function` and the
+    functions of this package that it goes through read, and the attributes that they read of modules."""
+    def note(owner):
+        for name in names & owner.keys() - _LIVE:
+            if (id(owner), name) in found:
+                continue
+            value = owner[name]
+            found[id(owner), name] = (owner, name, value)
+            if name != 'load':
+                follow(value)
+
+    def follow(value):
+        if isinstance(value, types.ModuleType):
+            note(vars(value))
+        elif isinstance(value, types.FunctionType) and value.__module__.startswith(__package__):
+            _relied(value, found)
+
+    names = {name for code in _codes(function.__code__) for name in code.co_names} - {function.__name__}
+    note(function.__globals__)
+    # (modules that another function has been found to read, of which this one reads other attributes)
+    for name in names & function.__globals__.keys():
+        if isinstance(function.__globals__[name], types.ModuleType):
+            note(vars(function.__globals__[name]))
+    for cell in function.__closure__ or ():
+        follow(cell.cell_contents)
+
+
+def native(op):
+    """Decorator of an op that csrc/host.cpp can take."""
+    origin = getattr(op, 'origin_function', op)
+    found = {}
+    _relied(origin, found)
+    entries = []
+    if origin is not op:
+        entries = [(op.__dict__, 'origin_function', origin)] + [(None, name, conf) for name, conf in op.configurators.items()]
+        for conf in op.configurators.values():
+            if isinstance(conf, types.FunctionType):
+                _relied(conf, found)
+    native_ops[origin.__name__] = (None if origin is op else op, list(found.values()) + entries)
+    return op
 
 
 def last_error():
@@ -215,6 +259,3 @@ def workspace(nbytes, device):
     """Scratch buffer owned by the caller side of the ABI (torch's caching allocator)."""
     return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
 
-
-_helpers = [(globals(), name, globals()[name]) for name in ('load', 'call', 'query', 'stream_of', 'workspace')]
-_helpers += [(vars(stream_table), name, getattr(stream_table, name)) for name in ('_find', 'stream_shape')]

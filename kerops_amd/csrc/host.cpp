@@ -8,8 +8,8 @@
 // The Python functions stay what defines an op.  A function here takes a call only if nothing about it is unusual and
 // returns None otherwise, whereupon the caller goes on with the Python function: wrong shapes, types or devices (it
 // raises the op's own error), copies (a weight that is not contiguous), tensor subclasses, torch function and dispatch
-// modes, tracing, vmap, tensors of another than the current device, knobs passed by keyword, replaced configurators or
-// replaced helpers of the modules involved (`watch`).  Launch tables are read on every call.
+// modes, tracing, vmap, tensors of another than the current device, knobs passed by keyword, a replaced function, configurator
+// or module-level name that the Python function of the call would read (`watch`).  Launch tables are read on every call.
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
@@ -26,6 +26,7 @@
 #include <climits>
 #include <initializer_list>
 #include <optional>
+#include <utility>
 #include <vector>
 
 #include "../../include/kerops_hip.h"
@@ -63,12 +64,16 @@ enum Op {
     kOps
 };
 
+// The entries of one dictionary that have to be what they were.  A dictionary's version (no two states of any dictionaries
+// share one) says that nothing was written to it since they were last compared.
 struct Watched {
-    PyObject *dict, *key, *value;  // dict nullptr: the op's configurators of the moment
+    PyObject* dict;  // nullptr: the op's configurators of the moment
+    std::vector<std::pair<PyObject*, PyObject*>> entries;
+    uint64_t version = 0;
 };
 struct Relied {
     PyObject* op_dict = nullptr;  // the ConfiguredFunction's attributes (nullptr: a plain function)
-    std::vector<Watched> entries;
+    std::vector<Watched> dicts;
 };
 std::array<Relied, kOps> relied;
 std::array<PyObject*, kOps> op_names;
@@ -104,14 +109,28 @@ bool plain_thread()
            (c10::impl::tls_local_dispatch_key_set().included_.raw_repr() & ~usual) == 0;
 }
 
+bool as_before(PyObject* dict, Watched& w)
+{
+#if PY_VERSION_HEX < 0x030C0000
+    const uint64_t version = ((PyDictObject*)dict)->ma_version_tag;
+    if (version == w.version) return true;
+#endif
+    for (const auto& [key, value] : w.entries)
+        if (PyDict_GetItem(dict, key) != value) return false;
+#if PY_VERSION_HEX < 0x030C0000
+    w.version = version;
+#endif
+    return true;
+}
+
 bool steady(Op op)
 {
-    const Relied& r = relied[op];
+    Relied& r = relied[op];
     PyObject* configurators = r.op_dict ? PyDict_GetItem(r.op_dict, k_configurators) : nullptr;
     if (r.op_dict && !(configurators && PyDict_CheckExact(configurators))) return false;
-    for (const Watched& w : r.entries)
-        if (PyDict_GetItem(w.dict ? w.dict : configurators, w.key) != w.value) return false;
-    return !r.entries.empty() && plain_thread();
+    for (Watched& w : r.dicts)
+        if (!as_before(w.dict ? w.dict : configurators, w)) return false;
+    return !r.dicts.empty() && plain_thread();
 }
 
 // ---- arguments ----
@@ -871,12 +890,18 @@ PyObject* setup(PyObject*, PyObject* args)
         Relied r;
         if (op_dict != Py_None) r.op_dict = op_dict, Py_INCREF(op_dict);
         for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
-            Watched w;
-            if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "OOO", &w.dict, &w.key, &w.value)) return nullptr;
-            if (w.dict == Py_None && r.op_dict) w.dict = nullptr;
-            else if (!PyDict_Check(w.dict)) return PyErr_Format(PyExc_RuntimeError, "%U: not a dictionary", op_names[op]);
-            Py_XINCREF(w.dict), Py_INCREF(w.key), Py_INCREF(w.value);
-            r.entries.push_back(w);
+            PyObject *dict, *key, *value;
+            if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "OOO", &dict, &key, &value)) return nullptr;
+            if (dict == Py_None && r.op_dict) dict = nullptr;
+            else if (!PyDict_Check(dict)) return PyErr_Format(PyExc_RuntimeError, "%U: not a dictionary", op_names[op]);
+            size_t d = 0;
+            while (d < r.dicts.size() && r.dicts[d].dict != dict) ++d;
+            if (d == r.dicts.size()) {
+                Py_XINCREF(dict);
+                r.dicts.push_back({dict, {}});
+            }
+            Py_INCREF(key), Py_INCREF(value);
+            r.dicts[d].entries.emplace_back(key, value);
         }
         relied[op] = std::move(r);
     }

@@ -11,7 +11,7 @@ from ..settings.stream_table import stream_knob
 from ._common import next_power_of_2, numel_no_channels, require_cuda, stream_waves
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('AddStats', 'num_warps'),
            blocks=stream_knob('AddStats', 'blocks'), segment=stream_knob('AddStats', 'segment'))
 def AddStats(
@@ -43,7 +43,7 @@ def AddStats(
     return output, mean, sqmean
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('AddStatsBackward', 'num_warps', 'add_grad'),
            blocks=stream_knob('AddStatsBackward', 'blocks', 'add_grad'),
            segment=stream_knob('AddStatsBackward', 'segment', 'add_grad'))

@@ -14,7 +14,7 @@ from ..settings.stream_table import stream_knob, stream_shape
 from ._common import next_power_of_2, require_cuda, stream_waves
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('AvgPoolCeilStats', 'num_warps'),
            blocks=stream_knob('AvgPoolCeilStats', 'blocks'), segment=stream_knob('AvgPoolCeilStats', 'segment'))
 def AvgPoolCeilStats(x, *, l1_cache_bytes: ConfigurableArg, num_warps: ConfigurableArg, blocks: ConfigurableArg,
@@ -51,7 +51,7 @@ def AvgPoolCeilStats(x, *, l1_cache_bytes: ConfigurableArg, num_warps: Configura
     return output, mean, sqmean
 
 
-@_lib.native()
+@_lib.native
 @configure(blocks=stream_knob('ApplyBNReLUAvgPoolCeilStats', 'blocks'),
            num_warps=stream_knob('ApplyBNReLUAvgPoolCeilStats', 'num_warps'),
            segment=stream_knob('ApplyBNReLUAvgPoolCeilStats', 'segment'))
@@ -96,7 +96,7 @@ def _backward_knob(key):
     return knob
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=_backward_knob('num_warps'), blocks=_backward_knob('blocks'),
            segment=_backward_knob('segment'))
 def AvgPoolCeilStatsBackward(

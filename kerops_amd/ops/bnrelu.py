@@ -13,7 +13,7 @@ from ..settings.stream_table import stream_knob
 from ._common import next_power_of_2, numel_no_channels, require_cuda, stream_waves
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('ApplyBNReLU', 'num_warps'),
            blocks=stream_knob('ApplyBNReLU', 'blocks'), segment=stream_knob('ApplyBNReLU', 'segment'))
 def ApplyBNReLU(
@@ -42,7 +42,7 @@ def ApplyBNReLU(
     return output
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('ApplyBNReLUBackward', 'num_warps'),
            blocks=stream_knob('ApplyBNReLUBackward', 'blocks'), segment=stream_knob('ApplyBNReLUBackward', 'segment'))
 def ApplyBNReLUBackward(

@@ -41,7 +41,7 @@ def lanec(channels):
     return _LANE_C[channels]
 
 
-@_lib.native('warps', 'dblock', 'wtile', 'lanec', 'nearest_conv_shape')
+@_lib.native
 @configure(
     ACCTYPE='float32',
     num_warps=lambda x: warps(x.shape[1], x.shape[4]),

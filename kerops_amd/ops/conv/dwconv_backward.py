@@ -18,7 +18,7 @@ def served(channels):
     return {8: 0, 16: 0, 32: 0, 64: 0, 128: 0}[channels]
 
 
-@_lib.native('served')
+@_lib.native
 @configure(H_chunk=lambda x: served(x.shape[1]), out_dtype=torch.float16)
 def DWConvBackward(x, grad, weight, *, H_chunk: ConfigurableArg, out_dtype: ConfigurableArg):
     """x, grad (N,C,H,W,D) fp16 channels_last_3d, weight [3,3,3,C] fp16 -> (grad_x like x, grad_w [3,3,3,C]).

@@ -10,7 +10,7 @@ from ... import _lib
 from .._common import cl3d, next_power_of_2, require_cuda
 
 
-@_lib.native()
+@_lib.native
 def DWConvStats(x, weight):
     """Returns (y, mean, sqmean): y = DWConv(x, weight) (bit-identical), mean / sqmean = Stats(y)
     (fp32, per channel; fp32 partial sums per workgroup, added in fp64 in a fixed order)."""

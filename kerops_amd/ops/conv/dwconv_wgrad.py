@@ -49,7 +49,7 @@ def ilp(channels):
     return {8: 1, 16: 1, 32: 1, 64: 1, 128: 1}[channels]
 
 
-@_lib.native('warps', 'dblock', 'wtile', 'lanec', 'ilp', 'nearest_conv_shape')
+@_lib.native
 @configure(
     ACCTYPE='float32',
     num_warps=lambda x: warps(x.shape[1]),

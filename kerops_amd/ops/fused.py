@@ -31,7 +31,7 @@ def PointwiseLinear(x, weight, relu_in=False):
     return out
 
 
-@_lib.native()
+@_lib.native
 @configure(reserved=0)
 def DWSepBlock(x, dw_weight, scale, shift, pw_weight, *, reserved: ConfigurableArg):
     """Returns (y fp16 (N,Cout,H,W,D) channels_last_3d, absmax fp32 1-element device tensor)."""

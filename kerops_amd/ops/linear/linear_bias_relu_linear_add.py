@@ -23,7 +23,7 @@ def ilp(channels):
     return {16: 1, 32: 1, 64: 1}[channels]
 
 
-@_lib.native('dblock', 'ilp')
+@_lib.native
 @configure(num_warps=4, D_block=lambda x: dblock(x.shape[1]), ILP=lambda x: ilp(x.shape[1]))
 def LinBReLULinAdd(x, weight_up, weight_down, bias, add_other, *, num_warps: ConfigurableArg,
                    D_block: ConfigurableArg, ILP: ConfigurableArg):

@@ -20,7 +20,7 @@ def dblock(channels):
     return {16: 64, 32: 64, 64: 64}[channels]
 
 
-@_lib.native('dblock')
+@_lib.native
 @configure(num_warps=4, D_block=lambda x: dblock(x.shape[1]), ILP=1, out_dtype=torch.float16)
 def LinBReLULinBackward(x, grad, weight_up, weight_down, bias, *, num_warps: ConfigurableArg,
                         D_block: ConfigurableArg, ILP: ConfigurableArg, out_dtype: ConfigurableArg):

@@ -19,7 +19,7 @@ def ilp(in_channels):
     return {16: 1, 32: 1, 64: 1, 128: 1}[in_channels]
 
 
-@_lib.native('ilp')
+@_lib.native
 @configure(num_warps=4, D_block=32, ILP=lambda x: ilp(x.shape[1]))
 def ReLULinearAdd(x, weight, add_other, *, num_warps: ConfigurableArg, D_block: ConfigurableArg,
                   ILP: ConfigurableArg):
@@ -46,7 +46,7 @@ def ReLULinearAdd(x, weight, add_other, *, num_warps: ConfigurableArg, D_block: 
     return output
 
 
-@_lib.native()
+@_lib.native
 def ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other):
     """ReLULinearAdd(ApplyBNReLU(x, bn_weight, bn_bias), weight, add_other) in one pass, bit-identical to that
     composition (kerops/ops/bnrelu.py:11-42 then kerops/ops/linear/relu_linear_add.py:20-52): the normalised

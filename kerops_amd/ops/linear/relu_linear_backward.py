@@ -27,7 +27,7 @@ def dblock(in_channels):
     return {16: 64, 32: 64, 64: 64, 128: 64}[in_channels]
 
 
-@_lib.native('warps', 'dblock')
+@_lib.native
 @configure(
     num_warps=lambda x: warps(x.shape[1]),
     D_block=lambda x: dblock(x.shape[1]),
@@ -80,7 +80,7 @@ def ReLULinearBackward(
     return x_grad, (weight_grad if direct else weight_grad.to(out_dtype))
 
 
-@_lib.native()
+@_lib.native
 def ApplyBNReLULinearBackward(x, bn_weight, bn_bias, grad, weight):
     """Gradients of ApplyBNReLULinearAdd(x, bn_weight, bn_bias, weight, add_other) in one pass over x and grad.
     Returns (dx like x, bn_weight_grad fp32, bn_bias_grad fp32, weight_grad fp16): dx bit-identical to ApplyBNReLU,

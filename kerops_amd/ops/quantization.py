@@ -23,7 +23,7 @@ def _dense(x):
     )
 
 
-@_lib.native()
+@_lib.native
 @configure(num_warps=stream_knob('QuantUint8Window', 'num_warps'), l1_cache_bytes=get_l1_cache,
            blocks=stream_knob('QuantUint8Window', 'blocks'), segment=stream_knob('QuantUint8Window', 'segment'))
 def QuantUint8Window(x, window, *, num_warps: ConfigurableArg, l1_cache_bytes: ConfigurableArg,
@@ -42,7 +42,7 @@ def QuantUint8Window(x, window, *, num_warps: ConfigurableArg, l1_cache_bytes: C
     return output
 
 
-@_lib.native()
+@_lib.native
 @configure(num_warps=stream_knob('DequantUint8Window', 'num_warps'), l1_cache_bytes=get_l1_cache,
            blocks=stream_knob('DequantUint8Window', 'blocks'), segment=stream_knob('DequantUint8Window', 'segment'))
 def DequantUint8Window(x, init_dtype, window, *, num_warps: ConfigurableArg, l1_cache_bytes: ConfigurableArg,
@@ -73,7 +73,7 @@ def AbsMax(y, *, blocks: ConfigurableArg):
     return out
 
 
-@_lib.native()
+@_lib.native
 @configure(blocks=stream_knob('QuantInt8Sym', 'blocks', 'y'), num_warps=stream_knob('QuantInt8Sym', 'num_warps', 'y'),
            segment=stream_knob('QuantInt8Sym', 'segment', 'y'))
 def QuantInt8Sym(y, absmax=None, *, blocks: ConfigurableArg, num_warps: ConfigurableArg, segment: ConfigurableArg):

@@ -11,7 +11,7 @@ from ..settings.stream_table import stream_knob
 from ._common import next_power_of_2, numel_no_channels, require_cuda, stream_waves
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('Stats', 'num_warps'),
            blocks=stream_knob('Stats', 'blocks'), segment=stream_knob('Stats', 'segment'))
 def Stats(x, *, l1_cache_bytes: ConfigurableArg, num_warps: ConfigurableArg, blocks: ConfigurableArg,
@@ -40,7 +40,7 @@ def Stats(x, *, l1_cache_bytes: ConfigurableArg, num_warps: ConfigurableArg, blo
     return mean, sqmean
 
 
-@_lib.native()
+@_lib.native
 @configure(l1_cache_bytes=get_l1_cache, num_warps=stream_knob('StatsBackward', 'num_warps'),
            blocks=stream_knob('StatsBackward', 'blocks'), segment=stream_knob('StatsBackward', 'segment'))
 def StatsBackward(

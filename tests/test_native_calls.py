@@ -128,6 +128,41 @@ def test_native_calls_built_for_another_version_are_refused(host, monkeypatch, o
     assert _lib.host is host
 
 
+# what the Python function of an op reads of this package when it is called
+READ = {'AvgPoolCeilStatsBackward': {'stream_shape', 'require_cuda', 'stream_waves', 'ceil', '_find', 'call', 'stream_of'},
+        'Stats': {'numel_no_channels', 'require_cuda', 'stream_waves', 'next_power_of_2', 'query', 'workspace', '_find'},
+        'QuantUint8Window': {'_dense', 'require_cuda', 'stream_waves', 'BUILT_WAVES'},
+        'DWConv': {'warps', 'dblock', 'wtile', 'lanec', 'nearest_conv_shape', 'require_cuda', 'next_power_of_2', 'load'},
+        'DWConvStats': {'cl3d', 'require_cuda', 'next_power_of_2', 'workspace'}}
+
+
+@pytest.mark.parametrize('name', OPS)
+def test_everything_that_a_python_function_reads_is_compared(host, name):
+    found = {}
+    _lib._relied(getattr(OPS[name], 'origin_function', OPS[name]), found)
+    compared = {(id(owner), key) for owner, key, _ in _lib.native_ops[name][1]}
+    assert set(found) <= compared, 'a name defined behind its op'  # (the list is made where the op is defined)
+    assert READ.get(name, set()) <= {key for _, key, _ in _lib.native_ops[name][1]}
+    assert not hasattr(OPS[name], 'origin_function') or (id(OPS[name].__dict__), 'origin_function') in compared
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', OPS)
+def test_a_call_with_a_replaced_name_is_left_to_the_python_function(host, monkeypatch, name):
+    args = arguments(name, 'plain' if name != 'DWSepBlock' else 'odd', DEV)
+    call = getattr(host, name)
+    assert call(*args) is not None
+    for owner, key, value in _lib.native_ops[name][1]:
+        if owner is None:
+            owner = OPS[name].configurators
+        if owner.get('__name__', '').split('.')[0] == 'torch' or not callable(value) or isinstance(value, type):
+            continue
+        with monkeypatch.context() as m:
+            m.setitem(owner, key, functools.partial(value))
+            assert call(*args) is None, key
+        assert call(*args) is not None, key
+
+
 def _clone(op):
     return functools.wraps(op)(type(op)(op.origin_function, op.signature, op.configurable_args, op.usual_args, **op.configurators))
 
