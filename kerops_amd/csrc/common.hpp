@@ -403,7 +403,8 @@ static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots
     }
     return {part, best_h};
 }
-// offsets inside one (W, D, C) plane are 32-bit in the convolution kernels (W, D, C positive)
+// offsets inside one (W, D, C) plane are 32-bit in the convolution kernels (W, D, C positive): an element's index is an int,
+// its byte offset a uint32_t (doubled as an int it would overflow from 2^30 elements on)
 static inline bool plane_exceeds_i32(int W, int D, int C)
 {
     const int64_t wd = (int64_t)W * D;  // < 2^62

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
             const int w = w0 - 1 + wq, d = d0 - 1 + dq;
             const bool ok = (blk < Cfg::NGB) && (wq < Cfg::R) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
             const int cbyte = (cs * 16 - Cfg::rot(dq)) & (PB - 1);
-            gvo[i] = ok ? (uint32_t)(((w * D + d) * C + cslab) * 2 + cbyte) : 0u;
+            gvo[i] = ok ? ((uint32_t)(w * D + d) * C + cslab) * 2u + cbyte : 0u;
             // chunks no other workgroup reads (the patch without its border ring) take the streaming hint
             const bool interior = NTI && (wq >= 2) && (wq <= TW - 1) && (dq >= 2) && (dq <= TD - 1);
             gmask[i] = __ballot(ok && !interior);
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
             const int w = w0 + wq, d = d0 + dq;
             const bool ok = (blk < Cfg::NXB) && (wq < TW) && (w < W) && (d < D);
             const int cbyte = (cs * 16 - Cfg::rot(dq)) & (PB - 1);
-            xvo[i] = ok ? (uint32_t)(((w * D + d) * C + cslab) * 2 + cbyte) : 0u;
+            xvo[i] = ok ? ((uint32_t)(w * D + d) * C + cslab) * 2u + cbyte : 0u;
             xmask[i] = __ballot(ok);
             xlds[i] = lds0 + Cfg::XOFF + (blk < Cfg::NXB ? blk : 0) * 1024;
         }
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void dwconv_bwd_dma_kernel(const WgArgs
             for (int o = 0; o < RO; ++o) {
                 const int w = w0 + ra + o, d = d0 + pgrp + rr;
                 const bool ok = (w < W) && (d < D);
-                ooff[o] = ok ? (uint32_t)(((w * D + d) * C + cslab) * 2 + cb) : 0u;
+                ooff[o] = ok ? ((uint32_t)(w * D + d) * C + cslab) * 2u + cb : 0u;
                 omask[o] = __ballot(ok);
             }
             float4_t T[RO][CPL];  // dx tiles, four planes in a ring of registers

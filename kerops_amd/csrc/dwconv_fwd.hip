@@ -205,7 +205,7 @@ __device__ __forceinline__ void dwconv_fwd_body(const FwdArgs& a, half8_t (&lds)
         const int cq = r - dq * CG;
         const int w = w0 - 1 + wq, d = d0 - 1 + dq;
         gval[j] = (q < NCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-        goff[j] = gval[j] ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
+        goff[j] = gval[j] ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : 0u;
         ldst[j] = gval[j] ? q : NCH;
         // halo chunks outside the volume never change: zero them once in both buffers
         if (q < NCH && !gval[j]) {
@@ -227,7 +227,7 @@ __device__ __forceinline__ void dwconv_fwd_body(const FwdArgs& a, half8_t (&lds)
         lbase[k] = (wl * PD + dl) * SC + cl * CL;  // in halves
         const int w = w0 + wl, d = d0 + dl;
         oval[k] = (w < W) && (d < D);
-        ooff[k] = oval[k] ? (uint32_t)(((w * D + d) * C + cslab + cl * CL) * 2) : 0u;
+        ooff[k] = oval[k] ? ((uint32_t)(w * D + d) * C + cslab + cl * CL) * 2u : 0u;
     }
 
     float a0[P][CL], a1[P][CL], a2[P][CL];
@@ -521,7 +521,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
         Order::decode(ch, wq, dq, cq);
         const int w = w0 - 1 + wq, d = d0 - 1 + dq;
         const bool ok = (ch < Cfg::NXCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-        xgo[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : kNoVoxel;
+        xgo[j] = ok ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : kNoVoxel;
         xls[j] = ch < Cfg::NXCH ? lds_swizzle<PB>(wq * PDP + dq, cq * 16) : Cfg::DUMP;
     }
 
@@ -597,7 +597,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     for (int i = 0; i < NY2; ++i) {
         const int c = t + i * NT, row = c / (COUT / 8), cc = c - row * (COUT / 8);
         const int w = w0 + row / TD, d = d0 + row % TD;
-        y2go[i] = (w < W && d < D) ? (uint32_t)(((w * D + d) * COUT + cc * 8) * 2) : kNoVoxel;
+        y2go[i] = (w < W && d < D) ? ((uint32_t)(w * D + d) * COUT + cc * 8) * 2u : kNoVoxel;
     }
     const uint32_t y2_bytes = (uint32_t)((int64_t)W * D * COUT * 2);
     half_t* yn2 = MODE == 2 ? a.y2 + (int64_t)n * H * W * D * COUT : nullptr;
@@ -623,7 +623,7 @@ __device__ __forceinline__ void dwconv_fwd_mfma_segment(const FwdArgs& a, unsign
     const int ord = ot_swz(opos, ocq * 16);
     const int ow = w0 + opos / TD, odd = d0 + opos % TD;
     const bool ovalid = (ow < W) && (odd < D);
-    const uint32_t ogo = ovalid ? (uint32_t)(((ow * D + odd) * C + cslab + ocq * 8) * 2) : kNoVoxel;
+    const uint32_t ogo = ovalid ? ((uint32_t)(ow * D + odd) * C + cslab + ocq * 8) * 2u : kNoVoxel;
     int pending_row = -1;
     auto flush_row = [&](int par) {  // stores the plane that the previous step left in output tile par, if it did
         if constexpr (BOUNCE) {

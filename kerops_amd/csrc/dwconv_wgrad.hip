@@ -97,7 +97,7 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::NT >= 512 || Cfg::STRAIGHT) ? 4 : 3)
         const int cq = r - dq * CG;
         const int w = w0 - 1 + wq, d = d0 - 1 + dq;
         const bool ok = (q < NCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-        goff[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
+        goff[j] = ok ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : 0u;
         ldst[j] = ok ? q : NCH;
         if (q < NCH && !ok) {
             const half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::NT >= 512 || Cfg::STRAIGHT) ? 4 : 3)
         const int w = w0 + wl, d = d0 + dl;
         pv0[k] = (w < W) && (d < D);
         pv1[k] = (w < W) && (d + 1 < D);
-        poff[k] = pv0[k] ? (uint32_t)(((w * D + d) * C + cslab + cl * CL) * 2) : 0u;
+        poff[k] = pv0[k] ? ((uint32_t)(w * D + d) * C + cslab + cl * CL) * 2u : 0u;
     }
 
     float acc[27][CL];
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NT >= 512 ? 4 : 3) void dwconv_wgrad_
             Order::decode(ch, wq, dq, cq);
             const int w = w0 - 1 + wq, d = d0 - 1 + dq;
             const bool ok = (ch < Cfg::NXCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-            xgo[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
+            xgo[j] = ok ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : 0u;
             xls[j] = ok ? Cfg::swz(wq * PDP + dq, cq * 16) : -1;
         }
     #pragma unroll
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NT >= 512 ? 4 : 3) void dwconv_wgrad_
             const int dq = rem / CG, cq = rem - dq * CG;
             const int w = w0 + wq, d = d0 + dq;
             const bool ok = (ch < Cfg::NGCH) && (w < W) && (d < D);
-            ggo[j] = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
+            ggo[j] = ok ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : 0u;
             gls[j] = ok ? Cfg::swz(wq * TD + dq, cq * 16) : -1;
         }
 
@@ -744,7 +744,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_bwd_split_kernel(const WgAr
         const int dq = rem / CG, cq = rem - dq * CG;
         const int w = w0 - 1 + wq, d = d0 - 1 + dq;
         const bool ok = (ts < Cfg::NCH) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
-        go = ok ? (uint32_t)(((w * D + d) * C + cslab + cq * 8) * 2) : 0u;
+        go = ok ? ((uint32_t)(w * D + d) * C + cslab + cq * 8) * 2u : 0u;
         ls = ok ? lds_swizzle<PB>(wq * PDP + dq, cq * 16) : -1;
         // x: the patch alone (the weight gradient is summed over the x positions of the patch against the g
         // positions around them, so that only one of the two tensors is read with a halo)
@@ -752,7 +752,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_bwd_split_kernel(const WgAr
         const int xrem = ts - xwq * (TD * CG);
         const int xdq = xrem / CG, xcq = xrem - xdq * CG;
         const bool xok = (ts < Cfg::NXCH) && (w0 + xwq < W) && (d0 + xdq < D);
-        xgo = xok ? (uint32_t)((((w0 + xwq) * D + d0 + xdq) * C + cslab + xcq * 8) * 2) : 0u;
+        xgo = xok ? ((uint32_t)((w0 + xwq) * D + d0 + xdq) * C + cslab + xcq * 8) * 2u : 0u;
         xls = xok ? lds_swizzle<PB>(xwq * TD + xdq, xcq * 16) : -1;
         return true;
     };
@@ -823,7 +823,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_bwd_split_kernel(const WgAr
             const int ord = ot_swz(opos, ocq * 16);
             const int ow = w0 + opos / TD, odd = d0 + opos % TD;
             const bool ovalid = (ow < W) && (odd < D);
-            const uint32_t ogo = ovalid ? (uint32_t)(((ow * D + odd) * C + cslab + ocq * 8) * 2) : 0u;
+            const uint32_t ogo = ovalid ? ((uint32_t)(ow * D + odd) * C + cslab + ocq * 8) * 2u : 0u;
             parity = 0;
             prefetch(hs - 1, xpre0, gpre0);
             prefetch(hs, xpre1, gpre1);

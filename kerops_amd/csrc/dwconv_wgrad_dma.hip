@@ -199,7 +199,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_wgrad_dma_kernel(const WgAr
             const int w = w0 - 1 + wq, d = d0 - 1 + dq;
             const bool ok = (blk < Cfg::NXB) && (wq < Cfg::R) && (w >= 0) && (w < W) && (d >= 0) && (d < D);
             const int cbyte = (cs * 16 - Cfg::rot(dq)) & (PB - 1);
-            xvo[i] = ok ? (uint32_t)(((w * D + d) * C + cslab) * 2 + cbyte) : 0u;
+            xvo[i] = ok ? ((uint32_t)(w * D + d) * C + cslab) * 2u + cbyte : 0u;
             const bool interior = NTI && (wq >= 2) && (wq <= TW - 1) && (dq >= 2) && (dq <= TD - 1);
             xmask[i] = __ballot(ok && !interior);
             xmask_in[i] = __ballot(ok && interior);
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(Cfg::NT, 4) void dwconv_wgrad_dma_kernel(const WgAr
             const int w = w0 + wq, d = d0 + dq;
             const bool ok = (blk < Cfg::NGB) && (wq < TW) && (w < W) && (d < D);
             const int cbyte = (cs * 16 - Cfg::rot(dq)) & (PB - 1);
-            gvo[i] = ok ? (uint32_t)(((w * D + d) * C + cslab) * 2 + cbyte) : 0u;
+            gvo[i] = ok ? ((uint32_t)(w * D + d) * C + cslab) * 2u + cbyte : 0u;
             gmask[i] = __ballot(ok);
             glds[i] = lds0 + (blk < Cfg::NGB ? blk : 0) * 1024;
         }

@@ -10,6 +10,7 @@ from kerops_amd.ops.addition import AddStats, AddStatsBackward
 from kerops_amd.ops.avgpool import AvgPoolCeilStats, AvgPoolCeilStatsBackward
 from kerops_amd.ops.bnrelu import ApplyBNReLU, ApplyBNReLUBackward
 from kerops_amd.ops.conv import DWConv, DWConvBackward, DWConvStats, DWConvWGRAD
+from kerops_amd.ops.fused import DWSepBlock
 from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackward, LinBReLULinAdd,
                                    LinBReLULinBackward, ReLULinearAdd, ReLULinearBackward)
 from kerops_amd.ops.quantization import DequantUint8Window, QuantInt8Sym, QuantUint8Window
@@ -375,3 +376,58 @@ def test_depthwise_marches_of_any_length(c, w, d, h_chunk):
     assert torch.equal(bits(dx), bits(dx_ref))
     # fp32 sums of a few thousand products in another order
     assert ((gw - gw_ref).norm() / gw_ref.norm()).item() < 1e-5
+
+
+# planes of just under 2^31 elements (the largest accepted): the byte offsets of the buffer accesses go up to 2^32 - 16
+@pytest.mark.parametrize('c,w,d', [(8, 16383, 16384), (64, 5793, 5792)])
+def test_depthwise_planes_up_to_four_gigabytes(c, w, d):
+    gen = torch.Generator(DEV).manual_seed(c)
+    x = torch.randn(1, 1, w, d, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3)
+    taps = (torch.randn(3, 3, 3, c, device=DEV, generator=gen) / 27 ** 0.5).half()
+    rows = 40
+    half = 2 ** 31 // (2 * c * d)  # the row of W with the voxel at byte 2^31
+    # an output depends on its neighbours alone: the rows of a narrower plane around the place, without its edge rows
+    parts = [(0, rows, 0, rows - 1), (half - rows // 2, half + rows // 2, 1, rows - 1), (w - rows, w, 1, rows)]
+    y, _, _ = DWConvStats(x, taps)
+    assert torch.equal(y, DWConv(x, taps))
+    dx, gw = DWConvBackward(x, x, taps, out_dtype=torch.float32)
+    for a, b, first, last in parts:
+        sub = x[:, :, :, a:b].contiguous(memory_format=torch.channels_last_3d)
+        for whole, part in ((y, DWConv(sub, taps)), (dx, DWConvBackward(sub, sub, taps)[0])):
+            assert torch.equal(bits(whole[:, :, :, a + first:a + last]), bits(part[:, :, :, first:last]))
+    del y, dx
+    # the centre tap's gradient of x with itself is a sum of squares: all of the plane, or a part of it is missing
+    flat_x = x.permute(0, 2, 3, 4, 1).reshape(-1, c)
+    square = sum(t.double().square().sum(0) for t in flat_x.split(1 << 22))
+    assert ((gw[1, 1, 1] - square).abs() <= 1e-4 * square).all()
+
+
+def test_fused_block_planes_up_to_four_gigabytes():
+    w, d = 4095, 4096
+    gen = torch.Generator(DEV).manual_seed(1)
+    x = torch.randn(1, 1, w, d, 64, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3)
+    taps = (torch.randn(3, 3, 3, 64, device=DEV, generator=gen) / 27 ** 0.5).half()
+    scale, shift = torch.rand(64, device=DEV, generator=gen) + 0.5, torch.randn(64, device=DEV, generator=gen) * 0.1
+    mix = (torch.randn(64, 128, device=DEV, generator=gen) / 8).half()
+    y, peak = DWSepBlock(x, taps, scale, shift, mix)
+    assert peak.item() == max(t.abs().amax().item() for t in y.permute(0, 2, 3, 4, 1).reshape(-1, 128).split(1 << 22))
+    for a, b, first, last in ((0, 40, 0, 39), (2028, 2068, 1, 39), (w - 40, w, 1, 40)):
+        part, _ = DWSepBlock(x[:, :, :, a:b].contiguous(memory_format=torch.channels_last_3d), taps, scale, shift, mix)
+        assert torch.equal(bits(y[:, :, :, a + first:a + last]), bits(part[:, :, :, first:last]))
+
+
+def test_pool_backward_rows_up_to_four_gigabytes():
+    n, c, h, w, d = 1, 8, 650, 650, 635
+    gen = torch.Generator(DEV).manual_seed(2)
+    grad, pooled = (torch.randn(n, h // 2, w // 2, (d + 1) // 2, c, device=DEV, generator=gen, dtype=torch.float16) for _ in range(2))
+    mg, sg = torch.randn(c, device=DEV, generator=gen) * 1e7, torch.randn(c, device=DEV, generator=gen) * 1e7
+    m = torch.tensor(float(pooled.numel() // c), device=DEV)
+    dx = AvgPoolCeilStatsBackward(grad.permute(0, 4, 1, 2, 3), mg, sg, pooled.permute(0, 4, 1, 2, 3), (n, c, h, w, d))
+    out = dx.permute(0, 2, 3, 4, 1)
+    taps = torch.full(((d + 1) // 2,), 8.0, device=DEV)
+    taps[-1] = 4.0
+    for a in (*range(0, 325, 40), 162, 163, 324):  # (byte 2^31 is in the rows of 162)
+        g, o = grad[0, a].float(), pooled[0, a].float()
+        ref = ((g + mg / m + 2.0 * o * sg / m) / taps[:, None]).half().repeat_interleave(2, 0).repeat_interleave(2, 1)[:, :d]
+        for row in (2 * a, 2 * a + 1):
+            assert torch.equal(bits(out[0, row]), bits(ref))
