@@ -157,7 +157,9 @@ int kerops_dwconv_bwd_f16_out(const void* x, const void* g, const void* wt, void
 /* Per-channel mean and mean of squares over M = numel / C voxels, fp32.
  * Replaces the zero-fill of mean/sqmean and the `_Stats_cl3d_impl[(grid,)](...)`
  * launch: kerops/ops/stats.py:27-31 (kernel kerops/kernels/stats.py:6-23).
- * Two-pass and deterministic instead of float atomics. */
+ * Two-pass and deterministic instead of float atomics.  With blocks = 0 the workgroups hand over their sums with what their
+ * rounding to fp32 left if the workspace has room for it (the one that the query with blocks = 0 asks for does): a smaller
+ * workspace that is still accepted can change the last bits. */
 int64_t kerops_stats_workspace_bytes(int64_t M, int32_t C, int32_t blocks);
 int kerops_stats_f16(const void* x, float* mean, float* sqmean, int64_t M, int32_t C, void* workspace,
                      int64_t workspace_bytes, int32_t blocks, int32_t waves, int32_t segment, void* stream);

@@ -45,11 +45,12 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_fwd_kernel(const ha
                                                                         const float* __restrict__ bb,
                                                                         half_t* __restrict__ y, float* __restrict__ ws,
                                                                         const PoolDims p, int64_t nchunks,
-                                                                        int segments)
+                                                                        int segments, int pairs)
 {
     typedef typename HVec<V>::type hv;
-    __shared__ float red[4 * 2 * 64 * V];
+    __shared__ double red[4 * 2 * 64 * V];
     const ChunkWalk<U> wk(nchunks, segments != 0);
+    // (in fp32 over all steps: fp64 takes the registers of a second window in flight, and few workgroups pool few windows)
     float acc[2][V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[0][j] = acc[1][j] = 0.0f;
@@ -184,7 +185,9 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_fwd_kernel(const ha
         load_window(i, wn);
         finish_window(i, wn);
     }
-    block_channel_partials_any<2, V>(acc, p.CG, red, ws + (int64_t)blockIdx.x * 2 * p.CG * V);
+    ChannelTotals<V> sums;
+    sums.take(acc);
+    sums.write(p.CG, red, ws, pairs);
 }
 
 // PERM (16-byte chunks, even D, whole wavefronts inside one pooled row, fewer than 64 channels): a wavefront's 64
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_bwd_rows_kernel(
 // step: 1 = interleaved (one window per thread in flight), 2 = contiguous runs of two chunks per thread (two
 // windows, 16 loads, in flight).  Built-in choices by the size of the volume that is pooled; the largest measured at
 // (1,64,350,350,128).  GPU time per launch in a row of launches at 64 channels, inputs from memory:
-//   forward   24 / 48 / 96 / 192 MiB: (1280,4,1) or (256,4,1) 13.8 / 19.5 / 30.3 / 49.1 us, here 13.4 / 18.2 / 27.7 / 46.2
+//   forward   24 / 48 / 96 / 192 MiB: (1280,4,1) or (256,4,1) 14.4 / 20.1 / 30.4 / 49.3 us, here 11.6 / 16.1 / 25.2 / 43.8
 //   backward  24 / 48 / 96 / 192 MiB: (768,4,1) or (256,4,1) 8.4 / 14.8 / 27.5 / 49.2, here 7.2 / 13.1 / 26.1 / 45.9
 struct PoolDefault {
     int64_t below;  // bytes
@@ -392,7 +395,6 @@ constexpr PoolDefault kDefPoolBwd[] = {{32 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 
 // 95 MiB 26.3 / 24.6; 256 workgroups are too few (67 MiB 27.5, 368 137), 1024 to 4096 no better
 constexpr PoolDefault kDefPoolBwdRows[] = {{6 * kMiB, 512, 4, 1}, {kAnySize, 512, 4, 2}};
 constexpr PoolDefault kDefPoolBwdRows8[] = {{6 * kMiB, 512, 4, 1}, {64 * kMiB, 512, 4, 2}, {kAnySize, 512, 4, 1}};
-constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
 
 // Backward: the condition of the redistributing stores (PERM), and where the kernel in output order is the faster one.
 // us with results stored from where they are computed or redistributed, each with its best shape / in output order:
@@ -505,15 +507,16 @@ static int pool_fwd_run(const char* op, const void* x, const float* bw, const fl
     hipStream_t s = (hipStream_t)stream;
     float* ws = (float*)workspace;
     const int seg = sh.segment != 1;
+    const bool pairs = sum_pairs(blocks, sh.blocks, 2 * C, (int64_t)N * H * W * D * C * 2, workspace_bytes);
     const bool ntld = C >= 64;  // voxel rows of whole 128-byte lines
 #define KEROPS_POOL_GO(Uv, B)                                                                                      \
     KEROPS_DISPATCH_V(C, {                                                                                         \
         if (ntld)                                                                                                  \
             hipLaunchKernelGGL((avgpool_fwd_kernel<V, Uv, B, true>), dim3(sh.blocks), dim3(sh.threads), 0, s,      \
-                               (const half_t*)x, bw, bb, (half_t*)y, ws, p, nchunks, seg);                         \
+                               (const half_t*)x, bw, bb, (half_t*)y, ws, p, nchunks, seg, pairs);                         \
         else                                                                                                       \
             hipLaunchKernelGGL((avgpool_fwd_kernel<V, Uv, B, false>), dim3(sh.blocks), dim3(sh.threads), 0, s,     \
-                               (const half_t*)x, bw, bb, (half_t*)y, ws, p, nchunks, seg);                         \
+                               (const half_t*)x, bw, bb, (half_t*)y, ws, p, nchunks, seg, pairs);                         \
     })
     if (bw) {
         if (sh.segment == 2) KEROPS_POOL_GO(2, true);
@@ -526,7 +529,7 @@ static int pool_fwd_run(const char* op, const void* x, const float* bw, const fl
     rc = check_launch(op);
     if (rc != KEROPS_OK) return rc;
     const double Mo = (double)N * p.Ho * p.Wo * p.Do;
-    launch_reduce_rows(ws, sh.blocks, 2 * C, mean, sqmean, C, 1.0 / Mo, s);
+    launch_reduce_rows(ws, sh.blocks, 2 * C, mean, sqmean, C, 1.0 / Mo, s, pairs);
     return check_launch(op);
 }
 

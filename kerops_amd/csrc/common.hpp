@@ -730,25 +730,25 @@ constexpr int kStreamMaxThreads = 1024;
 // Sums of N values per lane over the lanes of a wavefront with the same lane % CG (CG <= 64 a power of two), pairs first at a
 // distance of 32 lanes, then 16, ...  A step halves the values that a lane goes on with: it hands the other half of them to
 // its partner, so N = 16 takes 8 + 4 + 2 + 1 exchanges, each step's in flight together, and one for every step after that.
-// (A butterfly per value is N log2(64 / CG) exchanges one after the other, 96 at CG = 1: Stats of (1,8,64,64,32) 10.7 us, here 5.4,
-// AddStats of (1,16,128,128,128) 40.4 and 36.1.)
+// (A butterfly per value is N log2(64 / CG) exchanges one after the other, 96 at CG = 1: with fp32 values Stats of (1,8,64,64,32)
+// 10.7 us, here 5.4, AddStats of (1,16,128,128,128) 40.4 and 36.1.)
 // `store(base, v)`: called with the N >> steps values that the lane has, the first of them number `base`, by one lane each.
-template <int N, int OFF = 32, class Store>
-__device__ __forceinline__ void wave_sums(float (&v)[N], int CG, int lane, int base, int spare, Store store)
+template <int N, int OFF = 32, class T, class Store>
+__device__ __forceinline__ void wave_sums(T (&v)[N], int CG, int lane, int base, int spare, Store store)
 {
     if constexpr (OFF > 0) {
         if (OFF >= CG) {  // (uniform)
             if constexpr (N > 1) {
                 const bool up = (lane & OFF) != 0;
-                float w[N / 2];
+                T w[N / 2];
 #pragma unroll
                 for (int k = 0; k < N / 2; ++k) {
-                    const float keep = up ? v[N / 2 + k] : v[k], give = up ? v[k] : v[N / 2 + k];
+                    const T keep = up ? v[N / 2 + k] : v[k], give = up ? v[k] : v[N / 2 + k];
                     w[k] = keep + __shfl_xor(give, OFF, 64);
                 }
                 wave_sums<N / 2, OFF / 2>(w, CG, lane, base + (up ? N / 2 : 0), spare, store);
             } else {
-                float w[1] = {v[0] + __shfl_xor(v[0], OFF, 64)};
+                T w[1] = {v[0] + __shfl_xor(v[0], OFF, 64)};
                 wave_sums<1, OFF / 2>(w, CG, lane, base, spare | OFF, store);  // both partners hold the sum
             }
             return;
@@ -760,42 +760,77 @@ __device__ __forceinline__ void wave_sums(float (&v)[N], int CG, int lane, int b
     }
 }
 
-// Sum NACC*V per-thread accumulators over the threads of a workgroup (up to 1024) that own the same channel group
-// (thread t owns group t % CG, CG <= 64 a power of two) and write the workgroup's partial [NACC][CG*V] to `dst`.  The
-// wavefronts hand their sums over in rounds of four through LDS (`red`: 4*NACC*CG*V floats); thread o keeps the running
-// sums of the outputs o, o + threads, ... (at most NACC*512 / 256 = 2*NACC of them) and adds the rounds in a fixed order.
-template <int NACC, int V>
-__device__ __forceinline__ void block_channel_partials_any(float (&acc)[NACC][V], int CG, float* red, float* dst)
-{
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave, nthr = blockDim.x, nwaves = nthr / kWave;
-    const int cols = CG * V, nout = NACC * cols;
-    float flat[NACC * V];
+typedef float fp32_pair_t __attribute__((ext_vector_type(2)));  // a sum rounded to fp32 and what the rounding left
+
+// Per-channel sums of a thread, then of its workgroup, in fp64.  A kernel adds the values of one step of its walk in fp32.  How
+// many steps a thread takes, and how many workgroups there are, goes with the launch shape, which is chosen for its speed:
+// with fp32 sums from step to step, over the lanes and in a workgroup's row, the error against 64 bits went with it.
+// Relative errors, zero-mean values, all-fp32 sums / now: dscale of ApplyBNReLUBackward of (1,64,192,192,128) 316e-9 / 32e-9,
+// dshift 69e-9 / 27e-9, mean of AddStats of (1,128,136,136,128) 43e-9 / 25e-9, of AvgPoolCeilStats of (1,64,61,63,63) 42e-9 /
+// 25e-9.  Time: 0.3 us for the exchanges in fp64, 0.4 for the pairs, up to 3 % of the largest ApplyBNReLUBackward.
+template <int V>
+struct ChannelTotals {
+    double tot[2 * V];
+    __device__ __forceinline__ ChannelTotals()
+    {
 #pragma unroll
-    for (int a = 0; a < NACC; ++a)
+        for (int j = 0; j < 2 * V; ++j) tot[j] = 0.0;
+    }
+    __device__ __forceinline__ void take(float (&acc)[2][V])  // and clears acc
+    {
 #pragma unroll
-        for (int j = 0; j < V; ++j) flat[a * V + j] = acc[a][j];
-    constexpr int kMine = 2 * NACC;
-    float run[kMine];
+        for (int j = 0; j < V; ++j) {
+            tot[j] += (double)acc[0][j];
+            tot[V + j] += (double)acc[1][j];
+            acc[0][j] = acc[1][j] = 0.0f;
+        }
+    }
+    // Adds the threads of the workgroup (up to 1024) that own the same channel group (thread t owns group t % CG, CG <= 64 a
+    // power of two) and writes the workgroup's row of the workspace, [2][CG*V] sums as fp32 or, `pairs`, as fp32_pair_t.  The
+    // wavefronts hand their sums over in rounds of four through LDS (`red`: 4*2*CG*V doubles); thread o keeps the running
+    // sums of the outputs o, o + threads, ... (at most four of them: 2*512 / 256) and adds the rounds in a fixed order.
+    __device__ __forceinline__ void write(int CG, double* red, float* ws, bool pairs)
+    {
+        const int t = threadIdx.x, lane = t % kWave, wave = t / kWave, nthr = blockDim.x, nwaves = nthr / kWave;
+        const int cols = CG * V, nout = 2 * cols;
+        constexpr int kMine = 4;
+        double run[kMine];
 #pragma unroll
-    for (int m = 0; m < kMine; ++m) run[m] = 0.0f;
-    for (int r = 0; r < nwaves; r += 4) {
-        if (wave >= r && wave < r + 4)
-            wave_sums<NACC * V>(flat, CG, lane, 0, 0, [&](int k, float v) {
-                red[((wave - r) * NACC + k / V) * cols + (lane & (CG - 1)) * V + k % V] = v;
-            });
-        __syncthreads();
+        for (int m = 0; m < kMine; ++m) run[m] = 0.0;
+        for (int r = 0; r < nwaves; r += 4) {
+            if (wave >= r && wave < r + 4)
+                wave_sums<2 * V>(tot, CG, lane, 0, 0, [&](int k, double v) {
+                    red[((wave - r) * 2 + k / V) * cols + (lane & (CG - 1)) * V + k % V] = v;
+                });
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < kMine; ++m) {
+                const int o = t + m * nthr;
+                if (o < nout) run[m] += ((red[o] + red[nout + o]) + (red[2 * nout + o] + red[3 * nout + o]));
+            }
+            if (r + 4 < nwaves) __syncthreads();
+        }
 #pragma unroll
         for (int m = 0; m < kMine; ++m) {
             const int o = t + m * nthr;
-            if (o < nout) run[m] += (red[o] + red[nout + o]) + (red[2 * nout + o] + red[3 * nout + o]);
+            if (o < nout) {
+                const float high = (float)run[m];
+                // (an infinite sum has no rest)
+                const float low = __builtin_isfinite(high) ? (float)(run[m] - (double)high) : 0.0f;
+                const int64_t at = (int64_t)blockIdx.x * nout + o;
+                if (pairs) reinterpret_cast<fp32_pair_t*>(ws)[at] = fp32_pair_t{high, low};
+                else ws[at] = high;
+            }
         }
-        __syncthreads();
     }
-#pragma unroll
-    for (int m = 0; m < kMine; ++m) {
-        const int o = t + m * nthr;
-        if (o < nout) dst[o] = run[m];
-    }
+};
+
+constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
+// `pairs` of ChannelTotals::write: where the launch shape is the library's own choice and the scratch memory has room for them (a
+// workspace query with blocks = 0 does), unless the tensor is so small that its sums are short.
+static inline bool sum_pairs(int blocks_asked, int blocks, int ncols, int64_t bytes, int64_t workspace_bytes)
+{
+    return blocks_asked <= 0 && workspace_bytes / (int64_t)sizeof(fp32_pair_t) >= (int64_t)blocks * ncols && bytes >= (8 << 20);
 }
 
 // Column sums in fp64 by a workgroup of 1024, in a fixed order: a slice of threads per row, N rows of a slice in flight at
@@ -847,15 +882,19 @@ __device__ __forceinline__ double sum_lines(const float* __restrict__ ws, int nr
     return v;
 }
 
-// 16 columns of any row-major fp32 buffer, column j (below ncols) per lane of 16: returned by the threads below 16
-__device__ __forceinline__ double sum_columns(const float* __restrict__ ws, int nrows, int64_t pitch, int j, int ncols,
+// 16 columns of any row-major buffer, column j (below ncols) per lane of 16: returned by the threads below 16.  T: float or
+// fp32_pair_t.
+__device__ __forceinline__ double wide(float v) { return (double)v; }
+__device__ __forceinline__ double wide(fp32_pair_t v) { return (double)v[0] + (double)v[1]; }
+template <class T>
+__device__ __forceinline__ double sum_columns(const T* __restrict__ ws, int nrows, int64_t pitch, int j, int ncols,
                                               double (&part)[16][17])
 {
     const int t = threadIdx.x;
-    const float* col = ws + (j < ncols ? j : ncols - 1);
+    const T* col = ws + (j < ncols ? j : ncols - 1);
     double s = 0.0;
     auto row = [&](int r) { return col[r * pitch]; };
-    auto add = [&](float v, bool exists) { s += exists ? (double)v : 0.0; };
+    auto add = [&](T v, bool exists) { s += exists ? wide(v) : 0.0; };
     if (nrows <= 256) sum_slices<4>(nrows, t / 16, 64, row, add);
     else sum_slices<8>(nrows, t / 16, 64, row, add);
     s += __shfl_xor(s, 16, 64);
@@ -873,7 +912,7 @@ __device__ __forceinline__ double sum_columns(const float* __restrict__ ws, int 
 // out[j] = scale * sum_r ws[r*ncols + j] for j < ncols, summed in fp64 in a fixed order;
 // columns [0, split) go to out0, the rest to out1.  (Kernel lives in core.hip.)
 void launch_reduce_rows(const float* ws, int nrows, int ncols, float* out0, float* out1, int split, double scale,
-                        hipStream_t stream);
+                        hipStream_t stream, bool pairs = false);
 // the same for a multiple of 32 columns and scale 1, the results in out0 rounded to fp16
 void launch_reduce_rows_f16(const float* ws, int nrows, int ncols, half_t* out0, float* out1, int split,
                             hipStream_t stream);

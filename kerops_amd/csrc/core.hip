@@ -64,7 +64,8 @@ namespace kerops {
 
 // Sums the rows of a partial buffer column by column in a fixed order (fp64, sum_columns) and writes scale * sum to out0
 // (columns below split) or out1.  A workgroup owns 16 columns.
-__global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restrict__ ws, int nrows, int ncols,
+template <class T>
+__global__ __launch_bounds__(1024) void reduce_rows_kernel(const T* __restrict__ ws, int nrows, int ncols,
                                                            float* __restrict__ out0, float* __restrict__ out1,
                                                            int split, double scale)
 {
@@ -97,8 +98,13 @@ __global__ __launch_bounds__(1024) void reduce_lines_kernel(const float* __restr
 }
 
 void launch_reduce_rows(const float* ws, int nrows, int ncols, float* out0, float* out1, int split, double scale,
-                        hipStream_t stream)
+                        hipStream_t stream, bool pairs)
 {
+    if (pairs) {
+        hipLaunchKernelGGL((reduce_rows_kernel<fp32_pair_t>), dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream,
+                           reinterpret_cast<const fp32_pair_t*>(ws), nrows, ncols, out0, out1, split, scale);
+        return;
+    }
     // A line's 32 columns per workgroup pay where the columns fill the chip.  The statistics of up to 512 channels are
     // few columns of up to 4096 rows, which a narrower split spreads over twice the workgroups (256 columns: statistics
     // and pool of (1,128,103,82,48) 105.0 us, 107.0 by lines).
@@ -107,7 +113,7 @@ void launch_reduce_rows(const float* ws, int nrows, int ncols, float* out0, floa
                            out0, out1, split, scale);
         return;
     }
-    hipLaunchKernelGGL(reduce_rows_kernel, dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream, ws, nrows, ncols,
+    hipLaunchKernelGGL((reduce_rows_kernel<float>), dim3(ceil_div(ncols, 16)), dim3(1024), 0, stream, ws, nrows, ncols,
                        out0, out1, split, scale);
 }
 

@@ -7,8 +7,8 @@
 // segment per workgroup and step): a thread moves V = min(8, C) consecutive channels per
 // access (16 bytes for C >= 8), consecutive lanes take consecutive chunks, and every stride
 // of the walk is a multiple of the number of channel groups, so a thread keeps one channel
-// group for its whole life: per-channel parameters sit in registers and per-channel sums
-// are plain per-thread fp32 accumulators.  Reductions finish with wavefront shuffles, one LDS
+// group for its whole life: per-channel parameters and sums (ChannelTotals) sit in registers.
+// Reductions finish with wavefront shuffles, one LDS
 // hop per workgroup, a [workgroups][..] partial buffer and a small fp64 second pass:
 // no float atomics, identical bits on every run.
 #include "common.hpp"
@@ -19,11 +19,12 @@ namespace kerops {
 template <int V, int U, bool ADD>
 __global__ __launch_bounds__(kStreamMaxThreads) void stats_kernel(const half_t* x, const half_t* y, half_t* z,
                                                                   float* __restrict__ ws, int64_t nchunks, int CG,
-                                                                  int segments)
+                                                                  int segments, int pairs)
 {
     typedef typename HVec<V>::type hv;
-    __shared__ float red[4 * 2 * 64 * V];
+    __shared__ double red[4 * 2 * 64 * V];
     const ChunkWalk<U> wk(nchunks, segments != 0);
+    ChannelTotals<V> sums;
     float acc[2][V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[0][j] = acc[1][j] = 0.0f;
@@ -69,9 +70,11 @@ __global__ __launch_bounds__(kStreamMaxThreads) void stats_kernel(const half_t* 
                 acc[1][j] += __builtin_fmaf(f0, f0, f1 * f1) + __builtin_fmaf(f2, f2, f3 * f3);
             }
         }
+        sums.take(acc);
     }
     for (int64_t i = wk.tail; i < nchunks; i += wk.T) body(i);
-    block_channel_partials_any<2, V>(acc, CG, red, ws + (int64_t)blockIdx.x * 2 * CG * V);
+    sums.take(acc);
+    sums.write(CG, red, ws, pairs);
 }
 
 // ---------------------------------------------------------- stats backward
@@ -158,10 +161,10 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const hal
                                                                        const float* __restrict__ bv,
                                                                        const half_t* __restrict__ g,
                                                                        half_t* __restrict__ dx, float* __restrict__ ws,
-                                                                       int64_t nchunks, int CG, int segments)
+                                                                       int64_t nchunks, int CG, int segments, int pairs)
 {
     typedef typename HVec<V>::type hv;
-    __shared__ float red[4 * 2 * 64 * V];
+    __shared__ double red[4 * 2 * 64 * V];
     const ChunkWalk<U> wk(nchunks, segments != 0);
     const int cg = (int)(wk.first % CG);
     float w[V], nb[V];
@@ -170,10 +173,13 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const hal
         w[j] = wv[cg * V + j];
         nb[j] = -bv[cg * V + j];
     }
-    float acc[2][V];  // [0] = dW, [1] = dB
+    ChannelTotals<V> sums;
+    float acc[2][V];  // [0] = dW, [1] = dB, of a step
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[0][j] = acc[1][j] = 0.0f;
-    auto body = [&](int64_t k, const hv& xv, const hv& gv) {
+    // (chunk i from chunk `at` on: in the loop `at` is the workgroup's and i the thread, scalar base addresses and one offset
+    // register for all accesses.  With an address per access and thread the sums had to leave the registers.)
+    auto body = [&](int64_t at, int64_t i, const hv& xv, const hv& gv) {
         hv o;
 #pragma unroll
         for (int j = 0; j < V; ++j) {
@@ -185,21 +191,24 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const hal
             acc[0][j] = __builtin_fmaf(xf, gm, acc[0][j]);
             acc[1][j] += gm;
         }
-        st_stream<V>(dx, k, o);
+        st_stream<V>(dx + at * V, i, o);
     };
+    const uint32_t t = threadIdx.x;
     for (int64_t k = 0; k < wk.nfull; ++k) {
-        const int64_t i = k * wk.step + wk.first;
+        const int64_t at = k * wk.step + (wk.first - t);
         hv xv[U], gv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            xv[u] = ld_stream<V>(x, i + u * wk.su);
-            gv[u] = ld_stream<V>(g, i + u * wk.su);
+            xv[u] = ld_stream<V>(x + (at + u * wk.su) * V, t);
+            gv[u] = ld_stream<V>(g + (at + u * wk.su) * V, t);
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) body(i + u * wk.su, xv[u], gv[u]);
+        for (int u = 0; u < U; ++u) body(at + u * wk.su, t, xv[u], gv[u]);
+        sums.take(acc);
     }
-    for (int64_t i = wk.tail; i < nchunks; i += wk.T) body(i, ld_stream<V>(x, i), ld_stream<V>(g, i));
-    block_channel_partials_any<2, V>(acc, CG, red, ws + (int64_t)blockIdx.x * 2 * CG * V);
+    for (int64_t i = wk.tail; i < nchunks; i += wk.T) body(0, i, ld_stream<V>(x, i), ld_stream<V>(g, i));
+    sums.take(acc);
+    sums.write(CG, red, ws, pairs);
 }
 
 // ------------------------------------------------------------ quantisers
@@ -449,12 +458,13 @@ using namespace kerops;
 // wavefronts win while a tensor is small: a workgroup of sixteen is placed on a compute unit only as a whole and pays
 // its slowest wavefront at either end.  GPU time per launch in a row of launches, inputs from memory, C = 16 and 64 alike:
 //   BN-ReLU            0.5 / 8 / 48 / 192 MiB: (256,16,8) or (1280,16,4) 6.1 / 7.9 / 20.4 / 67.0 us, here 2.8 / 4.9 / 18.7 / 65.3
-//   its backward       8 / 48 / 96 / 384 MiB: (768,4,1) or (1536,16,4) 13.0 / 34.2 / 78.8 / 215, here 12.6 / 31.9 / 55.1 / 196;
-//                      1.9 GiB 1002, 1011 with 256 workgroups
-//   add + statistics   8 / 48 / 96 / 1914 MiB: (1280,4,8) or (1280,16,8) 12.2 / 34.2 / 67.0 / 1048, here 9.2 / 28.6 / 52.3 / 1015;
+//   its backward       8 / 48 / 96 / 384 MiB: (768,4,1) or (1536,16,4) 14.1 / 34.5 / 78.1 / 215, here 11.2 / 31.3 / 55.4 / 203; one
+//                      shape for all sizes, at 1.9 GiB within 2 % of the best.  (256,4,1), the best before the sums were taken in
+//                      fp64, leaves a wavefront per SIMD, whose additions then hide behind nothing: 120 M elements 134, here 121
+//   add + statistics   8 / 48 / 96 / 1914 MiB: (1280,4,8) or (1280,16,8) 14.2 / 34.0 / 72.8 / 1061, here 10.5 / 30.0 / 53.6 / 1050;
 //                      (256,4,1) / (512,4,4) at 12 / 24 / 64 / 160 MiB: 12.1 / 17.9 / 35.7 / 83.4 and 11.4 / 17.4 / 36.9 / 86.1
 //   its backward       2 / 24 / 64 MiB: (1536,16,1) or (512,4,4) 8.1 / 17.9 / 37.4, here 5.2 / 15.3 / 36.3
-//   statistics         2 / 64 / 100 MiB: 5.9 / 15.4 / 21.3 (what lies between these shapes is less than the noise)
+//   statistics         2 / 64 / 100 MiB: 7.8 / 18.1 / 22.9 (what lies between these shapes is less than the noise)
 //   window quantiser   2 / 24 / 64 / 128 MiB in: (512,16,8) or (256,4,8) 6.6 / 9.3 / 21.2 / 36.7, here 3.4 / 8.8 / 19.1 / 36.7
 //   its inverse        2 / 24 / 48 MiB out: (1536,16,8) 5.1 / 10.1 / 18.1, here 3.1 / 8.7 / 15.9
 //   int8 quantiser     16 / 48 / 96 MiB in: (256,4,4) or (4096,16,4) 10.2 / 26.8 / 29.0, here 7.2 / 15.6 / 27.9
@@ -476,7 +486,7 @@ constexpr SizedDefault kDefAddStats[] = {{40 * kMiB, {512, 4, 4}}, {kAnySize, {2
 constexpr SizedDefault kDefStatsBwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {4096, 16, 4}}};
 constexpr SizedDefault kDefAddStatsBwd[] = {{112 * kMiB, {1024, 4, 4}}, {kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefBnReluFwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {1280, 16, 4}}};
-constexpr SizedDefault kDefBnReluBwd[] = {{40 * kMiB, {512, 4, 4}}, {1536 * kMiB, {256, 4, 1}}, {kAnySize, {1536, 16, 4}}};
+constexpr SizedDefault kDefBnReluBwd[] = {{kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefQuantU8[] = {{56 * kMiB, {1536, 4, 4}}, {112 * kMiB, {1536, 4, 8}}, {kAnySize, {256, 4, 8}}};
 constexpr SizedDefault kDefDequantU8[] = {{3 * kMiB, {1024, 4, 1}}, {56 * kMiB, {2048, 4, 8}}, {kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefQuantI8[] = {{160 * kMiB, {2048, 4, 4}}, {256 * kMiB, {1536, 16, 4}}, {kAnySize, {4096, 16, 4}}};
@@ -491,7 +501,6 @@ const StreamDefault& default_shape(const SizedDefault (&table)[N], int64_t bytes
     return table[i].shape;
 }
 constexpr int kMaxStreamBlocks = 65536;
-constexpr int kMaxDefaultBlocks = 4096;  // workspace queries with blocks = 0 size for this many partials
 
 int resolve_shape(const char* op, const StreamDefault& def, int64_t work_items, bool wide8, int blocks, int waves,
                   int segment, StreamShape* out)
@@ -597,18 +606,19 @@ static int stats_common(const char* op, const StreamDefault& def, const void* x,
     hipStream_t s = (hipStream_t)stream;
     float* ws = (float*)workspace;
     const int seg = sh.segment != 1;
+    const bool pairs = sum_pairs(blocks, sh.blocks, 2 * C, channel_bytes(M, C), workspace_bytes);
     KEROPS_DISPATCH_VU(C, sh, {
         if (add) {
             hipLaunchKernelGGL((stats_kernel<V, U, true>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x,
-                               (const half_t*)y, (half_t*)z, ws, nchunks, CG, seg);
+                               (const half_t*)y, (half_t*)z, ws, nchunks, CG, seg, pairs);
         } else {
             hipLaunchKernelGGL((stats_kernel<V, U, false>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x,
-                               (const half_t*)nullptr, (half_t*)nullptr, ws, nchunks, CG, seg);
+                               (const half_t*)nullptr, (half_t*)nullptr, ws, nchunks, CG, seg, pairs);
         }
     });
     rc = check_launch(op);
     if (rc != KEROPS_OK) return rc;
-    launch_reduce_rows(ws, sh.blocks, 2 * C, mean, sqmean, C, 1.0 / (double)M, s);
+    launch_reduce_rows(ws, sh.blocks, 2 * C, mean, sqmean, C, 1.0 / (double)M, s, pairs);
     return check_launch(op);
 }
 
@@ -729,13 +739,14 @@ extern "C" int kerops_bnrelu_bwd_f16(const void* x, const float* wv, const float
     hipStream_t s = (hipStream_t)stream;
     float* ws = (float*)workspace;
     const int seg = sh.segment != 1;
+    const bool pairs = sum_pairs(blocks, sh.blocks, 2 * C, channel_bytes(M, C), workspace_bytes);
     KEROPS_DISPATCH_VU(C, sh, {
         hipLaunchKernelGGL((bnrelu_bwd_kernel<V, U>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x, wv,
-                           bv, (const half_t*)g, (half_t*)dx, ws, M * CG, CG, seg);
+                           bv, (const half_t*)g, (half_t*)dx, ws, M * CG, CG, seg, pairs);
     });
     rc = check_launch("bnrelu_bwd");
     if (rc != KEROPS_OK) return rc;
-    launch_reduce_rows(ws, sh.blocks, 2 * C, dW, dB, C, 1.0, s);
+    launch_reduce_rows(ws, sh.blocks, 2 * C, dW, dB, C, 1.0, s, pairs);
     return check_launch("bnrelu_bwd");
 }
 

@@ -15,6 +15,7 @@ from kerops_amd.ops.linear import (ApplyBNReLULinearAdd, ApplyBNReLULinearBackwa
                                    LinBReLULinBackward, ReLULinearAdd, ReLULinearBackward)
 from kerops_amd.ops.quantization import DequantUint8Window, QuantInt8Sym, QuantUint8Window
 from kerops_amd.ops.stats import Stats, StatsBackward
+from kerops_amd.settings import stream_table
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
@@ -376,6 +377,73 @@ def test_depthwise_marches_of_any_length(c, w, d, h_chunk):
     assert torch.equal(bits(dx), bits(dx_ref))
     # fp32 sums of a few thousand products in another order
     assert ((gw - gw_ref).norm() / gw_ref.norm()).item() < 1e-5
+
+
+def channel_sums(*terms):
+    """Sums over the voxels in 64 bits, a part of the tensors at a time; terms: (function, tensors ...)."""
+    out = []
+    for f, *ts in terms:
+        parts = zip(*(t.permute(0, 2, 3, 4, 1).reshape(-1, t.shape[1]).split(1 << 18) for t in ts))
+        out.append(sum(f(*(p.double() for p in part)).sum(0) for part in parts))
+    return out
+
+
+# Zero-mean values, whose sums are small against their terms: the error of a channel sum against 64 bits, over the size of the
+# sums.  Rounding a sum to fp32 is at most 2^-25 to 2^-24 of it, evenly spread: 2^-24 / sqrt(3) = 3.4e-8 in the mean square.
+# Sums of fp16 values (mean, dshift) have no other error: the few of a step of the walk are nearly exact.  Products
+# (dscale) are rounded as a step adds them, four in a row: sqrt(1 + (1 + 2 + 3 + 4) / 4) times as much, 6.4e-8.  10 % for
+# the spread of 64 to 128 channels.
+@pytest.mark.parametrize('c,shape', [(64, (1, 86, 86, 88)), (128, (1, 136, 136, 128)), (8, (1, 123, 125, 123))])
+def test_channel_sums_of_the_built_in_shapes_have_no_chains(c, shape):
+    gen = torch.Generator(DEV).manual_seed(c)
+    n, h, w, d = shape
+    x, y = (torch.randn(n, h, w, d, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3) for _ in range(2))
+    scale, shift = torch.rand(c, device=DEV, generator=gen) + 0.5, torch.randn(c, device=DEV, generator=gen) * 0.1
+    one, ten_percent = 2.0 ** -24 / 3 ** 0.5, 1.1
+
+    def check(got, total, bound):
+        assert ((got.double() - total).norm() / total.norm()).item() < bound * one * ten_percent
+
+    v = x.numel() // c
+    z, mean, _ = AddStats(x, y)
+    check(mean, channel_sums((lambda t: t, z))[0] / v, 1.0)
+    del z
+    dx, dscale, dshift = ApplyBNReLUBackward(x, scale, shift, y)
+    on = (dx != 0) | (y == 0)  # (scale > 0: the gradient is zero where the ReLU is, or y itself)
+    for got, total, bound in zip((dscale, dshift), channel_sums((lambda t, g, m: t * g * m, x, y, on), (lambda g, m: g * m, y, on)),
+                                 ((1 + 10 / 4) ** 0.5, 1.0)):
+        check(got, total, bound)
+    # (Stats and the pooling have shapes in the table for the largest tensors, whose workgroups hand over fp32 sums)
+    if x.numel() * 2 >= stream_table.SMALL_BYTES:
+        return
+    check(Stats(x)[0], channel_sums((lambda t: t, x))[0] / v, 1.0)
+    pmean = AvgPoolCeilStats(x)[1]
+    # (all windows of a voxel's sample have 8, 4, 2 or 1 voxels: a voxel counts with one over that number)
+    weight = torch.ones(h, w, d, device=DEV, dtype=torch.float64)
+    for axis, e in enumerate((h, w, d)):
+        edge = torch.full((e,), 0.5, device=DEV, dtype=torch.float64)
+        if e % 2:
+            edge[-1] = 1.0
+        weight *= edge.view([-1 if a == axis else 1 for a in range(3)])
+    weight = weight.expand(1, 1, h, w, d)
+    windows = n * -(-h // 2) * -(-w // 2) * -(-d // 2)
+    check(pmean, channel_sums((lambda t, k: t * k, x, weight))[0] / windows, 1.0)
+
+
+def test_channel_sums_that_are_not_finite():
+    c, v = 64, 80000  # (9.8 MiB: rows of pairs)
+    gen = torch.Generator(DEV).manual_seed(3)
+    x = torch.randn(1, v, 1, 1, c, device=DEV, generator=gen).half().permute(0, 4, 1, 2, 3)
+    x[0, 1, 5], x[0, 2, 7], x[0, 3, 9], x[0, 3, 11] = float('inf'), float('nan'), float('-inf'), float('-inf')
+    inf, nan = float('inf'), float('nan')
+    one, zero = torch.ones(c, device=DEV), torch.zeros(c, device=DEV)
+    for mean, sqmean in (Stats(x), AddStats(x, torch.zeros_like(x))[1:], AvgPoolCeilStats(x)[1:]):
+        assert mean[1] == inf and sqmean[1] == inf and mean[3] == -inf and sqmean[3] == inf
+        assert mean[2].isnan() and sqmean[2].isnan()
+        assert mean[4:].isfinite().all() and sqmean[4:].isfinite().all() and mean[0].isfinite()
+    _, dscale, dshift = ApplyBNReLUBackward(torch.ones_like(x), one, zero, x)
+    for got in (dscale, dshift):
+        assert torch.equal(got[1:4].nan_to_num(7.0), torch.tensor([inf, nan, -inf], device=DEV).nan_to_num(7.0)) and got[4:].isfinite().all()
 
 
 # planes of just under 2^31 elements (the largest accepted): the byte offsets of the buffer accesses go up to 2^32 - 16
