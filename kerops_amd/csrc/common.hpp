@@ -762,6 +762,15 @@ __device__ __forceinline__ void wave_sums(T (&v)[N], int CG, int lane, int base,
 
 typedef float fp32_pair_t __attribute__((ext_vector_type(2)));  // a sum rounded to fp32 and what the rounding left
 
+// element `i` of a workspace of fp32 sums or, `pairs`, of fp32_pair_t
+__device__ __forceinline__ void store_sum(float* ws, int64_t i, double sum, bool pairs)
+{
+    const float high = (float)sum;
+    // (an infinite sum has no rest)
+    if (pairs) reinterpret_cast<fp32_pair_t*>(ws)[i] = fp32_pair_t{high, __builtin_isfinite(high) ? (float)(sum - (double)high) : 0.0f};
+    else ws[i] = high;
+}
+
 // Per-channel sums of a thread, then of its workgroup, in fp64.  A kernel adds the values of one step of its walk in fp32.  How
 // many steps a thread takes, and how many workgroups there are, goes with the launch shape, which is chosen for its speed:
 // with fp32 sums from step to step, over the lanes and in a workgroup's row, the error against 64 bits went with it.
@@ -813,14 +822,7 @@ struct ChannelTotals {
 #pragma unroll
         for (int m = 0; m < kMine; ++m) {
             const int o = t + m * nthr;
-            if (o < nout) {
-                const float high = (float)run[m];
-                // (an infinite sum has no rest)
-                const float low = __builtin_isfinite(high) ? (float)(run[m] - (double)high) : 0.0f;
-                const int64_t at = (int64_t)blockIdx.x * nout + o;
-                if (pairs) reinterpret_cast<fp32_pair_t*>(ws)[at] = fp32_pair_t{high, low};
-                else ws[at] = high;
-            }
+            if (o < nout) store_sum(ws, (int64_t)blockIdx.x * nout + o, run[m], pairs);
         }
     }
 };

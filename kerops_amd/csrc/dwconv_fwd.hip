@@ -57,6 +57,7 @@ struct FwdArgs {
     half_t* y2;         // [N][H][W][D][cout]
     float* amax_ws;     // one max|y2| per workgroup
     float* stats_ws;    // mode 3: per workgroup [2][slab channels] sums of y and y*y (y as stored, fp16)
+    bool stats_pairs;   // ... as fp32_pair_t
     int H, W, D, C;
     int n_wt, n_dt, n_hc, n_slab, h_chunk;
     uint32_t nblocks;
@@ -915,16 +916,19 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NT >= 512 ? 4 : 3) void dwconv_fwd_mf
         const int b = lane / 4, rr = lane % 4;
         const int q = b % NQ, sub = b / NQ;
         // lanes of a wavefront that share the channel pair differ in rr (lane bits 0-1) and sub (the bits above q)
-        float v4[4] = {ssum[0], ssum[1], ssq[0], ssq[1]};
+        const float v1[4] = {ssum[0], ssum[1], ssq[0], ssq[1]};
+        double v4[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            v4[i] += __shfl_xor(v4[i], 1);
-            v4[i] += __shfl_xor(v4[i], 2);
+            float v = v1[i] + __shfl_xor(v1[i], 1);
+            v += __shfl_xor(v, 2);
+            v4[i] = (double)v;
 #pragma unroll
             for (int m = 4 * NQ; m < kWave; m <<= 1) v4[i] += __shfl_xor(v4[i], m);
         }
         __syncthreads();  // the staging buffers are free now
-        float* sred = reinterpret_cast<float*>(smem);  // [wavefront][2 NQ channels][sum, sum of squares]
+        double* sred = reinterpret_cast<double*>(smem);  // [wavefront][2 NQ channels][sum, sum of squares]
+        static_assert(Cfg::NWAVE * 2 * NQ * 2 * 8 <= SMEM_BYTES, "the sums fit the staging buffers");
         if (rr == 0 && sub == 0) {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
@@ -936,10 +940,10 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NT >= 512 ? 4 : 3) void dwconv_fwd_mf
         if (t < 2 * SC) {  // wavefronts that share a half of the slab, in a fixed order
             const int st = t / SC, ch = t % SC;
             const int hf = ch / (2 * NQ), cl = ch % (2 * NQ);
-            float acc = 0.0f;
+            double acc = 0.0;
 #pragma unroll
             for (int pp = 0; pp < Cfg::NPART; ++pp) acc += sred[((pp * Cfg::NHALF + hf) * 2 * NQ + cl) * 2 + st];
-            a.stats_ws[(int64_t)ws_row * 2 * SC + st * SC + ch] = acc;
+            store_sum(a.stats_ws, (int64_t)ws_row * 2 * SC + t, acc, a.stats_pairs);
         }
     }
 }
@@ -1019,7 +1023,8 @@ static int launch_fwd_mfma(const FwdArgs& base, int N, int h_chunk, hipStream_t 
 
 // Adds the per-workgroup sums in a fixed order (fp64, sum_columns) and divides by the number of voxels: one workgroup per
 // slab and 16 of its 2 SC columns (SC sums, SC sums of squares); row r of the workspace belongs to slab r % n_slab.
-__global__ __launch_bounds__(1024) void dwconv_stats_reduce_kernel(const float* __restrict__ ws, uint32_t nblocks,
+template <class T>
+__global__ __launch_bounds__(1024) void dwconv_stats_reduce_kernel(const T* __restrict__ ws, uint32_t nblocks,
                                                                    int n_slab, int SC, double inv_count,
                                                                    float* __restrict__ mean, float* __restrict__ sqmean)
 {
@@ -1233,6 +1238,16 @@ static int dwconv_stats_check(int32_t N, int32_t H, int32_t W, int32_t D, int32_
     return KEROPS_OK;
 }
 
+// Half a round of long marches (the split takes it where it is the faster one) has half the workgroups, with sums of twice the
+// length: they hand over what the rounding to fp32 leaves as well, in as many rows as a full round has (relative error of the
+// mean against 64 bits, zero-mean values, (1,32,54,54,56) / (1,128,34,34,36): 53e-9 / 41e-9 with fp32 sums of half a round,
+// 36e-9 / 33e-9 of a full one, 24e-9 / 29e-9 so, at 0.2 us of 13).
+static bool dwconv_stats_pairs(const FwdArgs& a)
+{
+    const uint32_t cus = (uint32_t)device_geometry().cus;
+    return a.nblocks > cus / 2 && a.nblocks <= cus;
+}
+
 extern "C" int64_t kerops_dwconv_stats_workspace_bytes(int32_t N, int32_t H, int32_t W, int32_t D, int32_t C)
 {
     int rc = dwconv_stats_check(N, H, W, D, C);
@@ -1246,7 +1261,7 @@ extern "C" int64_t kerops_dwconv_stats_workspace_bytes(int32_t N, int32_t H, int
         return plan_fwd_mfma<cg(), tw(), td(), nt()>(a, N, 0, true, true);
     });
     if (rc != KEROPS_OK) return rc;
-    return (int64_t)a.nblocks * 2 * std::min(C, 64) * (int64_t)sizeof(float);
+    return (int64_t)a.nblocks * 2 * std::min(C, 64) * (int64_t)(dwconv_stats_pairs(a) ? sizeof(fp32_pair_t) : sizeof(float));
 }
 
 extern "C" int kerops_dwconv_stats_f16(const void* x, const void* wt, void* y, float* mean, float* sqmean,
@@ -1279,6 +1294,7 @@ extern "C" int kerops_dwconv_stats_f16(const void* x, const void* wt, void* y, f
         using Cfg = FmCfg<cg(), tw(), td(), nt()>;
         int r = plan_fwd_mfma<cg(), tw(), td(), nt()>(a, N, 0, true, true);
         if (r != KEROPS_OK) return r;
+        a.stats_pairs = dwconv_stats_pairs(a);
         if (a.stream_interior)
             hipLaunchKernelGGL((dwconv_fwd_mfma_kernel<Cfg, 3, 0, true>), dim3(xcd_padded_grid(a.nblocks, a.n_xcd)), dim3(Cfg::NT), 0,
                                s, a);
@@ -1288,8 +1304,13 @@ extern "C" int kerops_dwconv_stats_f16(const void* x, const void* wt, void* y, f
     });
     if (rc != KEROPS_OK) return rc;
     const double inv_count = 1.0 / ((double)N * H * W * D);
-    hipLaunchKernelGGL(dwconv_stats_reduce_kernel, dim3(a.n_slab * ceil_div(2 * std::min(C, 64), 16)), dim3(1024), 0, s, (const float*)workspace, a.nblocks,
-                       a.n_slab, std::min(C, 64), inv_count, mean, sqmean);
+    const dim3 grid(a.n_slab * ceil_div(2 * std::min(C, 64), 16));
+    if (a.stats_pairs)
+        hipLaunchKernelGGL((dwconv_stats_reduce_kernel<fp32_pair_t>), grid, dim3(1024), 0, s, (const fp32_pair_t*)workspace, a.nblocks,
+                           a.n_slab, std::min(C, 64), inv_count, mean, sqmean);
+    else
+        hipLaunchKernelGGL((dwconv_stats_reduce_kernel<float>), grid, dim3(1024), 0, s, (const float*)workspace, a.nblocks, a.n_slab,
+                           std::min(C, 64), inv_count, mean, sqmean);
     return check_launch("dwconv_stats_reduce");
 }
 

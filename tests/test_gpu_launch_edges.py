@@ -430,6 +430,21 @@ def test_channel_sums_of_the_built_in_shapes_have_no_chains(c, shape):
     check(pmean, channel_sums((lambda t, k: t * k, x, weight))[0] / windows, 1.0)
 
 
+# the same for the convolution with statistics where half a round of workgroups marches over twice the rows (and, the last, where
+# a full round does).  A lane's sums over a march are fp32 here: 20 % for them and the spread
+@pytest.mark.parametrize('c,shape', [(16, (1, 58, 58, 60)), (32, (1, 54, 54, 56)), (64, (1, 44, 42, 44)), (128, (1, 34, 34, 36)), (64, (1, 18, 16, 20))])
+def test_sums_of_the_convolution_with_statistics(c, shape):
+    one, errors = 2.0 ** -24 / 3 ** 0.5, []
+    for seed in range(8):
+        gen = torch.Generator(DEV).manual_seed(seed)
+        x = torch.randn(*shape, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3)
+        y, mean, sqmean = DWConvStats(x, (torch.randn(3, 3, 3, c, device=DEV, generator=gen) / 27 ** 0.5).half())
+        total, squares = (t * c / x.numel() for t in channel_sums((lambda t: t, y), (lambda t: t * t, y)))
+        errors.append(((mean.double() - total).norm() / total.norm()).square().item())
+        assert ((sqmean.double() - squares).norm() / squares.norm()).item() < 1e-6
+    assert (sum(errors) / len(errors)) ** 0.5 < 1.2 * one
+
+
 def test_channel_sums_that_are_not_finite():
     c, v = 64, 80000  # (9.8 MiB: rows of pairs)
     gen = torch.Generator(DEV).manual_seed(3)
