@@ -114,6 +114,8 @@ __device__ __forceinline__ void wait_loads_in_flight()
 {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// until every vector memory access of the wavefront has completed (the compiler's own accesses; it sees this wait)
+__device__ __forceinline__ void wait_all_accesses() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 __device__ __forceinline__ const char* uniform_ptr(const char* p)
 {
     const uint64_t v = reinterpret_cast<uint64_t>(p);

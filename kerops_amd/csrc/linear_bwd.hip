@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
                                                                         const half_t* __restrict__ Wm,
                                                                         half_t* __restrict__ dx, float* __restrict__ ws,
                                                                         int64_t V, const float* __restrict__ scale,
-                                                                        const float* __restrict__ shift)
+                                                                        const float* __restrict__ shift, int drain)
 {
     constexpr int CGI = CIN / 8, ROW = CIN * COUT + (AFFINE ? 2 * CIN : 0);  // ROW: floats of a row of the workspace
     using Cfg = LbCfg<CIN, COUT, AFFINE>;
@@ -229,6 +229,7 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
     for (; tile < ntiles; tile += gridDim.x) {
         const int64_t v0 = tile * Cfg::TILE;
         half8_t xraw[AFFINE ? NLX : 1];
+        if (!AFFINE && drain) wait_all_accesses();  // (uniform)
         // ---- stage the tile (rows past V are zero: they add nothing to dW) ----
 #pragma unroll
         for (int j = 0; j < NLX; ++j) {
@@ -413,7 +414,8 @@ __global__ __launch_bounds__(kLbThreads, 2) void relu_linear_bwd_kernel(const ha
 // 16 -> 16 has the fewest bytes in flight and the shortest rows of sums and takes four.  In volumes of half a million
 // voxels and more, where the rows of sums are few against the tiles, three pay at 32 -> 32 (0.2 M voxels 13.7 us with
 // two, 14.5 with three; 0.9 M 36.9 and 34.8; 15.7 M 523 and 492) and 16 -> 128 (0.2 M 19.1 and 19.7; 0.9 M 57.6 and
-// 55.4; 4 M 231 and 219), and 16 -> 16 has one more than it needs (4 M: 68.9 with four, 66.2 with three).
+// 55.4; with stores left in flight 4 M 217 and 224, but the sums of two are longer by half, which costs bits), and 16 -> 16
+// has one more than it needs (4 M: 68.9 with four, 66.2 with three).
 static int lb_blocks(int64_t V, int cin, int cout, bool affine)
 {
     const bool narrow = cin == 16 && cout == 16 && !affine;
@@ -423,18 +425,34 @@ static int lb_blocks(int64_t V, int cin, int cout, bool affine)
     return (int)std::max<int64_t>(1, std::min<int64_t>(ntiles, per_cu * device_geometry().cus));
 }
 
+// Voxels from which a wavefront of the plain kernel waits for its stores before it goes on.  Large volumes run at the memory's rate,
+// and then some pairs are the fastest where a workgroup reads and writes in turns, as it did with a condition around every
+// store (us without / with the wait: 16 -> 16 at 4 M voxels 66.4 / 66.0, 30 M 501 / 474; 16 -> 32 at 16 M 332 / 326; 16 -> 64 at 4 M
+// 135 / 130, 16 M 538 / 514; 32 -> 16 at 16 M 454 / 449; 32 -> 32 at 4 M 129 / 125, 16 M 526 / 490; 32 -> 64 at 16 M 677 / 666;
+// 32 -> 128 at 4 M 268 / 257; 64 -> 32 at 4 M 214 / 213, 16 M 898 / 878; 64 -> 128 at 4 M 356 / 342), others are not (16 -> 32
+// at 4 M 84.8 / 87.1, 16 -> 128 at 4 M 224 / 227, 64 -> 64 at 16 M 1083 / 1089, 128 -> 64 at 8 M 911 / 954).
+static constexpr int64_t lb_drain_from(int cin, int cout)
+{
+    constexpr int64_t kVoxels = 1000;
+    if (cin == 128 || (cin == 64 && cout < 128 && cout != 32) || (cin == 16 && cout == 128)) return INT64_MAX;
+    if (cout == 2 * cin && cin <= 32) return 12000 * kVoxels;
+    if (cin == 32 && cout == 16) return 6000 * kVoxels;
+    if ((cin == 16 && cout == 16) || (cin == 64 && cout == 32)) return 3000 * kVoxels;
+    return cout == 128 ? 700 * kVoxels : 2000 * kVoxels;  // 32 -> 128, 64 -> 128; 16 -> 64, 32 -> 32
+}
+
 // daffine: the AFFINE kernel's [2][CIN] sums, null without scale and shift
 template <int CIN, int COUT>
 static int launch_lb(const half_t* x, const float* scale, const float* shift, const half_t* g, const half_t* Wm,
                      half_t* dx, void* dW, int dw_dtype, float* daffine, float* ws, int64_t V, hipStream_t s)
 {
-    const int blocks = lb_blocks(V, CIN, COUT, scale != nullptr);
+    const int blocks = lb_blocks(V, CIN, COUT, scale != nullptr), drain = V >= lb_drain_from(CIN, COUT);
     if (scale)
         hipLaunchKernelGGL((relu_linear_bwd_kernel<CIN, COUT, true>), dim3(blocks), dim3(kLbThreads), 0, s, x, g, Wm, dx,
-                           ws, V, scale, shift);
+                           ws, V, scale, shift, drain);
     else
         hipLaunchKernelGGL((relu_linear_bwd_kernel<CIN, COUT, false>), dim3(blocks), dim3(kLbThreads), 0, s, x, g, Wm,
-                           dx, ws, V, scale, shift);
+                           dx, ws, V, scale, shift, drain);
     int rc = check_launch("relu_linear_bwd");
     if (rc != KEROPS_OK) return rc;
     const int ncols = CIN * COUT + (scale ? 2 * CIN : 0);

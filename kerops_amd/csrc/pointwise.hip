@@ -35,14 +35,41 @@ struct PwCfg {
     // Workgroups per compute unit of the persistent loop: as few as keep the memory pipe full, which also have the fewest
     // prologues.  With a residual two, at 16 -> 16, whose tiles have the fewest bytes, three (us with 2 / 3 / 4: 16 -> 16 at
     // 0.9 M voxels 16.3 / 15.7 / 15.8, 32 -> 32 at 0.9 M 29.7 / 31.4 / 31.4 and at 4 M 126 / 136 / 139, 64 -> 32 at 2 M
-    // 84.8 / 91.3 / 89.9, 64 -> 128 at 0.9 M 99.0 / 100.2 / 99.3, 16 -> 64 at 4 M 197 / 198 / 200).
+    // 84.8 / 91.3 / 89.9, 64 -> 128 at 0.9 M 99.0 / 100.2 / 99.3).
+    // Large volumes run at the memory's rate whatever the number, and then the order of reads and writes counts: some pairs
+    // are the fastest with another number, or where a wavefront waits for its stores before it goes on (`drain`), reading and
+    // writing in turns as with a condition around every store.  us with the choice above / this one:
+    //   16 -> 16 at 16 M 261 / 250, 30 M 505 / 480; 16 -> 32 at 30 M 938 / 900; 16 -> 64 at 8 M 409 / 407, 16 M 883 / 843;
+    //   32 -> 64 at 8 M 472 / 467, 16 M 924 / 916; 32 -> 16 at 2 M 44.2 / 43.1, 16 M 365 / 349; 64 -> 32 with the batch-norm map at
+    //   4 M 173 / 172, 16 M 741 / 726; 64 -> 64 at 4 M 261 / 257, 8 M 543 / 523; 128 -> 16 at 2 M 123 / 122, 8 M 491 / 487;
+    //   128 -> 32 at 2 M 136 / 134, 8 M 573 / 563
+    struct Large {
+        int64_t from;  // voxels
+        int per_cu;
+        bool drain;
+    };
+    static constexpr int64_t kVoxels = 1000;
+    static constexpr Large large()
+    {
+        if (CIN == 16 && COUT == 16) return {6000 * kVoxels, 2, false};
+        if (CIN == 16 && COUT == 32) return {12000 * kVoxels, 3, true};
+        if (CIN == 16 && COUT == 64) return {3000 * kVoxels, 3, false};
+        if (CIN == 32 && COUT == 64) return {6000 * kVoxels, 3, false};
+        if (CIN == 32 && COUT == 16) return {700 * kVoxels, 3, true};
+        if (CIN == 64 && COUT == 32) return {3000 * kVoxels, 2, true};
+        if (CIN == 64 && COUT == 64) return {3000 * kVoxels, 3, false};
+        if (CIN == 128 && COUT == 16) return {1500 * kVoxels, 2, true};
+        if (CIN == 128 && COUT == 32) return {700 * kVoxels, 3, false};
+        return {INT64_MAX, 0, false};
+    }
+    static bool drains(int64_t V, bool add) { return add && large().drain && V >= large().from; }
     // Without a residual a tile has half the bytes: four, where their LDS fits (64 -> 128, 0.1 M voxels 16.1 with four,
     // 13.2 with the three that fit, 4 M 284 and 285; 128 -> 128 24.3 with four, 18.6 with the two that fit, 4 M 387 and 391).
     static constexpr int LDS_BYTES = kPwWaves * TILE_HALVES * 2 + MT * KS * 64 * 16 + 2 * CIN * 4 + 64;
     static constexpr int FITS = 160 * 1024 / LDS_BYTES;
     static int64_t workgroups(int64_t V, bool add)
     {
-        const int per_cu = add ? (CIN + COUT == 32 ? 3 : 2) : (FITS < 4 ? FITS : 4);
+        const int per_cu = !add ? (FITS < 4 ? FITS : 4) : V >= large().from ? large().per_cu : CIN + COUT == 32 ? 3 : 2;
         return std::max<int64_t>(1, std::min<int64_t>(ceil_div64(V, 32 * kPwWaves), (int64_t)per_cu * device_geometry().cus));
     }
 };
@@ -54,8 +81,8 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
                                                                const half_t* __restrict__ Wm,
                                                                const half_t* __restrict__ add,
                                                                half_t* __restrict__ out, float* __restrict__ amax_ws,
-                                                               int64_t V, const float* __restrict__ scale = nullptr,
-                                                               const float* __restrict__ shift = nullptr)
+                                                               int64_t V, const float* __restrict__ scale,
+                                                               const float* __restrict__ shift, int drain)
 {
     using Cfg = PwCfg<CIN, COUT>;
     constexpr int MT = Cfg::MT, KS = Cfg::KS;
@@ -142,6 +169,7 @@ __global__ __launch_bounds__(kPwThreads) void pointwise_kernel(const half_t* __r
     for (int64_t r = 0; r < nrounds; ++r) {
         const int64_t tidx = (r * gridDim.x + blockIdx.x) * kPwWaves + wave;
         const int64_t v0 = tidx * 32;
+        if (HAS_ADD && drain) wait_all_accesses();  // (uniform)
         if constexpr (!HAS_ADD) load_x(tidx + tiles_per_round, xn);
         {
             if constexpr (AFFINE) {
@@ -262,19 +290,20 @@ static int launch_pw(const half_t* x, const half_t* Wm, const half_t* add, half_
         return KEROPS_E_BADARG;
     }
     const int blocks = absmax ? pointwise_blocks(V) : (int)PwCfg<CIN, COUT>::workgroups(V, add != nullptr);
+    const int drain = PwCfg<CIN, COUT>::drains(V, add != nullptr);
     if (scale) {  // the affine map ends in a ReLU of its own
         if (add) {
             hipLaunchKernelGGL((pointwise_kernel<CIN, COUT, false, true, false, true>), dim3(blocks), dim3(kPwThreads), 0,
-                               s, x, Wm, add, out, amax_ws, V, scale, shift);
+                               s, x, Wm, add, out, amax_ws, V, scale, shift, drain);
         } else {
             hipLaunchKernelGGL((pointwise_kernel<CIN, COUT, false, false, false, true>), dim3(blocks), dim3(kPwThreads),
-                               0, s, x, Wm, add, out, amax_ws, V, scale, shift);
+                               0, s, x, Wm, add, out, amax_ws, V, scale, shift, drain);
         }
         return check_launch("bnrelu_pointwise");
     }
 #define KEROPS_PW_GO(R, A, M)                                                                                    \
     hipLaunchKernelGGL((pointwise_kernel<CIN, COUT, R, A, M>), dim3(blocks), dim3(kPwThreads), 0, s, x, Wm, add, \
-                       out, amax_ws, V, nullptr, nullptr)
+                       out, amax_ws, V, nullptr, nullptr, drain)
     if (absmax) {
         if (relu_in) KEROPS_PW_GO(true, false, true);
         else KEROPS_PW_GO(false, false, true);

@@ -296,6 +296,27 @@ def test_inverted_bottleneck_either_side_of_a_volume_line(c, line):
     assert (out[:, :, tail].cpu().float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
 
 
+# either side of the volumes at which the pointwise ops change their number of workgroups, or wait for their stores
+@pytest.mark.parametrize('cin,cout,line', [(16, 16, 6000000), (16, 32, 12000000), (16, 64, 3000000), (32, 64, 6000000), (32, 16, 700000), (64, 32, 3000000),
+                                           (64, 64, 3000000), (128, 16, 1500000), (128, 32, 700000), (32, 32, 2000000), (32, 128, 700000)])
+def test_pointwise_ops_either_side_of_a_volume_line(cin, cout, line):
+    gen = torch.Generator(DEV).manual_seed(cin + cout)
+    x, add = (torch.randn(1, line, 1, 1, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3) for c in (cin, cout))
+    mix = (torch.randn(cin, cout, device=DEV, generator=gen) / cin ** 0.5).half()
+    scale, shift = torch.rand(cin, device=DEV, generator=gen) + 0.5, torch.randn(cin, device=DEV, generator=gen)
+    part = slice(0, line - 1)
+    low_x, low_add = x[:, :, part], add[:, :, part]
+    # every voxel's result is its own
+    for whole, below in ((ReLULinearAdd(x, mix, add), ReLULinearAdd(low_x, mix, low_add)),
+                         (ApplyBNReLULinearAdd(x, scale, shift, mix, add), ApplyBNReLULinearAdd(low_x, scale, shift, mix, low_add)),
+                         (ReLULinearBackward(x, add, mix)[0], ReLULinearBackward(low_x, low_add, mix)[0])):
+        assert torch.equal(whole[:, :, part], below)
+    tail = slice(line - 2000, line)
+    ref = oracle.pointwise(x[:, :, tail].cpu(), mix.cpu(), add=add[:, :, tail].cpu(), relu_in=True)
+    got = ReLULinearAdd(x, mix, add)[:, :, tail].cpu()
+    assert (got.float() - ref.float()).abs().max() <= 2.0 ** -8 * max(1.0, ref.abs().max().item())
+
+
 # the pooling backward in output order (8, 16 and, from 24 MiB on, 32 channels): single rows and voxels, runs of a wavefront
 # that end inside a row, many rounds of one workgroup, both sides of the 32-channel line
 @pytest.mark.parametrize('c,shape', [(8, (1, 1, 1, 1)), (8, (2, 3, 5, 7)), (8, (1, 2, 1, 65)), (8, (1, 9, 8, 64)), (16, (1, 1, 6, 31)),
