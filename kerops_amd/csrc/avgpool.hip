@@ -390,6 +390,10 @@ constexpr PoolDefault kDefPoolFwd[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 
 constexpr PoolDefault kDefPoolFwdBnRelu[] = {{256 * kMiB, 512, 4, 1}, {kAnySize, 256, 4, 2}};
 constexpr PoolDefault kDefPoolBwd[] = {{32 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
                                        {512 * kMiB, 256, 4, 2}, {kAnySize, 256, 4, 1}};
+// 8 and 16 channels with redistributed results; us with (256,4,1) / (256,4,2) / (512,4,1): C = 8, 765 MiB 189 / 178 / 181,
+// 1582 MiB 391 / 399 / 382; C = 16, 763 MiB 189 / 181 / 181, 1914 MiB 476 / 497 / 470
+constexpr PoolDefault kDefPoolBwdPerm[] = {{32 * kMiB, 768, 4, 1}, {56 * kMiB, 768, 4, 2}, {112 * kMiB, 512, 4, 1},
+                                           {1024 * kMiB, 256, 4, 2}, {kAnySize, 512, 4, 1}};
 // in output order (segment: output chunks per thread and step); us with (512,4,1) / (512,4,2): C = 8, 4 MiB 3.9 / 4.2, 11 6.4 /
 // 5.7, 49 15.9 / 16.1, 67 20.1 / 20.8, 184 48.3 / 50.2; C = 16, 9 MiB 6.1 / 5.5, 17 8.0 / 6.6, 100 27.0 / 25.5, 368 91.4 / 91.2; C = 32,
 // 95 MiB 26.3 / 24.6; 256 workgroups are too few (67 MiB 27.5, 368 137), 1024 to 4096 no better
@@ -564,8 +568,11 @@ extern "C" int kerops_avgpool_ceil_stats_bwd_f16(const void* inpgrad, const floa
     int64_t nchunks = 0;
     StreamShape sh;
     const bool rows = pool_bwd_by_rows(N, H, W, D, C);
-    int rc = pool_plan("avgpool_ceil_stats_bwd", !rows ? kDefPoolBwd : C == 8 ? kDefPoolBwdRows8 : kDefPoolBwdRows, N, H, W, D, C,
-                       blocks, waves, segment, &p, &nchunks, &sh, rows ? 2 : 1);
+    // redistribute the results for whole-line stores where a voxel row is narrower than a 128-byte line
+    const bool perm = pool_bwd_permutes(D, C);
+    const PoolDefault* def = perm && C < 32 ? kDefPoolBwdPerm : kDefPoolBwd;
+    if (rows) def = C == 8 ? kDefPoolBwdRows8 : kDefPoolBwdRows;
+    int rc = pool_plan("avgpool_ceil_stats_bwd", def, N, H, W, D, C, blocks, waves, segment, &p, &nchunks, &sh, rows ? 2 : 1);
     if (rc != KEROPS_OK) return rc;
     if (!inpgrad || !meangrad || !sqmeangrad || !output || !dx || !aligned16(inpgrad) || !aligned16(output) ||
         !aligned16(dx)) {
@@ -574,8 +581,6 @@ extern "C" int kerops_avgpool_ceil_stats_bwd_f16(const void* inpgrad, const floa
     }
     const float fMo = (float)((int64_t)N * p.Ho * p.Wo * p.Do);
     const int seg = sh.segment != 1;
-    // redistribute the results for whole-line stores where a voxel row is narrower than a 128-byte line
-    const bool perm = pool_bwd_permutes(D, C);
     if (rows) {
         PoolRows q;
         q.row = (uint32_t)D * p.CG;

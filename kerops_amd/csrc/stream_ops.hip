@@ -465,7 +465,8 @@ using namespace kerops;
 //                      (256,4,1) / (512,4,4) at 12 / 24 / 64 / 160 MiB: 12.1 / 17.9 / 35.7 / 83.4 and 11.4 / 17.4 / 36.9 / 86.1
 //   its backward       2 / 24 / 64 MiB: (1536,16,1) or (512,4,4) 8.1 / 17.9 / 37.4, here 5.2 / 15.3 / 36.3
 //   statistics         2 / 64 / 100 MiB: 7.8 / 18.1 / 22.9 (what lies between these shapes is less than the noise)
-//   window quantiser   2 / 24 / 64 / 128 MiB in: (512,16,8) or (256,4,8) 6.6 / 9.3 / 21.2 / 36.7, here 3.4 / 8.8 / 19.1 / 36.7
+//   window quantiser   2 / 24 / 64 / 128 MiB in: (512,16,8) or (256,4,8) 6.6 / 9.3 / 21.2 / 36.7, here 3.4 / 8.8 / 19.1 / 33.8;
+//                      130 / 180 / 239 / 255 MiB with (256,4,8) 36.6 / 48.8 / 65.2 / 70.2, here 33.8 / 46.5 / 61.4 / 65.5
 //   its inverse        2 / 24 / 48 MiB out: (1536,16,8) 5.1 / 10.1 / 18.1, here 3.1 / 8.7 / 15.9
 //   int8 quantiser     16 / 48 / 96 MiB in: (256,4,4) or (4096,16,4) 10.2 / 26.8 / 29.0, here 7.2 / 15.6 / 27.9
 // Up to 4 % of a launch separates neighbouring lines of a table.  The shapes of the largest tensors were measured at
@@ -487,7 +488,8 @@ constexpr SizedDefault kDefStatsBwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB,
 constexpr SizedDefault kDefAddStatsBwd[] = {{112 * kMiB, {1024, 4, 4}}, {kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefBnReluFwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {1280, 16, 4}}};
 constexpr SizedDefault kDefBnReluBwd[] = {{kAnySize, {512, 4, 4}}};
-constexpr SizedDefault kDefQuantU8[] = {{56 * kMiB, {1536, 4, 4}}, {112 * kMiB, {1536, 4, 8}}, {kAnySize, {256, 4, 8}}};
+constexpr SizedDefault kDefQuantU8[] = {{56 * kMiB, {1536, 4, 4}}, {112 * kMiB, {1536, 4, 8}}, {192 * kMiB, {4096, 4, 4}},
+                                        {256 * kMiB, {4096, 16, 4}}, {kAnySize, {256, 4, 8}}};
 constexpr SizedDefault kDefDequantU8[] = {{3 * kMiB, {1024, 4, 1}}, {56 * kMiB, {2048, 4, 8}}, {kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefQuantI8[] = {{160 * kMiB, {2048, 4, 4}}, {256 * kMiB, {1536, 16, 4}}, {kAnySize, {4096, 16, 4}}};
 // (called ahead of the argument checks)

@@ -9,7 +9,8 @@
 The reference keys its launch tables by channel count (kerops/ops/conv/dwconv.py:10-17); so does this one.  An op's
 entry maps a key to a shape:
 
-    "8", "16", ...   the channel count of the tensor (measured at (1, C, 350, 350, 128))
+    "8", "16", ...   the channel count of the tensor (measured at (1, C, 350, 350, 128), "8" at twice that: below
+                     SMALL_BYTES no tensor reads them)
     "small"          tensors below SMALL_BYTES, whatever their channel count: what is best for them goes by their size
                      alone, so the table leaves them to the library's rule (zeros) as long as nobody enters a shape
     "default"        every other case (channel counts without an entry, tensors that are not 5-D)

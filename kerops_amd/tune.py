@@ -180,9 +180,9 @@ def apply_streams(result, write=False, note='', key='default'):
         stream_table.save(note=note)
 
 
-# `--streams --all`: the tensors behind each key of the stream table.  "default" (channel counts without an entry)
-# repeats the 64-channel measurement; "small" stays with the library's rule by size.
-STREAM_CLASSES = (('8', (1, 8, 350, 350, 128)), ('16', (1, 16, 350, 350, 128)), ('32', (1, 32, 350, 350, 128)),
+# `--streams --all`: the tensors behind each key of the stream table, each large enough to read that key.  "default"
+# (channel counts without an entry) repeats the 64-channel measurement; "small" stays with the library's rule by size.
+STREAM_CLASSES = (('8', (1, 8, 350, 350, 256)), ('16', (1, 16, 350, 350, 128)), ('32', (1, 32, 350, 350, 128)),
                   ('64', (1, 64, 350, 350, 128)), ('128', (1, 128, 350, 350, 128)))
 
 
@@ -193,14 +193,16 @@ def main():
     ap.add_argument('--ops', nargs='*', default=None, help='with --streams: only these ops')
     ap.add_argument('--all', action='store_true', help='with --streams: every class of the stream table')
     ap.add_argument('--key', default=None, help='with --streams: table key to file the result under (default: the '
-                                                'channel count of --shape)')
+                                                'key a tensor of --shape reads)')
     ap.add_argument('--shape', type=int, nargs=5, default=[1, 64, 350, 350, 128], metavar=('N', 'C', 'H', 'W', 'D'))
     ap.add_argument('--channels', type=int, nargs='*', default=None)
     ap.add_argument('--h-chunks', type=int, nargs='*', default=[0])
     ap.add_argument('--apply', action='store_true')
     args = ap.parse_args()
     if args.streams:
-        classes = STREAM_CLASSES if args.all else ((args.key or str(args.shape[1]), tuple(args.shape)),)
+        from .settings import stream_table
+        own_key = stream_table.table_key(args.shape[1], 2 * math.prod(args.shape))
+        classes = STREAM_CLASSES if args.all else ((args.key or own_key, tuple(args.shape)),)
         for key, shape in classes:
             res = tune_streams(shape, ops=args.ops, verbose=not args.all)
             for op, (blocks, warps, segment, ms) in res.items():
@@ -210,7 +212,6 @@ def main():
             if key == '64':
                 apply_streams(res, key='default')
         if args.write:
-            from .settings import stream_table
             stream_table.save(note='measured by kerops_amd.tune --streams on ' + torch.cuda.get_device_name(0) + ': keys '
                               + ', '.join(f'{k} at {sh}' for k, sh in classes) + '; "default" repeats 64')
         return

@@ -336,11 +336,39 @@ def test_pool_backward_rows(c, shape, knobs):
     assert torch.equal(bits(dx.cpu()), bits(oracle.avgpool_ceil_stats_bwd(grad, mg, sg, pooled, (n, c, h, w, d))))
 
 
+# either side of the sizes at which the built-in launch shapes of the pooling backward and its order change: rows of
+# 128 voxels, whose results the kernel in input order redistributes, and of 127
+@pytest.mark.parametrize('c,mib', [(c, mib) for c in (8, 16, 32) for mib in (6, 24, 64, 192)] + [(8, 512), (16, 512), (8, 1024), (16, 1024)])
+@pytest.mark.parametrize('d', [127, 128])
+def test_pool_backward_either_side_of_a_size_line(c, mib, d):
+    gen = torch.Generator(DEV).manual_seed(c + mib)
+    w = 256
+    line = (mib << 20) // (2 * c * w * d)
+    for h in (line, line + 1):
+        small = (1, -(-h // 2), w // 2, 64)
+        grad, pooled = (torch.randn(*small, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3) for _ in range(2))
+        mg, sg = (torch.randn(c, device=DEV, generator=gen) for _ in range(2))
+        args = (grad, mg, sg, pooled, (1, c, h, w, d))
+        # every element is the same whatever the shape
+        assert torch.equal(AvgPoolCeilStatsBackward(*args), AvgPoolCeilStatsBackward(*args, blocks=2000, num_warps=8, segment=1))
+        part = 2 * min(4, h // 2)  # the last rows against the oracle: whole windows, and the rest of an odd height
+        lo = h - h % 2 - part
+        ref_args = [t[:, :, lo // 2:].cpu() for t in (grad, pooled)]
+        count = grad.numel() // c
+        # (the oracle takes its mean over the part's windows)
+        scale = ref_args[0].numel() // c / count
+        ref = oracle.avgpool_ceil_stats_bwd(ref_args[0], mg.cpu() * scale, sg.cpu() * scale, ref_args[1], (1, c, h - lo, w, d))
+        got = AvgPoolCeilStatsBackward(*args)[:, :, lo:].cpu()
+        # a rounding to fp16, of up to 2^-11, of either
+        assert ((got.float() - ref.float()).norm() / ref.float().norm()).item() < 2.0 ** -10
+
+
 # one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
-@pytest.mark.parametrize('mib', [3, 14, 20, 40, 56, 112, 160])
+@pytest.mark.parametrize('mib', [3, 14, 20, 32, 40, 56, 112, 160, 192, 256, 384, 512])
 @pytest.mark.parametrize('off', [-1, 1])
-def test_stream_ops_either_side_of_a_size_line(mib, off):
+def test_stream_ops_either_side_of_a_size_line(mib, off, monkeypatch):
     c = 64
+    monkeypatch.setattr(stream_table, '_table', {})  # the library's shapes, at every size
     v = (mib << 20) // (2 * c) + off
     gen = torch.Generator(DEV).manual_seed(mib)
     x, y = (torch.randn(1, v, 1, 1, c, device=DEV, generator=gen).half().permute(0, 4, 1, 2, 3) for _ in range(2))

@@ -194,6 +194,14 @@ def test_stream_table_feeds_the_stream_ops_live():
     assert stream_table.stream_knob('NoSuchOp', 'blocks')(big) == 0
 
 
+def test_stream_classes_are_measured_where_their_key_is_read():
+    import math
+    from kerops_amd import tune
+    from kerops_amd.settings import stream_table
+    for key, shape in tune.STREAM_CLASSES:
+        assert stream_table.table_key(shape[1], 2 * math.prod(shape)) == key, (key, shape)
+
+
 def test_stream_table_round_trips_through_its_file(tmp_path):
     from kerops_amd.settings import stream_table
 
