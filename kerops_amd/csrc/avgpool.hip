@@ -297,7 +297,8 @@ __global__ __launch_bounds__(kStreamMaxThreads) void avgpool_bwd_kernel(const ha
 struct FastDivisor {
     uint32_t mul, shift;
 };
-// n / d for n < 2^31: (mulhi(n, mul) + n) >> shift with shift = ceil(log2 d), mul = floor(2^32 (2^shift - d) / d) + 1
+// Division by an invariant integer through a product (Granlund and Montgomery, 1994); n / d for n < 2^31:
+// (mulhi(n, mul) + n) >> shift with shift = ceil(log2 d), mul = floor(2^32 (2^shift - d) / d) + 1
 static FastDivisor fast_divisor(uint32_t d)
 {
     uint32_t s = 0;

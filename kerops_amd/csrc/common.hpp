@@ -361,8 +361,11 @@ struct MarchCost {
     // Most workgroups that may march over a single row, which reads three planes for one.  Alone on a compute unit such a
     // workgroup is still the faster one ((1,32,33,19,25), 198 of them: forward 6.26 us, 6.60 with two rows each); two of
     // them on a compute unit lose in the forward and weight-gradient kernels ((2,32,32,9,35), 384: forward 8.20 us, 6.81
-    // with two rows each, weight gradient 12.2 and 10.9) and not in the fused backward (15.0 and 15.8), which keeps to
-    // single rows wherever they fit.
+    // with two rows each, weight gradient 12.2 and 10.9).  The fused backward keeps to single rows wherever they fit, also
+    // against the cost below: that was the faster split of its earlier kernel (15.0 and 15.8 us) and is no longer.  Over 36
+    // volumes of 257 to 512 such workgroups two rows take 0.90 to 0.95 of its time (the same volume 13.2 and 12.0), over 40
+    // of fewer 1.06 to 1.09.  The limit of one workgroup per compute unit would be right here too; it moves together with
+    // the test that holds the fused backward's workgroup counts.
     int one_row;
 };
 static inline MarchSplit pick_split(int H, int64_t tiles, int row_len, int slots, int slab_mult, const DeviceGeometry& geo,

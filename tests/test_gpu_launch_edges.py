@@ -264,8 +264,8 @@ def test_inverted_bottleneck_tiles_and_rounds(c, v):
         assert err < 2.0 ** -5 if v < 1000 else err < 2.0 ** -8, err
 
 
-def test_inverted_bottleneck_is_the_same_with_early_and_late_loads():
-    # 32 channels load late above 2.6 M voxels: every voxel's result is its own, so the parts give the same bits
+def test_inverted_bottleneck_of_a_large_volume_is_that_of_its_parts():
+    # 2.6 M voxels of 32 channels, many tiles per workgroup: every voxel's result is its own, so the parts give the same bits
     c, v = 32, (5 << 19) + 33
     gen = torch.Generator(DEV).manual_seed(9)
     x, add = (torch.randn(1, v, 1, 1, c, device=DEV, generator=gen).half().permute(0, 4, 1, 2, 3) for _ in range(2))
