@@ -781,7 +781,7 @@ __device__ __forceinline__ void store_sum(float* ws, int64_t i, double sum, bool
 // with fp32 sums from step to step, over the lanes and in a workgroup's row, the error against 64 bits went with it.
 // Relative errors, zero-mean values, all-fp32 sums / now: dscale of ApplyBNReLUBackward of (1,64,192,192,128) 316e-9 / 32e-9,
 // dshift 69e-9 / 27e-9, mean of AddStats of (1,128,136,136,128) 43e-9 / 25e-9, of AvgPoolCeilStats of (1,64,61,63,63) 42e-9 /
-// 25e-9.  Time: 0.3 us for the exchanges in fp64, 0.4 for the pairs, up to 3 % of the largest ApplyBNReLUBackward.
+// 25e-9.  Time: 0.3 us for the exchanges in fp64, 0.4 for the pairs, 1 to 2 % of the largest ApplyBNReLUBackward.
 template <int V>
 struct ChannelTotals {
     double tot[2 * V];

@@ -155,7 +155,11 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_fwd_kernel(const hal
     for (int64_t i = wk.tail; i < nchunks; i += wk.T) st_stream<V>(y, i, act(ld_stream<V>(x, i)));
 }
 
-template <int V, int U>
+// TOGETHER: the results of a step are stored one after the other at its end, not each as it is there, with two to four chunks
+// of loads still to come.  That is what keeps sixteen wavefronts per workgroup, and with them the largest tensors, at the rate
+// of memory: 16 waves, apart / together 1.9 GiB 1101 / 1010 us, 3.7 GiB 2208 / 2005; four waves, 3.7 GiB 2169 / 2214, 957 MiB
+// 505 / 520.
+template <int V, int U, bool TOGETHER>
 __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const half_t* __restrict__ x,
                                                                        const float* __restrict__ wv,
                                                                        const float* __restrict__ bv,
@@ -177,9 +181,9 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const hal
     float acc[2][V];  // [0] = dW, [1] = dB, of a step
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[0][j] = acc[1][j] = 0.0f;
-    // (chunk i from chunk `at` on: in the loop `at` is the workgroup's and i the thread, scalar base addresses and one offset
-    // register for all accesses.  With an address per access and thread the sums had to leave the registers.)
-    auto body = [&](int64_t at, int64_t i, const hv& xv, const hv& gv) {
+    // (in the loop `at` is the workgroup's: scalar base addresses and one offset register for all accesses.  With an address per
+    // access and thread the sums had to leave the registers.)
+    auto body = [&](const hv& xv, const hv& gv) {
         hv o;
 #pragma unroll
         for (int j = 0; j < V; ++j) {
@@ -191,22 +195,30 @@ __global__ __launch_bounds__(kStreamMaxThreads) void bnrelu_bwd_kernel(const hal
             acc[0][j] = __builtin_fmaf(xf, gm, acc[0][j]);
             acc[1][j] += gm;
         }
-        st_stream<V>(dx + at * V, i, o);
+        return o;
     };
     const uint32_t t = threadIdx.x;
     for (int64_t k = 0; k < wk.nfull; ++k) {
         const int64_t at = k * wk.step + (wk.first - t);
-        hv xv[U], gv[U];
+        hv xv[U], gv[U], ov[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             xv[u] = ld_stream<V>(x + (at + u * wk.su) * V, t);
             gv[u] = ld_stream<V>(g + (at + u * wk.su) * V, t);
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) body(at + u * wk.su, t, xv[u], gv[u]);
+        for (int u = 0; u < U; ++u) {
+            ov[u] = body(xv[u], gv[u]);
+            if (!TOGETHER) st_stream<V>(dx + (at + u * wk.su) * V, t, ov[u]);
+        }
         sums.take(acc);
+        if (TOGETHER) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) st_stream<V>(dx + (at + u * wk.su) * V, t, ov[u]);
+        }
     }
-    for (int64_t i = wk.tail; i < nchunks; i += wk.T) body(0, i, ld_stream<V>(x, i), ld_stream<V>(g, i));
+    for (int64_t i = wk.tail; i < nchunks; i += wk.T) st_stream<V>(dx, i, body(ld_stream<V>(x, i), ld_stream<V>(g, i)));
     sums.take(acc);
     sums.write(CG, red, ws, pairs);
 }
@@ -458,10 +470,12 @@ using namespace kerops;
 // wavefronts win while a tensor is small: a workgroup of sixteen is placed on a compute unit only as a whole and pays
 // its slowest wavefront at either end.  GPU time per launch in a row of launches, inputs from memory, C = 16 and 64 alike:
 //   BN-ReLU            0.5 / 8 / 48 / 192 MiB: (256,16,8) or (1280,16,4) 6.1 / 7.9 / 20.4 / 67.0 us, here 2.8 / 4.9 / 18.7 / 65.3
-//   its backward       8 / 48 / 96 / 384 MiB: (768,4,1) or (1536,16,4) 14.1 / 34.5 / 78.1 / 215, here 11.2 / 31.3 / 55.4 / 203; one
-//                      shape for all sizes, at 1.9 GiB within 2 % of the best.  (256,4,1), the best before the sums were taken in
-//                      fp64, leaves a wavefront per SIMD, whose additions then hide behind nothing: 120 M elements 134, here 121
-//   add + statistics   8 / 48 / 96 / 1914 MiB: (1280,4,8) or (1280,16,8) 14.2 / 34.0 / 72.8 / 1061, here 10.5 / 30.0 / 53.6 / 1050;
+//   its backward       8 / 48 / 96 / 384 MiB: (768,4,1) or (1536,16,4) 14.1 / 34.5 / 78.1 / 215, here 11.2 / 31.3 / 55.4 / 203;
+//                      1100 / 1300 / 1500 / 1914 / 3828 MiB: (512,4,4) 587 / 700 / 824 / 1070 / 2162-2266, (1536,16,4) 589 / 698 / 806 /
+//                      1032 / 1966-2021.  (256,4,1), the best before the sums were taken in fp64, leaves a wavefront per SIMD, whose
+//                      additions then hide behind nothing: 120 M elements 134, here 121
+//   add + statistics   8 / 48 / 96 MiB: (1280,4,8) or (1280,16,8) 14.2 / 34.0 / 72.8, here 10.5 / 30.0 / 53.6;
+//                      957 / 1300 / 1500 / 1914 / 3828 MiB: (256,4,1) 499 / 692 / 792 / 1028 / 2081, (3072,16,4) 524 / 687 / 785 / 966 / 1996;
 //                      (256,4,1) / (512,4,4) at 12 / 24 / 64 / 160 MiB: 12.1 / 17.9 / 35.7 / 83.4 and 11.4 / 17.4 / 36.9 / 86.1
 //   its backward       2 / 24 / 64 MiB: (1536,16,1) or (512,4,4) 8.1 / 17.9 / 37.4, here 5.2 / 15.3 / 36.3
 //   statistics         2 / 64 / 100 MiB: 7.8 / 18.1 / 22.9 (what lies between these shapes is less than the noise)
@@ -483,11 +497,11 @@ struct SizedDefault {
 };
 constexpr int64_t kMiB = 1ll << 20, kAnySize = INT64_MAX;
 constexpr SizedDefault kDefStats[] = {{384 * kMiB, {512, 4, 4}}, {kAnySize, {256, 4, 8}}};
-constexpr SizedDefault kDefAddStats[] = {{40 * kMiB, {512, 4, 4}}, {kAnySize, {256, 4, 1}}};
+constexpr SizedDefault kDefAddStats[] = {{40 * kMiB, {512, 4, 4}}, {1536 * kMiB, {256, 4, 1}}, {kAnySize, {3072, 16, 4}}};
 constexpr SizedDefault kDefStatsBwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {4096, 16, 4}}};
 constexpr SizedDefault kDefAddStatsBwd[] = {{112 * kMiB, {1024, 4, 4}}, {kAnySize, {512, 4, 4}}};
 constexpr SizedDefault kDefBnReluFwd[] = {{14 * kMiB, {1024, 4, 4}}, {256 * kMiB, {512, 4, 4}}, {kAnySize, {1280, 16, 4}}};
-constexpr SizedDefault kDefBnReluBwd[] = {{kAnySize, {512, 4, 4}}};
+constexpr SizedDefault kDefBnReluBwd[] = {{1280 * kMiB, {512, 4, 4}}, {kAnySize, {1536, 16, 4}}};
 constexpr SizedDefault kDefQuantU8[] = {{56 * kMiB, {1536, 4, 4}}, {112 * kMiB, {1536, 4, 8}}, {192 * kMiB, {4096, 4, 4}},
                                         {256 * kMiB, {4096, 16, 4}}, {kAnySize, {256, 4, 8}}};
 constexpr SizedDefault kDefDequantU8[] = {{3 * kMiB, {1024, 4, 1}}, {56 * kMiB, {2048, 4, 8}}, {kAnySize, {512, 4, 4}}};
@@ -743,8 +757,13 @@ extern "C" int kerops_bnrelu_bwd_f16(const void* x, const float* wv, const float
     const int seg = sh.segment != 1;
     const bool pairs = sum_pairs(blocks, sh.blocks, 2 * C, channel_bytes(M, C), workspace_bytes);
     KEROPS_DISPATCH_VU(C, sh, {
-        hipLaunchKernelGGL((bnrelu_bwd_kernel<V, U>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x, wv,
-                           bv, (const half_t*)g, (half_t*)dx, ws, M * CG, CG, seg, pairs);
+        constexpr bool kTogether = V == 8 && U == 4;  // (eight chunks of results at once do not fit the registers)
+        if (kTogether && sh.threads > 512)
+            hipLaunchKernelGGL((bnrelu_bwd_kernel<V, U, kTogether>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x,
+                               wv, bv, (const half_t*)g, (half_t*)dx, ws, M * CG, CG, seg, pairs);
+        else
+            hipLaunchKernelGGL((bnrelu_bwd_kernel<V, U, false>), dim3(sh.blocks), dim3(sh.threads), 0, s, (const half_t*)x, wv,
+                               bv, (const half_t*)g, (half_t*)dx, ws, M * CG, CG, seg, pairs);
     });
     rc = check_launch("bnrelu_bwd");
     if (rc != KEROPS_OK) return rc;

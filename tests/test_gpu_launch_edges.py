@@ -364,7 +364,7 @@ def test_pool_backward_either_side_of_a_size_line(c, mib, d):
 
 
 # one voxel to either side of the sizes at which the built-in launch shapes of the stream ops change
-@pytest.mark.parametrize('mib', [3, 14, 20, 32, 40, 56, 112, 160, 192, 256, 384, 512])
+@pytest.mark.parametrize('mib', [3, 14, 20, 32, 40, 56, 112, 160, 192, 256, 384, 512, 1280, 1536])
 @pytest.mark.parametrize('off', [-1, 1])
 def test_stream_ops_either_side_of_a_size_line(mib, off, monkeypatch):
     c = 64
@@ -442,7 +442,7 @@ def channel_sums(*terms):
 # Sums of fp16 values (mean, dshift) have no other error: the few of a step of the walk are nearly exact.  Products
 # (dscale) are rounded as a step adds them, four in a row: sqrt(1 + (1 + 2 + 3 + 4) / 4) times as much, 6.4e-8.  10 % for
 # the spread of 64 to 128 channels.
-@pytest.mark.parametrize('c,shape', [(64, (1, 86, 86, 88)), (128, (1, 136, 136, 128)), (8, (1, 123, 125, 123))])
+@pytest.mark.parametrize('c,shape', [(64, (1, 86, 86, 88)), (128, (1, 136, 136, 128)), (8, (1, 123, 125, 123)), (64, (1, 236, 236, 228))])
 def test_channel_sums_of_the_built_in_shapes_have_no_chains(c, shape):
     gen = torch.Generator(DEV).manual_seed(c)
     n, h, w, d = shape
