@@ -429,16 +429,19 @@ static int lb_blocks(int64_t V, int cin, int cout, bool affine)
 // and then some pairs are the fastest where a workgroup reads and writes in turns, as it did with a condition around every
 // store (us without / with the wait: 16 -> 16 at 4 M voxels 66.4 / 66.0, 30 M 501 / 474; 16 -> 32 at 16 M 332 / 326; 16 -> 64 at 4 M
 // 135 / 130, 16 M 538 / 514; 32 -> 16 at 16 M 454 / 449; 32 -> 32 at 4 M 129 / 125, 16 M 526 / 490; 32 -> 64 at 16 M 677 / 666;
-// 32 -> 128 at 4 M 268 / 257; 64 -> 32 at 4 M 214 / 213, 16 M 898 / 878; 64 -> 128 at 4 M 356 / 342), others are not (16 -> 32
-// at 4 M 84.8 / 87.1, 16 -> 128 at 4 M 224 / 227, 64 -> 64 at 16 M 1083 / 1089, 128 -> 64 at 8 M 911 / 954).
+// 32 -> 128 at 4 M 268 / 257; 64 -> 32 at 4 M 214 / 213, 16 M 898 / 878; 64 -> 128 at 12 M 1086 / 1033), others are not (16 -> 32
+// at 4 M 84.8 / 87.1, 16 -> 128 at 4 M 224 / 227, 64 -> 64 at 16 M 1083 / 1089, 128 -> 64 at 8 M 911 / 954).  Behind other ops a
+// launch without the wait can be the faster one where in a row of its own it is not: 64 -> 128 behind the forward op, both,
+// at 0.9 M 169 / 172, 2 M 367 / 377, 4 M 743 / 753 (alone 350 / 336), 6 M 1142 / 1140, 8 M 1567 / 1540; the other pairs gain or
+// are equal there too (32 -> 128 at 2 M 329 / 323, 32 -> 32 at 4 M 254 / 250, 16 -> 64 at 4 M 326 / 320).
 static constexpr int64_t lb_drain_from(int cin, int cout)
 {
     constexpr int64_t kVoxels = 1000;
     if (cin == 128 || (cin == 64 && cout < 128 && cout != 32) || (cin == 16 && cout == 128)) return INT64_MAX;
     if (cout == 2 * cin && cin <= 32) return 12000 * kVoxels;
-    if (cin == 32 && cout == 16) return 6000 * kVoxels;
+    if ((cin == 32 && cout == 16) || (cin == 64 && cout == 128)) return 6000 * kVoxels;
     if ((cin == 16 && cout == 16) || (cin == 64 && cout == 32)) return 3000 * kVoxels;
-    return cout == 128 ? 700 * kVoxels : 2000 * kVoxels;  // 32 -> 128, 64 -> 128; 16 -> 64, 32 -> 32
+    return cout == 128 ? 700 * kVoxels : 2000 * kVoxels;  // 32 -> 128; 16 -> 64, 32 -> 32
 }
 
 // daffine: the AFFINE kernel's [2][CIN] sums, null without scale and shift

@@ -298,7 +298,7 @@ def test_inverted_bottleneck_either_side_of_a_volume_line(c, line):
 
 # either side of the volumes at which the pointwise ops change their number of workgroups, or wait for their stores
 @pytest.mark.parametrize('cin,cout,line', [(16, 16, 6000000), (16, 32, 12000000), (16, 64, 3000000), (32, 64, 6000000), (32, 16, 700000), (64, 32, 3000000),
-                                           (64, 64, 3000000), (128, 16, 1500000), (128, 32, 700000), (32, 32, 2000000), (32, 128, 700000)])
+                                           (64, 64, 3000000), (128, 16, 1500000), (128, 32, 700000), (32, 32, 2000000), (32, 128, 700000), (64, 128, 6000000)])
 def test_pointwise_ops_either_side_of_a_volume_line(cin, cout, line):
     gen = torch.Generator(DEV).manual_seed(cin + cout)
     x, add = (torch.randn(1, line, 1, 1, c, device=DEV, generator=gen, dtype=torch.float16).permute(0, 4, 1, 2, 3) for c in (cin, cout))
